@@ -6,13 +6,14 @@
 // padded rows/columns of the weights stay zero (their gradients are zero and Adam keeps them
 // at zero), so the padded network equals the unpadded one.
 //
-// GEMM: C[M x N] = A[M x K] B[K x N], 64 x 64 tile per 256-thread workgroup, each wavefront
-// computes a 32 x 32 quarter as 2 x 2 MFMA 16x16x32 blocks; A and B are staged through LDS
-// with k contiguous, so that each lane's MFMA operand (8 consecutive k) is one 16-byte read.
+// GEMM: C[M x N] = A[M x K] B[K x N], BM x BN tile per 256-thread workgroup, each wavefront a
+// quarter of it as 16 x 16 MFMA 16x16x32 blocks; A and B are staged through LDS with k
+// contiguous, so that each lane's MFMA operand (8 consecutive k) is one 16-byte read.
 // A is either row-major [M x K] or its transpose ([K x M], for dW = dZ^T H); B is either
 // [K x N] row-major (dX = dZ W) or [N x K] row-major (forward: B = W^T).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <cstring>
@@ -25,10 +26,13 @@
 namespace mlp {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int TM = 64, TN = 64, TK = 32, THREADS = 256;
+constexpr int TK = 64, THREADS = 256;
 constexpr int LDK = TK + 8;  // LDS row stride in bf16 (pads rows apart by 16 bytes)
+constexpr int GROUP = 8;     // layers per grouped launch
 
 __device__ inline __bf16 to_bf16(float f) { return (__bf16)f; }  // round to nearest even
 __device__ inline float silu(float z) { return z / (1.0f + __expf(-z)); }
@@ -38,271 +42,333 @@ __device__ inline float dsilu(float z) {
 }
 
 enum Epi {
-  EPI_BIAS_SILU = 0,  // Z = acc + b (fp32 out0), H = bf16(silu(Z)) (out1)
-  EPI_BIAS = 1,       // Y = acc + b (fp32 out0)
-  EPI_DSILU = 2,      // dZ = bf16(acc * silu'(Z)), Z read from aux (fp32)
-  EPI_F32 = 3,        // plain fp32 store (weight gradients)
+  EPI_BIAS_SILU = 0,  // Z = acc + b (fp32 out0, unless null), H = bf16(silu(Z)) (out1)
+  EPI_OUT = 1,        // y = omean + oscale (acc + b), the real rows and columns only (out0)
+  EPI_DSILU = 2,      // dZ = bf16(acc * silu'(Z)), Z read from aux (fp32) (out1)
+  EPI_F32 = 3,        // plain fp32 store (weight gradients) (out0)
+  EPI_LOSS = 4,       // Y = acc + b, dY = bf16(2 (Y - t') w / (batch dout)) (out1), loss partials
+};
+
+// One product and what its epilogue reads and writes (ldc: row pitch of out0 / out1 / aux).
+struct GemmArgs {
+  int K, lda, ldb, ldc;
+  const __bf16* A;
+  const __bf16* B;
+  const float* bias;
+  const float* aux;      // EPI_DSILU: Z; EPI_LOSS: the targets t [batch][dout]
+  float* out0;
+  __bf16* out1;
+  const float* omean;    // EPI_OUT, EPI_LOSS
+  const float* oscale;
+  const float* wt;       // EPI_LOSS: per-output weights or null
+  float* part;           // EPI_LOSS: one partial sum per workgroup
+  int batch, dout;       // EPI_OUT, EPI_LOSS: the unpadded extents
+};
+
+// One TK-deep slice of an operand tile of R rows (rows = m of A, n of B) from memory into
+// registers, then into LDS as [row][k].  T = false: memory is [row][k], 16 bytes (8 k) per load.
+// T = true: memory is [k][row]; a thread loads a pair of rows for 8 consecutive k (8 loads of
+// 4 bytes) and transposes the 8 x 2 block in registers, so that LDS gets 16-byte stores
+// either way.
+template <int R, bool T>
+struct Slice {
+  static constexpr int NV = T ? (R * TK / 16 + THREADS - 1) / THREADS
+                              : (R * TK / 8 + THREADS - 1) / THREADS;
+  static constexpr int ITEMS = T ? R * TK / 16 : R * TK / 8;
+  bf16x8 v[NV][T ? 2 : 1];
+  __device__ __forceinline__ void load(const __bf16* __restrict__ g, int ld, int r0, int k0) {
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {
+      const int t = threadIdx.x + u * THREADS;
+      if (ITEMS % THREADS && t >= ITEMS) continue;
+      if (!T) {
+        const int r = t / (TK / 8), kc = (t % (TK / 8)) * 8;
+        v[u][0] = *reinterpret_cast<const bf16x8*>(&g[(size_t)(r0 + r) * ld + k0 + kc]);
+      } else {
+        const int kc = (t / (R / 2)) * 8, r = (t % (R / 2)) * 2;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const bf16x2 w = *reinterpret_cast<const bf16x2*>(&g[(size_t)(k0 + kc + e) * ld + r0 + r]);
+          v[u][0][e] = w[0];
+          v[u][T ? 1 : 0][e] = w[1];
+        }
+      }
+    }
+  }
+  __device__ __forceinline__ void store(__bf16* s) const {
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {
+      const int t = threadIdx.x + u * THREADS;
+      if (ITEMS % THREADS && t >= ITEMS) continue;
+      if (!T) {
+        const int r = t / (TK / 8), kc = (t % (TK / 8)) * 8;
+        *reinterpret_cast<bf16x8*>(&s[r * LDK + kc]) = v[u][0];
+      } else {
+        const int kc = (t / (R / 2)) * 8, r = (t % (R / 2)) * 2;
+        *reinterpret_cast<bf16x8*>(&s[r * LDK + kc]) = v[u][0];
+        *reinterpret_cast<bf16x8*>(&s[(r + 1) * LDK + kc]) = v[u][T ? 1 : 0];
+      }
+    }
+  }
 };
 
 // A: if !TA, A[m][k] = Ag[m * lda + k]; if TA, A[m][k] = Ag[k * lda + m]
 // B: if TB,  B[k][n] = Bg[n * ldb + k]; if !TB, B[k][n] = Bg[k * ldb + n]
-// Tile BM x BN (64 x 64, or 32 x 32 when the 64-tile grid would leave compute units idle):
-// four wavefronts in a 2 x 2 arrangement, each owning (BM/2) x (BN/2) as 16 x 16 MFMA blocks.
-// Each output element sums its K-slices in the same order whatever the tile, so both tiles
-// give the same bits.
+// Tile (m0, n0) of BM x BN: four wavefronts in a 2 x 2 arrangement, each owning (BM/2) x (BN/2)
+// as 16 x 16 MFMA blocks.  The matrices are small enough to sit in the caches, so a tile is bound
+// by the round trips of its K-slices, not by the matrix cores: TK = 64, two LDS buffers with one
+// barrier per slice, and PF slices of loads in flight in registers ahead of the one in LDS.  A
+// 512-deep layer of 64 rows takes 4.6 us like this (6.1 us with one slice ahead, 8.4-11 us with
+// 32-deep slices and none ahead, as k_gemm had before).  The transposed operands hold 4-byte
+// pairs, so one slice ahead is all that pays (weight gradients 12.9 us, 18.5 with three).  Each
+// output element sums its 32-deep K-steps in the same order whatever the tile, so every tile
+// gives the same bits.
 template <int BM, int BN, bool TA, bool TB, int EPI>
-__global__ void __launch_bounds__(THREADS)
-    k_gemm(int M, int N, int K, const __bf16* __restrict__ Ag, int lda,
-           const __bf16* __restrict__ Bg, int ldb, const float* __restrict__ bias,
-           const float* __restrict__ aux, float* __restrict__ out0, void* __restrict__ out1,
-           int ldc) {
+__device__ __forceinline__ void gemm_tile(const GemmArgs& q, int m0, int n0) {
   constexpr int FM = BM / 32, FN = BN / 32;  // MFMA blocks per wavefront
-  __shared__ __attribute__((aligned(16))) __bf16 As[BM * LDK];
-  __shared__ __attribute__((aligned(16))) __bf16 Bs[BN * LDK];
+  __shared__ __attribute__((aligned(16))) __bf16 smem[2 * (BM + BN) * LDK];
+  // buffer c: A rows, then B rows
+  auto As = [&](int c) { return smem + c * (BM + BN) * LDK; };
+  auto Bs = [&](int c) { return smem + c * (BM + BN) * LDK + BM * LDK; };
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
   const int wm = (wv >> 1) * (BM / 2), wn = (wv & 1) * (BN / 2);
   f32x4 acc[FM][FN];
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int k0 = 0; k0 < K; k0 += TK) {
-    // stage A (BM x 32) and B (32 x BN as [n][k]): 8 bf16 per thread, BM * 4 (BN * 4) threads
-    if (tid < BM * 4) {
-      if (!TA) {
-        const int r = tid >> 2, kc = (tid & 3) * 8;
-        *reinterpret_cast<bf16x8*>(&As[r * LDK + kc]) =
-            *reinterpret_cast<const bf16x8*>(&Ag[(size_t)(m0 + r) * lda + k0 + kc]);
-      } else {
-        const int kk = tid / (BM / 8), mc = (tid % (BM / 8)) * 8;
-        const bf16x8 v = *reinterpret_cast<const bf16x8*>(&Ag[(size_t)(k0 + kk) * lda + m0 + mc]);
+  // PF slices in flight in registers ahead of the one in LDS
+  constexpr int PF = TA || !TB ? (BM >= 64 ? 1 : 2) : (BM >= 64 ? 3 : 4);
+  Slice<BM, TA> sa[PF];
+  Slice<BN, !TB> sb[PF];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) As[(mc + e) * LDK + kk] = v[e];
-      }
+  for (int p = 0; p < PF; ++p)
+    if (p * TK < q.K) {
+      sa[p].load(q.A, q.lda, m0, p * TK);
+      sb[p].load(q.B, q.ldb, n0, p * TK);
     }
-    if (tid < BN * 4) {
-      if (TB) {
-        const int r = tid >> 2, kc = (tid & 3) * 8;
-        *reinterpret_cast<bf16x8*>(&Bs[r * LDK + kc]) =
-            *reinterpret_cast<const bf16x8*>(&Bg[(size_t)(n0 + r) * ldb + k0 + kc]);
-      } else {
-        const int kk = tid / (BN / 8), nc = (tid % (BN / 8)) * 8;
-        const bf16x8 v = *reinterpret_cast<const bf16x8*>(&Bg[(size_t)(k0 + kk) * ldb + n0 + nc]);
+  int cur = 0;
+  for (int kb = 0; kb < q.K; kb += PF * TK) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) Bs[(nc + e) * LDK + kk] = v[e];
+    for (int p = 0; p < PF; ++p) {
+      const int k0 = kb + p * TK;
+      if (k0 >= q.K) break;
+      // buffer `cur` was last read two slices ago, before the previous slice's barrier
+      sa[p].store(As(cur));
+      sb[p].store(Bs(cur));
+      __syncthreads();
+      if (k0 + PF * TK < q.K) {
+        sa[p].load(q.A, q.lda, m0, k0 + PF * TK);
+        sb[p].load(q.B, q.ldb, n0, k0 + PF * TK);
       }
+#pragma unroll
+      for (int kk = 0; kk < TK; kk += 32) {
+        // operands: lane holds row (lane % 16), k = 8 (lane / 16) .. +7
+        bf16x8 a[FM], b[FN];
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+          a[i] = *reinterpret_cast<const bf16x8*>(
+              &As(cur)[(wm + i * 16 + (lane & 15)) * LDK + kk + 8 * (lane >> 4)]);
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+          b[j] = *reinterpret_cast<const bf16x8*>(
+              &Bs(cur)[(wn + j * 16 + (lane & 15)) * LDK + kk + 8 * (lane >> 4)]);
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+      }
+      cur ^= 1;
     }
-    __syncthreads();
-    // operands: lane holds row (lane % 16), k = 8 (lane / 16) .. +7
-    bf16x8 a[FM], b[FN];
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-      a[i] = *reinterpret_cast<const bf16x8*>(&As[(wm + i * 16 + (lane & 15)) * LDK + 8 * (lane >> 4)]);
-#pragma unroll
-    for (int j = 0; j < FN; ++j)
-      b[j] = *reinterpret_cast<const bf16x8*>(&Bs[(wn + j * 16 + (lane & 15)) * LDK + 8 * (lane >> 4)]);
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-      for (int j = 0; j < FN; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-    __syncthreads();
   }
   // result: lane holds rows 4 (lane / 16) + r, column lane % 16 of each 16 x 16 block
+  float loss = 0.0f;
+  // the output goes through LDS: the rows of y have no alignment, so whole row segments of the
+  // tile are written by consecutive lanes instead of 16 columns of four rows per store
+  float* tile = reinterpret_cast<float*>(smem);
+  static_assert(BM * (BN + 1) * sizeof(float) <= sizeof(smem), "output tile in the operand buffers");
+  if (EPI == EPI_OUT) __syncthreads();
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
-    for (int j = 0; j < FN; ++j)
+    for (int j = 0; j < FN; ++j) {
+      const int col = n0 + wn + j * 16 + (lane & 15);
+      const float bias = EPI == EPI_BIAS_SILU || EPI == EPI_OUT || EPI == EPI_LOSS ? q.bias[col] : 0.0f;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int row = m0 + wm + i * 16 + 4 * (lane >> 4) + r;
-        const int col = n0 + wn + j * 16 + (lane & 15);
-        const size_t o = (size_t)row * ldc + col;
+        const size_t o = (size_t)row * q.ldc + col;
         const float v = acc[i][j][r];
         if (EPI == EPI_BIAS_SILU) {
-          const float zz = v + bias[col];
-          out0[o] = zz;
-          reinterpret_cast<__bf16*>(out1)[o] = to_bf16(silu(zz));
-        } else if (EPI == EPI_BIAS) {
-          out0[o] = v + bias[col];
+          const float zz = v + bias;
+          if (q.out0) q.out0[o] = zz;
+          q.out1[o] = to_bf16(silu(zz));
+        } else if (EPI == EPI_OUT) {
+          tile[(row - m0) * (BN + 1) + col - n0] = v + bias;
         } else if (EPI == EPI_DSILU) {
-          reinterpret_cast<__bf16*>(out1)[o] = to_bf16(v * dsilu(aux[o]));
+          q.out1[o] = to_bf16(v * dsilu(q.aux[o]));
+        } else if (EPI == EPI_LOSS) {
+          // loss = mean((Y - t')^2 w) over batch x dout with t' = (t - omean) / oscale
+          float g = 0.0f;
+          if (row < q.batch && col < q.dout) {
+            const float w = q.wt ? q.wt[col] : 1.0f;
+            const float d =
+                (v + bias) - (q.aux[(size_t)row * q.dout + col] - q.omean[col]) / q.oscale[col];
+            const float inv = 1.0f / ((float)q.batch * (float)q.dout);
+            loss += d * d * w * inv;
+            g = 2.0f * d * w * inv;
+          }
+          q.out1[o] = to_bf16(g);
         } else {
-          out0[o] = v;
+          q.out0[o] = v;
         }
       }
+    }
+  if (EPI == EPI_OUT) {
+    __syncthreads();
+    const int c = tid % BN, col = n0 + c;
+    if (col < q.dout) {
+      const float om = q.omean[col], os = q.oscale[col];
+#pragma unroll 4
+      for (int r = tid / BN; r < BM && m0 + r < q.batch; r += THREADS / BN)
+        q.out0[(size_t)(m0 + r) * q.dout + col] = om + os * tile[r * (BN + 1) + c];
+    }
+  }
+  if (EPI == EPI_LOSS) {
+    __shared__ float red[THREADS / 64];
+#pragma unroll
+    for (int s = 32; s > 0; s >>= 1) loss += __shfl_down(loss, s);
+    if (lane == 0) red[wv] = loss;
+    __syncthreads();
+    if (tid == 0) q.part[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
+  }
 }
 
-// Forward GEMM of the larger batches: C[M x N] = A[M x K] W^T (A row-major, W [N x K]
-// row-major), 128 x 128 tile per 256-thread workgroup, each wavefront a 64 x 64 quarter as
-// 4 x 4 MFMA 16x16x32 blocks.  Two LDS buffers: while the MFMAs consume K-slice s, the
-// slice s + 1 is already in flight from HBM into registers and is stored to the other
-// buffer afterwards, so one barrier per slice separates the two.  Each output element adds
-// its K-slices in the same order as k_gemm, so both kernels give the same bits.
-template <int EPI>
+template <int BM, int BN, bool TA, bool TB, int EPI>
+__global__ void __launch_bounds__(THREADS) k_gemm(GemmArgs q, int tiles_n) {
+  // workgroup b runs on XCD b % 8 (round-robin dispatch): with a multiple of 8 tiles, each XCD
+  // takes a contiguous eighth of them, tiles_n tiles per row block, so that its L2 reads an
+  // eighth of A instead of all of it
+  const unsigned nb = gridDim.x, b = blockIdx.x;
+  const int t = (nb & 7u) ? (int)b : (int)((b & 7u) * (nb >> 3) + (b >> 3));
+  gemm_tile<BM, BN, TA, TB, EPI>(q, t / tiles_n * BM, t % tiles_n * BN);
+}
+
+// x[batch][din] fp32 -> X[Mp][Dp] bf16 with (x - mean) * scale, zero padding.  One column of
+// IN_ROWS rows per thread, neighbouring threads on neighbouring columns (the rows of x have no
+// 16-byte alignment), every load of a thread in flight together.
+constexpr int IN_ROWS = 8;
 __global__ void __launch_bounds__(THREADS)
-    k_gemm_fwd(int M, int N, int K, const __bf16* __restrict__ Ag, int lda,
-               const __bf16* __restrict__ Bg, int ldb, const float* __restrict__ bias,
-               float* __restrict__ out0, __bf16* __restrict__ out1, int ldc) {
-  constexpr int BM = 128, BN = 128, F = 4;
-  __shared__ __attribute__((aligned(16))) __bf16 As[2][BM * LDK];
-  __shared__ __attribute__((aligned(16))) __bf16 Bs[2][BN * LDK];
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-  const int wm = (wv >> 1) * 64, wn = (wv & 1) * 64;
-  // staging: thread t moves rows t >> 2 and 64 + (t >> 2), 8 k-values at (t & 3) * 8
-  const int sr = tid >> 2, sk = (tid & 3) * 8;
-  const __bf16* ga0 = Ag + (size_t)(m0 + sr) * lda + sk;
-  const __bf16* ga1 = Ag + (size_t)(m0 + 64 + sr) * lda + sk;
-  const __bf16* gb0 = Bg + (size_t)(n0 + sr) * ldb + sk;
-  const __bf16* gb1 = Bg + (size_t)(n0 + 64 + sr) * ldb + sk;
-  bf16x8 ra0 = *reinterpret_cast<const bf16x8*>(ga0), ra1 = *reinterpret_cast<const bf16x8*>(ga1);
-  bf16x8 rb0 = *reinterpret_cast<const bf16x8*>(gb0), rb1 = *reinterpret_cast<const bf16x8*>(gb1);
-  f32x4 acc[F][F];
+    k_input(int batch, int din, int Mp, int Dp, const float* __restrict__ x,
+            const float* __restrict__ mean, const float* __restrict__ scale,
+            __bf16* __restrict__ X) {
+  const int c = blockIdx.x * THREADS + threadIdx.x, r0 = blockIdx.y * IN_ROWS;
+  if (c >= Dp) return;
+  float v[IN_ROWS];
 #pragma unroll
-  for (int i = 0; i < F; ++i)
+  for (int e = 0; e < IN_ROWS; ++e)
+    v[e] = r0 + e < batch && c < din ? x[(size_t)(r0 + e) * din + c] : 0.0f;
+  const float mu = c < din ? mean[c] : 0.0f, sc = c < din ? scale[c] : 0.0f;
 #pragma unroll
-    for (int j = 0; j < F; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  *reinterpret_cast<bf16x8*>(&As[0][sr * LDK + sk]) = ra0;
-  *reinterpret_cast<bf16x8*>(&As[0][(64 + sr) * LDK + sk]) = ra1;
-  *reinterpret_cast<bf16x8*>(&Bs[0][sr * LDK + sk]) = rb0;
-  *reinterpret_cast<bf16x8*>(&Bs[0][(64 + sr) * LDK + sk]) = rb1;
-  __syncthreads();
-  int cur = 0;
-  for (int k0 = 0; k0 < K; k0 += TK) {
-    const bool more = k0 + TK < K;
-    if (more) {
-      ra0 = *reinterpret_cast<const bf16x8*>(ga0 + k0 + TK);
-      ra1 = *reinterpret_cast<const bf16x8*>(ga1 + k0 + TK);
-      rb0 = *reinterpret_cast<const bf16x8*>(gb0 + k0 + TK);
-      rb1 = *reinterpret_cast<const bf16x8*>(gb1 + k0 + TK);
-    }
-    bf16x8 a[F], b[F];
+  for (int e = 0; e < IN_ROWS; ++e)
+    X[(size_t)(r0 + e) * Dp + c] = to_bf16(r0 + e < batch && c < din ? (v[e] - mu) * sc : 0.0f);
+}
+
+// The weight and bias gradients of up to GROUP layers in one launch: they are independent of
+// each other once the backward chain has left every dZ_i.
+//   db_i[c] = sum over rows of dZ_i[r][c]: a workgroup takes CS_COLS columns; its threads bring
+// CS_ROWS rows at a time into LDS with every load in flight, and CS_COLS of them add a column
+// each in row order.  (One thread per column reading its rows from memory one after the other
+// took 53 us per layer at 512 rows.)
+//   dW_i = dZ_i^T H_{i-1} ([out x in], K = batch rows): one BM x BN tile per workgroup.
+// cfirst[i] / first[i]: layer i's first column / tile workgroup; the column sums come first.
+constexpr int CS_COLS = 32, CS_ROWS = 256;
+struct GroupArgs {
+  int n, first[GROUP + 1], tiles_n[GROUP], cfirst[GROUP + 1];
+  GemmArgs g[GROUP];
+  float* db[GROUP];
+};
+
+__device__ __forceinline__ void colsum(const __bf16* __restrict__ dZ, int rows, int ld, int c0,
+                                       float* __restrict__ db) {
+  __shared__ __attribute__((aligned(16))) __bf16 s[CS_ROWS][CS_COLS];
+  const int tid = threadIdx.x;
+  float sum = 0.0f;
+  for (int r0 = 0; r0 < rows; r0 += CS_ROWS) {
+    const int nr = min(CS_ROWS, rows - r0);  // rows are padded to a multiple of 128
 #pragma unroll
-    for (int i = 0; i < F; ++i)
-      a[i] = *reinterpret_cast<const bf16x8*>(&As[cur][(wm + i * 16 + (lane & 15)) * LDK + 8 * (lane >> 4)]);
-#pragma unroll
-    for (int j = 0; j < F; ++j)
-      b[j] = *reinterpret_cast<const bf16x8*>(&Bs[cur][(wn + j * 16 + (lane & 15)) * LDK + 8 * (lane >> 4)]);
-#pragma unroll
-    for (int i = 0; i < F; ++i)
-#pragma unroll
-      for (int j = 0; j < F; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-    if (more) {
-      const int nx = cur ^ 1;
-      *reinterpret_cast<bf16x8*>(&As[nx][sr * LDK + sk]) = ra0;
-      *reinterpret_cast<bf16x8*>(&As[nx][(64 + sr) * LDK + sk]) = ra1;
-      *reinterpret_cast<bf16x8*>(&Bs[nx][sr * LDK + sk]) = rb0;
-      *reinterpret_cast<bf16x8*>(&Bs[nx][(64 + sr) * LDK + sk]) = rb1;
+    for (int u = 0; u < CS_ROWS * CS_COLS / 8 / THREADS; ++u) {
+      const int t = tid + u * THREADS, r = t / (CS_COLS / 8), c = (t % (CS_COLS / 8)) * 8;
+      if (r < nr)
+        *reinterpret_cast<bf16x8*>(&s[r][c]) =
+            *reinterpret_cast<const bf16x8*>(&dZ[(size_t)(r0 + r) * ld + c0 + c]);
     }
     __syncthreads();
-    cur ^= 1;
-  }
-#pragma unroll
-  for (int i = 0; i < F; ++i)
-#pragma unroll
-    for (int j = 0; j < F; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = m0 + wm + i * 16 + 4 * (lane >> 4) + r;
-        const int col = n0 + wn + j * 16 + (lane & 15);
-        const size_t o = (size_t)row * ldc + col;
-        const float v = acc[i][j][r];
-        if (EPI == EPI_BIAS_SILU) {
-          const float zz = v + bias[col];
-          out0[o] = zz;
-          out1[o] = to_bf16(silu(zz));
-        } else {
-          out0[o] = v + bias[col];
-        }
-      }
-  (void)M, (void)N;
-}
-
-// x[batch][din] fp32 -> X[Mp][Dp] bf16 with (x - mean) * scale, zero padding
-__global__ void k_input(int batch, int din, int Mp, int Dp, const float* __restrict__ x,
-                        const float* __restrict__ mean, const float* __restrict__ scale,
-                        __bf16* __restrict__ X) {
-  const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= (long long)Mp * Dp) return;
-  const int r = (int)(q / Dp), c = (int)(q % Dp);
-  float v = 0.0f;
-  if (r < batch && c < din) v = (x[(size_t)r * din + c] - mean[c]) * scale[c];
-  X[q] = to_bf16(v);
-}
-
-// y[batch][dout] = omean + oscale * Y (fp32), per output
-__global__ void k_output(int batch, int dout, int ldy, const float* __restrict__ omean,
-                         const float* __restrict__ oscale, const float* __restrict__ Y,
-                         float* __restrict__ y) {
-  const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= (long long)batch * dout) return;
-  const int r = (int)(q / dout), c = (int)(q % dout);
-  y[q] = omean[c] + oscale[c] * Y[(size_t)r * ldy + c];
-}
-
-// loss = mean((Y - t')^2 w) over batch x dout with t' = (t - omean) / oscale;
-// dY = bf16(2 (Y - t') w / (batch dout))
-__global__ void k_loss(int batch, int dout, int Mp, int ldy, const float* __restrict__ omean,
-                       const float* __restrict__ oscale, const float* __restrict__ Y,
-                       const float* __restrict__ t,
-                       const float* __restrict__ wt, __bf16* __restrict__ dY,
-                       float* __restrict__ loss) {
-  __shared__ float red[256];
-  const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  float l = 0.0f;
-  if (q < (long long)Mp * ldy) {
-    const int r = (int)(q / ldy), c = (int)(q % ldy);
-    float g = 0.0f;
-    if (r < batch && c < dout) {
-      const float w = wt ? wt[c] : 1.0f;
-      const float d = Y[q] - (t[(size_t)r * dout + c] - omean[c]) / oscale[c];
-      const float inv = 1.0f / ((float)batch * (float)dout);
-      l = d * d * w * inv;
-      g = 2.0f * d * w * inv;
+    if (tid < CS_COLS) {
+#pragma unroll 32
+      for (int r = 0; r < nr; ++r) sum += (float)s[r][tid];
     }
-    dY[q] = to_bf16(g);
-  }
-  red[threadIdx.x] = l;
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
     __syncthreads();
   }
-  if (threadIdx.x == 0) atomicAdd(loss, red[0]);
+  if (tid < CS_COLS) db[c0 + tid] = sum;
 }
 
-// db[c] = sum over rows of dZ[r][c] (bf16 in, fp32 out), one thread per column
-__global__ void k_colsum(int rows, int cols, int ld, const __bf16* __restrict__ dZ,
-                         float* __restrict__ db) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= cols) return;
-  float s = 0.0f;
-  for (int r = 0; r < rows; ++r) s += (float)dZ[(size_t)r * ld + c];
-  db[c] = s;
+template <int BM, int BN>
+__global__ void __launch_bounds__(THREADS) k_grads(GroupArgs a) {
+  const int ncol = a.cfirst[a.n];
+  int i = 0;
+  if ((int)blockIdx.x < ncol) {
+    while ((int)blockIdx.x >= a.cfirst[i + 1]) ++i;
+    colsum(a.g[i].A, a.g[i].K, a.g[i].lda, (blockIdx.x - a.cfirst[i]) * CS_COLS, a.db[i]);
+    return;
+  }
+  const int b = blockIdx.x - ncol;
+  while (b >= a.first[i + 1]) ++i;
+  const int t = b - a.first[i];
+  const GemmArgs q = a.g[i];
+  gemm_tile<BM, BN, true, false, EPI_F32>(q, t / a.tiles_n[i] * BM, t % a.tiles_n[i] * BN);
 }
 
 // Adam on fp32 masters; refreshes the bf16 copy.  Padded entries have zero gradient and stay 0.
-__global__ void k_adam(long long n, float lr, float b1, float b2, float eps, float c1, float c2,
-                       float* __restrict__ w, const float* __restrict__ g, float* __restrict__ m,
-                       float* __restrict__ v, __bf16* __restrict__ wb) {
-  const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= n) return;
-  const float gg = g[q];
-  const float mm = b1 * m[q] + (1.0f - b1) * gg;
-  const float vv = b2 * v[q] + (1.0f - b2) * gg * gg;
-  m[q] = mm, v[q] = vv;
-  const float ww = w[q] - lr * (mm / c1) / (sqrtf(vv / c2) + eps);
-  w[q] = ww;
-  if (wb) wb[q] = to_bf16(ww);
-}
+// Up to 2 GROUP arrays (weights and biases) in one launch, four values per thread; first[i]:
+// array i's first workgroup.
+struct AdamArgs {
+  int n, first[2 * GROUP + 1];
+  long long len[2 * GROUP];
+  float lr, b1, b2, eps, c1, c2;
+  float* w[2 * GROUP];
+  const float* g[2 * GROUP];
+  float* m[2 * GROUP];
+  float* v[2 * GROUP];
+  __bf16* wb[2 * GROUP];
+};
 
-// zero-fill by a kernel (graph-capture safe, unlike a memset node)
-__global__ void k_zero(float* __restrict__ a, int n) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q < n) a[q] = 0.0f;
+__global__ void __launch_bounds__(THREADS) k_adam(AdamArgs a) {
+  int i = 0;
+  while (i + 1 < a.n && (int)blockIdx.x >= a.first[i + 1]) ++i;
+  const long long q = 4 * ((long long)(blockIdx.x - a.first[i]) * THREADS + threadIdx.x);
+  if (q >= a.len[i]) return;  // lengths are multiples of 64
+  f32x4 w = *reinterpret_cast<f32x4*>(a.w[i] + q), m = *reinterpret_cast<f32x4*>(a.m[i] + q),
+        v = *reinterpret_cast<f32x4*>(a.v[i] + q);
+  const f32x4 g = *reinterpret_cast<const f32x4*>(a.g[i] + q);
+  bf16x4 wb;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float gg = g[e];
+    // the fused products are written out: which of the two the compiler fuses is left to it
+    // otherwise, and Adam's division by |g| carries that rounding on through the steps
+    const float mm = __builtin_fmaf(1.0f - a.b1, gg, a.b1 * m[e]);
+    const float vv = __builtin_fmaf(gg, (1.0f - a.b2) * gg, a.b2 * v[e]);
+    m[e] = mm, v[e] = vv;
+    const float ww = w[e] - a.lr * (mm / a.c1) / (sqrtf(vv / a.c2) + a.eps);
+    w[e] = ww;
+    wb[e] = to_bf16(ww);
+  }
+  *reinterpret_cast<f32x4*>(a.m[i] + q) = m;
+  *reinterpret_cast<f32x4*>(a.v[i] + q) = v;
+  *reinterpret_cast<f32x4*>(a.w[i] + q) = w;
+  if (a.wb[i]) *reinterpret_cast<bf16x4*>(a.wb[i] + q) = wb;
 }
 
 __global__ void k_to_bf16(long long n, const float* __restrict__ a, __bf16* __restrict__ b) {
@@ -333,11 +399,10 @@ struct memb_mlp {
   __bf16* X = nullptr;             // [Mp][Dp]
   std::vector<float*> Z;           // hidden pre-activations [Mp][Wp]
   std::vector<__bf16*> H;          // hidden activations [Mp][Wp]
-  float* Y = nullptr;              // [Mp][Op]
-  __bf16* dY = nullptr;            // [Mp][Op]
-  __bf16* dZa = nullptr;           // [Mp][Wp] (two buffers, ping-pong)
-  __bf16* dZb = nullptr;
-  float* loss = nullptr;
+  std::vector<__bf16*> dZ;         // per layer, gradient of the pre-activation [Mp][out_p]
+  float* hpart = nullptr;          // loss partials, one per workgroup of the last layer, in
+  float* part = nullptr;           // pinned host memory; its device address
+  size_t npart = 0;
   float *mean = nullptr, *scale = nullptr;    // input normalisation [Dp]
   float *omean = nullptr, *oscale = nullptr;  // output de-normalisation [Op]
   long long step = 0;
@@ -366,85 +431,97 @@ int dalloc(memb_mlp* m, T** p, size_t n) {
   return MEMB_OK;
 }
 
+// 64 x 64 tiles where there is at least one per compute unit, 32 x 32 below (training batches,
+// small inference batches): a forward pass of 2048 rows takes 48 us with 64 x 64 hidden layers (256
+// tiles) and 54 us with 32 x 32; 4096 rows 67 and 78 us; a training step of 512 rows, whose
+// hidden layers have 64 tiles of 64 x 64, 142 us with 32 x 32.  128 x 128 tiles were slower
+// everywhere (8192 rows: 150 against 121 us).
 template <bool TA, bool TB, int EPI>
-int gemm(memb_mlp* m, int M, int N, int K, const __bf16* A, int lda, const __bf16* B, int ldb,
-         const float* bias, const float* aux, float* out0, void* out1, int ldc) {
-  if (M % 64 || N % 64 || K % 32) return mfail(m, MEMB_E_ARG, "gemm shape not padded");
-  if constexpr (!TA && TB && (EPI == EPI_BIAS_SILU || EPI == EPI_BIAS)) {
-    // forward layers of batches large enough to fill the chip with 128 x 128 tiles
-    if (M % 128 == 0 && N % 128 == 0 && (long long)(M / 128) * (N / 128) >= m->cus) {
-      k_gemm_fwd<EPI><<<dim3(N / 128, M / 128), THREADS, 0, m->stream>>>(
-          M, N, K, A, lda, B, ldb, bias, out0, reinterpret_cast<__bf16*>(out1), ldc);
-      XCHK(m, hipGetLastError());
-      return MEMB_OK;
-    }
-  }
-  if ((long long)(M / TM) * (N / TN) < 2LL * m->cus) {
-    // too few 64 x 64 tiles to fill the compute units (training batches): 32 x 32 tiles
-    k_gemm<32, 32, TA, TB, EPI><<<dim3(N / 32, M / 32), THREADS, 0, m->stream>>>(
-        M, N, K, A, lda, B, ldb, bias, aux, out0, out1, ldc);
-  } else {
-    k_gemm<TM, TN, TA, TB, EPI><<<dim3(N / TN, M / TM), THREADS, 0, m->stream>>>(
-        M, N, K, A, lda, B, ldb, bias, aux, out0, out1, ldc);
-  }
+int gemm(memb_mlp* m, int M, int N, const GemmArgs& q) {
+  if (M % 64 || N % 64 || q.K % TK) return mfail(m, MEMB_E_ARG, "gemm shape not padded");
+  const int b = (long long)(M / 64) * (N / 64) >= m->cus ? 64 : 32;
+  const unsigned grid = (unsigned)(M / b) * (N / b);
+  if (b == 64)
+    k_gemm<64, 64, TA, TB, EPI><<<grid, THREADS, 0, m->stream>>>(q, N / b);
+  else
+    k_gemm<32, 32, TA, TB, EPI><<<grid, THREADS, 0, m->stream>>>(q, N / b);
+  m->npart = grid;
   XCHK(m, hipGetLastError());
   return MEMB_OK;
 }
 
-int forward(memb_mlp* m, int batch, const float* x) {
+// The hidden layers; keep: store the pre-activations Z for a backward pass.
+int forward_hidden(memb_mlp* m, int batch, const float* x, bool keep) {
   const int Mp = pad128(batch);
-  k_input<<<nblk((long long)Mp * m->Dp), 256, 0, m->stream>>>(batch, m->din, Mp, m->Dp, x, m->mean,
-                                                            m->scale, m->X);
-  const __bf16* in = m->X;
-  int ldi = m->Dp;
-  for (int i = 0; i < m->nl; ++i) {
-    int rc;
-    if (i < m->nl - 1)
-      rc = gemm<false, true, EPI_BIAS_SILU>(m, Mp, m->out_p[i], m->in_p[i], in, ldi, m->Wb[i],
-                                            m->in_p[i], m->b[i], nullptr, m->Z[i], m->H[i],
-                                            m->out_p[i]);
-    else
-      rc = gemm<false, true, EPI_BIAS>(m, Mp, m->out_p[i], m->in_p[i], in, ldi, m->Wb[i],
-                                       m->in_p[i], m->b[i], nullptr, m->Y, nullptr, m->out_p[i]);
+  k_input<<<dim3(nblk(m->Dp, THREADS), Mp / IN_ROWS), THREADS, 0, m->stream>>>(
+      batch, m->din, Mp, m->Dp, x, m->mean, m->scale, m->X);
+  for (int i = 0; i < m->nl - 1; ++i) {
+    GemmArgs q{};
+    q.K = q.lda = q.ldb = m->in_p[i], q.ldc = m->out_p[i];
+    q.A = i == 0 ? m->X : m->H[i - 1], q.B = m->Wb[i], q.bias = m->b[i];
+    q.out0 = keep ? m->Z[i] : nullptr, q.out1 = m->H[i];
+    int rc = gemm<false, true, EPI_BIAS_SILU>(m, Mp, m->out_p[i], q);
     if (rc) return rc;
-    if (i < m->nl - 1) in = m->H[i], ldi = m->out_p[i];
   }
   return MEMB_OK;
 }
 
-int backward(memb_mlp* m, int batch, const float* x, const float* t, const float* wt, float* loss) {
-  int rc = forward(m, batch, x);
+// The arguments of the last layer's product, whose epilogue forms the output or the loss
+GemmArgs last_layer(const memb_mlp* m, int batch) {
+  const int i = m->nl - 1;
+  GemmArgs q{};
+  q.K = q.lda = q.ldb = m->in_p[i], q.ldc = m->out_p[i];
+  q.A = i == 0 ? m->X : m->H[i - 1], q.B = m->Wb[i], q.bias = m->b[i];
+  q.omean = m->omean, q.oscale = m->oscale, q.batch = batch, q.dout = m->dout;
+  return q;
+}
+
+// Forward, loss and every gradient, enqueued; the nloss loss partials are in hpart once the
+// stream has come this far.
+int backward(memb_mlp* m, int batch, const float* x, const float* t, const float* wt,
+             size_t& nloss) {
+  int rc = forward_hidden(m, batch, x, true);
   if (rc) return rc;
-  const int Mp = pad128(batch);
-  k_zero<<<1, 64, 0, m->stream>>>(m->loss, 1);
-  k_loss<<<nblk((long long)Mp * m->Op), 256, 0, m->stream>>>(batch, m->dout, Mp, m->Op,
-                                                            m->omean, m->oscale, m->Y, t, wt,
-                                                            m->dY, m->loss);
-  const __bf16* dcur = m->dY;  // gradient w.r.t. the current layer's pre-activation
-  int ldd = m->Op;
-  for (int i = m->nl - 1; i >= 0; --i) {
-    const __bf16* hin = i == 0 ? m->X : m->H[i - 1];
-    const int ldh = i == 0 ? m->Dp : m->out_p[i - 1];
-    // dW_i = dZ_i^T H_{i-1}: [out x in], K = Mp
-    if ((rc = gemm<true, false, EPI_F32>(m, m->out_p[i], m->in_p[i], Mp, dcur, ldd, hin, ldh,
-                                         nullptr, nullptr, m->gW[i], nullptr, m->in_p[i])))
-      return rc;
-    k_colsum<<<nblk(m->out_p[i]), 256, 0, m->stream>>>(Mp, m->out_p[i], ldd, dcur, m->gb[i]);
-    if (i > 0) {
-      // dZ_{i-1} = (dZ_i W_i) * silu'(Z_{i-1}): [Mp x in], K = out
-      __bf16* dst = (i & 1) ? m->dZa : m->dZb;
-      if ((rc = gemm<false, false, EPI_DSILU>(m, Mp, m->in_p[i], m->out_p[i], dcur, ldd, m->Wb[i],
-                                              m->in_p[i], nullptr, m->Z[i - 1], nullptr, dst,
-                                              m->in_p[i])))
-        return rc;
-      dcur = dst, ldd = m->in_p[i];
+  const int Mp = pad128(batch), last = m->nl - 1;
+  {
+    GemmArgs q = last_layer(m, batch);
+    q.aux = t, q.wt = wt, q.out1 = m->dZ[last], q.part = m->part;
+    if ((rc = gemm<false, true, EPI_LOSS>(m, Mp, m->out_p[last], q))) return rc;
+    nloss = m->npart;
+  }
+  for (int i = last; i > 0; --i) {
+    // dZ_{i-1} = (dZ_i W_i) * silu'(Z_{i-1}): [Mp x in], K = out
+    GemmArgs q{};
+    q.K = q.lda = m->out_p[i], q.ldb = q.ldc = m->in_p[i];
+    q.A = m->dZ[i], q.B = m->Wb[i], q.aux = m->Z[i - 1], q.out1 = m->dZ[i - 1];
+    if ((rc = gemm<false, false, EPI_DSILU>(m, Mp, m->in_p[i], q))) return rc;
+  }
+  for (int i0 = 0; i0 < m->nl; i0 += GROUP) {
+    const int n = std::min(GROUP, m->nl - i0);
+    GroupArgs g{};
+    g.n = n;
+    for (int k = 0; k < n; ++k) {
+      const int i = i0 + k;
+      g.tiles_n[k] = m->in_p[i] / 64;
+      g.first[k + 1] = g.first[k] + m->out_p[i] / 64 * g.tiles_n[k];
+      GemmArgs& q = g.g[k];
+      q.K = Mp, q.lda = m->out_p[i], q.ldb = q.ldc = m->in_p[i];
+      q.A = m->dZ[i], q.B = i == 0 ? m->X : m->H[i - 1], q.out0 = m->gW[i];
+      g.cfirst[k + 1] = g.cfirst[k] + m->out_p[i] / CS_COLS;
+      g.db[k] = m->gb[i];
     }
+    k_grads<64, 64><<<g.cfirst[n] + g.first[n], THREADS, 0, m->stream>>>(g);
   }
   XCHK(m, hipGetLastError());
-  if (loss) {
-    XCHK(m, hipMemcpyAsync(loss, m->loss, sizeof(float), hipMemcpyDeviceToHost, m->stream));
-    XCHK(m, hipStreamSynchronize(m->stream));
-  }
+  return MEMB_OK;
+}
+
+// Waits for the step and adds its loss partials in workgroup order.
+int read_loss(memb_mlp* m, size_t nloss, float* loss) {
+  XCHK(m, hipStreamSynchronize(m->stream));
+  float s = 0.0f;
+  for (size_t i = 0; i < nloss; ++i) s += m->hpart[i];
+  *loss = s;
   return MEMB_OK;
 }
 }  // namespace
@@ -491,10 +568,15 @@ int memb_mlp_create(memb_mlp** out, int din, int width, int nhidden, int dout, i
       return rc;
     m->Z.push_back(z), m->H.push_back(h);
   }
-  if ((rc = dalloc(m, &m->X, (size_t)m->Mp * m->Dp)) || (rc = dalloc(m, &m->Y, (size_t)m->Mp * m->Op)) ||
-      (rc = dalloc(m, &m->dY, (size_t)m->Mp * m->Op)) ||
-      (rc = dalloc(m, &m->dZa, (size_t)m->Mp * m->Wp)) ||
-      (rc = dalloc(m, &m->dZb, (size_t)m->Mp * m->Wp)) || (rc = dalloc(m, &m->loss, 1)) ||
+  for (int i = 0; i < m->nl; ++i) {
+    __bf16* d;
+    if ((rc = dalloc(m, &d, (size_t)m->Mp * m->out_p[i]))) return rc;
+    m->dZ.push_back(d);
+  }
+  const size_t parts = (size_t)(m->Mp / 32) * (m->Op / 32);  // the smallest tile's workgroups
+  XCHK(m, hipHostMalloc((void**)&m->hpart, parts * sizeof(float), hipHostMallocMapped));
+  XCHK(m, hipHostGetDevicePointer((void**)&m->part, m->hpart, 0));
+  if ((rc = dalloc(m, &m->X, (size_t)m->Mp * m->Dp)) ||
       (rc = dalloc(m, &m->mean, (size_t)m->Dp)) || (rc = dalloc(m, &m->scale, (size_t)m->Dp)) ||
       (rc = dalloc(m, &m->omean, (size_t)m->Op)) || (rc = dalloc(m, &m->oscale, (size_t)m->Op)))
     return rc;
@@ -509,6 +591,7 @@ void memb_mlp_destroy(memb_mlp* m) {
   (void)hipSetDevice(m->device);
   if (m->stream) (void)hipStreamSynchronize(m->stream);
   for (void* p : m->allocs) (void)hipFree(p);
+  if (m->hpart) (void)hipHostFree(m->hpart);
   if (m->own) (void)hipStreamDestroy(m->own);
   delete m;
 }
@@ -603,40 +686,49 @@ int memb_mlp_init(memb_mlp* m, uint64_t seed) {
 int memb_mlp_forward(memb_mlp* m, int batch, const float* x, float* y) {
   if (!m || batch <= 0 || batch > m->maxb || !x || !y) return MEMB_E_ARG;
   XCHK(m, hipSetDevice(m->device));
-  int rc = forward(m, batch, x);
+  int rc = forward_hidden(m, batch, x, false);
   if (rc) return rc;
-  k_output<<<nblk((long long)batch * m->dout), 256, 0, m->stream>>>(batch, m->dout, m->Op,
-                                                                   m->omean, m->oscale, m->Y, y);
-  XCHK(m, hipGetLastError());
-  return MEMB_OK;
+  GemmArgs q = last_layer(m, batch);
+  q.out0 = y;
+  return gemm<false, true, EPI_OUT>(m, pad128(batch), m->out_p[m->nl - 1], q);
 }
 
 int memb_mlp_grad_only(memb_mlp* m, int batch, const float* x, const float* t, const float* wt,
                        float* loss) {
   if (!m || batch <= 0 || batch > m->maxb || !x || !t) return MEMB_E_ARG;
   XCHK(m, hipSetDevice(m->device));
-  return backward(m, batch, x, t, wt, loss);
+  size_t nloss = 0;
+  int rc = backward(m, batch, x, t, wt, nloss);
+  if (rc || !loss) return rc;
+  return read_loss(m, nloss, loss);
 }
 
 int memb_mlp_train_step(memb_mlp* m, int batch, const float* x, const float* t, const float* wt,
                         float lr, float* loss) {
   if (!m || batch <= 0 || batch > m->maxb || !x || !t) return MEMB_E_ARG;
   XCHK(m, hipSetDevice(m->device));
-  int rc = backward(m, batch, x, t, wt, loss);
+  size_t nloss = 0;
+  int rc = backward(m, batch, x, t, wt, nloss);
   if (rc) return rc;
   ++m->step;
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   const float c1 = 1.0f - std::pow(b1, (float)m->step), c2 = 1.0f - std::pow(b2, (float)m->step);
-  for (int i = 0; i < m->nl; ++i) {
-    const long long nw = (long long)m->out_p[i] * m->in_p[i];
-    k_adam<<<nblk(nw), 256, 0, m->stream>>>(nw, lr, b1, b2, eps, c1, c2, m->W[i], m->gW[i],
-                                             m->mW[i], m->vW[i], m->Wb[i]);
-    k_adam<<<nblk(m->out_p[i]), 256, 0, m->stream>>>(m->out_p[i], lr, b1, b2, eps, c1, c2,
-                                                      m->b[i], m->gb[i], m->mb[i], m->vb[i],
-                                                      nullptr);
+  for (int i0 = 0; i0 < m->nl; i0 += GROUP) {
+    AdamArgs a{};
+    a.lr = lr, a.b1 = b1, a.b2 = b2, a.eps = eps, a.c1 = c1, a.c2 = c2;
+    auto add = [&](long long n, float* w, float* g, float* mo, float* vo, __bf16* wb) {
+      const int k = a.n++;
+      a.len[k] = n, a.w[k] = w, a.g[k] = g, a.m[k] = mo, a.v[k] = vo, a.wb[k] = wb;
+      a.first[k + 1] = a.first[k] + (int)nblk(n / 4, THREADS);
+    };
+    for (int i = i0; i < std::min(i0 + GROUP, m->nl); ++i) {
+      add((long long)m->out_p[i] * m->in_p[i], m->W[i], m->gW[i], m->mW[i], m->vW[i], m->Wb[i]);
+      add(m->out_p[i], m->b[i], m->gb[i], m->mb[i], m->vb[i], nullptr);
+    }
+    k_adam<<<a.first[a.n], THREADS, 0, m->stream>>>(a);
   }
   XCHK(m, hipGetLastError());
-  return MEMB_OK;
+  return loss ? read_loss(m, nloss, loss) : MEMB_OK;
 }
 
 }  // extern "C"
