@@ -8,7 +8,7 @@
  *       complagrforces      forcing.f90:11-114   (force grid = harmonic grid: TRSSPH is the
  *                                                 identity)
  *       cal_spectral_force  sph.f90:1523-1755
- *     -> memb_traction_f64_dev, one workgroup per capsule, every capsule in one launch.
+ *     -> memb_traction_f64_dev, three kernels over batches of capsules.
  *
  *  2. A learned surrogate of that law: an MLP from the capsule's real spherical-harmonic
  *     shape coefficients to the traction at its points, run and trained with hand-written
@@ -63,6 +63,15 @@ int memb_ncoef(const memb_plan* p);
 int memb_traction_f64_dev(memb_plan* p, int64_t ncap, double gs, double eb, const double* x,
                           const double* y, const double* z, double* fx, double* fy, double* fz,
                           double* nx, double* ny, double* nz, double* area);
+
+/* The same law with its node phase in the oracle's order of operations, for finite differences of
+ * the law (the surrogate's Jacobian), which see nothing but its rounding: results agree with
+ * memb_traction_f64_dev to 1e-10 of the largest component.  The first call on a plan builds
+ * tables and waits, so it cannot be captured. */
+int memb_traction_ordered_f64_dev(memb_plan* p, int64_t ncap, double gs, double eb,
+                                  const double* x, const double* y, const double* z, double* fx,
+                                  double* fy, double* fz, double* nx, double* ny, double* nz,
+                                  double* area);
 
 /* Shape coefficients of ncap capsules (device): coef[c * 3 (L+1)^2 + ...], packed as above.
  * The analysis of cal_3dcrd_spectral_coeff (sph1.f90:29-37). */

@@ -173,6 +173,7 @@ def load_memb() -> ctypes.CDLL:
         "memb_npts": (I, [P]),
         "memb_ncoef": (I, [P]),
         "memb_traction_f64_dev": (I, [P, I64, D, D] + [P] * 10),
+        "memb_traction_ordered_f64_dev": (I, [P, I64, D, D] + [P] * 10),
         "memb_coeffs_f64_dev": (I, [P, I64, P, P, P, P]),
         "memb_geometry_f64_dev": (I, [P, I64, P, P, P, P, P, P, P, P]),
         "memb_traction_select_f64_dev": (I, [P, I64, P, D, D] + [P] * 10),

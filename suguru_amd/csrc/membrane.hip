@@ -1,5 +1,5 @@
-// membrane.hip -- the reference's FP64 capsule membrane law on gfx950, one workgroup per
-// capsule (libmemb.so, C ABI in include/memb.h).
+// membrane.hip -- the reference's FP64 capsule membrane law on gfx950, three kernels over
+// batches of capsules (libmemb.so, C ABI in include/memb.h).
 //
 // Per capsule (forcing.f90:11-114 with the force grid equal to the harmonic grid):
 //   1. shape coefficients: longitude DFT per latitude, then Gauss-Legendre quadrature
@@ -15,11 +15,14 @@
 // the unit-sphere reference state) are built once per degree by memb_plan_create.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/memb.h"
@@ -27,39 +30,35 @@
 namespace memb {
 
 constexpr int NQ = 15;        // derivatives of total order <= 4
-constexpr int RING = 3;       // fine latitude rings processed together
-constexpr int THREADS = 128;     // per capsule workgroup (two wavefronts)
-constexpr int NREF = 56;      // reference-state doubles per fine node
+constexpr int NREF = 36;      // reference-state doubles per fine node
 constexpr int LMAX = 23;
+constexpr int ND_THREADS = 128;  // per workgroup of the node kernel (two wavefronts)
+constexpr int SH_THREADS = 256;  // per workgroup of the shape and filter kernels
+constexpr int AB_SLOTS = 4;   // rings whose coefficients are in LDS
+constexpr int F_SLOTS = 3;    // rings whose outputs are in LDS
 
-__host__ __device__ inline int qidx(int kt, int kp) {
-  const int s = kt + kp;
-  return s * (s + 1) / 2 + kp;
+__host__ __device__ constexpr int qidx(int kt, int kp) {
+  return (kt + kp) * (kt + kp + 1) / 2 + kp;
 }
+// Harmonics (m, n = m + d) packed with m fastest: for one d, neighbouring m are neighbours, in
+// the tables as in the coefficients, so that threads that own an m each read them coalesced
+// and without bank conflicts while they walk d.
+__host__ __device__ constexpr int tidx(int N, int d, int m) { return d * N - d * (d - 1) / 2 + m; }
 
+// Colatitudes come in pairs (theta, pi - theta): P_n^m(pi - theta) = (-1)^(n + m) P_n^m(theta),
+// and each theta-derivative adds a sign, so tables hold the northern ring of a pair only.
 struct Tables {
-  int L, N, np2, nt, np;       // N = L+1 coarse latitudes; nt = 2N, np = 2 np2
+  int L, N, np2, nt, np, NT;   // N = L+1 coarse latitudes; nt = 2N, np = 2 np2; NT harmonics
   const double* w2;            // [N] coarse Gauss weights
-  const double* w;             // [nt] fine Gauss weights
   const double* s2;            // [N] sin(theta) coarse
-  const double* Pc;            // [N][N][N] (i, m, n) coarse Pbar
-  const double* Pcd;           // [N][N][N] coarse dPbar/dtheta
-  const double* Pfd;           // [nt][5][N][N] fine theta-derivatives 0..4
-  const double* Pfa;           // [nt][N][N] fine Pbar, degrees <= L
-  const double* cs2;           // [np2][N] cos(m phi_j) coarse
-  const double* sn2;
-  const double* csf;           // [np][N] fine
-  const double* snf;
-  const double* ref;           // [nt*np][NREF] unit-sphere state (mode 0 reads it)
-};
-
-// ---- per-node geometry and law (device versions of the oracle's formulas) ------------------
-struct Geom {
-  double a[2][3], n[3], J;
-  double g[2][2], gd[2][2][2];
-  double G[2][2], Gd[2][2][2], Gdd[2][2][2][2];
-  double b[2][2], bd[2][2][2], bdd[2][2][2][2];
-  double Gam[2][2][2], Gamd[2][2][2][2];
+  const double* WPc;           // [N][NT] w2 Pbar, coarse (analysis of the shape)
+  const double* Pc;            // [(N+1)/2][NT] coarse Pbar, northern rings
+  const double* Pcd;           // [(N+1)/2][NT] coarse dPbar/dtheta, northern rings
+  const double* Pfd;           // [N][5][NT] fine theta-derivatives 0..4, northern rings
+  const double* WPf;           // [N][NT] w Pbar, fine northern rings (the filter's quadrature)
+  const double2* e2;           // [np2] cos, sin(2 pi q / np2)
+  const double2* ef;           // [np] cos, sin(2 pi q / np)
+  const double* ref;           // [NREF][nt*np] unit-sphere state (the law reads it)
 };
 
 __device__ inline double dot3(const double* u, const double* v) {
@@ -69,12 +68,6 @@ __device__ inline void cross3(const double* u, const double* v, double* r) {
   r[0] = u[1] * v[2] - u[2] * v[1];
   r[1] = u[2] * v[0] - u[0] * v[2];
   r[2] = u[0] * v[1] - u[1] * v[0];
-}
-__device__ inline void mul2(const double X[2][2], const double Y[2][2], double R[2][2]) {
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) R[i][j] = X[i][0] * Y[0][j] + X[i][1] * Y[1][j];
 }
 
 // v of the adjacent lane (lanes 2k and 2k + 1 swap): DPP quad_perm [1, 0, 3, 2] on the two
@@ -86,698 +79,818 @@ __device__ __forceinline__ double swap_pair(double v) {
   return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-// X[c][q]: derivatives of coordinate c; returns the node geometry
-__device__ void geometry(const double (*X)[NQ], Geom& o) {
-  double x1[2][3], x2[2][2][3], x3[2][2][2][3], x4[2][2][2][2][3];
+// ---- per-node geometry and law -----------------------------------------------------------------
+// Tensors that are symmetric in a pair of indices keep one value per sum of the pair: a metric
+// g[a + b], its derivatives gd[c][a + b] and gdd[c + d][a + b].  Everything past the surface's
+// own derivatives is scalar: with D21[s][b] = x_,s . x_,b (s the number of phi-derivatives of
+// the second derivative) and so on, the Christoffel symbols are Gam[l][s] = G[l][p] D21[s][p],
+// n_,c = -b_cl a^l turns the derivatives of the curvature into products of b, Gam and
+// H[l][s] = x_,s(third) . a^l, and no contravariant vector or derivative of the normal is formed:
+// about 430 FMAs a node instead of 1000, with 36 instead of 56 values of reference state.
+struct Geom {
+  double n[3], x1[2][3];
+  double g[3], gd[2][3], G[3], Gd[2][3], Gdd[3][3];
+  double b[3], bd[2][3], bdd[3][3];
+  double Gam[2][3], Gamd[2][2][3];  // [l][s], [derivative][l][s]
+};
+
+// the entries of R = X S (S symmetric, X full) that a symmetric result needs: (0,0), (0,1), (1,1)
+__device__ __forceinline__ void mul_fs(const double X[2][2], const double S[3], double R[2][2]) {
 #pragma unroll
-  for (int k = 0; k < 3; ++k)
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int a = 0; a < 2; ++a) {
-      x1[a][k] = X[k][qidx(1 - a, a)];
-#pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        x2[a][b][k] = X[k][qidx(2 - a - b, a + b)];
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-          x3[a][b][c][k] = X[k][qidx(3 - a - b - c, a + b + c)];
-#pragma unroll
-          for (int d = 0; d < 2; ++d) x4[a][b][c][d][k] = X[k][qidx(4 - a - b - c - d, a + b + c + d)];
-        }
-      }
-    }
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int k = 0; k < 3; ++k) o.a[a][k] = x1[a][k];
-  double cv[3], nd[2][3];
-  cross3(x1[0], x1[1], cv);
-  o.J = sqrt(dot3(cv, cv));
-  const double rJ = 1.0 / o.J;  // one division per node; the others multiply by it
-#pragma unroll
-  for (int k = 0; k < 3; ++k) o.n[k] = cv[k] * rJ;
-#pragma unroll
-  for (int c = 0; c < 2; ++c) {
-    double t1[3], t2[3], cd[3];
-    cross3(x2[0][c], x1[1], t1);
-    cross3(x1[0], x2[1][c], t2);
-#pragma unroll
-    for (int k = 0; k < 3; ++k) cd[k] = t1[k] + t2[k];
-    const double Jd = dot3(o.n, cd);
-#pragma unroll
-    for (int k = 0; k < 3; ++k) nd[c][k] = (cd[k] - Jd * o.n[k]) * rJ;
-  }
-  double gdd[2][2][2][2];
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      o.g[a][b] = dot3(x1[a], x1[b]);
-#pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        o.gd[c][a][b] = dot3(x2[a][c], x1[b]) + dot3(x1[a], x2[b][c]);
-#pragma unroll
-        for (int d = 0; d < 2; ++d)
-          gdd[c][d][a][b] = dot3(x3[a][c][d], x1[b]) + dot3(x2[a][c], x2[b][d]) +
-                            dot3(x2[a][d], x2[b][c]) + dot3(x1[a], x3[b][c][d]);
-      }
-    }
-  const double det = o.g[0][0] * o.g[1][1] - o.g[0][1] * o.g[1][0];
-  const double rdet = 1.0 / det;
-  o.G[0][0] = o.g[1][1] * rdet, o.G[1][1] = o.g[0][0] * rdet;
-  o.G[0][1] = -o.g[0][1] * rdet, o.G[1][0] = -o.g[1][0] * rdet;
-  double GdgG[2][2][2];
-#pragma unroll
-  for (int c = 0; c < 2; ++c) {
-    double t[2][2], u[2][2];
-    mul2(o.G, o.gd[c], t);
-    mul2(t, o.G, u);
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-      for (int b = 0; b < 2; ++b) GdgG[c][a][b] = u[a][b], o.Gd[c][a][b] = -u[a][b];
-  }
-#pragma unroll
-  for (int c = 0; c < 2; ++c)
-#pragma unroll
-    for (int d = 0; d < 2; ++d) {
-      double t1[2][2], t2[2][2], t3[2][2], t4[2][2], t5[2][2], gcd[2][2];
-      mul2(GdgG[d], o.gd[c], t1);
-      mul2(t1, o.G, t2);
-      mul2(GdgG[c], o.gd[d], t3);
-      mul2(t3, o.G, t4);
-#pragma unroll
-      for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) gcd[a][b] = gdd[c][d][a][b];
-      mul2(o.G, gcd, t1);
-      mul2(t1, o.G, t5);
-#pragma unroll
-      for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) o.Gdd[c][d][a][b] = t2[a][b] + t4[a][b] - t5[a][b];
-    }
-  double ac[2][3], acd[2][2][3];
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      ac[a][k] = o.G[a][0] * x1[0][k] + o.G[a][1] * x1[1][k];
-#pragma unroll
-      for (int c = 0; c < 2; ++c)
-        acd[c][a][k] = o.Gd[c][a][0] * x1[0][k] + o.Gd[c][a][1] * x1[1][k] +
-                       o.G[a][0] * x2[0][c][k] + o.G[a][1] * x2[1][c][k];
-    }
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      o.b[a][b] = dot3(x2[a][b], o.n);
-#pragma unroll
-      for (int c = 0; c < 2; ++c) o.bd[c][a][b] = dot3(x3[a][b][c], o.n) + dot3(x2[a][b], nd[c]);
-    }
-  double ndd[2][2][3];
-#pragma unroll
-  for (int c = 0; c < 2; ++c)
-#pragma unroll
-    for (int d = 0; d < 2; ++d)
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        double s = 0.0;
-#pragma unroll
-        for (int l = 0; l < 2; ++l) s += o.bd[d][c][l] * ac[l][k] + o.b[c][l] * acd[d][l][k];
-        ndd[c][d][k] = -s;
-      }
-#pragma unroll
-  for (int c = 0; c < 2; ++c)
-#pragma unroll
-    for (int d = 0; d < 2; ++d)
-#pragma unroll
-      for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-          o.bdd[c][d][a][b] = dot3(x4[a][b][c][d], o.n) + dot3(x3[a][b][c], nd[d]) +
-                              dot3(x3[a][b][d], nd[c]) + dot3(x2[a][b], ndd[c][d]);
-#pragma unroll
-  for (int b = 0; b < 2; ++b)
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        o.Gam[b][a][c] = dot3(x2[a][c], ac[b]);
-#pragma unroll
-        for (int l = 0; l < 2; ++l)
-          o.Gamd[l][b][a][c] = dot3(x3[a][c][l], ac[b]) + dot3(x2[a][c], acd[l][b]);
-      }
+    for (int j = 0; j < 2; ++j) R[i][j] = X[i][0] * S[j] + X[i][1] * S[1 + j];
 }
 
-// load q1 a1 + q2 a2 + q3 n at one node (sph.f90:1615-1700; membmodel.c:60-79)
-__device__ void law(const Geom& o, const double* __restrict__ R, double gs, double eb,
-                    double f[3]) {
-  double A[2][2], Ad[2][2][2], Add[2][2][2][2], B[2][2], Bd[2][2][2], Bdd[2][2][2][2];
+// X[c][q]: derivatives of coordinate c.  BEND: the second derivatives of metric and curvature
+// too, which only the bending moment needs (they are what reads the third and fourth
+// derivatives of the surface).
+template <bool BEND>
+__device__ __forceinline__ void geometry(const double (&X)[3][BEND ? NQ : 6], Geom& o) {
+  double x2[3][3];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) (&A[0][0])[q] = R[q], (&B[0][0])[q] = R[28 + q];
+  for (int k = 0; k < 3; ++k) {
+    o.x1[0][k] = X[k][qidx(1, 0)], o.x1[1][k] = X[k][qidx(0, 1)];
 #pragma unroll
-  for (int q = 0; q < 8; ++q) (&Ad[0][0][0])[q] = R[4 + q], (&Bd[0][0][0])[q] = R[32 + q];
+    for (int s = 0; s < 3; ++s) x2[s][k] = X[k][qidx(2 - s, s)];
+  }
+  double cv[3];
+  cross3(o.x1[0], o.x1[1], cv);
+  const double rJ = 1.0 / sqrt(dot3(cv, cv));
 #pragma unroll
-  for (int q = 0; q < 16; ++q) (&Add[0][0][0][0])[q] = R[12 + q], (&Bdd[0][0][0][0])[q] = R[40 + q];
-  const double detA = A[0][0] * A[1][1] - A[0][1] * A[0][1];
-  const double deta = o.g[0][0] * o.g[1][1] - o.g[0][1] * o.g[0][1];
+  for (int k = 0; k < 3; ++k) o.n[k] = cv[k] * rJ;
+  double D21[3][2];
+#pragma unroll
+  for (int s = 0; s < 3; ++s) {
+    o.b[s] = dot3(x2[s], o.n);
+#pragma unroll
+    for (int p = 0; p < 2; ++p) D21[s][p] = dot3(x2[s], o.x1[p]);
+  }
+  o.g[0] = dot3(o.x1[0], o.x1[0]), o.g[1] = dot3(o.x1[0], o.x1[1]), o.g[2] = dot3(o.x1[1], o.x1[1]);
+  const double rdet = 1.0 / (o.g[0] * o.g[2] - o.g[1] * o.g[1]);
+  o.G[0] = o.g[2] * rdet, o.G[1] = -o.g[1] * rdet, o.G[2] = o.g[0] * rdet;
+  double U[2][2][2];  // U[c] = G g_,c
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    o.gd[c][0] = 2.0 * D21[c][0];
+    o.gd[c][1] = D21[c][1] + D21[1 + c][0];
+    o.gd[c][2] = 2.0 * D21[1 + c][1];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) U[c][i][j] = o.G[i] * o.gd[c][j] + o.G[1 + i] * o.gd[c][1 + j];
+    o.Gd[c][0] = -(U[c][0][0] * o.G[0] + U[c][0][1] * o.G[1]);
+    o.Gd[c][1] = -(U[c][0][0] * o.G[1] + U[c][0][1] * o.G[2]);
+    o.Gd[c][2] = -(U[c][1][0] * o.G[1] + U[c][1][1] * o.G[2]);
+  }
+#pragma unroll
+  for (int l = 0; l < 2; ++l)
+#pragma unroll
+    for (int s = 0; s < 3; ++s) o.Gam[l][s] = o.G[l] * D21[s][0] + o.G[1 + l] * D21[s][1];
+  if (!BEND) return;
+  double D31[4][2], D22[3][3], N3[4], N4[5], H[2][4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    double v[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) v[k] = X[k][BEND ? qidx(3 - s, s) : 0];
+    N3[s] = dot3(v, o.n);
+#pragma unroll
+    for (int p = 0; p < 2; ++p) D31[s][p] = dot3(v, o.x1[p]);
+#pragma unroll
+    for (int l = 0; l < 2; ++l) H[l][s] = o.G[l] * D31[s][0] + o.G[1 + l] * D31[s][1];
+  }
+#pragma unroll
+  for (int s = 0; s < 5; ++s) {
+    double v[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) v[k] = X[k][BEND ? qidx(4 - s, s) : 0];
+    N4[s] = dot3(v, o.n);
+  }
+#pragma unroll
+  for (int s = 0; s < 3; ++s)
+#pragma unroll
+    for (int t = s; t < 3; ++t) D22[s][t] = D22[t][s] = dot3(x2[s], x2[t]);
+#pragma unroll
+  for (int e = 0; e < 3; ++e) {  // (c, d) = (0, 0), (0, 1), (1, 1)
+    const int c = e >> 1, d = (e + 1) >> 1;
+    const double gdd[3] = {2.0 * (D31[e][0] + D22[c][d]),
+                           (D31[e][1] + D31[1 + e][0]) + (D22[c][1 + d] + D22[d][1 + c]),
+                           2.0 * (D31[1 + e][1] + D22[1 + c][1 + d])};
+    double V[2][2], M[2][2], Y[2][2], Z[2][2];  // M = U_d U_c G, Z = G g_,cd G
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        V[i][j] = U[d][i][0] * U[c][0][j] + U[d][i][1] * U[c][1][j];
+        Y[i][j] = o.G[i] * gdd[j] + o.G[1 + i] * gdd[1 + j];
+      }
+    mul_fs(V, o.G, M);
+    mul_fs(Y, o.G, Z);
+    o.Gdd[e][0] = 2.0 * M[0][0] - Z[0][0];
+    o.Gdd[e][1] = (M[0][1] + M[1][0]) - Z[0][1];
+    o.Gdd[e][2] = 2.0 * M[1][1] - Z[1][1];
+  }
+  double W[2][2][3];  // W[d][l][s] = x_,s . (a^l)_,d
+#pragma unroll
+  for (int d = 0; d < 2; ++d)
+#pragma unroll
+    for (int l = 0; l < 2; ++l)
+#pragma unroll
+      for (int s = 0; s < 3; ++s) {
+        W[d][l][s] = (o.Gd[d][l] * D21[s][0] + o.Gd[d][1 + l] * D21[s][1]) +
+                     (o.G[l] * D22[s][d] + o.G[1 + l] * D22[s][1 + d]);
+        o.Gamd[d][l][s] = H[l][s + d] + W[d][l][s];
+      }
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+#pragma unroll
+    for (int s = 0; s < 3; ++s)
+      o.bd[c][s] = N3[s + c] - (o.b[c] * o.Gam[0][s] + o.b[c + 1] * o.Gam[1][s]);
+#pragma unroll
+  for (int e = 0; e < 3; ++e) {
+    const int c = e >> 1, d = (e + 1) >> 1;
+#pragma unroll
+    for (int s = 0; s < 3; ++s) {
+      double t = N4[s + e];
+#pragma unroll
+      for (int l = 0; l < 2; ++l) {
+        t -= o.b[d + l] * H[l][s + c] + o.b[c + l] * H[l][s + d];
+        t -= o.bd[d][c + l] * o.Gam[l][s] + o.b[c + l] * W[d][l][s];
+      }
+      o.bdd[e][s] = t;
+    }
+  }
+}
+
+// load q1 a1 + q2 a2 + q3 n at one node (sph.f90:1615-1700; membmodel.c:60-79); R: the node's
+// reference state, field q at R[q * rs]
+template <bool BEND>
+__device__ __forceinline__ void law(const Geom& o, const double* __restrict__ R, long long rs,
+                                    double gs, double eb, double f[3]) {
+  double A[3], Ad[2][3];
+#pragma unroll
+  for (int s = 0; s < 3; ++s) {
+    A[s] = R[s * rs];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) Ad[c][s] = R[(3 + 3 * c + s) * rs];
+  }
+  const double detA = A[0] * A[2] - A[1] * A[1];
+  const double deta = o.g[0] * o.g[2] - o.g[1] * o.g[1];
   const double I2 = detA * deta - 1.0;
   const double Js = sqrt(1.0 + I2);
   const double rJs = 1.0 / Js, rI = 1.0 / (I2 + 1.0);  // one division each
-  double I2d[2], Jsd[2];
-#pragma unroll
-  for (int c = 0; c < 2; ++c) {
-    const double dA = Ad[c][0][0] * A[1][1] + A[0][0] * Ad[c][1][1] - 2.0 * A[0][1] * Ad[c][0][1];
-    const double da = o.gd[c][0][0] * o.g[1][1] + o.g[0][0] * o.gd[c][1][1] -
-                      2.0 * o.g[0][1] * o.gd[c][0][1];
-    I2d[c] = dA * deta + da * detA;
-    Jsd[c] = 0.5 * rJs * I2d[c];
-  }
   const double w1 = 0.5 * gs;
   const double w2 = -0.5 * gs * (rI * rI);
-  double w2d[2];
+  const double tA = 2.0 * rJs * w1, tG = 2.0 * Js * w2;  // T = tA A + tG G
+  double T[3], Td[2][3];
 #pragma unroll
-  for (int c = 0; c < 2; ++c) w2d[c] = gs * (rI * rI * rI) * I2d[c];
-  double T[2][2], Td[2][2][2];
+  for (int s = 0; s < 3; ++s) T[s] = tA * A[s] + tG * o.G[s];
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+  for (int c = 0; c < 2; ++c) {
+    const double dA = Ad[c][0] * A[2] + A[0] * Ad[c][2] - 2.0 * A[1] * Ad[c][1];
+    const double da = o.gd[c][0] * o.g[2] + o.g[0] * o.gd[c][2] - 2.0 * o.g[1] * o.gd[c][1];
+    const double I2d = dA * deta + da * detA;
+    const double Jsd = 0.5 * rJs * I2d;
+    const double w2d = gs * (rI * rI * rI) * I2d;
+    const double uA = -2.0 * (rJs * rJs) * Jsd * w1, uG = 2.0 * Jsd * w2 + 2.0 * Js * w2d;
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      T[a][b] = 2.0 * rJs * w1 * A[a][b] + 2.0 * Js * w2 * o.G[a][b];
+    for (int s = 0; s < 3; ++s)
+      Td[c][s] = (uA * A[s] + tA * Ad[c][s]) + (uG * o.G[s] + tG * o.Gd[c][s]);
+  }
+  double tr[2];  // Gam^a_al
 #pragma unroll
-      for (int c = 0; c < 2; ++c)
-        Td[c][a][b] = -2.0 * (rJs * rJs) * Jsd[c] * w1 * A[a][b] + 2.0 * rJs * w1 * Ad[c][a][b] +
-                      2.0 * Jsd[c] * w2 * o.G[a][b] + 2.0 * Js * w2d[c] * o.G[a][b] +
-                      2.0 * Js * w2 * o.Gd[c][a][b];
-    }
+  for (int l = 0; l < 2; ++l) tr[l] = o.Gam[0][l] + o.Gam[1][1 + l];
   double q[2];
 #pragma unroll
-  for (int b = 0; b < 2; ++b) {
-    double s = Td[0][0][b] + Td[1][1][b];
+  for (int b = 0; b < 2; ++b)
+    q[b] = (Td[0][b] + Td[1][1 + b]) + (tr[0] * T[b] + tr[1] * T[1 + b]) +
+           (o.Gam[b][0] * T[0] + 2.0 * o.Gam[b][1] * T[1] + o.Gam[b][2] * T[2]);
+  double q3 = T[0] * o.b[0] + 2.0 * T[1] * o.b[1] + T[2] * o.b[2];
+  if (BEND) {
+    double B[3], Bd[2][3];
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
+    for (int s = 0; s < 3; ++s) {
+      B[s] = R[(18 + s) * rs];
 #pragma unroll
-      for (int l = 0; l < 2; ++l) s += o.Gam[a][a][l] * T[l][b] + o.Gam[b][a][l] * T[a][l];
-    q[b] = s;
-  }
-  double q3 = 0.0;
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b) q3 += T[a][b] * o.b[a][b];
-  if (eb != 0.0) {
-    double K[2][2], Kd[2][2][2], Kdd[2][2][2][2];
+      for (int c = 0; c < 2; ++c) Bd[c][s] = R[(21 + 3 * c + s) * rs];
+    }
+    // K^a_c = A^pa B_cp - G^pa b_cp, its first derivatives, and in dds the contraction of
+    // (G^bc K^a_c),ab; K[c][a], Kd[l][c][a]
+    double K[2][2], Kd[2][2][2];
 #pragma unroll
     for (int c = 0; c < 2; ++c)
 #pragma unroll
       for (int a = 0; a < 2; ++a) {
-        double s = 0.0;
+        K[c][a] = (A[a] * B[c] + A[1 + a] * B[c + 1]) - (o.G[a] * o.b[c] + o.G[1 + a] * o.b[c + 1]);
 #pragma unroll
-        for (int cp = 0; cp < 2; ++cp) s += A[cp][a] * B[c][cp] - o.G[cp][a] * o.b[c][cp];
-        K[c][a] = s;
+        for (int l = 0; l < 2; ++l)
+          Kd[l][c][a] = (Ad[l][a] * B[c] + Ad[l][1 + a] * B[c + 1] + A[a] * Bd[l][c] +
+                         A[1 + a] * Bd[l][c + 1]) -
+                        (o.Gd[l][a] * o.b[c] + o.Gd[l][1 + a] * o.b[c + 1] + o.G[a] * o.bd[l][c] +
+                         o.G[1 + a] * o.bd[l][c + 1]);
+      }
+    double dds = 0.0;
 #pragma unroll
-        for (int l = 0; l < 2; ++l) {
-          double t = 0.0;
+    for (int e = 0; e < 3; ++e) {  // derivatives l, k with l + k = e
+      const int l = e >> 1, k = (e + 1) >> 1;
+      double Add[3], Bdd[3];
 #pragma unroll
-          for (int cp = 0; cp < 2; ++cp)
-            t += Ad[l][cp][a] * B[c][cp] + A[cp][a] * Bd[l][c][cp] - o.Gd[l][cp][a] * o.b[c][cp] -
-                 o.G[cp][a] * o.bd[l][c][cp];
-          Kd[l][c][a] = t;
+      for (int s = 0; s < 3; ++s) Add[s] = R[(9 + 3 * e + s) * rs], Bdd[s] = R[(27 + 3 * e + s) * rs];
+      double Kdd[2][2];
 #pragma unroll
-          for (int k = 0; k < 2; ++k) {
-            double u = 0.0;
+      for (int c = 0; c < 2; ++c)
 #pragma unroll
-            for (int cp = 0; cp < 2; ++cp)
-              u += Add[l][k][cp][a] * B[c][cp] + Ad[k][cp][a] * Bd[l][c][cp] +
-                   Ad[l][cp][a] * Bd[k][c][cp] + A[cp][a] * Bdd[l][k][c][cp] -
-                   o.Gdd[l][k][cp][a] * o.b[c][cp] - o.Gd[k][cp][a] * o.bd[l][c][cp] -
-                   o.Gd[l][cp][a] * o.bd[k][c][cp] - o.G[cp][a] * o.bdd[l][k][c][cp];
-            Kdd[l][k][c][a] = u;
+        for (int a = 0; a < 2; ++a) {
+          double u = 0.0, v = 0.0;
+#pragma unroll
+          for (int p = 0; p < 2; ++p) {
+            u += Add[p + a] * B[c + p] + A[p + a] * Bdd[c + p];
+            v += o.Gdd[e][p + a] * o.b[c + p] + o.G[p + a] * o.bdd[e][c + p];
+            if (l == k) {
+              u += 2.0 * (Ad[l][p + a] * Bd[l][c + p]);
+              v += 2.0 * (o.Gd[l][p + a] * o.bd[l][c + p]);
+            } else {
+              u += Ad[k][p + a] * Bd[l][c + p] + Ad[l][p + a] * Bd[k][c + p];
+              v += o.Gd[k][p + a] * o.bd[l][c + p] + o.Gd[l][p + a] * o.bd[k][c + p];
+            }
           }
+          Kdd[c][a] = u - v;
         }
-      }
-    double M[2][2], Md[2][2][2], dds = 0.0;
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        double m = 0.0, md0 = 0.0, md1 = 0.0;
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-          m += o.G[b][c] * K[c][a];
-          md0 += o.Gd[0][b][c] * K[c][a] + o.G[b][c] * Kd[0][c][a];
-          md1 += o.Gd[1][b][c] * K[c][a] + o.G[b][c] * Kd[1][c][a];
-          dds += o.Gdd[b][a][b][c] * K[c][a] + o.Gd[a][b][c] * Kd[b][c][a] +
-                 o.Gd[b][b][c] * Kd[a][c][a] + o.G[b][c] * Kdd[b][a][c][a];
-        }
-        M[a][b] = m, Md[0][a][b] = md0, Md[1][a][b] = md1;
-      }
-    M[1][0] = M[0][1];
-    Md[0][1][0] = Md[0][0][1], Md[1][1][0] = Md[1][0][1];
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        M[a][b] *= eb;
-        Md[0][a][b] *= eb, Md[1][a][b] *= eb;
-      }
-    dds *= eb;
-    double Q[2], Qc = dds;
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      double s = 0.0;
+      // (a, b) with a + b = e: once for a = b, both orders for e = 1
 #pragma unroll
       for (int a = 0; a < 2; ++a) {
-        s += Md[a][a][b];
+        const int b = e - a;
+        if (b < 0 || b > 1) continue;
 #pragma unroll
-        for (int l = 0; l < 2; ++l) {
-          s += o.Gam[a][a][l] * M[l][b] + o.Gam[b][a][l] * M[a][l];
-          Qc += o.Gamd[b][a][a][l] * M[l][b] + o.Gam[a][a][l] * Md[b][l][b] +
-                o.Gamd[b][b][a][l] * M[a][l] + o.Gam[b][a][l] * Md[b][a][l];
-        }
+        for (int c = 0; c < 2; ++c)
+          dds += (o.Gdd[e][b + c] * K[c][a] + o.G[b + c] * Kdd[c][a]) +
+                 (o.Gd[a][b + c] * Kd[b][c][a] + o.Gd[b][b + c] * Kd[a][c][a]);
       }
-      Q[b] = s;
+    }
+    double M[3], Md[2][3];  // (a, b) = (0, 0), (0, 1), (1, 1); the moment is symmetric
+#pragma unroll
+    for (int s = 0; s < 3; ++s) {
+      const int a = s >> 1, b = (s + 1) >> 1;
+      M[s] = eb * (o.G[b] * K[0][a] + o.G[b + 1] * K[1][a]);
+#pragma unroll
+      for (int l = 0; l < 2; ++l)
+        Md[l][s] = eb * ((o.Gd[l][b] * K[0][a] + o.Gd[l][b + 1] * K[1][a]) +
+                         (o.G[b] * Kd[l][0][a] + o.G[b + 1] * Kd[l][1][a]));
+    }
+    double Q[2], Qc = eb * dds;
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      Q[b] = (Md[0][b] + Md[1][1 + b]) + (tr[0] * M[b] + tr[1] * M[1 + b]) +
+             (o.Gam[b][0] * M[0] + 2.0 * o.Gam[b][1] * M[1] + o.Gam[b][2] * M[2]);
+      Qc += (o.Gam[b][0] * Md[b][0] + 2.0 * o.Gam[b][1] * Md[b][1] + o.Gam[b][2] * Md[b][2]);
+      // Gam^a_al,b M^lb
+#pragma unroll
+      for (int l = 0; l < 2; ++l)
+        Qc += (o.Gamd[b][0][l] + o.Gamd[b][1][1 + l]) * M[l + b];
     }
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
+    for (int l = 0; l < 2; ++l)  // Gam^a_al (M^lb_,b + Q^l)
+      Qc += tr[l] * ((Md[0][l] + Md[1][1 + l]) + Q[l]);
 #pragma unroll
-      for (int l = 0; l < 2; ++l) Qc += Q[l] * o.Gam[b][b][l];
+    for (int s = 0; s < 3; ++s)  // Gam^b_al,b M^al
+      Qc += (s == 1 ? 2.0 : 1.0) * (o.Gamd[0][0][s] + o.Gamd[1][1][s]) * M[s];
     double bm[2][2];
 #pragma unroll
     for (int b = 0; b < 2; ++b)
 #pragma unroll
-      for (int a = 0; a < 2; ++a) bm[b][a] = o.G[0][a] * o.b[b][0] + o.G[1][a] * o.b[b][1];
+      for (int a = 0; a < 2; ++a) bm[b][a] = o.G[a] * o.b[b] + o.G[1 + a] * o.b[b + 1];
     q[0] -= bm[0][0] * Q[0] + bm[1][0] * Q[1];
     q[1] -= bm[0][1] * Q[0] + bm[1][1] * Q[1];
     q3 += Qc;
   }
 #pragma unroll
-  for (int k = 0; k < 3; ++k) f[k] = q[0] * o.a[0][k] + q[1] * o.a[1][k] + q3 * o.n[k];
+  for (int k = 0; k < 3; ++k) f[k] = q[0] * o.x1[0][k] + q[1] * o.x1[1][k] + q3 * o.n[k];
 }
 
-// ---- the per-capsule kernel ---------------------------------------------------------------
-// MODE 0: the law; 1: the reference state of one capsule (the unit sphere) into `ref`;
-// 2: shape coefficients only; 3: geometry only (unit normal and point area on the force
-// grid, no load).  Persistent: workgroup b handles capsules b, b + gridDim.x, ...
-// LDS: coarse coefficients [3][N][N] a and b, the longitude factors of both grids (2 (np + np2)
-// values), then a work region reused by the phases.
-// scratch: per workgroup, longitude DFT of the 2x-grid outputs [nt][6][N][2].
-// Registers: capped for two wavefronts per SIMD (256 VGPRs, about 42 of them spilled).  With
-// no cap the law takes 256 VGPRs + 40 AGPRs, one wavefront per SIMD, and runs 1.6x slower.
-// 128 threads per capsule and four capsules per CU (LDS: 39 KB each at L = 16); the per-node
-// phase takes chunks of 128 consecutive nodes, one per thread (step 2 below).
-// The transform loops carry `#pragma unroll 4`.  Their trip counts are run-time values, so
-// without the hint each iteration waits for its own table loads.  Each sum keeps its order,
-// so the output is bitwise unchanged; 1000 capsules at L = 16 take 1.32 instead of 1.47 ms
-// (unrolled by 8: 1.35 ms).
+// ---- the kernels ---------------------------------------------------------------------------------
+// The law of a batch is three kernels: shape (k_shape: coefficients and areas), nodes (k_nodes:
+// the doubled grid's load and its longitude DFT) and filter (k_filter).  Their data per capsule
+// slot: the coefficients [3][NT] (a, b) and the DFT rows [nt][N][6] (cos, sin sums).
+// As one kernel a capsule was one chain of 19 node chunks on one CU (478 us at degree 16,
+// whether 1 capsule or 1000 ran), with the registers of the node phase (256, 42 spilled) held
+// through the transforms.  Apart, the node phase spreads a few capsules over the chip (8
+// capsules: 56 us in all) and holds 232 registers, none spilled; the transforms run 16 wavefronts
+// a CU on tables read coalesced.  8000 capsules of degree 16: 4.74 -> 3.02 ms (shape 0.25, nodes
+// 2.40, filter 0.39); 301 of degree 23 without bending: 1053 -> 316 us.
+// Capsules: slot q holds capsule list[q], q < *cnt (list null: capsule c0 + q, q < n).
+struct Work {
+  int n;              // slots (list null), or the most there can be
+  const int* list;
+  const int* cnt;
+  long long c0;       // list null: slot q holds capsule c0 + q
+  double2* coef;      // [slot][3][NT]
+  double2* rows;      // [slot][nt][N][6]
+};
+__device__ __forceinline__ int work_n(const Work& w) { return w.list ? *w.cnt : w.n; }
+__device__ __forceinline__ long long work_cap(const Work& w, int q) { return w.list ? w.list[q] : w.c0 + q; }
+
+enum Shape {
+  SHAPE_LAW = 0,     // coefficients into the slot, areas
+  SHAPE_COEFFS = 1,  // coefficients packed into `out`
+  SHAPE_GEOM = 2,    // areas and unit normals of the force grid
+  SHAPE_REF = 3,     // coefficients into the slot only
+};
+
+// Coefficients of the three coordinates (the SPHEREPACK analysis of sph1.f90:29-79) and, from
+// them, x_theta and x_phi on the force grid: area |x_theta x x_phi| w / sin(theta) dphi
+// (sph3.f90:186-260; forcing.f90:91) and, for SHAPE_GEOM, the unit normal.
+// The raw coordinates carry the capsule's position, whose rounding lands in the near-zero high-m
+// coefficients and comes out of the fourth derivatives multiplied by m^4: the law sums every
+// point in order, as the reference does, so that it rounds there as the reference does.  The
+// geometry alone reads first derivatives: it takes the coordinates relative to the capsule's
+// first point and pairs points j and j + np2/2 (factors equal up to (-1)^m).
 template <int MODE>
-__global__ void __launch_bounds__(THREADS, 2)
-    k_mem(Tables T, long long ncap, double gs, double eb, const double* __restrict__ x,
-          const double* __restrict__ y, const double* __restrict__ z, double* __restrict__ o0,
-          double* __restrict__ o1, double* __restrict__ o2, double* __restrict__ o3,
-          double* __restrict__ o4, double* __restrict__ o5, double* __restrict__ o6,
-          double* __restrict__ scratch, const int* __restrict__ sel) {
+__global__ void __launch_bounds__(SH_THREADS)
+    k_shape(Tables T, Work wk, const double* __restrict__ x, const double* __restrict__ y,
+            const double* __restrict__ z, double* __restrict__ nx, double* __restrict__ ny,
+            double* __restrict__ nz, double* __restrict__ area, double* __restrict__ out,
+            const int* __restrict__ skip) {
   extern __shared__ double lds[];
+  constexpr bool REL = MODE == SHAPE_GEOM;
   const int tid = threadIdx.x;
-  const int N = T.N, NN = N * N, np2 = T.np2, nt = T.nt, np = T.np;
-  const int nc = N * np2, NT = N * (N + 1) / 2;  // NT: pairs (m, n >= m)
-  double* ca = lds;            // [3][N][N]
-  double* cb = ca + 3 * NN;    // [3][N][N]
-  // cos / sin(2 pi q / np) for q < np, then the same for q < np2: every longitude factor
-  // cos / sin(m phi_j) of the fine (force) grid is entry (m j) mod np (np2) of these, so the
-  // transforms read them from LDS instead of from the [j][m] tables in HBM
-  double* tcf = cb + 3 * NN;
-  double* tsf = tcf + np;
-  double* tc2 = tsf + np;
-  double* ts2 = tc2 + np2;
-  double* U = ts2 + np2;       // work region
-  double* scr = scratch + (size_t)blockIdx.x * nt * 6 * N * 2;  // >= 6 nc doubles too
-  for (int q = tid; q < np; q += THREADS) tcf[q] = T.csf[q * N + 1], tsf[q] = T.snf[q * N + 1];
-  for (int q = tid; q < np2; q += THREADS) tc2[q] = T.cs2[q * N + 1], ts2[q] = T.sn2[q * N + 1];
-  __syncthreads();
-  for (long long cap = blockIdx.x; cap < ncap; cap += gridDim.x) {
-    if (sel && sel[cap] == 0) continue;  // (uniform in the workgroup)
-    const double* xyz[3] = {x + cap * nc, y + cap * nc, z + cap * nc};
-    // 1. analysis: longitude DFT per (c, i, m) into U, then quadrature per (c, m, n)
-    // one thread per (i, m) for the three coordinates, every point in order: the raw
-    // coordinates carry the capsule's position, and pairing points j and j + np2/2 (the
-    // phi -> phi + pi symmetry used for the outputs below) rounds the near-zero high-m
-    // coefficients differently enough for the fourth derivatives' m^4 to show (4x the
-    // difference to the oracle on an ellipsoid)
-    for (int t = tid; t < NN; t += THREADS) {
+  const int N = T.N, NN = N * N, np2 = T.np2, nc = N * np2, NT = T.NT, hp = N;
+  double2* te = reinterpret_cast<double2*>(lds);  // [np2]
+  double2* cf = te + np2;                         // [3][NT] coefficients (a, b)
+  double2* tmp = cf + 3 * NT;  // [6][N][N] partial sums of x_theta (0..2), x_phi (3..5); before:
+  double* pts = reinterpret_cast<double*>(tmp);   // [3][nc] the points and
+  double2* U = tmp + (3 * nc + 1) / 2;            // [3][N][N] their longitude DFT
+  for (int q = tid; q < np2; q += SH_THREADS) te[q] = T.e2[q];
+  const int n = work_n(wk);
+  for (int slot = blockIdx.x; slot < n; slot += gridDim.x) {
+    const long long cap = work_cap(wk, slot);
+    if (skip && skip[cap]) continue;  // uniform over the workgroup
+    for (int t = tid; t < 3 * nc; t += SH_THREADS) {
+      const int c = t / nc, q = t - c * nc;
+      const double* p = (c == 0 ? x : (c == 1 ? y : z)) + cap * nc;
+      pts[t] = REL ? p[q] - p[0] : p[q];
+    }
+    __syncthreads();
+    // longitude DFT, one thread per (i, m) for the three coordinates
+    for (int t = tid; t < NN; t += SH_THREADS) {
       const int i = t / N, m = t % N;
       double cs[3] = {0.0, 0.0, 0.0}, sn[3] = {0.0, 0.0, 0.0};
+      const double sg = (m & 1) ? -1.0 : 1.0;
       int q = 0;  // (m j) mod np2
       #pragma unroll 4
-      for (int j = 0; j < np2; ++j) {
-        const double c = tc2[q], s = ts2[q];
+      for (int j = 0; j < (REL ? hp : np2); ++j) {
+        const double2 e = te[q];
         q += m;
         if (q >= np2) q -= np2;
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
-          const double v = xyz[k][i * np2 + j];
-          cs[k] += v * c;
-          sn[k] += v * s;
+          const double* p = pts + k * nc + i * np2 + j;
+          const double v = REL ? p[0] + sg * p[hp] : p[0];
+          cs[k] += v * e.x;
+          sn[k] += v * e.y;
         }
       }
 #pragma unroll
-      for (int k = 0; k < 3; ++k) U[2 * (k * NN + t)] = cs[k], U[2 * (k * NN + t) + 1] = sn[k];
+      for (int k = 0; k < 3; ++k) U[k * NN + t] = make_double2(cs[k], sn[k]);
     }
     __syncthreads();
-    // one thread per (m, n >= m) for the three coordinates (entries n < m are never read)
-    for (int t = tid; t < NT; t += THREADS) {
-      int m = 0, n = t;
-      while (n >= N - m) n -= N - m, ++m;
-      n += m;
+    // quadrature, one thread per harmonic for the three coordinates
+    for (int t = tid; t < NT; t += SH_THREADS) {
+      int d = 0, m = t;
+      while (m >= N - d) m -= N - d, ++d;
       double sa[3] = {0.0, 0.0, 0.0}, sb[3] = {0.0, 0.0, 0.0};
       #pragma unroll 4
       for (int i = 0; i < N; ++i) {
-        const double p = T.w2[i] * T.Pc[(i * N + m) * N + n];
+        const double p = T.WPc[i * NT + t];
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
-          const int u = (c * N + i) * N + m;
-          sa[c] += p * U[2 * u];
-          sb[c] += p * U[2 * u + 1];
+        for (int k = 0; k < 3; ++k) {
+          const double2 u = U[(k * N + i) * N + m];
+          sa[k] += p * u.x;
+          sb[k] += p * u.y;
         }
       }
 #pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        ca[(c * N + m) * N + n] = 2.0 / np2 * sa[c];
-        cb[(c * N + m) * N + n] = -2.0 / np2 * sb[c];
+      for (int k = 0; k < 3; ++k) {
+        const double a = 2.0 / np2 * sa[k], b = -2.0 / np2 * sb[k];
+        if (MODE == SHAPE_COEFFS) {
+          // packed: a(m, n >= m) then b(m >= 1, n >= m), per coordinate
+          double* o = out + (cap * 3 + k) * NN;
+          o[m * N - m * (m - 1) / 2 + d] = a;
+          if (m >= 1) o[NT + (m - 1) * N - (m - 1) * (m - 2) / 2 - (m - 1) + d] = b;
+        } else {
+          cf[k * NT + t] = make_double2(a, b);
+          if (MODE != SHAPE_GEOM)
+            wk.coef[((size_t)slot * 3 + k) * NT + t] = make_double2(a, b);
+        }
       }
     }
     __syncthreads();
-    if (MODE == 2) {
-      // packed: a(m, n>=m) then b(m>=1, n>=m), per coordinate
-      for (int t = tid; t < 3 * NN; t += THREADS) {
-        const int c = t / NN, m = (t / N) % N, n = t % N;
-        if (n < m) continue;
-        const int pa = m * N - m * (m - 1) / 2 + (n - m);
-        o0[cap * 3 * NN + c * NN + pa] = ca[(c * N + m) * N + n];
-        if (m >= 1) {
-          const int pb = (N * (N + 1)) / 2 + (m - 1) * N - (m - 1) * (m - 2) / 2 - (m - 1) + (n - m);
-          o0[cap * 3 * NN + c * NN + pb] = cb[(c * N + m) * N + n];
+    if (MODE == SHAPE_LAW || MODE == SHAPE_GEOM) {
+      // x_theta and x_phi of coordinate c per (c, ring pair, m): the sums over even and odd d
+      // give the northern ring as E + O and the southern one as +-(E - O)
+      const int nh = (N + 1) / 2;
+      for (int t = tid; t < 3 * nh * N; t += SH_THREADS) {
+        const int c = t / (nh * N), u = t % (nh * N), i = u / N, m = u % N;
+        const double* Pt = T.Pcd + i * NT;
+        const double* Pp = T.Pc + i * NT;
+        double2 st[2] = {{0.0, 0.0}, {0.0, 0.0}}, sp[2] = {{0.0, 0.0}, {0.0, 0.0}};
+        int q = m;  // tidx(N, d, m)
+        for (int d = 0; d < N - m; d += 2) {
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            const bool on = d + e < N - m;
+            const int qq = on ? q : m;
+            const double2 v = cf[c * NT + qq];
+            const double a = on ? Pt[qq] : 0.0, b = on ? Pp[qq] : 0.0;
+            st[e].x += a * v.x, st[e].y += a * v.y;
+            sp[e].x += b * v.x, sp[e].y += b * v.y;
+            q += N - (d + e);
+          }
+        }
+        const double h = m == 0 ? 0.5 : 1.0;
+        double2* tt = tmp + c * NN + m;
+        double2* tp = tmp + (3 + c) * NN + m;
+        tt[i * N] = make_double2(h * (st[0].x + st[1].x), h * (st[0].y + st[1].y));
+        tp[i * N] = make_double2(h * (sp[0].x + sp[1].x), h * (sp[0].y + sp[1].y));
+        if (N - 1 - i > i) {
+          const int k = (N - 1 - i) * N;
+          tt[k] = make_double2(h * (st[1].x - st[0].x), h * (st[1].y - st[0].y));
+          tp[k] = make_double2(h * (sp[0].x - sp[1].x), h * (sp[0].y - sp[1].y));
         }
       }
       __syncthreads();
-      continue;
-    }
-    // 2. the 2x grid in chunks of W consecutive nodes, one node per thread (not for MODE 3:
-    //    geometry only).  A chunk of W <= (RING - 1) np nodes touches at most RING rings.
-    //    Ring r's coefficients and outputs live in slot r % RING of AB and F: its coefficients
-    //    are summed before the first chunk that touches it, its longitude DFT runs after the
-    //    chunk that completes it, and only ring r + RING takes the slot again, whose first node
-    //    lies (RING - 1) np + 1 >= W nodes after ring r's last (so in a later chunk).  With
-    //    W = THREADS every round of the per-node phase is full (one partial round per capsule
-    //    instead of one per group of RING rings).
-    double* AB = U;                          // [RING][3][5][N][2]
-    double* F = AB + RING * 3 * 5 * N * 2;   // [RING][np][6]
-    const int nnode = MODE == 3 ? 0 : nt * np;
-    const int W = min(THREADS, (RING - 1) * np);  // even: node pairs stay in one chunk
-    int rnext = 0, rdone = 0;  // first ring without coefficients / without its DFT
-    for (int n0 = 0; n0 < nnode; n0 += W) {
-      const int n1 = min(n0 + W, nnode);
-      const int rhi = (n1 - 1) / np;  // last ring of the chunk
-      // a thread sums the three coordinates of one (ring, k, m): each table load feeds six FMAs
-      for (int t = tid; t < (rhi + 1 - rnext) * 5 * N; t += THREADS) {
-        const int ring = rnext + t / (5 * N), k = (t / N) % 5, m = t % N;
-        const int r = ring % RING;
-        const double* Pd = T.Pfd + (((size_t)ring * 5 + k) * N + m) * N;
-        const double h = m == 0 ? 0.5 : 1.0;
-        double sa0 = 0.0, sb0 = 0.0, sa1 = 0.0, sb1 = 0.0, sa2 = 0.0, sb2 = 0.0;
-        #pragma unroll 4
-        for (int n = m; n < N; ++n) {
-          const double p = Pd[n];
-          sa0 += p * ca[m * N + n], sb0 += p * cb[m * N + n];
-          sa1 += p * ca[(N + m) * N + n], sb1 += p * cb[(N + m) * N + n];
-          sa2 += p * ca[(2 * N + m) * N + n], sb2 += p * cb[(2 * N + m) * N + n];
+      // node sums, one thread per (i, j < np2/2) and its partner j + np2/2: the even-m terms E
+      // and the odd-m terms O give E + O and E - O
+      for (int t = tid; t < N * hp; t += SH_THREADS) {
+        const int i = t / hp, j = t % hp;
+        double s[2][6];
+#pragma unroll
+        for (int f = 0; f < 6; ++f) s[0][f] = 0.0, s[1][f] = 0.0;
+        int q = 0;  // (m j) mod np2
+        for (int m = 0; m < N; m += 2) {
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            if (m + e >= N) break;
+            const double2 w = te[q];
+            q += j;
+            if (q >= np2) q -= np2;
+#pragma unroll
+            for (int f = 0; f < 6; ++f) {
+              const double2 v = tmp[f * NN + i * N + m + e];
+              s[e][f] += f < 3 ? v.x * w.x - v.y * w.y : (double)(m + e) * (-v.x * w.y - v.y * w.x);
+            }
+          }
         }
-        const int t0 = ((r * 3) * 5 + k) * N + m, cs = 5 * N;  // AB slot of coordinate 0; stride
-        AB[2 * t0] = h * sa0, AB[2 * t0 + 1] = h * sb0;
-        AB[2 * (t0 + cs)] = h * sa1, AB[2 * (t0 + cs) + 1] = h * sb1;
-        AB[2 * (t0 + 2 * cs)] = h * sa2, AB[2 * (t0 + 2 * cs) + 1] = h * sb2;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          double v[6], cr[3];
+#pragma unroll
+          for (int f = 0; f < 6; ++f) v[f] = e ? s[0][f] - s[1][f] : s[0][f] + s[1][f];
+          cross3(&v[0], &v[3], cr);
+          const double J = sqrt(dot3(cr, cr));
+          const size_t o = (size_t)cap * nc + i * np2 + j + e * hp;
+          if (MODE == SHAPE_GEOM) nx[o] = cr[0] / J, ny[o] = cr[1] / J, nz[o] = cr[2] / J;
+          area[o] = J * T.w2[i] / T.s2[i] * (2.0 * M_PI / np2);
+        }
       }
-      rnext = rhi + 1;
+      __syncthreads();
+    }
+  }
+}
+
+// The doubled grid: x and its derivatives up to 4th order (sph3.f90:9-182; to 2nd order without
+// bending, where nothing reads the others), per node the geometry and the load q1 a1 + q2 a2 +
+// q3 n (sph.f90:1523-1700), and the longitude DFT of load and normal, degrees <= L.
+// REF: the unit sphere's state of slot 0 into `refout` instead.
+//
+// A unit of work is a run of rings of one capsule; rings go in the order north, south, north
+// ... (ring 0, nt - 1, 1, nt - 2, ...).  A few capsules are cut into so many runs that the
+// workgroups in flight are all used (8 capsules of degree 16: one ring each), many are one run
+// each: a ring's sums do not depend on the cut.  Within a run, chunks of W consecutive nodes, one per
+// thread.  A chunk of W <= 2 np nodes touches at most three rings; ring r's coefficients live in
+// slot r % AB_SLOTS and are summed (with those of its pair) before the first chunk that touches
+// it, its outputs live in slot r % F_SLOTS until the DFT after the chunk that completes it.
+// Registers: two wavefronts per SIMD.
+template <bool REF, bool BEND>
+__global__ void __launch_bounds__(ND_THREADS, 2)
+    k_nodes(Tables T, Work wk, int most, double gs, double eb, double* __restrict__ refout) {
+  extern __shared__ double lds[];
+  constexpr int NK = BEND ? 5 : 3, NX = BEND ? NQ : 6;  // theta-derivatives, derivatives
+  const int tid = threadIdx.x;
+  const int N = T.N, nt = T.nt, np = T.np, hp = np / 2, NT = T.NT;
+  double2* te = reinterpret_cast<double2*>(lds);  // [np]
+  double2* cf = te + np;                          // [3][NT]
+  double2* AB = cf + 3 * NT;                      // [AB_SLOTS][N][3][NK]
+  double* F = reinterpret_cast<double*>(AB + AB_SLOTS * 3 * NK * N);  // [F_SLOTS][hp][2][6]
+  for (int q = tid; q < np; q += ND_THREADS) te[q] = T.ef[q];
+  // runs of rp rings (an even number, so that pairs stay together, or single rings)
+  const int n = work_n(wk);
+  if (n == 0) return;
+  const int want = min(nt, max(1, most / n));
+  int rp = (nt + want - 1) / want;
+  if (rp > 1) rp += rp & 1;
+  const int parts = (nt + rp - 1) / rp;
+  const int W = min(ND_THREADS, 2 * np);  // even: node pairs stay in one chunk
+  for (int u = blockIdx.x; u < n * parts; u += gridDim.x) {
+    const int slot = u / parts, s0 = (u - slot * parts) * rp, s1 = min(s0 + rp, nt);
+    __syncthreads();
+    for (int t = tid; t < 3 * NT; t += ND_THREADS) cf[t] = wk.coef[(size_t)slot * 3 * NT + t];
+    __syncthreads();
+    const int node0 = s0 * np, node1 = s1 * np;
+    int rnext = s0, rdone = s0;  // first ring without coefficients / without its DFT
+    for (int n0 = node0; n0 < node1; n0 += W) {
+      const int n1 = min(n0 + W, node1);
+      const int rhi = (n1 - 1) / np;  // last ring of the chunk
+      if (rhi >= rnext) {
+        // one thread per (ring pair, k, m) for the three coordinates: each table load feeds
+        // six FMAs and both rings of the pair, north E + O, south (-1)^k (E - O) of the sums over
+        // even and odd n - m
+        const int p0 = rnext >> 1, p1 = rhi >> 1;
+        for (int t = tid; t < (p1 - p0 + 1) * NK * N; t += ND_THREADS) {
+          const int p = p0 + t / (NK * N), k = (t / N) % NK, m = t % N;
+          const double* P = T.Pfd + ((size_t)p * 5 + k) * NT;
+          double2 s[2][3];
+#pragma unroll
+          for (int c = 0; c < 3; ++c) s[0][c] = s[1][c] = make_double2(0.0, 0.0);
+          int q = m;  // tidx(N, d, m)
+          #pragma unroll 2
+          for (int d = 0; d < N - m; d += 2) {
+            const bool two = d + 1 < N - m;
+            const int q1 = two ? q + N - d : q;
+            const double e0 = P[q], e1 = two ? P[q1] : 0.0;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+              const double2 v0 = cf[c * NT + q], v1 = cf[c * NT + q1];
+              s[0][c].x += e0 * v0.x, s[0][c].y += e0 * v0.y;
+              s[1][c].x += e1 * v1.x, s[1][c].y += e1 * v1.y;
+            }
+            q += 2 * (N - d) - 1;
+          }
+          const double h = m == 0 ? 0.5 : 1.0, hs = (k & 1) ? -h : h;
+#pragma unroll
+          for (int c = 0; c < 3; ++c) {
+            const int a = m * 3 * NK + c * NK + k;
+            AB[((2 * p) % AB_SLOTS) * 3 * NK * N + a] =
+                make_double2(h * (s[0][c].x + s[1][c].x), h * (s[0][c].y + s[1][c].y));
+            AB[((2 * p + 1) % AB_SLOTS) * 3 * NK * N + a] =
+                make_double2(hs * (s[0][c].x - s[1][c].x), hs * (s[0][c].y - s[1][c].y));
+          }
+        }
+        rnext = 2 * p1 + 2;
+      }
       __syncthreads();
       // Lanes 2k and 2k + 1 take the node pair (jj, jj + np/2) of one ring, whose factors
       // agree up to (-1)^m (phi -> phi + pi): lane 2k sums the even-m terms E and lane 2k + 1
       // the odd-m terms O, both at phi_jj; after one exchange node jj holds E + O and node
       // jj + np/2 holds E - O, and each lane goes on with its own node.
-      for (int pn = n0 + tid; pn < n1; pn += THREADS) {
-        const int par = pn & 1, pr = pn >> 1, hp = np / 2;
-        const int ring = pr / hp, jj = pr - ring * hp, j = jj + par * hp, r = ring % RING;
-        const int node = ring * np + j;
-        double X[3][NQ];
+      if (n0 + tid < n1) {
+        const int pn = n0 + tid;
+        const int par = pn & 1, pr = pn >> 1;
+        const int ring = pr / hp, jj = pr - ring * hp;
+        double X[3][NX];
 #pragma unroll
         for (int c = 0; c < 3; ++c)
 #pragma unroll
-          for (int q = 0; q < NQ; ++q) X[c][q] = 0.0;
+          for (int q = 0; q < NX; ++q) X[c][q] = 0.0;
         int q = par * jj;  // (m jj) mod np
-        const int dq = (2 * jj) % np;
-        for (int m = par; m < N; m += 2) {
-          const double cm = tcf[q], sm = tsf[q];
+        int dq = 2 * jj;
+        if (dq >= np) dq -= np;
+        const double2* ab = AB + (ring % AB_SLOTS) * 3 * NK * N + par * 3 * NK;
+        for (int m = par; m < N; m += 2, ab += 6 * NK) {
+          const double2 w = te[q];
           q += dq;
           if (q >= np) q -= np;
           const double m1 = (double)m, m2 = m1 * m1, m3 = m2 * m1, m4 = m2 * m2;
 #pragma unroll
           for (int c = 0; c < 3; ++c)
 #pragma unroll
-            for (int kt = 0; kt <= 4; ++kt) {
-              const int ab = ((r * 3 + c) * 5 + kt) * N + m;
-              const double A = AB[2 * ab], B = AB[2 * ab + 1];
-              const double h0 = A * cm - B * sm, h1 = -A * sm - B * cm;
+            for (int kt = 0; kt < NK; ++kt) {
+              const double2 v = ab[c * NK + kt];
+              const double h0 = v.x * w.x - v.y * w.y, h1 = -v.x * w.y - v.y * w.x;
               X[c][qidx(kt, 0)] += h0;
-              if (kt <= 3) X[c][qidx(kt, 1)] += m1 * h1;
-              if (kt <= 2) X[c][qidx(kt, 2)] -= m2 * h0;
-              if (kt <= 1) X[c][qidx(kt, 3)] -= m3 * h1;
-              if (kt == 0) X[c][qidx(0, 4)] += m4 * h0;
+              if (kt <= NK - 2) X[c][qidx(kt, 1)] += m1 * h1;
+              if (kt <= NK - 3) X[c][qidx(kt, 2)] -= m2 * h0;
+              if (BEND && kt <= 1) X[c][BEND ? qidx(kt, 3) : 0] -= m3 * h1;
+              if (BEND && kt == 0) X[c][BEND ? qidx(0, 4) : 0] += m4 * h0;
             }
         }
 #pragma unroll
         for (int c = 0; c < 3; ++c)
 #pragma unroll
-          for (int qq = 0; qq < NQ; ++qq) {
+          for (int qq = 0; qq < NX; ++qq) {
             const double other = swap_pair(X[c][qq]);
             X[c][qq] = par ? other - X[c][qq] : X[c][qq] + other;
           }
         Geom o;
-        geometry(X, o);
-        if (MODE == 1) {
-          double* R = o0 + node * NREF;
+        geometry<BEND>(X, o);
+        const long long nodes = (long long)nt * np;
+        if (REF) {
+          double* R = refout + pn;
 #pragma unroll
-          for (int q = 0; q < 4; ++q) R[q] = (&o.G[0][0])[q], R[28 + q] = (&o.b[0][0])[q];
+          for (int s = 0; s < 3; ++s) {
+            R[s * nodes] = o.G[s], R[(18 + s) * nodes] = o.b[s];
 #pragma unroll
-          for (int q = 0; q < 8; ++q) R[4 + q] = (&o.Gd[0][0][0])[q], R[32 + q] = (&o.bd[0][0][0])[q];
+            for (int c = 0; c < 2; ++c)
+              R[(3 + 3 * c + s) * nodes] = o.Gd[c][s], R[(21 + 3 * c + s) * nodes] = o.bd[c][s];
 #pragma unroll
-          for (int q = 0; q < 16; ++q)
-            R[12 + q] = (&o.Gdd[0][0][0][0])[q], R[40 + q] = (&o.bdd[0][0][0][0])[q];
+            for (int e = 0; e < 3; ++e)
+              R[(9 + 3 * e + s) * nodes] = o.Gdd[e][s], R[(27 + 3 * e + s) * nodes] = o.bdd[e][s];
+          }
         } else {
-          double f[3];
-          law(o, T.ref + node * NREF, gs, eb, f);
-          double* Fo = F + ((size_t)r * np + j) * 6;
-          Fo[0] = f[0], Fo[1] = f[1], Fo[2] = f[2];
-          Fo[3] = o.n[0], Fo[4] = o.n[1], Fo[5] = o.n[2];
+          double f[6];
+          law<BEND>(o, T.ref + pn, nodes, gs, eb, f);
+#pragma unroll
+          for (int k = 0; k < 3; ++k) f[3 + k] = o.n[k];
+          // the DFT needs v_j + v_{j + np/2} for even and v_j - v_{j + np/2} for odd m
+          double* Fo = F + ((size_t)((ring % F_SLOTS) * hp + jj) * 2 + par) * 6;
+#pragma unroll
+          for (int k = 0; k < 6; ++k) {
+            const double other = swap_pair(f[k]);
+            Fo[k] = par ? other - f[k] : f[k] + other;
+          }
         }
       }
       __syncthreads();
-      if (MODE == 0 && n1 / np > rdone) {
-        // rings rdone .. n1 / np - 1 are complete: longitude DFT of their six outputs, degrees
-        // <= L only.  A thread sums three outputs for one (ring, m), so that each pair of
-        // table loads feeds six FMAs.
-        // Nodes j and j + np/2 share their factors up to (-1)^m (phi -> phi + pi), so the
-        // sum runs over the first half of the ring on v_j + (-1)^m v_{j + np/2}.
-        for (int t = tid; t < (n1 / np - rdone) * 2 * N; t += THREADS) {
-          const int ring = rdone + t / (2 * N), f0 = 3 * ((t / N) % 2), m = t % N;
-          const int r = ring % RING;
-          const double sg = (m & 1) ? -1.0 : 1.0;
-          const int hp = np / 2;
-          double cs0 = 0.0, sn0 = 0.0, cs1 = 0.0, sn1 = 0.0, cs2 = 0.0, sn2 = 0.0;
+      if (!REF && n1 / np > rdone) {
+        // rings rdone .. n1 / np - 1 are complete: longitude DFT of their six outputs, a thread
+        // for two outputs of one (ring, m)
+        for (int t = tid; t < (n1 / np - rdone) * 3 * N; t += ND_THREADS) {
+          const int ring = rdone + t / (3 * N), g = (t / N) % 3, m = t % N;
+          const double2* v =
+              reinterpret_cast<const double2*>(F + ((size_t)(ring % F_SLOTS) * hp * 2 + (m & 1)) * 6) + g;
+          double2 s0 = {0.0, 0.0}, s1 = {0.0, 0.0};
           int q = 0;  // (m j) mod np
           #pragma unroll 4
           for (int j = 0; j < hp; ++j) {
-            const double* v = F + ((size_t)r * np + j) * 6 + f0;
-            const double* w = v + (size_t)hp * 6;
-            const double c = tcf[q], s = tsf[q];
+            const double2 e = te[q], w = v[6 * j];
             q += m;
             if (q >= np) q -= np;
-            const double e0 = v[0] + sg * w[0], e1 = v[1] + sg * w[1], e2 = v[2] + sg * w[2];
-            cs0 += e0 * c, sn0 += e0 * s;
-            cs1 += e1 * c, sn1 += e1 * s;
-            cs2 += e2 * c, sn2 += e2 * s;
+            s0.x += w.x * e.x, s0.y += w.x * e.y;
+            s1.x += w.y * e.x, s1.y += w.y * e.y;
           }
-          double* s = scr + (((size_t)ring * 6 + f0) * N + m) * 2;
-          s[0] = cs0, s[1] = sn0;
-          s[2 * N] = cs1, s[2 * N + 1] = sn1;
-          s[4 * N] = cs2, s[4 * N + 1] = sn2;
+          double2* r = wk.rows + (((size_t)slot * nt + ring) * N + m) * 6 + 2 * g;
+          r[0] = s0, r[1] = s1;
         }
-        __syncthreads();
         rdone = n1 / np;
       }
     }
-    if (MODE == 1) continue;
-    // 3. filter: quadrature of the 2x-grid outputs (degrees <= L), synthesis on the force
-    //    grid, two fields at a time (each table load feeds both); the area from the coarse
-    //    shape (sph3.f90:186-260)
-    // fc: the six fields' coefficients, packed by (m, n >= m) at pk(m) + n - m with
-    // pk(m) = m N - m (m - 1) / 2, [6][N (N + 1) / 2][2]; tmp: per (i, m) partial sums of the
-    // current pair of fields
-    double* fc = U;
-    double* tmp = U + 12 * NT;   // [2][N][N][2]
-    double* xt = scr;            // [nc][3] x_theta on the force grid (scratch reused)
-    double* xp = scr + (size_t)nc * 3;  // [nc][3] x_phi
-    if (MODE == 0) {
-      // quadrature of all six fields in one pass, one item per (m, n >= m) pair (each table
-      // load feeds twelve sums), 2 THREADS items per round.  The scratch rows of nq rings at
-      // a time are first copied into the tmp region (all of a thread's loads in flight, one
-      // wait per chunk): read in place, each iteration waited on its own scratch loads.
-      const int nq = N / 3;  // 12 N nq <= 4 NN doubles
-      double* stg = tmp;
-      for (int t0 = 0; t0 < NT; t0 += 2 * THREADS) {
-        int mm[2], nn[2];
-        double sa[2][6], sb[2][6];
+  }
+}
+
+// The dealias filter: quadrature of the doubled grid's load and normal (degrees <= L), synthesis
+// on the force grid (sph1.f90:723-951), unit normal (cal_unitO_filter, sph1.f90:1378-1406).  A
+// unit is one capsule, or with parts = 2 its load (0) or its normal (1).
+// The DFT rows come nq ring pairs at a time through LDS as the sum and the difference of the
+// pair's rings, which is what the harmonics of even and of odd n - m integrate.
+constexpr int FL_STAGE = 4;  // ring pairs per staged chunk
+__global__ void __launch_bounds__(SH_THREADS)
+    k_filter(Tables T, Work wk, int most, double* __restrict__ fx, double* __restrict__ fy,
+             double* __restrict__ fz, double* __restrict__ nx, double* __restrict__ ny,
+             double* __restrict__ nz) {
+  extern __shared__ double lds[];
+  const int tid = threadIdx.x;
+  const int N = T.N, NN = N * N, np2 = T.np2, nt = T.nt, nc = N * np2, NT = T.NT, hp = N;
+  const int nh = (N + 1) / 2;
+  double2* te = reinterpret_cast<double2*>(lds);  // [np2]
+  double2* fc = te + np2;                         // [3][NT] coefficients of the three fields
+  double2* stg = fc + 3 * NT;                     // [FL_STAGE][2][N][3] staged rows, then
+  double2* tmp = stg;                             // [3][N][N] partial sums
+  for (int q = tid; q < np2; q += SH_THREADS) te[q] = T.e2[q];
+  const int n = work_n(wk);
+  const int parts = 2 * n <= most ? 2 : 1;
+  for (int u = blockIdx.x; u < n * parts; u += gridDim.x) {
+    const int slot = u / parts;
+    const long long cap = work_cap(wk, slot);
+    for (int g = parts == 2 ? u - slot * 2 : 0; g < (parts == 2 ? u - slot * 2 + 1 : 2); ++g) {
+      const double2* rows = wk.rows + (size_t)slot * nt * N * 6 + 3 * g;
+      // quadrature, one thread per harmonic and field; up to 4 items a thread (NT <= 300)
+      double2 acc[4];
 #pragma unroll
-        for (int k = 0; k < 2; ++k) {
-          int m = 0, n = min(t0 + k * THREADS + tid, NT - 1);
-          while (n >= N - m) n -= N - m, ++m;
-          mm[k] = m, nn[k] = n + m;
-#pragma unroll
-          for (int f = 0; f < 6; ++f) sa[k][f] = 0.0, sb[k][f] = 0.0;
+      for (int k = 0; k < 4; ++k) acc[k] = make_double2(0.0, 0.0);
+      for (int c0 = 0; c0 < N; c0 += FL_STAGE) {
+        const int cr = min(FL_STAGE, N - c0);
+        __syncthreads();  // the previous chunk (and unit) is consumed
+        for (int e = tid; e < cr * 3 * N; e += SH_THREADS) {
+          const int r = e / (3 * N), k = e - r * 3 * N;  // k = 3 m + field
+          const size_t a = (size_t)(2 * (c0 + r)) * N * 6 + (k / 3) * 6 + k % 3;
+          const double2 v = rows[a], w = rows[a + (size_t)N * 6];
+          stg[(r * 2) * 3 * N + k] = make_double2(v.x + w.x, v.y + w.y);
+          stg[(r * 2 + 1) * 3 * N + k] = make_double2(v.x - w.x, v.y - w.y);
         }
-        for (int c0 = 0; c0 < nt; c0 += nq) {
-          const int cr = min(nq, nt - c0);
-          __syncthreads();  // the previous chunk is consumed
-          const double2* src = reinterpret_cast<const double2*>(scr + (size_t)c0 * 12 * N);
-          double2* dst = reinterpret_cast<double2*>(stg);
-          for (int e = tid; e < cr * 6 * N; e += THREADS) dst[e] = src[e];
-          __syncthreads();
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const int it = tid + k * SH_THREADS;
+          if (it >= 3 * NT) break;
+          const int f = it / NT, t = it - f * NT;
+          int d = 0, m = t;
+          while (m >= N - d) m -= N - d, ++d;
+          const double2* s = stg + (d & 1) * 3 * N + 3 * m + f;
           for (int r = 0; r < cr; ++r) {
-            const int i = c0 + r;
+            const double p = T.WPf[(c0 + r) * NT + t];
+            const double2 v = s[r * 6 * N];
+            acc[k].x += p * v.x;
+            acc[k].y += p * v.y;
+          }
+        }
+      }
+      __syncthreads();
 #pragma unroll
-            for (int k = 0; k < 2; ++k) {
-              const double p = T.w[i] * T.Pfa[((size_t)i * N + mm[k]) * N + nn[k]];
-              const double* sr = stg + ((size_t)r * 6 * N + mm[k]) * 2;
+      for (int k = 0; k < 4; ++k) {
+        const int it = tid + k * SH_THREADS;
+        if (it < 3 * NT) fc[it] = make_double2(2.0 / T.np * acc[k].x, -2.0 / T.np * acc[k].y);
+      }
+      __syncthreads();
+      // partial sums per (field, ring pair, m): northern ring E + O, southern ring E - O
+      for (int t = tid; t < 3 * nh * N; t += SH_THREADS) {
+        const int f = t / (nh * N), w = t % (nh * N), i = w / N, m = w % N;
+        const double* P = T.Pc + i * NT;
+        double2 s[2] = {{0.0, 0.0}, {0.0, 0.0}};
+        int q = m;  // tidx(N, d, m)
+        #pragma unroll 2
+        for (int d = 0; d < N - m; d += 2) {
+          const bool two = d + 1 < N - m;
+          const int q1 = two ? q + N - d : q;
+          const double a = P[q], b = two ? P[q1] : 0.0;
+          const double2 v0 = fc[f * NT + q], v1 = fc[f * NT + q1];
+          s[0].x += a * v0.x, s[0].y += a * v0.y;
+          s[1].x += b * v1.x, s[1].y += b * v1.y;
+          q += 2 * (N - d) - 1;
+        }
+        const double h = m == 0 ? 0.5 : 1.0;
+        double2* o = tmp + f * NN + m;
+        o[i * N] = make_double2(h * (s[0].x + s[1].x), h * (s[0].y + s[1].y));
+        if (N - 1 - i > i)
+          o[(N - 1 - i) * N] = make_double2(h * (s[0].x - s[1].x), h * (s[0].y - s[1].y));
+      }
+      __syncthreads();
+      // node sums of the three fields, one thread per (i, j < np2/2) and its partner j + np2/2
+      for (int t = tid; t < N * hp; t += SH_THREADS) {
+        const int i = t / hp, j = t % hp;
+        double s[2][3] = {{0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}};
+        int q = 0;  // (m j) mod np2
+        for (int m = 0; m < N; m += 2) {
 #pragma unroll
-              for (int f = 0; f < 6; ++f) {
-                sa[k][f] += p * sr[2 * f * N];
-                sb[k][f] += p * sr[2 * f * N + 1];
-              }
+          for (int e = 0; e < 2; ++e) {
+            if (m + e >= N) break;
+            const double2 w = te[q];
+            q += j;
+            if (q >= np2) q -= np2;
+#pragma unroll
+            for (int f = 0; f < 3; ++f) {
+              const double2 v = tmp[f * NN + i * N + m + e];
+              s[e][f] += v.x * w.x - v.y * w.y;
             }
           }
         }
 #pragma unroll
-        for (int k = 0; k < 2; ++k) {
-          const int t = t0 + k * THREADS + tid;
-          if (t < NT)
+        for (int e = 0; e < 2; ++e) {
+          double v[3];
 #pragma unroll
-            for (int f = 0; f < 6; ++f)
-              fc[2 * (f * NT + t)] = 2.0 / np * sa[k][f], fc[2 * (f * NT + t) + 1] = -2.0 / np * sb[k][f];
-        }
-      }
-      __syncthreads();
-    }
-    for (int f2 = MODE == 3 ? 6 : 0; f2 < 12; f2 += 2) {
-      if (f2 < 6) {
-        const double* fa = fc + 2 * f2 * NT;
-        const double* fb = fa + 2 * NT;
-        for (int t = tid; t < NN; t += THREADS) {
-          const int i = t / N, m = t % N;
-          const double h = m == 0 ? 0.5 : 1.0;
-          const int pk = m * N - m * (m - 1) / 2 - m;  // + n
-          double sa0 = 0.0, sb0 = 0.0, sa1 = 0.0, sb1 = 0.0;
-          #pragma unroll 4
-          for (int n = m; n < N; ++n) {
-            const double p = T.Pc[(i * N + m) * N + n];
-            const int u = pk + n;
-            sa0 += p * fa[2 * u];
-            sb0 += p * fa[2 * u + 1];
-            sa1 += p * fb[2 * u];
-            sb1 += p * fb[2 * u + 1];
-          }
-          tmp[2 * t] = h * sa0, tmp[2 * t + 1] = h * sb0;
-          tmp[2 * (NN + t)] = h * sa1, tmp[2 * (NN + t) + 1] = h * sb1;
-        }
-      } else {
-        // fi 6..8: x_theta, fi 9..11: x_phi of coordinate c, from the coarse shape
-        const int c0 = f2 < 9 ? f2 - 6 : f2 - 9, c1 = f2 + 1 < 9 ? f2 - 5 : f2 - 8;
-        const double* P0 = f2 < 9 ? T.Pcd : T.Pc;
-        const double* P1 = f2 + 1 < 9 ? T.Pcd : T.Pc;
-        for (int t = tid; t < NN; t += THREADS) {
-          const int i = t / N, m = t % N;
-          const double h = m == 0 ? 0.5 : 1.0;
-          const double* Q0 = P0 + (i * N + m) * N;
-          const double* Q1 = P1 + (i * N + m) * N;
-          double sa0 = 0.0, sb0 = 0.0, sa1 = 0.0, sb1 = 0.0;
-          #pragma unroll 4
-          for (int n = m; n < N; ++n) {
-            sa0 += Q0[n] * ca[(c0 * N + m) * N + n];
-            sb0 += Q0[n] * cb[(c0 * N + m) * N + n];
-            sa1 += Q1[n] * ca[(c1 * N + m) * N + n];
-            sb1 += Q1[n] * cb[(c1 * N + m) * N + n];
-          }
-          tmp[2 * t] = h * sa0, tmp[2 * t + 1] = h * sb0;
-          tmp[2 * (NN + t)] = h * sa1, tmp[2 * (NN + t) + 1] = h * sb1;
-        }
-      }
-      __syncthreads();
-      // the 2x-grid longitude DFT partials are dead once f2 >= 6: x_theta / x_phi reuse them.
-      // One thread per node (i, j < np2/2) and its partner j + np2/2, whose factors are the
-      // same up to (-1)^m (phi -> phi + pi).
-      const int hp2 = np2 / 2;
-      for (int t = tid; t < N * hp2; t += THREADS) {
-        const int i = t / hp2, j = t % hp2;
-        double v0 = 0.0, v1 = 0.0, w0 = 0.0, w1 = 0.0;  // v: node j, w: node j + np2/2
-        int q = 0;  // (m j) mod np2
-        #pragma unroll 4
-        for (int m = 0; m < N; ++m) {
-          const double A0 = tmp[2 * (i * N + m)], B0 = tmp[2 * (i * N + m) + 1];
-          const double A1 = tmp[2 * (NN + i * N + m)], B1 = tmp[2 * (NN + i * N + m) + 1];
-          const double cm = tc2[q], sm = ts2[q], sg = (m & 1) ? -1.0 : 1.0;
-          q += j;
-          if (q >= np2) q -= np2;
-          const double t0 = f2 < 9 ? A0 * cm - B0 * sm : (double)m * (-A0 * sm - B0 * cm);
-          const double t1 = f2 + 1 < 9 ? A1 * cm - B1 * sm : (double)m * (-A1 * sm - B1 * cm);
-          v0 += t0, w0 += sg * t0;
-          v1 += t1, w1 += sg * t1;
-        }
-        const double v[4] = {v0, v1, w0, w1};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int fi = f2 + (e & 1);
-          const int node = i * np2 + j + (e >> 1) * hp2;
-          if (fi < 6) {
-            double* dst = fi == 0 ? o0 : fi == 1 ? o1 : fi == 2 ? o2 : fi == 3 ? o3 : fi == 4 ? o4 : o5;
-            dst[(size_t)cap * nc + node] = v[e];
-          } else if (fi < 9) {
-            xt[(size_t)node * 3 + (fi - 6)] = v[e];
+          for (int f = 0; f < 3; ++f) v[f] = e ? s[0][f] - s[1][f] : s[0][f] + s[1][f];
+          const size_t o = (size_t)cap * nc + i * np2 + j + e * hp;
+          if (g == 0) {
+            fx[o] = v[0], fy[o] = v[1], fz[o] = v[2];
           } else {
-            xp[(size_t)node * 3 + (fi - 9)] = v[e];
+            const double r = sqrt(dot3(v, v));
+            nx[o] = v[0] / r, ny[o] = v[1] / r, nz[o] = v[2] / r;
           }
         }
       }
-      __syncthreads();
     }
-    // unit normal (cal_unitO_filter, sph1.f90:1378-1406) and point area
-    // surfmet * w_i / sin(theta_i) * dphi (forcing.f90:91; sph.f90:131)
-    for (int node = tid; node < nc; node += THREADS) {
-      const size_t o = (size_t)cap * nc + node;
-      double cr[3];
-      cross3(xt + (size_t)node * 3, xp + (size_t)node * 3, cr);
-      const double J = sqrt(dot3(cr, cr));
-      if (MODE == 0) {
-        const double a = o3[o], b = o4[o], c = o5[o];
-        const double r = sqrt(a * a + b * b + c * c);
-        o3[o] = a / r, o4[o] = b / r, o5[o] = c / r;
-      } else {
-        // MODE 3: the unit normal of the force grid itself, (x_t x x_p) / |x_t x x_p|
-        o3[o] = cr[0] / J, o4[o] = cr[1] / J, o5[o] = cr[2] / J;
-      }
-      const int i = node / np2;
-      o6[o] = J * T.w2[i] / T.s2[i] * (2.0 * M_PI / np2);
-    }
-    __syncthreads();
   }
 }
+
+// list[0 .. *cnt): the capsules of sel[0 .. n) that are set, in order.  One workgroup.
+constexpr int SL_THREADS = 1024;
+__global__ void __launch_bounds__(SL_THREADS)
+    k_select(int n, const int* __restrict__ sel, long long c0, int* __restrict__ list,
+             int* __restrict__ cnt) {
+  __shared__ int wsum[SL_THREADS / 64];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  int base = 0;
+  for (int b = 0; b < n; b += SL_THREADS) {
+    const bool on = b + tid < n && sel[c0 + b + tid] != 0;
+    const unsigned long long bal = __ballot(on);
+    if (lane == 0) wsum[wv] = __popcll(bal);
+    __syncthreads();
+    int before = 0, total = 0;
+    for (int w = 0; w < SL_THREADS / 64; ++w) {
+      before += w < wv ? wsum[w] : 0;
+      total += wsum[w];
+    }
+    if (on) list[base + before + __popcll(bal & __lanemask_lt())] = (int)(c0 + b + tid);
+    base += total;
+    __syncthreads();
+  }
+  if (tid == 0) *cnt = base;
+}
+
+}  // namespace memb
+
+#include "law_ordered.hpp"
+
+namespace memb {
 
 // ---- host tables ------------------------------------------------------------------------
 void gauss(int n, double* theta, double* w) {
@@ -851,6 +964,17 @@ void legendre_derivs(int nmax, double t, double* D /* [5][nmax][nmax] */) {
   }
 }
 
+// unit-sphere points of the force grid, x block, y block, z block (sph.f90:84-86)
+void sphere(int N, int np2, const double* theta, double* xyz) {
+  for (int i = 0; i < N; ++i)
+    for (int j = 0; j < np2; ++j) {
+      const double ph = 2.0 * M_PI * j / np2;
+      xyz[i * np2 + j] = std::sin(theta[i]) * std::sin(ph);
+      xyz[N * np2 + i * np2 + j] = std::sin(theta[i]) * std::cos(ph);
+      xyz[2 * N * np2 + i * np2 + j] = std::cos(theta[i]);
+    }
+}
+
 }  // namespace memb
 
 using namespace memb;
@@ -862,10 +986,14 @@ struct memb_plan {
   Tables T{};
   std::vector<void*> bufs;  // device allocations of the tables
   double* ref = nullptr;
-  double* scratch = nullptr;
-  size_t scratch_wg = 0;
-  int num_wg = 0;
-  size_t lds = 0;
+  // work of the law: capsule slots with their coefficients and DFT rows, and the list of the
+  // selected capsules of a batch with its length behind it
+  double2* coef = nullptr;
+  double2* rows = nullptr;
+  int* list = nullptr;
+  int slots = 0;
+  int num_wg = 0;  // node workgroups in flight
+  ordered::OrderedTables O{};  // built at the first use of the ordered law
 };
 
 namespace {
@@ -1188,160 +1316,46 @@ __global__ void __launch_bounds__(CS_THREADS)
   }
 }
 
-// Geometry only (unit normal and point area on the force grid) with the arithmetic of
-// k_mem<3> -- analysis of the three coordinates, x_theta and x_phi synthesised from the coarse
-// coefficients, n = (x_t x x_p) / |x_t x x_p|, area = |x_t x x_p| w_i / sin(theta_i) dphi
-// (forcing.f90:91; sph.f90:131) -- laid out for throughput rather than for the law's
-// registers: 256 threads per capsule, the longitude tables staged in LDS once per workgroup,
-// the six (i, m) partial sums of x_theta and x_phi in one pass, and one thread per node for
-// all six node sums, the cross product, the normal and the area.  Persistent over capsules.
-constexpr int GM_THREADS = 256;
-__global__ void __launch_bounds__(GM_THREADS)
-    k_geom(Tables T, long long ncap, const double* __restrict__ x, const double* __restrict__ y,
-           const double* __restrict__ z, double* __restrict__ nx, double* __restrict__ ny,
-           double* __restrict__ nz, double* __restrict__ area, const int* __restrict__ skip) {
-  extern __shared__ double lds[];
-  const int tid = threadIdx.x;
-  const int N = T.N, NN = N * N, np2 = T.np2, nc = N * np2, NT = N * (N + 1) / 2, hp = np2 / 2;
-  // cos / sin(2 pi q / np2), q < np2: the factor cos / sin(m phi_j) is entry (m j) mod np2, and
-  // nodes j and j + np2/2 share their factors up to (-1)^m (phi -> phi + pi)
-  double* tc = lds;
-  double* ts = tc + np2;
-  double* ca = ts + np2;            // [3][N][N]
-  double* cb = ca + 3 * NN;         // [3][N][N]
-  double* tmp = cb + 3 * NN;        // [6][N][N][2]: x_theta (0..2), x_phi (3..5) partial sums
-  double* pts = tmp;                // [3][nc] the capsule's points and
-  double* U = tmp + 3 * nc;         // [3][N][N][2] their longitude DFT, both dead before tmp
-  for (int q = tid; q < np2; q += GM_THREADS) tc[q] = T.cs2[q * N + 1], ts[q] = T.sn2[q * N + 1];
-  for (long long cap = blockIdx.x; cap < ncap; cap += gridDim.x) {
-    if (skip && skip[cap]) continue;  // uniform over the workgroup
-    // the capsule's points into LDS with coalesced loads
-    for (int t = tid; t < 3 * nc; t += GM_THREADS) {
-      const int c = t / nc, q = t - c * nc;
-      pts[t] = (c == 0 ? x : (c == 1 ? y : z))[cap * nc + q];
+// LDS of the three kernels (bytes)
+size_t lds_shape(const Tables& T) {
+  const int NN = T.N * T.N;
+  return (size_t)(T.np2 + 3 * T.NT + 6 * NN) * sizeof(double2);
+}
+size_t lds_nodes(const Tables& T, bool bend) {
+  return (size_t)(T.np + 3 * T.NT + AB_SLOTS * 3 * (bend ? 5 : 3) * T.N) * sizeof(double2) +
+         (size_t)F_SLOTS * T.np * 6 * sizeof(double);
+}
+size_t lds_filter(const Tables& T) {
+  const int NN = T.N * T.N;
+  return (size_t)(T.np2 + 3 * T.NT + std::max(FL_STAGE * 6 * T.N, 3 * NN)) * sizeof(double2);
+}
+
+// The law of ncap capsules (those with sel != 0), in batches of the plan's slots.
+int run_law(memb_plan* p, long long ncap, double gs, double eb, const double* x, const double* y,
+            const double* z, double* fx, double* fy, double* fz, double* nx, double* ny,
+            double* nz, double* area, const int* sel) {
+  const Tables& T = p->T;
+  const int most = p->num_wg;
+  for (long long c0 = 0; c0 < ncap; c0 += p->slots) {
+    const int n = (int)std::min<long long>(p->slots, ncap - c0);
+    Work w{};
+    w.n = n, w.c0 = c0, w.coef = p->coef, w.rows = p->rows;
+    if (sel) {
+      w.list = p->list, w.cnt = p->list + p->slots;
+      k_select<<<1, SL_THREADS, 0, p->stream>>>(n, sel, c0, p->list, p->list + p->slots);
     }
-    __syncthreads();
-    // longitude DFT, one thread per (i, m) for the three coordinates, every point in order
-    // (the raw coordinates are not paired by the phi -> phi + pi symmetry, as in the law)
-    for (int t = tid; t < NN; t += GM_THREADS) {
-      const int i = t / N, m = t % N;
-      double cs[3] = {0.0, 0.0, 0.0}, sn[3] = {0.0, 0.0, 0.0};
-      int q = 0;  // (m j) mod np2
-      #pragma unroll 4
-      for (int j = 0; j < np2; ++j) {
-        const double c = tc[q], s = ts[q];
-        q += m;
-        if (q >= np2) q -= np2;
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-          const double v = pts[k * nc + i * np2 + j];
-          cs[k] += v * c;
-          sn[k] += v * s;
-        }
-      }
-#pragma unroll
-      for (int k = 0; k < 3; ++k) U[2 * (k * NN + t)] = cs[k], U[2 * (k * NN + t) + 1] = sn[k];
-    }
-    __syncthreads();
-    // quadrature, one thread per (m, n >= m) for the three coordinates (n < m is never read)
-    for (int t = tid; t < NT; t += GM_THREADS) {
-      int m = 0, n = t;
-      while (n >= N - m) n -= N - m, ++m;
-      n += m;
-      double sa[3] = {0.0, 0.0, 0.0}, sb[3] = {0.0, 0.0, 0.0};
-      #pragma unroll 4
-      for (int i = 0; i < N; ++i) {
-        const double p = T.w2[i] * T.Pc[(i * N + m) * N + n];
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-          const int u = (k * N + i) * N + m;
-          sa[k] += p * U[2 * u];
-          sb[k] += p * U[2 * u + 1];
-        }
-      }
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        ca[(k * N + m) * N + n] = 2.0 / np2 * sa[k];
-        cb[(k * N + m) * N + n] = -2.0 / np2 * sb[k];
-      }
-    }
-    __syncthreads();
-    // x_theta and x_phi of coordinate c per (c, i, m): both from the same coefficients
-    for (int t = tid; t < 3 * NN; t += GM_THREADS) {
-      const int c = t / NN, u = t % NN, i = u / N, m = u % N;
-      const double h = m == 0 ? 0.5 : 1.0;
-      const double* Pt = T.Pcd + (i * N + m) * N;
-      const double* Pp = T.Pc + (i * N + m) * N;
-      double sa0 = 0.0, sb0 = 0.0, sa1 = 0.0, sb1 = 0.0;
-      #pragma unroll 4
-      for (int n = m; n < N; ++n) {
-        const double a = ca[(c * N + m) * N + n], b = cb[(c * N + m) * N + n];
-        sa0 += Pt[n] * a;
-        sb0 += Pt[n] * b;
-        sa1 += Pp[n] * a;
-        sb1 += Pp[n] * b;
-      }
-      tmp[2 * t] = h * sa0, tmp[2 * t + 1] = h * sb0;
-      tmp[2 * (3 * NN + t)] = h * sa1, tmp[2 * (3 * NN + t) + 1] = h * sb1;
-    }
-    __syncthreads();
-    // node sums, one thread per (i, j < np2/2) and its partner j + np2/2; normal and area
-    for (int t = tid; t < N * hp; t += GM_THREADS) {
-      const int i = t / hp, j = t % hp;
-      double d[2][6];
-#pragma unroll
-      for (int f = 0; f < 6; ++f) d[0][f] = 0.0, d[1][f] = 0.0;
-      int q = 0;  // (m j) mod np2
-      #pragma unroll 2
-      for (int m = 0; m < N; ++m) {
-        const double cm = tc[q], sm = ts[q], sg = (m & 1) ? -1.0 : 1.0;
-        q += j;
-        if (q >= np2) q -= np2;
-#pragma unroll
-        for (int f = 0; f < 6; ++f) {
-          const double A = tmp[2 * (f * NN + i * N + m)], B = tmp[2 * (f * NN + i * N + m) + 1];
-          const double e = f < 3 ? A * cm - B * sm : (double)m * (-A * sm - B * cm);
-          d[0][f] += e;
-          d[1][f] += sg * e;
-        }
-      }
-#pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        double cr[3];
-        cross3(&d[e][0], &d[e][3], cr);
-        const double J = sqrt(dot3(cr, cr));
-        const size_t o = (size_t)cap * nc + i * np2 + j + e * hp;
-        nx[o] = cr[0] / J, ny[o] = cr[1] / J, nz[o] = cr[2] / J;
-        area[o] = J * T.w2[i] / T.s2[i] * (2.0 * M_PI / np2);
-      }
-    }
-    __syncthreads();
+    k_shape<SHAPE_LAW><<<n, SH_THREADS, lds_shape(T), p->stream>>>(
+        T, w, x, y, z, nullptr, nullptr, nullptr, area, nullptr, nullptr);
+    const int gn = (int)std::min<long long>(most, (long long)n * T.nt);
+    if (eb != 0.0)
+      k_nodes<false, true><<<gn, ND_THREADS, lds_nodes(T, true), p->stream>>>(T, w, most, gs, eb,
+                                                                             nullptr);
+    else
+      k_nodes<false, false><<<gn, ND_THREADS, lds_nodes(T, false), p->stream>>>(T, w, most, gs,
+                                                                               eb, nullptr);
+    k_filter<<<2 * n <= most ? 2 * n : n, SH_THREADS, lds_filter(T), p->stream>>>(
+        T, w, most, fx, fy, fz, nx, ny, nz);
   }
-}
-
-size_t geom_lds_bytes(const Tables& T) {
-  const int N = T.N, NN = N * N;
-  // the two longitude tables, the coefficients, and the partial sums (which hold the points
-  // and their longitude DFT before)
-  return (size_t)(2 * T.np2 + 6 * NN + std::max(12 * NN, 3 * N * T.np2 + 6 * NN)) * sizeof(double);
-}
-
-size_t lds_bytes(const Tables& T) {
-  const int N = T.N, NN = N * N;
-  size_t work = std::max<size_t>(3 * NN * 2, (size_t)RING * 3 * 5 * N * 2 + (size_t)RING * T.np * 6);
-  // phase 3: the six fields' packed coefficients and the partial sums of two fields
-  work = std::max<size_t>(work, (size_t)6 * N * (N + 1) + 4 * NN);
-  return (6 * NN + 2 * (T.np + T.np2) + work) * sizeof(double);
-}
-
-template <int MODE>
-int launch(memb_plan* p, long long ncap, double gs, double eb, const double* x, const double* y,
-           const double* z, double* o0, double* o1, double* o2, double* o3, double* o4,
-           double* o5, double* o6, const int* sel = nullptr) {
-  const int nwg = (int)std::min<long long>(ncap, p->num_wg);
-  if (nwg <= 0) return MEMB_OK;
-  k_mem<MODE><<<nwg, THREADS, p->lds, p->stream>>>(p->T, ncap, gs, eb, x, y, z, o0, o1, o2, o3,
-                                                   o4, o5, o6, p->scratch, sel);
   MCHK(p, hipGetLastError());
   return MEMB_OK;
 }
@@ -1365,89 +1379,91 @@ int memb_plan_create(memb_plan** out, int L, int device) {
   p->stream = p->own;
   Tables& T = p->T;
   T.L = L, T.N = L + 1, T.np2 = 2 * (L + 1), T.nt = 2 * T.N, T.np = 2 * T.np2;
-  const int N = T.N, nt = T.nt, np = T.np, np2 = T.np2;
+  T.NT = T.N * (T.N + 1) / 2;
+  const int N = T.N, nt = T.nt, np = T.np, np2 = T.np2, NT = T.NT, nh = (N + 1) / 2;
   std::vector<double> th2(N), w2(N), th(nt), w(nt), s2(N);
   gauss(N, th2.data(), w2.data());
   gauss(nt, th.data(), w.data());
   for (int i = 0; i < N; ++i) s2[i] = std::sin(th2[i]);
-  std::vector<double> Pc((size_t)N * N * N), Pcd((size_t)N * N * N), Pfd((size_t)nt * 5 * N * N),
-      Pfa((size_t)nt * N * N), D(5 * N * N);
+  std::vector<double> WPc((size_t)N * NT), Pc((size_t)nh * NT), Pcd((size_t)nh * NT),
+      Pfd((size_t)N * 5 * NT), WPf((size_t)N * NT), D(5 * N * N);
+  auto each = [&](auto&& f) {  // f(packed index, index into D's [m][n])
+    for (int d = 0; d < N; ++d)
+      for (int m = 0; m < N - d; ++m) f(tidx(N, d, m), m * N + m + d);
+  };
   for (int i = 0; i < N; ++i) {
     legendre_derivs(N, th2[i], D.data());
-    std::copy(D.begin(), D.begin() + N * N, Pc.begin() + (size_t)i * N * N);
-    std::copy(D.begin() + N * N, D.begin() + 2 * N * N, Pcd.begin() + (size_t)i * N * N);
+    each([&](int t, int q) {
+      WPc[(size_t)i * NT + t] = w2[i] * D[q];
+      if (i < nh) Pc[(size_t)i * NT + t] = D[q], Pcd[(size_t)i * NT + t] = D[N * N + q];
+    });
+    legendre_derivs(N, th[i], D.data());  // the northern half of the doubled grid
+    each([&](int t, int q) {
+      for (int k = 0; k < 5; ++k) Pfd[((size_t)i * 5 + k) * NT + t] = D[k * N * N + q];
+      WPf[(size_t)i * NT + t] = w[i] * D[q];
+    });
   }
-  for (int i = 0; i < nt; ++i) {
-    legendre_derivs(N, th[i], D.data());
-    std::copy(D.begin(), D.end(), Pfd.begin() + (size_t)i * 5 * N * N);
-    std::copy(D.begin(), D.begin() + N * N, Pfa.begin() + (size_t)i * N * N);
-  }
-  std::vector<double> cs2((size_t)np2 * N), sn2((size_t)np2 * N), csf((size_t)np * N),
-      snf((size_t)np * N);
-  // cos / sin(m phi_j) with the angle reduced first, 2 pi ((m j) mod n) / n, as the longitude
-  // FFT's twiddle factors are formed (hrfft.f:214-267): exact to the last bit of cos / sin
-  // of an angle below 2 pi, where m phi_j itself (up to 2 pi L) carries 1e-14 of rounding
-  // that the fourth phi derivatives multiply by m^4
-  for (int j = 0; j < np2; ++j)
-    for (int m = 0; m < N; ++m) {
-      const double ph = 2.0 * M_PI * ((m * j) % np2) / np2;
-      cs2[j * N + m] = std::cos(ph), sn2[j * N + m] = std::sin(ph);
+  // cos / sin(m phi_j) is entry (m j) mod n of cos / sin(2 pi q / n): the angle is reduced first,
+  // as the longitude FFT's twiddle factors are formed (hrfft.f:214-267): exact to the last bit
+  // of cos / sin of an angle below 2 pi, where m phi_j itself (up to 2 pi L) carries 1e-14 of
+  // rounding that the fourth phi derivatives multiply by m^4
+  auto unit = [](int n) {
+    std::vector<double> e(2 * (size_t)n);
+    for (int q = 0; q < n; ++q) {
+      const double a = 2.0 * M_PI * q / n;
+      e[2 * q] = std::cos(a), e[2 * q + 1] = std::sin(a);
     }
-  for (int j = 0; j < np; ++j)
-    for (int m = 0; m < N; ++m) {
-      const double ph = 2.0 * M_PI * ((m * j) % np) / np;
-      csf[j * N + m] = std::cos(ph), snf[j * N + m] = std::sin(ph);
-    }
-  if ((rc = upload(p, w2, &T.w2)) || (rc = upload(p, w, &T.w)) || (rc = upload(p, s2, &T.s2)) ||
+    return e;
+  };
+  const double *e2 = nullptr, *ef = nullptr;
+  if ((rc = upload(p, w2, &T.w2)) || (rc = upload(p, s2, &T.s2)) || (rc = upload(p, WPc, &T.WPc)) ||
       (rc = upload(p, Pc, &T.Pc)) || (rc = upload(p, Pcd, &T.Pcd)) ||
-      (rc = upload(p, Pfd, &T.Pfd)) || (rc = upload(p, Pfa, &T.Pfa)) ||
-      (rc = upload(p, cs2, &T.cs2)) || (rc = upload(p, sn2, &T.sn2)) ||
-      (rc = upload(p, csf, &T.csf)) || (rc = upload(p, snf, &T.snf)))
+      (rc = upload(p, Pfd, &T.Pfd)) || (rc = upload(p, WPf, &T.WPf)) ||
+      (rc = upload(p, unit(np2), &e2)) || (rc = upload(p, unit(np), &ef)))
     return bail(rc);
-  p->lds = lds_bytes(T);
+  T.e2 = reinterpret_cast<const double2*>(e2), T.ef = reinterpret_cast<const double2*>(ef);
   int cus = 256;
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device);
-  p->num_wg = 4 * cus;  // four capsule workgroups per CU (LDS and the register cap allow it)
-  // per workgroup: longitude DFT of the 2x-grid outputs, and the force-grid basis vectors
-  p->scratch_wg = std::max<size_t>((size_t)nt * 6 * N * 2, (size_t)N * np2 * 6);
-  void* s = nullptr;
-  if (hipMalloc(&s, p->scratch_wg * p->num_wg * sizeof(double)) != hipSuccess)
-    return bail(fail(p, MEMB_E_HIP, "hipMalloc scratch failed"));
-  p->bufs.push_back(s);
-  p->scratch = (double*)s;
-  // the reference state: the unit sphere through the same kernel (sph.f90:56-70, 152-161)
-  void* r = nullptr;
-  if (hipMalloc(&r, (size_t)nt * np * NREF * sizeof(double)) != hipSuccess)
-    return bail(fail(p, MEMB_E_HIP, "hipMalloc reference state failed"));
-  p->bufs.push_back(r);
-  p->ref = (double*)r;
+  p->num_wg = 4 * cus;  // node workgroups in flight: four per CU (LDS and registers allow it)
+  p->slots = 8 * cus;   // capsules per batch: two full rounds of them
+  auto alloc = [&](auto** d, size_t bytes) {
+    void* q = nullptr;
+    if (hipMalloc(&q, bytes) != hipSuccess) return false;
+    p->bufs.push_back(q);
+    *d = reinterpret_cast<std::remove_reference_t<decltype(**d)>*>(q);
+    return true;
+  };
+  if (!alloc(&p->coef, (size_t)p->slots * 3 * NT * sizeof(double2)) ||
+      !alloc(&p->rows, (size_t)p->slots * nt * N * 6 * sizeof(double2)) ||
+      !alloc(&p->list, (size_t)(p->slots + 1) * sizeof(int)) ||
+      !alloc(&p->ref, (size_t)NREF * nt * np * sizeof(double)))
+    return bail(fail(p, MEMB_E_HIP, "hipMalloc of the plan's work arrays failed"));
+  // the reference state: the unit sphere through the same kernels (sph.f90:56-70, 152-161)
   std::vector<double> sx((size_t)N * np2 * 3);
-  for (int i = 0; i < N; ++i)
-    for (int j = 0; j < np2; ++j) {
-      const double ph = 2.0 * M_PI * j / np2;
-      sx[i * np2 + j] = std::sin(th2[i]) * std::sin(ph);
-      sx[N * np2 + i * np2 + j] = std::sin(th2[i]) * std::cos(ph);
-      sx[2 * N * np2 + i * np2 + j] = std::cos(th2[i]);
-    }
+  sphere(N, np2, th2.data(), sx.data());
   const double* dsx = nullptr;
   if ((rc = upload(p, sx, &dsx))) return bail(rc);
-  T.ref = nullptr;
-  // scratch stride is per workgroup; one capsule uses workgroup 0's region
-  if (hipFuncSetAttribute((const void*)k_mem<0>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                          (int)p->lds) != hipSuccess ||
-      hipFuncSetAttribute((const void*)k_mem<1>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                          (int)p->lds) != hipSuccess ||
-      hipFuncSetAttribute((const void*)k_mem<2>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                          (int)p->lds) != hipSuccess ||
-      hipFuncSetAttribute((const void*)k_mem<3>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                          (int)p->lds) != hipSuccess ||
-      hipFuncSetAttribute((const void*)k_geom, hipFuncAttributeMaxDynamicSharedMemorySize,
-                          (int)geom_lds_bytes(p->T)) != hipSuccess)
+  auto big = [&](const void* f, size_t lds) {
+    return hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
+  };
+  if (!big((const void*)k_shape<SHAPE_LAW>, lds_shape(T)) ||
+      !big((const void*)k_shape<SHAPE_COEFFS>, lds_shape(T)) ||
+      !big((const void*)k_shape<SHAPE_GEOM>, lds_shape(T)) ||
+      !big((const void*)k_shape<SHAPE_REF>, lds_shape(T)) ||
+      !big((const void*)k_nodes<true, true>, lds_nodes(T, true)) ||
+      !big((const void*)k_nodes<false, true>, lds_nodes(T, true)) ||
+      !big((const void*)k_nodes<false, false>, lds_nodes(T, false)) ||
+      !big((const void*)k_filter, lds_filter(T)))
     return bail(fail(p, MEMB_E_HIP, "hipFuncSetAttribute failed"));
-  if ((rc = launch<1>(p, 1, 0.0, 0.0, dsx, dsx + N * np2, dsx + 2 * N * np2, p->ref, nullptr,
-                      nullptr, nullptr, nullptr, nullptr, nullptr)))
-    return bail(rc);
-  if (hipStreamSynchronize(p->stream) != hipSuccess)
+  T.ref = nullptr;
+  Work wk{};
+  wk.n = 1, wk.coef = p->coef, wk.rows = p->rows;
+  k_shape<SHAPE_REF><<<1, SH_THREADS, lds_shape(T), p->stream>>>(
+      T, wk, dsx, dsx + N * np2, dsx + 2 * N * np2, nullptr, nullptr, nullptr, nullptr, nullptr,
+      nullptr);
+  k_nodes<true, true><<<nt, ND_THREADS, lds_nodes(T, true), p->stream>>>(T, wk, nt, 0.0, 0.0,
+                                                                        p->ref);
+  if (hipGetLastError() != hipSuccess || hipStreamSynchronize(p->stream) != hipSuccess)
     return bail(fail(p, MEMB_E_HIP, "reference state failed"));
   T.ref = p->ref;
   *out = p;
@@ -1490,7 +1506,77 @@ int memb_traction_f64_dev(memb_plan* p, int64_t ncap, double gs, double eb, cons
   if (ncap > 0 && !(x && y && z && fx && fy && fz && nx && ny && nz && area))
     return fail(p, MEMB_E_ARG, "null pointer");
   MCHK(p, hipSetDevice(p->device));
-  return launch<0>(p, ncap, gs, eb, x, y, z, fx, fy, fz, nx, ny, nz, area);
+  return run_law(p, ncap, gs, eb, x, y, z, fx, fy, fz, nx, ny, nz, area, nullptr);
+}
+
+// Tables and reference state of the ordered node phase, once per plan (waits).
+static int ordered_tables(memb_plan* p) {
+  if (p->O.ref) return MEMB_OK;
+  const Tables& T = p->T;
+  const int N = T.N, nt = T.nt, NT = T.NT, np2 = T.np2;
+  std::vector<double> th(nt), w(nt), th2(N), w2(N), D(5 * N * N), Pfd((size_t)nt * 5 * NT);
+  gauss(nt, th.data(), w.data());
+  gauss(N, th2.data(), w2.data());
+  for (int i = 0; i < nt; ++i) {
+    legendre_derivs(N, th[i], D.data());
+    for (int k = 0; k < 5; ++k)
+      for (int d = 0; d < N; ++d)
+        for (int m = 0; m < N - d; ++m)
+          Pfd[((size_t)i * 5 + k) * NT + tidx(N, d, m)] = D[(k * N + m) * N + m + d];
+  }
+  int rc;
+  if ((rc = upload(p, Pfd, &p->O.Pfd))) return rc;
+  std::vector<double> sx((size_t)N * np2 * 3);
+  sphere(N, np2, th2.data(), sx.data());
+  const double* dsx = nullptr;
+  if ((rc = upload(p, sx, &dsx))) return rc;
+  void* ref = nullptr;
+  MCHK(p, hipMalloc(&ref, (size_t)nt * T.np * ordered::NREF * sizeof(double)));
+  p->bufs.push_back(ref);
+  const int lds = (int)ordered::lds_bytes(T);
+  MCHK(p, hipFuncSetAttribute((const void*)ordered::k_nodes_ordered<true>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+  MCHK(p, hipFuncSetAttribute((const void*)ordered::k_nodes_ordered<false>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+  Work wk{};
+  wk.n = 1, wk.coef = p->coef, wk.rows = p->rows;
+  k_shape<SHAPE_REF><<<1, SH_THREADS, lds_shape(T), p->stream>>>(
+      T, wk, dsx, dsx + N * np2, dsx + 2 * N * np2, nullptr, nullptr, nullptr, nullptr, nullptr,
+      nullptr);
+  ordered::k_nodes_ordered<true><<<1, ordered::THREADS, lds, p->stream>>>(T, p->O, wk, 0.0, 0.0,
+                                                                         (double*)ref);
+  MCHK(p, hipGetLastError());
+  MCHK(p, hipStreamSynchronize(p->stream));
+  p->O.ref = (const double*)ref;
+  return MEMB_OK;
+}
+
+int memb_traction_ordered_f64_dev(memb_plan* p, int64_t ncap, double gs, double eb,
+                                  const double* x, const double* y, const double* z, double* fx,
+                                  double* fy, double* fz, double* nx, double* ny, double* nz,
+                                  double* area) {
+  if (!p) return MEMB_E_ARG;
+  if (!p->T.ref) return fail(p, MEMB_E_STATE, "plan not initialised");
+  if (ncap < 0) return fail(p, MEMB_E_ARG, "ncap < 0");
+  if (ncap > 0 && !(x && y && z && fx && fy && fz && nx && ny && nz && area))
+    return fail(p, MEMB_E_ARG, "null pointer");
+  MCHK(p, hipSetDevice(p->device));
+  int rc = ordered_tables(p);
+  if (rc) return rc;
+  const Tables& T = p->T;
+  for (long long c0 = 0; c0 < ncap; c0 += p->slots) {
+    const int n = (int)std::min<long long>(p->slots, ncap - c0);
+    Work w{};
+    w.n = n, w.c0 = c0, w.coef = p->coef, w.rows = p->rows;
+    k_shape<SHAPE_LAW><<<n, SH_THREADS, lds_shape(T), p->stream>>>(
+        T, w, x, y, z, nullptr, nullptr, nullptr, area, nullptr, nullptr);
+    ordered::k_nodes_ordered<false><<<n, ordered::THREADS, ordered::lds_bytes(T), p->stream>>>(
+        T, p->O, w, gs, eb, nullptr);
+    k_filter<<<2 * n <= p->num_wg ? 2 * n : n, SH_THREADS, lds_filter(T), p->stream>>>(
+        T, w, p->num_wg, fx, fy, fz, nx, ny, nz);
+  }
+  MCHK(p, hipGetLastError());
+  return MEMB_OK;
 }
 
 int memb_coeffs_f64_dev(memb_plan* p, int64_t ncap, const double* x, const double* y,
@@ -1499,8 +1585,16 @@ int memb_coeffs_f64_dev(memb_plan* p, int64_t ncap, const double* x, const doubl
   if (ncap < 0) return fail(p, MEMB_E_ARG, "ncap < 0");
   if (ncap > 0 && !(x && y && z && coef)) return fail(p, MEMB_E_ARG, "null pointer");
   MCHK(p, hipSetDevice(p->device));
-  return launch<2>(p, ncap, 0.0, 0.0, x, y, z, coef, nullptr, nullptr, nullptr, nullptr, nullptr,
-                   nullptr);
+  if (ncap == 0) return MEMB_OK;
+  // (uses no slot: it may run beside the law on another stream)
+  Work w{};
+  w.n = (int)std::min<long long>(ncap, INT_MAX);
+  if (ncap > w.n) return fail(p, MEMB_E_ARG, "more than 2^31 - 1 capsules");
+  k_shape<SHAPE_COEFFS><<<(unsigned)std::min<long long>(ncap, p->num_wg), SH_THREADS,
+                          lds_shape(p->T), p->stream>>>(p->T, w, x, y, z, nullptr, nullptr,
+                                                        nullptr, nullptr, coef, nullptr);
+  MCHK(p, hipGetLastError());
+  return MEMB_OK;
 }
 
 int memb_geometry_f64_dev(memb_plan* p, int64_t ncap, const double* x, const double* y,
@@ -1512,10 +1606,13 @@ int memb_geometry_f64_dev(memb_plan* p, int64_t ncap, const double* x, const dou
     return fail(p, MEMB_E_ARG, "null pointer");
   MCHK(p, hipSetDevice(p->device));
   if (ncap == 0) return MEMB_OK;
-  // three 256-thread workgroups per CU (LDS: 3 x 42 KB at L = 16)
-  const unsigned nwg = (unsigned)std::min<long long>(ncap, (long long)p->num_wg * 3 / 4);
-  k_geom<<<nwg, GM_THREADS, geom_lds_bytes(p->T), p->stream>>>(p->T, ncap, x, y, z, nx, ny, nz,
-                                                               area, skip);
+  // (uses no slot: it may run beside the law on another stream)
+  Work w{};
+  w.n = (int)std::min<long long>(ncap, INT_MAX);
+  if (ncap > w.n) return fail(p, MEMB_E_ARG, "more than 2^31 - 1 capsules");
+  k_shape<SHAPE_GEOM><<<(unsigned)std::min<long long>(ncap, p->num_wg), SH_THREADS,
+                        lds_shape(p->T), p->stream>>>(p->T, w, x, y, z, nx, ny, nz, area, nullptr,
+                                                      skip);
   MCHK(p, hipGetLastError());
   return MEMB_OK;
 }
@@ -1530,7 +1627,7 @@ int memb_traction_select_f64_dev(memb_plan* p, int64_t ncap, const int* sel, dou
   if (ncap > 0 && !(sel && x && y && z && fx && fy && fz && nx && ny && nz && area))
     return fail(p, MEMB_E_ARG, "null pointer");
   MCHK(p, hipSetDevice(p->device));
-  return launch<0>(p, ncap, gs, eb, x, y, z, fx, fy, fz, nx, ny, nz, area, sel);
+  return run_law(p, ncap, gs, eb, x, y, z, fx, fy, fz, nx, ny, nz, area, sel);
 }
 
 int memb_corot_f64_dev(memb_plan* p, int64_t ncap, const double* X, const double* x,

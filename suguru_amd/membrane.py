@@ -56,6 +56,14 @@ class MembranePlan:
             self.h, ncap, float(gs), float(eb), _ptr(x), _ptr(y), _ptr(z), _ptr(fx), _ptr(fy),
             _ptr(fz), _ptr(nx), _ptr(ny), _ptr(nz), _ptr(area)))
 
+    def traction_ordered_dev(self, x, y, z, gs, eb, fx, fy, fz, nx, ny, nz, area):
+        """The law in the oracle's order of operations (memb_traction_ordered_f64_dev), for
+        finite differences; the first call on a plan waits."""
+        ncap = x.numel() // self.npts
+        self._check(self.lib.memb_traction_ordered_f64_dev(
+            self.h, ncap, float(gs), float(eb), _ptr(x), _ptr(y), _ptr(z), _ptr(fx), _ptr(fy),
+            _ptr(fz), _ptr(nx), _ptr(ny), _ptr(nz), _ptr(area)))
+
     def coeffs_dev(self, x, y, z, coef):
         ncap = x.numel() // self.npts
         self._check(self.lib.memb_coeffs_f64_dev(self.h, ncap, _ptr(x), _ptr(y), _ptr(z),

@@ -184,13 +184,15 @@ class Surrogate:
     def upload(self, a):
         return self.torch.from_numpy(np.ascontiguousarray(a, dtype=np.float64).reshape(-1)).to(self.dev)
 
-    def law(self, x, y, z):
-        """FP64 law on device point arrays [ncap * npts]: (f [3, n], normal [3, n], area [n])."""
+    def law(self, x, y, z, ordered=False):
+        """FP64 law on device point arrays [ncap * npts]: (f [3, n], normal [3, n], area [n]).
+        ordered: in the oracle's order of operations, for differences of the law."""
         t = self.torch
         n = x.numel()
         with self._streamed():
             out = [t.empty(n, dtype=t.float64, device=self.dev) for _ in range(7)]
-            self.plan.traction_dev(x, y, z, self.gs, self.eb, *out)
+            fn = self.plan.traction_ordered_dev if ordered else self.plan.traction_dev
+            fn(x, y, z, self.gs, self.eb, *out)
             res = t.stack(out[:3]), t.stack(out[3:6]), out[6]
         return res
 
@@ -208,7 +210,9 @@ class Surrogate:
 
     def build_jacobian(self, h=1e-6):
         """J = d f / d x at the unit sphere (FP64, [3 npts, 3 npts], x block, y block, z block),
-        by central differences of the GPU law: one batch of 2 x 3 npts perturbed spheres."""
+        by central differences of the GPU law: one batch of 2 x 3 npts perturbed spheres.  The
+        differences see the law's rounding, so it is evaluated in one fixed order of
+        operations: J agrees with the one of a surrogate saved earlier."""
         t = self.torch
         n, m = self.npts, self.dout
         with self._streamed():
@@ -218,7 +222,7 @@ class Surrogate:
             for sgn in (1.0, -1.0):
                 P = base + sgn * eye                   # capsule i: coordinate i moved by +-h
                 x, y, z = (P[:, k * n:(k + 1) * n].contiguous().view(-1) for k in range(3))
-                f, _, _ = self.law(x, y, z)
+                f, _, _ = self.law(x, y, z, ordered=True)
                 cols.append(f.view(3, m, n).permute(1, 0, 2).reshape(m, m))  # [capsule][3 n]
             J = ((cols[0] - cols[1]) / (2 * h)).T      # column i = d f / d x_i
             self.JT = J.T.contiguous()
