@@ -138,18 +138,29 @@ struct FillSrc {
   long long sy, sz;
 };
 
+// The arrays of one launch: workgroup row blockIdx.y transforms src[y] into dst[y].  The three
+// momentum solves share their launches: at 64^3 cells a launch is 5 us of latency whatever it
+// holds (26 launches -> 15; with fewer planes per momentum workgroup as well, a step there takes
+// 104 us instead of 211; 512 x 512 x 250 cells 8.09 instead of 8.27 ms, from the eliminations).
+struct Arrays {
+  const double* src[3];
+  double* dst[3];
+};
+
 // Forward: real lines -> packed half spectra.  XMAJOR: element index fastest across threads
 // (x lines); otherwise line index fastest (y lines).  src and dst may be the same array (the
 // workgroup reads all of its lines before the first barrier and writes them after the last).
 // FILL (x lines of a compact array only): the lines are fillps's divergence (fs), not src.
 template <bool XMAJOR, bool FILL = false>
 __global__ void __launch_bounds__(FFT_THREADS)
-    k_rfft_fwd(const double* src, double* dst, int N, int logm,
+    k_rfft_fwd(Arrays arr, int N, int logm,
                int nl, int groups_per_plane, long long plane_src, long long plane_dst,
                long long gstride_src, long long gstride_dst, long long es_src, long long ls_src,
                long long es_dst, long long ls_dst, long long off_src,
                const double2* __restrict__ tw, FillSrc fs) {
   extern __shared__ double2 sm[];
+  const double* src = arr.src[blockIdx.y];
+  double* dst = arr.dst[blockIdx.y];
   const int M = N >> 1, logn = logm + 1, lognl = 31 - __clz(nl);
   const int blk = xcd_logical_block<XMAJOR>();
   const int kp = blk / groups_per_plane, gp = blk - kp * groups_per_plane;
@@ -214,12 +225,14 @@ __global__ void __launch_bounds__(FFT_THREADS)
 // Inverse: packed half spectra -> real lines (scaled by 1/M here, 1/2 in the split).
 template <bool XMAJOR>
 __global__ void __launch_bounds__(FFT_THREADS)
-    k_rfft_inv(const double* src, double* dst, int N, int logm,
+    k_rfft_inv(Arrays arr, int N, int logm,
                int nl, int groups_per_plane, long long plane_src, long long plane_dst,
                long long gstride_src, long long gstride_dst, long long es_src, long long ls_src,
                long long es_dst, long long ls_dst, long long off_dst,
                const double2* __restrict__ tw) {
   extern __shared__ double2 sm[];
+  const double* src = arr.src[blockIdx.y];
+  double* dst = arr.dst[blockIdx.y];
   const int M = N >> 1, logn = logm + 1, lognl = 31 - __clz(nl);
   const int blk = xcd_logical_block<XMAJOR>();
   const int kp = blk / groups_per_plane, gp = blk - kp * groups_per_plane;
@@ -310,9 +323,20 @@ __global__ void __launch_bounds__(256) k_ztab(int nkx, int nky, int ktot, int ne
 // One lane per (i, j) mode of the compact spectral array, the forward sweep's values stored
 // back into the array and read again by the back substitution (the path above 257 planes;
 // k_tri_seg below takes every smaller grid in one pass).
+// The systems of one launch: workgroup row blockIdx.y solves array p[y] with its coefficients.
+struct Systems {
+  double* p[3];
+  const double* a[3];
+  const double* c[3];
+  const double* ztab[3];
+};
+
 __global__ void __launch_bounds__(TRI_MODES)
-    k_tri(double* __restrict__ p, int itot, int jtot, int ktot, const double* __restrict__ a,
-          const double* __restrict__ c, const double* __restrict__ ztab) {
+    k_tri(Systems sys, int itot, int jtot, int ktot) {
+  double* __restrict__ p = sys.p[blockIdx.y];
+  const double* __restrict__ a = sys.a[blockIdx.y];
+  const double* __restrict__ c = sys.c[blockIdx.y];
+  const double* __restrict__ ztab = sys.ztab[blockIdx.y];
   const long long plane = (long long)itot * jtot;
   const long long m = (long long)blockIdx.x * TRI_MODES + threadIdx.x;
   if (m >= plane) return;
@@ -351,8 +375,11 @@ __global__ void __launch_bounds__(TRI_MODES)
 constexpr int TRS_LSEG = 16;                   // rows per segment (registers per lane: 2 x 16)
 constexpr int TRS_MAXSEG = 16;                 // segments (wavefronts) per workgroup
 __global__ void __launch_bounds__(TRI_MODES * TRS_MAXSEG)
-    k_tri_seg(double* __restrict__ p, int itot, int jtot, int ktot, const double* __restrict__ a,
-              const double* __restrict__ c, const double* __restrict__ ztab) {
+    k_tri_seg(Systems sys, int itot, int jtot, int ktot) {
+  double* __restrict__ p = sys.p[blockIdx.y];
+  const double* __restrict__ a = sys.a[blockIdx.y];
+  const double* __restrict__ c = sys.c[blockIdx.y];
+  const double* __restrict__ ztab = sys.ztab[blockIdx.y];
   __shared__ double fy0[TRS_MAXSEG][TRI_MODES], fg[TRS_MAXSEG][TRI_MODES];
   __shared__ double bx0[TRS_MAXSEG][TRI_MODES], bh[TRS_MAXSEG][TRI_MODES];
   __shared__ double xlast[TRI_MODES];
@@ -375,7 +402,15 @@ __global__ void __launch_bounds__(TRI_MODES * TRS_MAXSEG)
   // (selects, so that the arrays stay in registers)
   // (every load is in bounds: lanes past the last mode read mode 0, then discard it)
   const long long mm = live ? m : 0;
-  double r[TRS_LSEG], z[TRS_LSEG];
+  // (a and c of the segment's rows first: uniform over the wavefront and before any store, they
+  // are scalar loads)
+  double r[TRS_LSEG], z[TRS_LSEG], ak[TRS_LSEG], ck[TRS_LSEG];
+#pragma unroll
+  for (int t = 0; t < TRS_LSEG; ++t) {
+    const int k = k0 + min(t, max(n - 1, 0));
+    ak[t] = a[k], ck[t] = c[k];
+  }
+  const double alast = a[ktot - 1];
 #pragma unroll
   for (int t = 0; t < TRS_LSEG; ++t) {
     const int k = k0 + min(t, max(n - 1, 0));
@@ -388,9 +423,8 @@ __global__ void __launch_bounds__(TRI_MODES * TRS_MAXSEG)
     double y = 0.0, gm = 1.0;
 #pragma unroll
     for (int t = 0; t < TRS_LSEG; ++t) {
-      const double ak = a[k0 + min(t, max(n - 1, 0))];
-      const double yn = (r[t] - ak * y) * z[t];
-      const double gn = gm * (-(ak * z[t]));
+      const double yn = (r[t] - ak[t] * y) * z[t];
+      const double gn = gm * (-(ak[t] * z[t]));
       y = t < n ? yn : y;
       gm = t < n ? gn : gm;
     }
@@ -403,7 +437,7 @@ __global__ void __launch_bounds__(TRI_MODES * TRS_MAXSEG)
   double prev = yin;
 #pragma unroll
   for (int t = 0; t < TRS_LSEG; ++t) {
-    const double yn = (r[t] - a[k0 + min(t, max(n - 1, 0))] * prev) * z[t];
+    const double yn = (r[t] - ak[t] * prev) * z[t];
     prev = t < n ? yn : prev;
     r[t] = prev;
   }
@@ -412,7 +446,7 @@ __global__ void __launch_bounds__(TRI_MODES * TRS_MAXSEG)
     double nxt = 0.0;
     if (live) {
       const double zl = ztab[(long long)(ktot - 1) * zs + zb];
-      nxt = zl != 0.0 ? (p[(long long)(ktot - 1) * plane + m] - a[ktot - 1] * prev) / zl : 0.0;
+      nxt = zl != 0.0 ? (p[(long long)(ktot - 1) * plane + m] - alast * prev) / zl : 0.0;
       p[(long long)(ktot - 1) * plane + m] = nxt;
     }
     xlast[lane] = nxt;
@@ -422,7 +456,7 @@ __global__ void __launch_bounds__(TRI_MODES * TRS_MAXSEG)
     double x = 0.0, hm = 1.0;
 #pragma unroll
     for (int t = TRS_LSEG - 1; t >= 0; --t) {
-      const double d = c[k0 + min(t, max(n - 1, 0))] * z[t];
+      const double d = ck[t] * z[t];
       const double xn = r[t] - d * x;
       const double hn = hm * (-d);
       x = t < n ? xn : x;
@@ -437,7 +471,7 @@ __global__ void __launch_bounds__(TRI_MODES * TRS_MAXSEG)
   double nxt = xin;
 #pragma unroll
   for (int t = TRS_LSEG - 1; t >= 0; --t) {
-    const double d = c[k0 + min(t, max(n - 1, 0))] * z[t];
+    const double d = ck[t] * z[t];
     const double xn = r[t] - d * nxt;
     nxt = t < n ? xn : nxt;
     r[t] = nxt;
@@ -550,18 +584,18 @@ __device__ __forceinline__ void mom_cell(const FGrid& g, double rep, double dt, 
 }
 
 // fftuvw.f90:30-105 per interior cell, k-marching, into the compact arrays: a workgroup owns
-// an MR_TI x MR_TJ tile of (i, j) columns and MR_KB consecutive planes.  The six velocity fields' planes k-1, k, k+1 of the tile plus a
+// an MR_TI x MR_TJ tile of (i, j) columns and KB consecutive planes.  The six velocity fields' planes k-1, k, k+1 of the tile plus a
 // one-cell apron sit in an LDS ring of three; each step prefetches plane k+2 into registers
 // while it computes plane k, then stores it over plane k-1.  Every velocity value is read
 // from HBM once per tile (plus the apron and the two extra planes); p and the forces are read
 // directly.
-constexpr int MR_TI = 32, MR_TJ = 8, MR_KB = 32;
+constexpr int MR_TI = 32, MR_TJ = 8;
 constexpr int MR_W = MR_TI + 2, MR_H = MR_TJ + 2, MR_PL = MR_W * MR_H;
 constexpr int MR_T = MR_TI * MR_TJ;
 constexpr int MR_LD = (MR_PL + MR_T - 1) / MR_T;  // apron-plane cells per thread
 
 __global__ void __launch_bounds__(MR_T)
-    k_mom_rhs_march(FGrid g, double rep, double dt, const double* __restrict__ uo,
+    k_mom_rhs_march(FGrid g, int KB, double rep, double dt, const double* __restrict__ uo,
                     const double* __restrict__ vo, const double* __restrict__ wo,
                     const double* __restrict__ uoo, const double* __restrict__ voo,
                     const double* __restrict__ woo, const double* __restrict__ p,
@@ -572,8 +606,8 @@ __global__ void __launch_bounds__(MR_T)
   const double* src[6] = {uo, vo, wo, uoo, voo, woo};
   const int tx = threadIdx.x % MR_TI, ty = threadIdx.x / MR_TI;
   const int i0 = blockIdx.x * MR_TI, j0 = blockIdx.y * MR_TJ;  // apron origin (halo index)
-  const int kb0 = blockIdx.z * MR_KB + 1;
-  const int kb1 = min(kb0 + MR_KB - 1, g.ktot);
+  const int kb0 = blockIdx.z * KB + 1;
+  const int kb1 = min(kb0 + KB - 1, g.ktot);
   // the apron-plane cells this thread loads: c = tid + r MR_T
   long long off[MR_LD];
   bool ok[MR_LD];
@@ -730,9 +764,11 @@ __device__ __forceinline__ double kstep(const FGrid& g, const double* f, int kin
 // jtot) take an interior column (its ghost planes k = 0 and ktot+1, and k = ktot for w); the
 // rest one cell of a halo column: x halos i = 0, itot+1 for j = 0..jtot+1, then y halos
 // j = 0, jtot+1 for i = 1..itot, every k (halo index fastest).
-__global__ void __launch_bounds__(256) k_bound(FGrid g, double* __restrict__ f0,
-                                               double* __restrict__ f1, double* __restrict__ f2,
-                                               int nfields, int kind0) {
+// kinds: the field kinds of kstep, four bits each.
+struct Fields {
+  double* f[4];
+};
+__global__ void __launch_bounds__(256) k_bound(FGrid g, Fields fs, int nfields, unsigned kinds) {
   const long long nin = (long long)g.itot * g.jtot;
   const long long nxh = 2LL * (g.jtot + 2), nh = nxh + 2LL * g.itot, K = g.ktot + 2;
   const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -740,8 +776,8 @@ __global__ void __launch_bounds__(256) k_bound(FGrid g, double* __restrict__ f0,
     const int fi = (int)(t / nin);
     const long long r = t - fi * nin;
     const int i = 1 + (int)(r % g.itot), j = 1 + (int)(r / g.itot);
-    double* f = fi == 0 ? f0 : (fi == 1 ? f1 : f2);
-    const int kind = kind0 == 2 ? 2 : (fi == 2 ? 1 : 0);
+    double* f = fs.f[fi];
+    const int kind = (kinds >> (4 * fi)) & 15;
     f[fidx(g, i, j, 0)] = kstep(g, f, kind, i, j, 0);
     f[fidx(g, i, j, g.ktot + 1)] = kstep(g, f, kind, i, j, g.ktot + 1);
     if (kind == 1) f[fidx(g, i, j, g.ktot)] = 0.0;
@@ -762,8 +798,8 @@ __global__ void __launch_bounds__(256) k_bound(FGrid g, double* __restrict__ f0,
     j = hy < g.itot ? 0 : g.jtot + 1;
     i = 1 + (int)(hy % g.itot);
   }
-  double* f = fi == 0 ? f0 : (fi == 1 ? f1 : f2);
-  const int kind = kind0 == 2 ? 2 : (fi == 2 ? 1 : 0);
+  double* f = fs.f[fi];
+  const int kind = (kinds >> (4 * fi)) & 15;
   const int si = i == 0 ? g.itot : (i == g.itot + 1 ? 1 : i);
   const int sj = j == 0 ? g.jtot : (j == g.jtot + 1 ? 1 : j);
   f[fidx(g, i, j, k)] = kstep(g, f, kind, si, sj, k);
@@ -884,6 +920,7 @@ struct fld_ctx {
   FGrid g{};
   double rep = 0, dt = 0;
   int device = 0;
+  int cus = 256;
   hipStream_t own = nullptr, stream = nullptr;
   std::string err;
   long long ncomp = 0;                  // itot * jtot * ktot
@@ -980,8 +1017,8 @@ void tridiag(const fld_ctx* c, int e, std::vector<double>& a, std::vector<double
   }
 }
 
-// x transform of the interior lines of a field (or of a compact array), forward or inverse
-int fft_x(fld_ctx* c, bool inv, const double* src, bool src_field, double* dst, bool dst_field) {
+// x transforms of the interior lines of n fields (or compact arrays), forward or inverse
+int fft_x(fld_ctx* c, bool inv, int n, const Arrays& arr, bool src_field, bool dst_field) {
   const FGrid& g = c->g;
   const int N = g.itot, nl = c->xlines;
   const int gpp = g.jtot / nl;  // workgroups per k plane
@@ -991,67 +1028,74 @@ int fft_x(fld_ctx* c, bool inv, const double* src, bool src_field, double* dst, 
   const long long off = 1 + g.sy + g.sz;  // (1, 1, 1)
   // lines, plus the inverse's LDS copy of the twiddles
   const size_t lds = (size_t)nl * (N / 2 + 1) * sizeof(double2) + (inv ? (size_t)(N / 2) * sizeof(double2) : 0);
-  const unsigned nb = (unsigned)(gpp * g.ktot);
+  const dim3 nb((unsigned)(gpp * g.ktot), (unsigned)n);
   if (!inv)
     k_rfft_fwd<true><<<nb, FFT_THREADS, lds, c->stream>>>(
-        src, dst, N, c->logmx, nl, gpp, plane_s, plane_d, nl * row_s, nl * row_d, 1, row_s, 1,
-        row_d, src_field ? off : 0, c->tw_x, FillSrc{});
+        arr, N, c->logmx, nl, gpp, plane_s, plane_d, nl * row_s, nl * row_d, 1, row_s, 1, row_d,
+        src_field ? off : 0, c->tw_x, FillSrc{});
   else
     k_rfft_inv<true><<<nb, FFT_THREADS, lds, c->stream>>>(
-        src, dst, N, c->logmx, nl, gpp, plane_s, plane_d, nl * row_s, nl * row_d, 1, row_s, 1,
-        row_d, dst_field ? off : 0, c->tw_x);
+        arr, N, c->logmx, nl, gpp, plane_s, plane_d, nl * row_s, nl * row_d, 1, row_s, 1, row_d,
+        dst_field ? off : 0, c->tw_x);
   HIPF(c, hipGetLastError());
   return FLD_OK;
 }
 
-// y transform in place on a compact array
-int fft_y(fld_ctx* c, bool inv, double* a) {
+// y transforms in place on n compact arrays
+int fft_y(fld_ctx* c, bool inv, int n, double* const* a) {
   const FGrid& g = c->g;
   const int N = g.jtot, nl = inv ? c->ylines_i : c->ylines_f;
   const int gpp = g.itot / nl;
   const long long cp = (long long)g.itot * g.jtot;
-  const unsigned nb = (unsigned)(gpp * g.ktot);
+  const dim3 nb((unsigned)(gpp * g.ktot), (unsigned)n);
+  Arrays arr{};
+  for (int i = 0; i < n; ++i) arr.src[i] = arr.dst[i] = a[i];
   if (!inv)
     k_rfft_fwd<false><<<nb, FFT_THREADS, c->lds_yf, c->stream>>>(
-        a, a, N, c->logmy, nl, gpp, cp, cp, nl, nl, g.itot, 1, g.itot, 1, 0, c->tw_y, FillSrc{});
+        arr, N, c->logmy, nl, gpp, cp, cp, nl, nl, g.itot, 1, g.itot, 1, 0, c->tw_y, FillSrc{});
   else
     k_rfft_inv<false><<<nb, FFT_THREADS, c->lds_yi, c->stream>>>(
-        a, a, N, c->logmy, nl, gpp, cp, cp, nl, nl, g.itot, 1, g.itot, 1, 0, c->tw_y);
+        arr, N, c->logmy, nl, gpp, cp, cp, nl, nl, g.itot, 1, g.itot, 1, 0, c->tw_y);
   HIPF(c, hipGetLastError());
   return FLD_OK;
 }
 
-int tri(fld_ctx* c, double* a, int ne) {
+int tri(fld_ctx* c, int n, double* const* a, const int* ne) {
   const FGrid& g = c->g;
   const long long modes = (long long)g.itot * g.jtot;
-  const double* ac = c->coef[ne];
-  const double* cc = c->coef[ne] + g.ktot;
+  Systems sys{};
+  for (int i = 0; i < n; ++i)
+    sys.p[i] = a[i], sys.a[i] = c->coef[ne[i]], sys.c[i] = c->coef[ne[i]] + g.ktot,
+    sys.ztab[i] = c->ztab[ne[i]];
   const int nseg = std::max(1, (g.ktot - 1 + TRS_LSEG - 1) / TRS_LSEG);
+  const dim3 nb(nblocks(modes, TRI_MODES), (unsigned)n);
   if (nseg <= TRS_MAXSEG)
-    k_tri_seg<<<nblocks(modes, TRI_MODES), TRI_MODES * nseg, 0, c->stream>>>(
-        a, g.itot, g.jtot, g.ktot, ac, cc, c->ztab[ne]);
+    k_tri_seg<<<nb, TRI_MODES * nseg, 0, c->stream>>>(sys, g.itot, g.jtot, g.ktot);
   else
-    k_tri<<<nblocks(modes, TRI_MODES), TRI_MODES, 0, c->stream>>>(a, g.itot, g.jtot, g.ktot, ac,
-                                                                  cc, c->ztab[ne]);
+    k_tri<<<nb, TRI_MODES, 0, c->stream>>>(sys, g.itot, g.jtot, g.ktot);
   HIPF(c, hipGetLastError());
   return FLD_OK;
 }
 
-// solver1d after the forward x transform: y transform, eliminations, inverses into the
-// interior of `out`
-int solve_after_x(fld_ctx* c, double* a, int ne, double* out) {
+// n solver1d after the forward x transforms: y transforms, eliminations, inverses into the
+// interiors of `out`
+int solve_after_x(fld_ctx* c, int n, double* const* a, const int* ne, double* const* out) {
+  Arrays arr{};
+  for (int i = 0; i < n; ++i) arr.src[i] = a[i], arr.dst[i] = out[i];
   int rc;
-  if ((rc = fft_y(c, false, a)) || (rc = tri(c, a, ne)) || (rc = fft_y(c, true, a)) ||
-      (rc = fft_x(c, true, a, false, out, true)))
+  if ((rc = fft_y(c, false, n, a)) || (rc = tri(c, n, a, ne)) || (rc = fft_y(c, true, n, a)) ||
+      (rc = fft_x(c, true, n, arr, false, true)))
     return rc;
   return FLD_OK;
 }
 
-// solver1d on a compact right-hand side, result into the interior of `out`
-int solve_compact(fld_ctx* c, double* a, int ne, double* out) {
+// n solver1d on compact right-hand sides, results into the interiors of `out`
+int solve_compact(fld_ctx* c, int n, double* const* a, const int* ne, double* const* out) {
+  Arrays arr{};
+  for (int i = 0; i < n; ++i) arr.src[i] = arr.dst[i] = a[i];
   int rc;
-  if ((rc = fft_x(c, false, a, false, a, false))) return rc;
-  return solve_after_x(c, a, ne, out);
+  if ((rc = fft_x(c, false, n, arr, false, false))) return rc;
+  return solve_after_x(c, n, a, ne, out);
 }
 
 // fillps (the divergence of u, v, w over dt) already transformed in x, into the compact
@@ -1066,17 +1110,19 @@ int fft_x_fill(fld_ctx* c, const double* u, const double* v, const double* w, do
   const double dti = 1.0 / c->dt;
   const FillSrc fs{u, v, w, dti * g.dxi, dti * g.dyi, dti * g.dzi, g.sy, g.sz};
   k_rfft_fwd<true, true><<<nb, FFT_THREADS, lds, c->stream>>>(
-      nullptr, dst, N, c->logmx, nl, gpp, cp, cp, nl * row, nl * row, 1, row, 1, row, 0, c->tw_x,
-      fs);
+      Arrays{{nullptr, nullptr, nullptr}, {dst, nullptr, nullptr}}, N, c->logmx, nl, gpp, cp, cp,
+      nl * row, nl * row, 1, row, 1, row, 0, c->tw_x, fs);
   HIPF(c, hipGetLastError());
   return FLD_OK;
 }
 
-int bound(fld_ctx* c, double* f0, double* f1, double* f2, int nfields, int kind0) {
+// halos and wall ghosts of nfields fields; kinds: kstep's kind of each, four bits
+constexpr unsigned KIND_UVW = 0x100, KIND_P = 0x2, KIND_UVWP = 0x2100;
+int bound(fld_ctx* c, const Fields& fs, int nfields, unsigned kinds) {
   const FGrid& g = c->g;
   const long long n = ((long long)g.itot * g.jtot +
                        (2LL * (g.jtot + 2) + 2LL * g.itot) * (g.ktot + 2)) * nfields;
-  k_bound<<<nblocks(n, 256), 256, 0, c->stream>>>(g, f0, f1, f2, nfields, kind0);
+  k_bound<<<nblocks(n, 256), 256, 0, c->stream>>>(g, fs, nfields, kinds);
   HIPF(c, hipGetLastError());
   return FLD_OK;
 }
@@ -1123,6 +1169,7 @@ int fld_create(fld_ctx** out, const ibx_grid* gr, double rep, double dt, int dev
     return code;
   };
   if (hipSetDevice(device) != hipSuccess) return bail(FLD_E_HIP, "device");
+  (void)hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, device);
   if (hipStreamCreateWithFlags(&c->own, hipStreamNonBlocking) != hipSuccess)
     return bail(FLD_E_HIP, "stream");
   c->stream = c->own;
@@ -1218,12 +1265,11 @@ int fld_solver1d_dev(fld_ctx* c, double* p, int ne) {
   if (!p) return fail(c, FLD_E_ARG, "null field");
   if (ne < 1 || ne > 3) return fail(c, FLD_E_ARG, "ne must be 1, 2 or 3");
   HIPF(c, hipSetDevice(c->device));
-  int rc = fft_x(c, false, p, true, c->work[0], false);
+  Arrays arr{};
+  arr.src[0] = p, arr.dst[0] = c->work[0];
+  int rc = fft_x(c, false, 1, arr, true, false);
   if (rc) return rc;
-  if ((rc = fft_y(c, false, c->work[0])) || (rc = tri(c, c->work[0], ne)) ||
-      (rc = fft_y(c, true, c->work[0])) || (rc = fft_x(c, true, c->work[0], false, p, true)))
-    return rc;
-  return FLD_OK;
+  return solve_after_x(c, 1, c->work, &ne, &p);
 }
 
 int fld_fftuvw_dev(fld_ctx* c, double* unew, double* vnew, double* wnew, const double* uo,
@@ -1234,32 +1280,35 @@ int fld_fftuvw_dev(fld_ctx* c, double* unew, double* vnew, double* wnew, const d
   if (!(unew && vnew && wnew && uo && vo && wo && uoo && voo && woo && pnew && fx && fy && fz))
     return fail(c, FLD_E_ARG, "null field");
   HIPF(c, hipSetDevice(c->device));
-  const dim3 mgrid((unsigned)((c->grid.itot + MR_TI - 1) / MR_TI),
-                   (unsigned)((c->grid.jtot + MR_TJ - 1) / MR_TJ),
-                   (unsigned)((c->grid.ktot + MR_KB - 1) / MR_KB));
-  k_mom_rhs_march<<<mgrid, MR_T, 0, c->stream>>>(c->g, c->rep, c->dt, uo, vo, wo, uoo, voo, woo,
-                                                 pnew, fx, fy, fz, c->work[0], c->work[1],
+  // planes per workgroup: 32 (two extra planes read per 32) while that gives a workgroup for each
+  // of the two the LDS lets a compute unit hold, fewer on smaller grids, where the march along k
+  // is a serial chain of plane loads (64^3 cells: 66 us with 32 planes, 32 workgroups)
+  const unsigned ti = (unsigned)((c->grid.itot + MR_TI - 1) / MR_TI);
+  const unsigned tj = (unsigned)((c->grid.jtot + MR_TJ - 1) / MR_TJ);
+  int kb = 32;
+  while (kb > 2 && (long long)ti * tj * ((c->grid.ktot + kb - 1) / kb) < 2LL * c->cus) kb >>= 1;
+  const dim3 mgrid(ti, tj, (unsigned)((c->grid.ktot + kb - 1) / kb));
+  k_mom_rhs_march<<<mgrid, MR_T, 0, c->stream>>>(c->g, kb, c->rep, c->dt, uo, vo, wo, uoo, voo,
+                                                 woo, pnew, fx, fy, fz, c->work[0], c->work[1],
                                                  c->work[2]);
   HIPF(c, hipGetLastError());
-  int rc;
-  if ((rc = solve_compact(c, c->work[2], 3, wnew)) || (rc = solve_compact(c, c->work[0], 2, unew)) ||
-      (rc = solve_compact(c, c->work[1], 2, vnew)))
-    return rc;
-  return FLD_OK;
+  const int ne[3] = {2, 2, 3};
+  double* const out[3] = {unew, vnew, wnew};
+  return solve_compact(c, 3, c->work, ne, out);
 }
 
 int fld_bounduvw_dev(fld_ctx* c, double* u, double* v, double* w) {
   if (!c) return FLD_E_ARG;
   if (!(u && v && w)) return fail(c, FLD_E_ARG, "null field");
   HIPF(c, hipSetDevice(c->device));
-  return bound(c, u, v, w, 3, 0);
+  return bound(c, Fields{{u, v, w, nullptr}}, 3, KIND_UVW);
 }
 
 int fld_boundp_dev(fld_ctx* c, double* p) {
   if (!c) return FLD_E_ARG;
   if (!p) return fail(c, FLD_E_ARG, "null field");
   HIPF(c, hipSetDevice(c->device));
-  return bound(c, p, nullptr, nullptr, 1, 2);
+  return bound(c, Fields{{p, nullptr, nullptr, nullptr}}, 1, KIND_P);
 }
 
 int fld_fillps_dev(fld_ctx* c, const double* u, const double* v, const double* w, double* p) {
@@ -1289,17 +1338,18 @@ int fld_step_dev(fld_ctx* c, double* unew, double* vnew, double* wnew, double* p
   if (!(pnew && p)) return fail(c, FLD_E_ARG, "null field");
   int rc = fld_fftuvw_dev(c, unew, vnew, wnew, uo, vo, wo, uoo, voo, woo, pnew, fx, fy, fz);
   if (rc) return rc;
-  if ((rc = bound(c, unew, vnew, wnew, 3, 0))) return rc;
+  const int ne = 1;
+  if ((rc = bound(c, Fields{{unew, vnew, wnew, nullptr}}, 3, KIND_UVW))) return rc;
   if ((rc = fft_x_fill(c, unew, vnew, wnew, c->work[0])) ||
-      (rc = solve_after_x(c, c->work[0], 1, p)) || (rc = bound(c, p, nullptr, nullptr, 1, 2)))
+      (rc = solve_after_x(c, 1, c->work, &ne, &p)) ||
+      (rc = bound(c, Fields{{p, nullptr, nullptr, nullptr}}, 1, KIND_P)))
     return rc;
   // correc and pnew += p fused (the reference's bounduvw between them reads neither p nor
   // pnew), then bounduvw and boundp(pnew)
   k_correc_addp<<<nblocks(c->ncomp, 256), 256, 0, c->stream>>>(c->g, c->dt, unew, vnew, wnew, p,
                                                                pnew);
   HIPF(c, hipGetLastError());
-  if ((rc = bound(c, unew, vnew, wnew, 3, 0))) return rc;
-  return bound(c, pnew, nullptr, nullptr, 1, 2);
+  return bound(c, Fields{{unew, vnew, wnew, pnew}}, 4, KIND_UVWP);
 }
 
 int fld_indicator_div_dev(fld_ctx* c, const double* gx, const double* gy, const double* gz,
@@ -1316,15 +1366,15 @@ static int ind_finish(fld_ctx* c, double* indi, double* indic, double* visc, dou
                       double* forcez, double lambda, double visc0, double sin_t, double cos_t,
                       double tcoef) {
   int rc;
-  if ((rc = bound(c, indi, nullptr, nullptr, 1, 2))) return rc;  // boundind(indi)
+  if ((rc = bound(c, Fields{{indi, nullptr, nullptr, nullptr}}, 1, KIND_P))) return rc;  // boundind(indi)
   k_ind_shift<<<nblocks(c->ncomp, 256), 256, 0, c->stream>>>(c->g, indi, indic);
   HIPF(c, hipGetLastError());
-  if ((rc = bound(c, indic, nullptr, nullptr, 1, 2))) return rc;  // boundind(indic)
+  if ((rc = bound(c, Fields{{indic, nullptr, nullptr, nullptr}}, 1, KIND_P))) return rc;  // boundind(indic)
   k_ind_finish<<<nblocks(c->ncomp, 256), 256, 0, c->stream>>>(c->g, indic, visc, forcey, forcez,
                                                               lambda, visc0, sin_t, -cos_t,
                                                               tcoef);
   HIPF(c, hipGetLastError());
-  return bound(c, visc, nullptr, nullptr, 1, 2);  // boundp(visc)
+  return bound(c, Fields{{visc, nullptr, nullptr, nullptr}}, 1, KIND_P);  // boundp(visc)
 }
 
 static bool ind_args_ok(double lambda, double visc0, double sin_t, double cos_t, double tcoef) {
@@ -1356,7 +1406,8 @@ int fld_indicator_dev(fld_ctx* c, const double* gx, const double* gy, const doub
   // solver1d(indi, 0) are the pressure solve, ne = 1), solution into the interior of indi
   k_ind_div<<<nblocks(c->ncomp, 256), 256, 0, c->stream>>>(c->g, gx, gy, gz, c->work[0], nullptr);
   HIPF(c, hipGetLastError());
-  int rc = solve_compact(c, c->work[0], 1, indi);
+  const int ne = 1;
+  int rc = solve_compact(c, 1, c->work, &ne, &indi);
   if (rc) return rc;
   return ind_finish(c, indi, indic, visc, forcey, forcez, lambda, visc0, sin_t, cos_t, tcoef);
 }
