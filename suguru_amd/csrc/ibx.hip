@@ -244,7 +244,32 @@ struct ObjBufs {
   unsigned* cover;           // coverage bitmap, 1 bit per cell
   int* meta;                 // OB_META queue counters
   long long icap;            // item capacity
+  ObjLimit lim;              // item extent
 };
+
+// Items of a launch: 2048 cells where there are enough of them to fill the chip, fewer where a
+// capsule or a few would otherwise leave it idle: an item is one workgroup's chain over its
+// candidates, so that smaller items end sooner, while candidates near an item's faces are prepared
+// once for each item they reach.  The line lies at the items that 2048 cells would give,
+// estimated from the points per capsule (about one per h^2 of surface).  Spread + interpolation
+// with items of 2048 / 1024 / 512 / 256 cells: 1 capsule of radius 8h (4 items of 2048) 107 / 96 /
+// 91 / 83 us; radius 10.6h: 4 capsules (32) 156 / 132 / 117 / 105, 16 (127) 162 / 130 / 118 / 129,
+// 30 (240) 171 / 138 / 144 / -, 60 (480) 181 / 160 / 177 / -, 1000 (7900) 1108 / 1306 / 1725 / -.
+// times: the most items one of 2048 cells can turn into.
+struct ObjChoice {
+  ObjLimit lim;
+  int times;
+};
+ObjChoice obj_choice(long long ncap, long long npts) {
+  if (ncap > 0 && ncap <= 256 && npts > 0) {
+    const double edge = 2.0 * std::sqrt((double)npts / (double)ncap / (4.0 * M_PI)) + 4.0;
+    const double est = (double)ncap * std::max(1.0, edge * edge * edge / 2048.0);
+    if (est <= 64) return {{16, 256}, 16};
+    if (est <= 160) return {{16, 512}, 8};
+    if (est <= 600) return {{16, 1024}, 4};
+  }
+  return {{OB_BX, OB_NC}, 1};
+}
 
 // Sizes (bytes) of the object-spread work buffers for ncap capsules on the context's grid;
 // items are sized separately (ObjSizes::per_item bytes per item of capacity).
@@ -278,9 +303,11 @@ ObjSizes obj_sizes(const ibx_ctx* c, long long ncap) {
 }
 
 // The allocating path: context-owned buffers, grown on demand.
-int obj_bufs_alloc(ibx_ctx* c, long long ncap, ObjBufs& ob) {
+int obj_bufs_alloc(ibx_ctx* c, long long ncap, long long npts, ObjBufs& ob) {
   const ObjSizes z = obj_sizes(c, ncap);
-  const long long icap = z.icap_want;
+  const ObjChoice ch = obj_choice(ncap, npts);
+  const long long icap = z.icap_want * ch.times;
+  ob.lim = ch.lim;
   int rc;
   if ((rc = ensure(c, c->oboxes, z.boxes)) || (rc = ensure(c, c->onbm, z.nbm)) ||
       (rc = ensure(c, c->ocnt, z.cnt)) || (rc = ensure(c, c->obinm, z.binm)) ||
@@ -302,7 +329,7 @@ int obj_bufs_alloc(ibx_ctx* c, long long ncap, ObjBufs& ob) {
 // The no-allocation path: the same buffers carved out of this device's fixed work array, each
 // aligned to 256 bytes.  The item capacity is what the array has left (at most the allocating
 // path's); a call that needs more items than that reports IBX_E_CAPACITY at the next ibx_sync.
-int obj_bufs_scratch(ibx_ctx* c, long long ncap, ObjBufs& ob) {
+int obj_bufs_scratch(ibx_ctx* c, long long ncap, long long npts, ObjBufs& ob) {
   if (!c->scratch) return fail(c, IBX_E_STATE, "no work array address for this device");
   const ObjSizes z = obj_sizes(c, ncap);
   auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
@@ -316,7 +343,11 @@ int obj_bufs_scratch(ibx_ctx* c, long long ncap, ObjBufs& ob) {
                     " MiB of work buffers, more than the fixed " +
                     std::to_string(kScratchBytes >> 20) + " MiB array");
   const long long fit = (long long)((kScratchBytes - fixed - 3 * 256) / ObjSizes::per_item);
-  const long long icap = std::min<long long>(z.icap_want, fit);
+  // small items only where the array holds all that the larger ones could turn into
+  ObjChoice ch = obj_choice(ncap, npts);
+  if (fit < z.icap_want * ch.times) ch = {{OB_BX, OB_NC}, 1};
+  const long long icap = std::min<long long>(z.icap_want * ch.times, fit);
+  ob.lim = ch.lim;
   unsigned char* p = (unsigned char*)c->scratch;
   auto take = [&](size_t b) {
     unsigned char* q = p;
@@ -343,32 +374,37 @@ int enqueue_spread_obj(ibx_ctx* c, const TileCfg& cf, bool cc, long long ncap,
                        const long long* d_off, long long npts, const double* x,
                        const double* y, const double* z, const double* f1, const double* f2,
                        const double* f3, const double* area, double* o1, double* o2, double* o3,
-                       const ObjBufs& ob, hipEvent_t ev_tile, hipEvent_t ev_tile_end,
-                       hipEvent_t ev_split, hipEvent_t ev_before) {
+                       const ObjBufs& ob, bool check, hipEvent_t ev_tile,
+                       hipEvent_t ev_tile_end, hipEvent_t ev_split, hipEvent_t ev_before) {
   if (npts >= OB_MAXPTS) return fail(c, IBX_E_ARG, "object spread: more than 2^27 points");
   const int klo = cc ? 0 : 1, khi = cc ? c->grid.ktot + 1 : c->grid.ktot;
   const long long ncells = c->gd.sz * (long long)(c->grid.ktot + 2);
   const ObjSizes zs = obj_sizes(c, ncap);
   const long long nw = zs.nw, nbw = zs.nbw, icap = ob.icap;
   const int nwd = zs.nwd;
+  const ObjLimit lim = ob.lim;
   int* meta = ob.meta;
   unsigned* cover = ob.cover;
-  k_obj_clear<<<blocks_for(std::max<long long>(std::max(nw, nbw), OB_META), 256), 256, 0,
-                c->stream>>>(nw, cover, nbw, ob.binm, meta);
+  const bool chk = check && ncap > 0;
+  k_obj_clear<<<blocks_for(std::max({nw, nbw, (long long)OB_META, chk ? ncap : 0}), 256), 256, 0,
+                c->stream>>>(nw, cover, nbw, ob.binm, meta, ncap, chk ? d_off : nullptr, npts,
+                             c->d_err);
   if (npts > 0 && ncap > 0) {
     k_obj_boxes<<<(unsigned)ncap, 256, 0, c->stream>>>(
-        c->gd, klo, khi, d_off, x, y, z, ob.boxes, ob.cnt,
+        c->gd, klo, khi, lim, d_off, x, y, z, ob.boxes, ob.cnt,
         nwd, ob.binm, c->d_err);
-    k_obj_scan<<<1, 1024, 0, c->stream>>>(ncap, ob.cnt, ob.off,
-                                          (int)icap, meta, c->d_err);
-    k_obj_items<<<(unsigned)ncap, 256, 0, c->stream>>>(
-        c->gd, ncap, nwd, ob.boxes, ob.binm,
-        ob.off, ob.items, (int)icap, cover,
-        ob.nbm, c->d_err);
-    k_obj_sources<<<(unsigned)(c->num_cus * 4), 256, 0, c->stream>>>(
-        nwd, ob.boxes, ob.nbm,
-        ob.items, (int)icap, ob.src, ob.nsrc, meta,
-        c->d_err);
+#define ITEM_ARGS                                                                              \
+  c->gd, lim, ncap, nwd, ob.boxes, ob.binm, ob.off, ob.cnt, ob.items, (int)icap, cover, ob.nbm, \
+      ob.src, ob.nsrc, meta, c->d_err
+    if (ncap <= OB_FUSE) {
+      k_obj_items<true><<<(unsigned)ncap, 256, 0, c->stream>>>(ITEM_ARGS);
+    } else {
+      k_obj_scan<<<1, 1024, 0, c->stream>>>(ncap, ob.cnt, ob.off, (int)icap, meta, c->d_err);
+      k_obj_items<false><<<(unsigned)ncap, 256, 0, c->stream>>>(ITEM_ARGS);
+      k_obj_sources<<<(unsigned)(c->num_cus * 4), 256, 0, c->stream>>>(
+          nwd, ob.boxes, ob.nbm, ob.items, (int)icap, ob.src, ob.nsrc, meta, c->d_err);
+    }
+#undef ITEM_ARGS
   }
   // another stream's work (the interpolation) joins here, before the persistent kernel
   // takes every compute unit
@@ -409,17 +445,18 @@ int enqueue_spread_obj(ibx_ctx* c, const TileCfg& cf, bool cc, long long ncap,
 int enqueue_spread(ibx_ctx* c, int cfgid, bool cc, long long ncap, const long long* d_off,
                    long long npts, const double* x, const double* y, const double* z,
                    const double* f1, const double* f2, const double* f3, const double* area,
-                   double* o1, double* o2, double* o3, bool size_entries,
+                   double* o1, double* o2, double* o3, bool size_entries, bool check = false,
                    hipEvent_t ev_tile = nullptr, hipEvent_t ev_split = nullptr,
                    hipEvent_t ev_tile_end = nullptr, hipEvent_t ev_before = nullptr) {
   const TileCfg& cf = kCfgs[cfgid];
   if (cf.obj) {
     ObjBufs ob;
-    int rc = obj_bufs_alloc(c, ncap, ob);
+    int rc = obj_bufs_alloc(c, ncap, npts, ob);
     if (rc) return rc;
     return enqueue_spread_obj(c, cf, cc, ncap, d_off, npts, x, y, z, f1, f2, f3, area, o1, o2,
-                              o3, ob, ev_tile, ev_tile_end, ev_split, ev_before);
+                              o3, ob, check, ev_tile, ev_tile_end, ev_split, ev_before);
   }
+  if (check && ncap > 0) k_check_off<<<1, 256, 0, c->stream>>>(ncap, d_off, npts, c->d_err);
   TileGeom tg = geom(c->grid, cf, cc);
   int rc;
   if ((rc = ensure(c, c->tcount, (size_t)tg.ntiles * sizeof(unsigned)))) return rc;
@@ -737,10 +774,8 @@ static int spread_dev(ibx_ctx* c, bool cc, int64_t ncap, const int64_t* cap_off,
   if (rc) return rc;
   HIPCHK(c, hipSetDevice(c->device));
   // the offset table lives in HBM: checked on the device before anything indexes through it
-  if (ncap > 0)
-    k_check_off<<<1, 256, 0, c->stream>>>(ncap, (const long long*)cap_off, npts, c->d_err);
   return enqueue_spread(c, c->cfg, cc, ncap, (const long long*)cap_off, npts, x, y, z, f1, f2,
-                        f3, area, o1, o2, o3, true);
+                        f3, area, o1, o2, o3, true, true);
 }
 
 int ibx_spread_f64_dev(ibx_ctx* c, int64_t ncap, const int64_t* cap_off, int64_t npts,
@@ -761,16 +796,14 @@ int ibx_spread_f64_dev_noalloc(ibx_ctx* c, int64_t ncap, const int64_t* cap_off,
                            forcez);
   if (rc) return rc;
   ObjBufs ob;
-  if ((rc = obj_bufs_scratch(c, ncap, ob))) return rc;
+  if ((rc = obj_bufs_scratch(c, ncap, npts, ob))) return rc;
   HIPCHK(c, hipSetDevice(c->device));
-  if (ncap > 0)
-    k_check_off<<<1, 256, 0, c->stream>>>(ncap, (const long long*)cap_off, npts, c->d_err);
   // the context's configuration when it is an object one, else the default object one (the
   // tile spread sizes its candidate list per call)
   const int cfg = kCfgs[c->cfg].obj ? c->cfg : kDefaultCfg;
   return enqueue_spread_obj(c, kCfgs[cfg], false, ncap, (const long long*)cap_off, npts, x, y,
-                            z, fx, fy, fz, area, forcex, forcey, forcez, ob, nullptr, nullptr,
-                            nullptr, nullptr);
+                            z, fx, fy, fz, area, forcex, forcey, forcez, ob, true, nullptr,
+                            nullptr, nullptr, nullptr);
 }
 
 int ibx_spread_cc_f64_dev(ibx_ctx* c, int64_t ncap, const int64_t* cap_off, int64_t npts,
@@ -1018,7 +1051,7 @@ static int batch_enqueue(ibx_batch* b, bool size_entries, const hipEvent_t* ev =
   }
   rc = enqueue_spread(c, b->cfg, false, b->ncap, (const long long*)b->d_off.p, b->npts, q.x,
                       q.y, q.z, q.fx, q.fy, q.fz, q.area, q.forcex, q.forcey, q.forcez,
-                      size_entries, ev ? ev[2] : nullptr, nullptr, ev ? ev[3] : nullptr,
+                      size_entries, false, ev ? ev[2] : nullptr, nullptr, ev ? ev[3] : nullptr,
                       ov ? c->ev_join : nullptr);
   if (rc) return rc;
   if (ov) HIPCHK(c, hipStreamWaitEvent(c->stream, c->ev_join, 0));  // (already joined)
@@ -1191,7 +1224,7 @@ int ibx_batch_profile(ibx_batch* b, int reps, double* us) {
       HIPCHK(c, hipEventRecord(ev[1], c->stream));
       rc = enqueue_spread(c, b->cfg, false, b->ncap, (const long long*)b->d_off.p, b->npts, q.x,
                           q.y, q.z, q.fx, q.fy, q.fz, q.area, q.forcex, q.forcey, q.forcez,
-                          false, ev[2], pass == 1 ? ev[4] : nullptr);
+                          false, false, ev[2], pass == 1 ? ev[4] : nullptr);
       if (rc) return rc;
       HIPCHK(c, hipEventRecord(ev[3], c->stream));
       HIPCHK(c, hipEventSynchronize(ev[3]));

@@ -932,26 +932,38 @@ constexpr int OB_META = OB_QSTRIDE * 9;
 // boxes: [nobj][6] clamped window bounds xa, xb, ya, yb, za, zb of object o = 9 p + nb
 // (xa > xb: no candidate)
 
-// the coverage bitmap (bit = linear cell index), the bin masks and the counters
+// the coverage bitmap (bit = linear cell index), the bin masks and the counters; and, with
+// `off`, k_check_off's check of the device-held offset table in the same launch
 __global__ void __launch_bounds__(256) k_obj_clear(long long nw, unsigned* __restrict__ cover,
                                                    long long nbw,
                                                    unsigned long long* __restrict__ binm,
-                                                   int* __restrict__ meta) {
+                                                   int* __restrict__ meta, long long ncap,
+                                                   const long long* __restrict__ off,
+                                                   long long npts, int* __restrict__ err) {
   const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (off && q < ncap) {
+    const long long a = off[q], b = off[q + 1];
+    if (b < a || (q == 0 && a != 0) || (q == ncap - 1 && b != npts)) atomicOr(err, ERR_OFFSETS);
+  }
   if (q < nw) cover[q] = 0u;
   if (q < nbw) binm[q] = 0ull;
   if (q < OB_META) meta[q] = 0;
 }
 
+// Extent of the items of a launch: at most bx cells in x and y and nc cells.
+struct ObjLimit {
+  int bx, nc;
+};
+
 // Item grid of one object box: cx x cy x cz sub-boxes of extent nx x ny x nz (the last ones
-// cut short), at most OB_BX x OB_BX x OB_NZ and OB_NC cells each.
+// cut short), within the launch's limit and OB_NZ planes each.
 struct ObjGrid {
   int cx, cy, cz, nx, ny, nz;
-  __device__ explicit ObjGrid(const int* b) {
+  __device__ explicit ObjGrid(const int* b, ObjLimit l) {
     const int X = b[1] - b[0] + 1, Y = b[3] - b[2] + 1, Z = b[5] - b[4] + 1;
-    cx = (X + OB_BX - 1) / OB_BX, cy = (Y + OB_BX - 1) / OB_BX;
+    cx = (X + l.bx - 1) / l.bx, cy = (Y + l.bx - 1) / l.bx;
     nx = (X + cx - 1) / cx, ny = (Y + cy - 1) / cy;
-    nz = max(1, min(min(Z, OB_NZ), OB_NC / (nx * ny)));
+    nz = max(1, min(min(Z, OB_NZ), l.nc / (nx * ny)));
     cz = (Z + nz - 1) / nz;
   }
   __device__ int count() const { return cx * cy * cz; }
@@ -982,7 +994,7 @@ struct ObjBins {
 
 // One workgroup per capsule: the clamped window boxes of its nine objects (boxes[o], o =
 // 9 p + nb), its registration in the coarse bins, and its number of items (cnt[p]).
-__global__ void __launch_bounds__(256) k_obj_boxes(GridD g, int klo, int khi,
+__global__ void __launch_bounds__(256) k_obj_boxes(GridD g, int klo, int khi, ObjLimit lim,
                                                    const long long* __restrict__ cap_off,
                                                    const double* __restrict__ x,
                                                    const double* __restrict__ y,
@@ -1056,7 +1068,7 @@ __global__ void __launch_bounds__(256) k_obj_boxes(GridD g, int klo, int khi,
     const int nb = tid;
     const bool has = B[nb][0] <= B[nb][1];
     for (int e = 0; e < 6; ++e) boxes[(p * 9 + nb) * 6 + e] = has ? B[nb][e] : (e & 1 ? 0 : 1);
-    ncnt[nb] = has ? ObjGrid(B[nb]).count() : 0;
+    ncnt[nb] = has ? ObjGrid(B[nb], lim).count() : 0;
     if (has) {
       const ObjBins bins(g);
       int r[6];
@@ -1129,29 +1141,100 @@ __device__ __forceinline__ bool boxes_meet(const int* a, const int* b) {
          a[3] >= b[2] && a[4] <= b[5] && a[5] >= b[4];
 }
 
+// The objects whose boxes meet an item's box, in ascending o, into src[item][0..nsrc[item]), by
+// one wavefront.  Candidates: the neighbours of the item's capsule (the item's box lies in its
+// capsule's union box), bits of row[0..nwd).
+__device__ __forceinline__ void obj_item_sources(const ObjItem& it, int item, int nwd,
+                                                 const unsigned long long* row,
+                                                 const int* __restrict__ boxes,
+                                                 int* __restrict__ src, int* __restrict__ nsrc,
+                                                 int* __restrict__ err) {
+  const int lane = threadIdx.x & 63;
+  const int xa = it.x0, xb = it.x0 + it.nx - 1, ya = it.y0, yb = it.y0 + it.ny - 1, za = it.z0,
+            zb = it.z0 + it.nz - 1;
+  int n = 0;
+  for (int w0 = 0; w0 < nwd; w0 += 64) {
+    const unsigned long long word = w0 + lane < nwd ? row[w0 + lane] : 0ull;
+    unsigned long long nzw = __ballot(word != 0ull);
+    while (nzw) {  // words ascending, then bits ascending: capsules ascending
+      const int l = __builtin_ctzll(nzw);
+      nzw &= nzw - 1;
+      const unsigned lo32 = (unsigned)__shfl((int)(unsigned)word, l),
+                     hi32 = (unsigned)__shfl((int)(unsigned)(word >> 32), l);
+      unsigned long long bits = ((unsigned long long)hi32 << 32) | lo32;
+      while (bits) {
+        const long long q = (long long)(w0 + l) * 64 + __builtin_ctzll(bits);
+        bits &= bits - 1;
+        bool h = false;
+        if (lane < 9) {
+          const int* b = boxes + (q * 9 + lane) * 6;
+          h = b[0] <= b[1] && b[0] <= xb && b[1] >= xa && b[2] <= yb && b[3] >= ya &&
+              b[4] <= zb && b[5] >= za;
+        }
+        const unsigned long long hb = __ballot(h);
+        if (h) {
+          const int pos = n + __popcll(hb & __lanemask_lt());
+          if (pos < OB_NSRC) src[(long long)item * OB_NSRC + pos] = (int)(q * 9 + lane);
+        }
+        n += __popcll(hb);
+      }
+    }
+  }
+  if (lane == 0) {
+    nsrc[item] = min(n, OB_NSRC);
+    if (n > OB_NSRC) atomicOr(err, ERR_CAPACITY);
+  }
+}
+
 // One workgroup per capsule p: its items (slots off[p] ... below icap; the items of an
 // object partition its box, c fastest), its boxes' cells in the coverage bitmap, and its
 // neighbour mask: bit q of nbm[p][0..nwd) is set iff a box of capsule q meets a box of p
 // (p itself included when it has a box); the candidates q are the capsules registered in
 // the bins that p's boxes overlap.
-__global__ void __launch_bounds__(256) k_obj_items(GridD g, long long ncap, int nwd,
+// FUSE (at most OB_FUSE capsules): the workgroup also adds up the item counts before its own
+// (k_obj_scan's work) and lists its items' sources (k_obj_sources'), whose neighbour mask it
+// holds in LDS: two launches fewer, 7 us of the 83 us a transfer of one capsule takes.
+constexpr int OB_FUSE = 1024;
+template <bool FUSE>
+__global__ void __launch_bounds__(256) k_obj_items(GridD g, ObjLimit lim, long long ncap, int nwd,
                                                    const int* __restrict__ boxes,
                                                    const unsigned long long* __restrict__ binm,
                                                    const int* __restrict__ off,
+                                                   const int* __restrict__ cnt,
                                                    ObjItem* __restrict__ items, int icap,
                                                    unsigned* __restrict__ cover,
                                                    unsigned long long* __restrict__ nbm,
-                                                   const int* __restrict__ err) {
+                                                   int* __restrict__ src, int* __restrict__ nsrc,
+                                                   int* __restrict__ meta,
+                                                   int* __restrict__ err) {
   if (offsets_bad(err)) return;
   __shared__ int B[9][6];
+  __shared__ int first;
   const int tid = threadIdx.x;
   const long long p = blockIdx.x;
   if (tid < 54) B[tid / 6][tid % 6] = boxes[p * 54 + tid];
+  if (FUSE && tid == 0) first = 0;
   __syncthreads();
-  int at = off[p];
+  int at;
+  if (FUSE) {
+    int v = 0;
+    for (long long q = tid; q < p; q += 256) v += cnt[q];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o);
+    if ((tid & 63) == 0 && v) atomicAdd(&first, v);
+    __syncthreads();
+    at = first;
+    if (tid == 0 && p == ncap - 1) {
+      meta[0] = at + cnt[p];
+      if (meta[0] > icap) atomicOr(err, ERR_CAPACITY);
+    }
+  } else {
+    at = off[p];
+  }
+  const int at0 = at;
   for (int nb = 0; nb < 9; ++nb) {
     if (B[nb][0] > B[nb][1]) continue;  // uniform
-    const ObjGrid og(B[nb]);
+    const ObjGrid og(B[nb], lim);
     for (int t = tid; t < og.count(); t += 256) {
       if (at + t >= icap) break;  // flagged by k_obj_scan
       const int a = t / (og.cy * og.cz), b = (t / og.cz) % og.cy, c = t % og.cz;
@@ -1244,14 +1327,49 @@ __global__ void __launch_bounds__(256) k_obj_items(GridD g, long long ncap, int 
       }
     }
     __syncthreads();
-    for (int t = tid; t < wn; t += 256) nbm[p * nwd + w0 + t] = res[t];
+    if (!FUSE)
+      for (int t = tid; t < wn; t += 256) nbm[p * nwd + w0 + t] = res[t];
     __syncthreads();
+  }
+  if (FUSE) {  // nwd <= OB_FUSE / 64 <= OB_NWC: one chunk, its mask still in res
+    // seven items per wavefront, nine lanes (image slots) each; capsules ascending
+    const int lane = tid & 63, grp = lane / 9, nb = lane % 9;
+    for (int i0 = at0 + 7 * (tid >> 6); i0 < min(at, icap); i0 += 28) {
+      const int item = i0 + grp;
+      const bool on = grp < 7 && item < min(at, icap);
+      ObjItem it{};
+      if (on) it = items[item];
+      int n = 0;
+      for (int w = 0; w < nwd; ++w) {
+        unsigned long long bits = res[w];
+        while (bits) {
+          const long long q = (long long)w * 64 + __builtin_ctzll(bits);
+          bits &= bits - 1;
+          bool h = false;
+          if (on) {
+            const int* b = boxes + (q * 9 + nb) * 6;
+            h = b[0] <= b[1] && b[0] <= it.x0 + it.nx - 1 && b[1] >= it.x0 &&
+                b[2] <= it.y0 + it.ny - 1 && b[3] >= it.y0 && b[4] <= it.z0 + it.nz - 1 &&
+                b[5] >= it.z0;
+          }
+          const unsigned mine = (unsigned)(__ballot(h) >> (9 * grp)) & 0x1ffu;
+          if (h) {
+            const int pos = n + __popc(mine & ((1u << nb) - 1u));
+            if (pos < OB_NSRC) src[(long long)item * OB_NSRC + pos] = (int)(q * 9 + nb);
+          }
+          n += __popc(mine);
+        }
+      }
+      if (on && nb == 0) {
+        nsrc[item] = min(n, OB_NSRC);
+        if (n > OB_NSRC) atomicOr(err, ERR_CAPACITY);
+      }
+    }
   }
 }
 
-// One wavefront per item (grid-stride): the objects whose boxes meet the item's box, in
-// ascending o, into src[item][0..nsrc[item]).  Candidates: the neighbours of the item's
-// capsule (the item's box lies in its capsule's union box).
+
+// One wavefront per item (grid-stride): its sources (batches beyond OB_FUSE capsules).
 __global__ void __launch_bounds__(256) k_obj_sources(int nwd, const int* __restrict__ boxes,
                                                      const unsigned long long* __restrict__ nbm,
                                                      const ObjItem* __restrict__ items,
@@ -1260,47 +1378,12 @@ __global__ void __launch_bounds__(256) k_obj_sources(int nwd, const int* __restr
                                                      int* __restrict__ meta,
                                                      int* __restrict__ err) {
   if (offsets_bad(err)) return;
-  const int lane = threadIdx.x & 63;
   const int nitems = min(meta[0], icap);
   const int waves = gridDim.x * (blockDim.x >> 6);
   for (int item = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); item < nitems;
        item += waves) {
     const ObjItem it = items[item];
-    const int xa = it.x0, xb = it.x0 + it.nx - 1, ya = it.y0, yb = it.y0 + it.ny - 1,
-              za = it.z0, zb = it.z0 + it.nz - 1;
-    const unsigned long long* row = nbm + (long long)it.p * nwd;
-    int n = 0;
-    for (int w0 = 0; w0 < nwd; w0 += 64) {
-      const unsigned long long word = w0 + lane < nwd ? row[w0 + lane] : 0ull;
-      unsigned long long nzw = __ballot(word != 0ull);
-      while (nzw) {  // words ascending, then bits ascending: capsules ascending
-        const int l = __builtin_ctzll(nzw);
-        nzw &= nzw - 1;
-        const unsigned lo32 = (unsigned)__shfl((int)(unsigned)word, l),
-                       hi32 = (unsigned)__shfl((int)(unsigned)(word >> 32), l);
-        unsigned long long bits = ((unsigned long long)hi32 << 32) | lo32;
-        while (bits) {
-          const long long q = (long long)(w0 + l) * 64 + __builtin_ctzll(bits);
-          bits &= bits - 1;
-          bool h = false;
-          if (lane < 9) {
-            const int* b = boxes + (q * 9 + lane) * 6;
-            h = b[0] <= b[1] && b[0] <= xb && b[1] >= xa && b[2] <= yb && b[3] >= ya &&
-                b[4] <= zb && b[5] >= za;
-          }
-          const unsigned long long hb = __ballot(h);
-          if (h) {
-            const int pos = n + __popcll(hb & __lanemask_lt());
-            if (pos < OB_NSRC) src[(long long)item * OB_NSRC + pos] = (int)(q * 9 + lane);
-          }
-          n += __popcll(hb);
-        }
-      }
-    }
-    if (lane == 0) {
-      nsrc[item] = min(n, OB_NSRC);
-      if (n > OB_NSRC) atomicOr(err, ERR_CAPACITY);
-    }
+    obj_item_sources(it, item, nwd, nbm + (long long)it.p * nwd, boxes, src, nsrc, err);
   }
 }
 
@@ -1668,7 +1751,9 @@ __global__ void __launch_bounds__(OB_THREADS, MINW)
   long long zu = blockIdx.x;
   const int xcd = blockIdx.x & 7;
   int qi = 0;  // queues tried so far (thread 0's view)
-  bool items_left = nitems > 0, zero_left = mine > 0;
+  // with more workgroups than items, the ones beyond them leave the queues to the others
+  // (each of which takes items until there are none): no round of eight empty queues
+  bool items_left = (int)blockIdx.x < nitems, zero_left = mine > 0;
   while (items_left || zero_left) {
     if (items_left) {
       // items: from the queue of this workgroup's XCD (a contiguous share, so that a
