@@ -31,18 +31,18 @@ def test_repeated_box_keeps_its_solution(ri, rj, kt):
     for shape, rep in ((small, (1, 1, 1)), (big, (1, rj, ri))):
         g = W.make_grid(*shape, H)
         s = FlowSolver(g, REP, DT)
-        s.set_stream(torch.cuda.current_stream().cuda_stream)
         f = []
         for a in inner:
             b = torch.zeros((kt + 2, shape[1] + 2, shape[0] + 2), dtype=torch.float64, device="cuda:0")
             b[1:-1, 1:-1, 1:-1] = dev(np.tile(a, rep))
             f.append(b.view(-1))
         uo, uoo, p, F = f[:3], f[3:6], f[6], f[7:10]
+        un = [torch.zeros_like(p) for _ in range(3)]
+        q = torch.zeros_like(p)
+        torch.cuda.synchronize()
         s.bounduvw(*uo)
         s.bounduvw(*uoo)
         s.boundp(p)
-        un = [torch.zeros_like(p) for _ in range(3)]
-        q = torch.zeros_like(p)
         s.step(*un, p, q, *uo, *uoo, *F)
         s.sync()
         got.append([a.view(kt + 2, shape[1] + 2, shape[0] + 2) for a in (*un, p, q)])

@@ -21,6 +21,7 @@ GS = 6250.0
 def run(torch, plan, xyz, eb, sel=None, ordered=False):
     n = xyz[0].numel()
     out = [torch.full((n,), -7.0, dtype=torch.float64, device="cuda:0") for _ in range(7)]
+    torch.cuda.synchronize()
     if sel is not None:
         plan.traction_select_dev(sel, *xyz, GS, eb, *out)
     elif ordered:
@@ -38,7 +39,6 @@ def test_splits_keep_the_bits(L, eb):
     from suguru_amd.membrane import MembranePlan
 
     plan = MembranePlan(L)
-    plan.set_stream(torch.cuda.current_stream().cuda_stream)
     n = plan.npts
     five = [torch.from_numpy(a).to("cuda:0") for a in capsules(L, 5, seed=3 * L + 1)]
     print(f"case: law splits L={L} eb={eb}, 5 capsules", flush=True)

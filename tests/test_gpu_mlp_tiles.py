@@ -38,13 +38,13 @@ def test_products_match_oracle(din, width, nh, dout, batch):
     omean, oscale = f(dout), rng.uniform(1.0, 3.0, dout).astype(np.float32)
     wt = rng.uniform(0.5, 1.5, dout).astype(np.float32)
     m = SurrogateMLP(din, width, nh, dout, max_batch=batch)
-    m.set_stream(torch.cuda.current_stream().cuda_stream)
     m.init(11)
     m.set_norm(mean, scale, omean, oscale)
     layers = [m.get_layer(i) for i in range(m.nl)]
     ref = MLPOracle(layers, mean, scale, oscale, out_mean=omean)
     d = [torch.from_numpy(a).to("cuda:0") for a in (x, t, wt)]
     y = torch.full((batch + 1, dout), 7.0, dtype=torch.float32, device="cuda:0")
+    torch.cuda.synchronize()
     m.forward(d[0], y, batch=batch)
     torch.cuda.synchronize()
     assert rel(y[:batch].cpu().numpy(), ref.predict(x)) < TOL

@@ -39,7 +39,6 @@ def test_spread_bits_by_capsule_count(grid, ncap, radius, degree):
     f = W.forces(caps.npts, ncap + 1)
     dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0")
     t = IBTransfer(g, 0)
-    t.set_stream(torch.cuda.current_stream().cuda_stream)
     try:
         off = dev(caps.cap_off)
         p = [dev(a) for a in (caps.x, caps.y, caps.z)]
@@ -48,6 +47,7 @@ def test_spread_bits_by_capsule_count(grid, ncap, radius, degree):
                        (dict(cc=True), O.lagr2eulrind)):
             out = [torch.full((g.ncells_halo,), np.nan, dtype=torch.float64, device="cuda:0")
                    for _ in range(3)]
+            torch.cuda.synchronize()
             t.spread_dev(off, *p, *d, *out, **kw)
             t.sync()
             want = fn(g, caps.cap_off, caps.x, caps.y, caps.z, *f, caps.area)
