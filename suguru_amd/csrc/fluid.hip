@@ -4,16 +4,18 @@
 // Layout.  The caller's fields are Fortran (0:i1,0:j1,0:k1) arrays, i fastest.  The solves work
 // in compact spectral arrays of itot x jtot x ktot doubles (i fastest), one per velocity
 // component; the pressure solve reuses the first.  A solve is five passes:
-//   1. x transform of every (j, k) line (k_rfft, lines contiguous),
-//   2. y transform of every (i, k) line (k_rfft, 8 neighbouring columns per workgroup: row
-//      segments of 64 bytes),
+//   1. x transform of every (j, k) line (k_x_fwd; lines contiguous),
+//   2. y transform of every (i, k) line (k_y; two neighbouring columns per complex line, row
+//      segments of 64 bytes and more per workgroup),
 //   3. Gaussian elimination in k per (i, j) mode (k_tri_seg: one lane per mode, the k rows in
 //      register-held segments joined through LDS, the per-mode reciprocal pivots read from a
 //      table built once per context; k_tri, two passes through the array, above 257 planes),
 //   4. y inverse, 5. x inverse (into the caller's field interior).
 // Transforms.  A real line of length N = 2M is transformed as M complex values
-// z_n = x_2n + i x_2n+1 (radix-2, in LDS, input bit-reversed on load), then split into the
-// half spectrum X_0 .. X_M.  Packed real layout of a line: [X_0, X_M, Re X_1, Im X_1, ...,
+// z_n = x_2n + i x_2n+1, then split into the half spectrum X_0 .. X_M; a pair of y lines as the
+// real and imaginary part of one complex line.  Lines of 16 .. 2048 (x) and 8 .. 1024 values (y)
+// go through registers (radix 8, fft_reg.hpp), the others through LDS (k_rfft: radix 4, input
+// bit-reversed on load).  Packed real layout of a line: [X_0, X_M, Re X_1, Im X_1, ...,
 // Re X_M-1, Im X_M-1]; position p carries wavenumber 0 (p = 0), M (p = 1) or p / 2.  The
 // second-difference eigenvalue of a position depends only on its wavenumber, which is what the
 // reference's xrt/yrt tables encode for VFFTPACK's layout (initsolver.f90:108-132).
@@ -23,9 +25,11 @@
 #include <cmath>
 #include <cstdint>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/fluid.h"
+#include "fft_reg.hpp"
 
 #pragma clang fp contract(off)
 
@@ -286,6 +290,228 @@ __global__ void __launch_bounds__(FFT_THREADS)
   for (int q = threadIdx.x; q < nl * N; q += blockDim.x) {
     const int l = XMAJOR ? q >> logn : q & (nl - 1), e = XMAJOR ? q & (N - 1) : q >> lognl;
     dst[bd + l * ls_dst + e * es_dst] = smd[2 * (l * (M + 1) + (e >> 1)) + (e & 1)] * sc;
+  }
+}
+
+// ---- register transforms --------------------------------------------------------------------
+// The transforms of lines that 8 values a thread cover (x lines of 16 .. 2048, y lines of
+// 8 .. 1024 values): radix-8 passes in registers with two or three exchanges through LDS, where the
+// kernels above go through LDS once per radix-4 pass and once more for the bit reversal, with a
+// workgroup barrier each.  Bound by memory: at 1024 x 512 x 256 an array takes 422 us forward and
+// 426 us inverse in x, 436 and 414 us in y (a copy of its 2.1 GB takes 438 us), 865 us with the
+// divergence as the source; the kernels above took 569, 579, 553, 610 and 1029 us.
+constexpr int REG_T = 256;  // threads of an x workgroup, and of a y workgroup up to 512 rows
+
+// two neighbouring values of a row (the rows of the caller's fields start at odd elements)
+struct __attribute__((packed, aligned(8))) Pair {
+  double x, y;
+};
+__device__ __forceinline__ double2 load2(const double* p) {
+  const Pair v = *reinterpret_cast<const Pair*>(p);
+  return make_double2(v.x, v.y);
+}
+__device__ __forceinline__ void store2(double* p, double2 v) {
+  *reinterpret_cast<Pair*>(p) = Pair{v.x, v.y};
+}
+
+// rows of the lines of one launch: line (j, k) at off + j row + k plane
+struct Rows {
+  long long off, row, plane;
+  __device__ __forceinline__ long long at(int j, int k) const { return off + j * row + k * plane; }
+};
+
+// x lines: one line of M = itot / 2 complex values per M/8 lanes, 2048 / M lines a workgroup.  With
+// M <= 512 a line stays within one wavefront and needs no workgroup barrier.
+template <int LOGM>
+struct XLine {
+  using Line = fft::Line<LOGM, (LOGM > 9)>;
+  static constexpr int M = Line::N, TPL = Line::TPL, PER = REG_T / TPL, PITCH = fft::pad(M) + 1;
+};
+
+template <int LOGM, bool FILL>
+__global__ void __launch_bounds__(REG_T)
+    k_x_fwd(Arrays arr, Rows rs, Rows rd, int logj, int lines, const double2* __restrict__ tw,
+            const double2* __restrict__ twm, FillSrc fs) {
+  using X = XLine<LOGM>;
+  constexpr int M = X::M, TPL = X::TPL;
+  constexpr bool WG = LOGM > 9;
+  __shared__ double2 sm[X::PER * X::PITCH];
+  const int t = threadIdx.x & (TPL - 1), own = threadIdx.x / TPL;
+  const int line = blockIdx.x * X::PER + own;
+  const bool live = line < lines;
+  const int ln = live ? line : lines - 1, k = ln >> logj, j = ln & ((1 << logj) - 1);
+  double2* buf = sm + own * X::PITCH;
+  double2 a[8];
+  if constexpr (FILL) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const long long c = 2 * (t + TPL * u) + 1 + fs.sy * (j + 1) + fs.sz * (k + 1);
+      const double2 w0 = load2(fs.w + c), w1 = load2(fs.w + c - fs.sz);
+      const double2 v0 = load2(fs.v + c), v1 = load2(fs.v + c - fs.sy);
+      const double2 u0 = load2(fs.u + c), u1 = load2(fs.u + c - 1);
+      a[u] = make_double2(((w0.x - w1.x) * fs.cz + (v0.x - v1.x) * fs.cy + (u0.x - u1.x) * fs.cx),
+                          ((w0.y - w1.y) * fs.cz + (v0.y - v1.y) * fs.cy + (u0.y - u1.y) * fs.cx));
+    }
+  } else {
+    const double* src = arr.src[blockIdx.y] + rs.at(j, k);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) a[u] = load2(src + 2 * (t + TPL * u));
+  }
+  typename X::Line lw;
+  lw.load(twm, t);
+  lw.template run<false>(a, buf, t);
+  // X_k = E_k + W^k O_k, E_k = (Z_k + conj Z_M-k) / 2, O_k = (Z_k - conj Z_M-k) / 2i
+  fft::line_sync<WG>();
+#pragma unroll
+  for (int u = 0; u < 8; ++u) buf[fft::pad(t + TPL * u)] = a[u];
+  fft::line_sync<WG>();
+  double* dst = arr.dst[blockIdx.y] + rd.at(j, k);
+#pragma unroll
+  for (int u = 0; u < 8; ++u) {
+    const int q = t + TPL * u;
+    const double2 b = buf[fft::pad((M - q) & (M - 1))], w = tw[q];
+    const double2 E = make_double2(0.5 * (a[u].x + b.x), 0.5 * (a[u].y - b.y));
+    const double2 O = make_double2(0.5 * (a[u].y + b.y), -0.5 * (a[u].x - b.x));
+    double2 v = fft::add(E, fft::mul(w, O));
+    if (u == 0 && t == 0) v = make_double2(a[0].x + a[0].y, a[0].x - a[0].y);
+    if (live) store2(dst + 2 * q, v);
+  }
+}
+
+template <int LOGM>
+__global__ void __launch_bounds__(REG_T)
+    k_x_inv(Arrays arr, Rows rs, Rows rd, int logj, int lines, const double2* __restrict__ tw,
+            const double2* __restrict__ twm) {
+  using X = XLine<LOGM>;
+  constexpr int M = X::M, TPL = X::TPL;
+  constexpr bool WG = LOGM > 9;
+  __shared__ double2 sm[X::PER * X::PITCH];
+  const int t = threadIdx.x & (TPL - 1), own = threadIdx.x / TPL;
+  const int line = blockIdx.x * X::PER + own;
+  const bool live = line < lines;
+  const int ln = live ? line : lines - 1, k = ln >> logj, j = ln & ((1 << logj) - 1);
+  double2* buf = sm + own * X::PITCH;
+  const double* src = arr.src[blockIdx.y] + rs.at(j, k);
+  double2 a[8];
+#pragma unroll
+  for (int u = 0; u < 8; ++u) a[u] = load2(src + 2 * (t + TPL * u));
+#pragma unroll
+  for (int u = 0; u < 8; ++u) buf[fft::pad(t + TPL * u)] = a[u];
+  fft::line_sync<WG>();
+  // Z_k = E_k + i O_k, E_k = (X_k + conj X_M-k) / 2, O_k = (X_k - conj X_M-k) conj(W^k) / 2
+#pragma unroll
+  for (int u = 0; u < 8; ++u) {
+    const int q = t + TPL * u;
+    const double2 b = buf[fft::pad((M - q) & (M - 1))], w = tw[q];
+    const double2 E = make_double2(0.5 * (a[u].x + b.x), 0.5 * (a[u].y - b.y));
+    const double2 D = make_double2(0.5 * (a[u].x - b.x), 0.5 * (a[u].y + b.y));
+    const double2 O = fft::mul(D, make_double2(w.x, -w.y));
+    double2 v = make_double2(E.x - O.y, E.y + O.x);
+    if (u == 0 && t == 0)
+      v = make_double2(0.5 * (a[0].x + a[0].y), 0.5 * (a[0].x - a[0].y));
+    a[u] = v;
+  }
+  typename X::Line lw;
+  lw.load(twm, t);
+  lw.template run<true>(a, buf, t);
+  const double sc = 1.0 / (double)M;
+  double* dst = arr.dst[blockIdx.y] + rd.at(j, k);
+  if (live) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      store2(dst + 2 * (t + TPL * u), make_double2(a[u].x * sc, a[u].y * sc));
+  }
+}
+
+// y lines: two neighbouring real columns are the real and imaginary part of one complex line of
+// N = jtot values (no twiddles in the split, 16-byte loads), neighbouring pairs on neighbouring
+// lanes.  A workgroup holds COLS pairs: 64-byte row segments at 512 rows, 128 at 256.
+template <int LOGN>
+struct YLine {
+  using Line = fft::Line<LOGN, true>;
+  static constexpr int N = Line::N, TPL = Line::TPL;
+  static constexpr int COLS = LOGN > 9 ? 4 : REG_T / TPL, T = COLS * TPL;
+  // the pairs of a row lie in different banks: pitch = 16 / COLS mod 16 sixteen-byte slots
+  static constexpr int SKEW = COLS >= 16 ? 1 : 16 / COLS;
+  static constexpr int PITCH = fft::pad(N) + (SKEW - fft::pad(N) % 16 + 16) % 16;
+};
+
+// the packed half spectra of a pair of columns from its complex spectrum: rows 2k and 2k + 1
+// (k = t + TPL u, u < 4) get Re and Im of X_k, rows 0 and 1 X_0 and X_N/2
+template <int LOGN>
+__device__ __forceinline__ void y_split(const double2 (&a)[8], double2* buf, int t,
+                                        double2 (&row)[8]) {
+  using Y = YLine<LOGN>;
+  __syncthreads();
+#pragma unroll
+  for (int u = 4; u < 8; ++u) buf[fft::pad(t + Y::TPL * u)] = a[u];
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const bool first = u == 0 && t == 0;
+    const int q = t + Y::TPL * u;
+    const double2 b = buf[fft::pad(first ? Y::N / 2 : Y::N - q)];
+    // A = (Z_k + conj Z_N-k) / 2, B = (Z_k - conj Z_N-k) / 2i
+    row[2 * u] = make_double2(0.5 * (a[u].x + b.x), 0.5 * (a[u].y + b.y));
+    row[2 * u + 1] = make_double2(0.5 * (a[u].y - b.y), -0.5 * (a[u].x - b.x));
+    if (first) row[0] = a[0], row[1] = b;
+  }
+}
+
+// the reverse: a[u] = Z_t+TPL u from the packed rows
+template <int LOGN>
+__device__ __forceinline__ void y_join(const double2 (&row)[8], double2* buf, int t,
+                                       double2 (&a)[8]) {
+  using Y = YLine<LOGN>;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const bool first = u == 0 && t == 0;
+    const int q = t + Y::TPL * u;
+    const double2 r = row[2 * u], i = row[2 * u + 1];  // (Re A, Re B), (Im A, Im B)
+    a[u] = first ? r : make_double2(r.x - i.y, i.x + r.y);
+    buf[fft::pad(first ? Y::N / 2 : Y::N - q)] = first ? i : make_double2(r.x + i.y, r.y - i.x);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 4; u < 8; ++u) a[u] = buf[fft::pad(t + Y::TPL * u)];
+}
+
+template <int LOGN, bool INV>
+__global__ void __launch_bounds__(YLine<LOGN>::T)
+    k_y(Arrays arr, int logc, long long pairs, const double2* __restrict__ twn) {
+  using Y = YLine<LOGN>;
+  __shared__ double2 sm[Y::COLS * Y::PITCH];
+  const int col = threadIdx.x & (Y::COLS - 1), t = threadIdx.x / Y::COLS;
+  const long long g = (long long)xcd_logical_block<false>() * Y::COLS + col;
+  const bool live = g < pairs;
+  const long long gg = live ? g : pairs - 1, k = gg >> logc, c = gg - (k << logc);
+  const long long pitch = 1LL << logc;  // pairs of a row
+  double2* p = reinterpret_cast<double2*>(arr.dst[blockIdx.y]) + k * (pitch << LOGN) + c;
+  double2* buf = sm + col * Y::PITCH;
+  double2 a[8], row[8];
+  typename Y::Line lw;
+  if constexpr (!INV) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) a[u] = p[(t + Y::TPL * u) * pitch];
+    lw.load(twn, t);
+    lw.template run<false>(a, buf, t);
+    y_split<LOGN>(a, buf, t, row);
+    if (live) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) p[(2 * (t + Y::TPL * (u >> 1)) + (u & 1)) * pitch] = row[u];
+    }
+  } else {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) row[u] = p[(2 * (t + Y::TPL * (u >> 1)) + (u & 1)) * pitch];
+    lw.load(twn, t);
+    y_join<LOGN>(row, buf, t, a);
+    lw.template run<true>(a, buf, t);
+    const double sc = 1.0 / (double)Y::N;
+    if (live) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        p[(t + Y::TPL * u) * pitch] = make_double2(a[u].x * sc, a[u].y * sc);
+    }
   }
 }
 
@@ -929,6 +1155,8 @@ struct fld_ctx {
   double* coef[4] = {nullptr, nullptr, nullptr, nullptr};  // a, c per ne (2 * ktot each)
   double2* tw_x = nullptr;
   double2* tw_y = nullptr;
+  double2* tw_xm = nullptr;  // exp(-2 pi i k / M), k < M = itot / 2
+  double2* tw_yn = nullptr;  // exp(-2 pi i k / jtot), k < jtot
   double* part = nullptr;  // chkdiv partials
   int logmx = 0, logmy = 0;
   size_t lds_yf = 0, lds_yi = 0;
@@ -960,11 +1188,11 @@ int ilog2(int n) {
 
 bool pow2(int n) { return n >= 2 && (n & (n - 1)) == 0; }
 
-// exp(-2 pi i k / n), k < n/2, from long-double sine and cosine
-std::vector<double2> twiddles(int n) {
-  std::vector<double2> t((size_t)std::max(1, n / 2));
+// exp(-2 pi i k / n), k < count, from long-double sine and cosine
+std::vector<double2> twiddles(int n, int count) {
+  std::vector<double2> t((size_t)std::max(1, count));
   const long double pi = 3.141592653589793238462643383279502884L;
-  for (int k = 0; k < n / 2; ++k) {
+  for (int k = 0; k < count; ++k) {
     const long double a = 2.0L * pi * (long double)k / (long double)n;
     t[(size_t)k] = make_double2((double)cosl(a), (double)(-sinl(a)));
   }
@@ -1017,8 +1245,60 @@ void tridiag(const fld_ctx* c, int e, std::vector<double>& a, std::vector<double
   }
 }
 
+// f(integral_constant<int, L>) for the run-time L in [LO, HI]
+template <int LO, int HI, class F>
+void with_log(int L, F&& f) {
+  if constexpr (LO <= HI) {
+    if (L == LO)
+      f(std::integral_constant<int, LO>{});
+    else
+      with_log<LO + 1, HI>(L, f);
+  }
+}
+
+bool reg_x(const fld_ctx* c) { return c->logmx >= 3 && c->logmx <= 10; }
+bool reg_y(const fld_ctx* c) { return c->logmy >= 2 && c->logmy <= 9; }
+
+// x transforms of n systems by the register kernels; fs: the pressure's divergence as the source
+int reg_fft_x(fld_ctx* c, bool inv, int n, const Arrays& arr, bool src_field, bool dst_field,
+              const FillSrc* fs) {
+  const FGrid& g = c->g;
+  const Rows field{1 + g.sy + g.sz, g.sy, g.sz}, compact{0, g.itot, (long long)g.itot * g.jtot};
+  const Rows rs = src_field ? field : compact, rd = dst_field ? field : compact;
+  const int lines = g.jtot * g.ktot, logj = c->logmy + 1;
+  with_log<3, 10>(c->logmx, [&](auto l) {
+    constexpr int L = decltype(l)::value;
+    const dim3 nb(nblocks(lines, XLine<L>::PER), (unsigned)n);
+    if (inv)
+      k_x_inv<L><<<nb, REG_T, 0, c->stream>>>(arr, rs, rd, logj, lines, c->tw_x, c->tw_xm);
+    else if (fs)
+      k_x_fwd<L, true><<<nb, REG_T, 0, c->stream>>>(arr, rs, rd, logj, lines, c->tw_x, c->tw_xm, *fs);
+    else
+      k_x_fwd<L, false><<<nb, REG_T, 0, c->stream>>>(arr, rs, rd, logj, lines, c->tw_x, c->tw_xm,
+                                                     FillSrc{});
+  });
+  HIPF(c, hipGetLastError());
+  return FLD_OK;
+}
+
+int reg_fft_y(fld_ctx* c, bool inv, int n, const Arrays& arr) {
+  const FGrid& g = c->g;
+  const long long pairs = (long long)(g.itot / 2) * g.ktot;
+  with_log<3, 10>(c->logmy + 1, [&](auto l) {
+    constexpr int L = decltype(l)::value;
+    const dim3 nb(nblocks(pairs, YLine<L>::COLS), (unsigned)n);
+    if (inv)
+      k_y<L, true><<<nb, YLine<L>::T, 0, c->stream>>>(arr, c->logmx, pairs, c->tw_yn);
+    else
+      k_y<L, false><<<nb, YLine<L>::T, 0, c->stream>>>(arr, c->logmx, pairs, c->tw_yn);
+  });
+  HIPF(c, hipGetLastError());
+  return FLD_OK;
+}
+
 // x transforms of the interior lines of n fields (or compact arrays), forward or inverse
 int fft_x(fld_ctx* c, bool inv, int n, const Arrays& arr, bool src_field, bool dst_field) {
+  if (reg_x(c)) return reg_fft_x(c, inv, n, arr, src_field, dst_field, nullptr);
   const FGrid& g = c->g;
   const int N = g.itot, nl = c->xlines;
   const int gpp = g.jtot / nl;  // workgroups per k plane
@@ -1050,6 +1330,7 @@ int fft_y(fld_ctx* c, bool inv, int n, double* const* a) {
   const dim3 nb((unsigned)(gpp * g.ktot), (unsigned)n);
   Arrays arr{};
   for (int i = 0; i < n; ++i) arr.src[i] = arr.dst[i] = a[i];
+  if (reg_y(c)) return reg_fft_y(c, inv, n, arr);
   if (!inv)
     k_rfft_fwd<false><<<nb, FFT_THREADS, c->lds_yf, c->stream>>>(
         arr, N, c->logmy, nl, gpp, cp, cp, nl, nl, g.itot, 1, g.itot, 1, 0, c->tw_y, FillSrc{});
@@ -1109,8 +1390,10 @@ int fft_x_fill(fld_ctx* c, const double* u, const double* v, const double* w, do
   const unsigned nb = (unsigned)(gpp * g.ktot);
   const double dti = 1.0 / c->dt;
   const FillSrc fs{u, v, w, dti * g.dxi, dti * g.dyi, dti * g.dzi, g.sy, g.sz};
+  const Arrays arr{{nullptr, nullptr, nullptr}, {dst, nullptr, nullptr}};
+  if (reg_x(c)) return reg_fft_x(c, false, 1, arr, false, false, &fs);
   k_rfft_fwd<true, true><<<nb, FFT_THREADS, lds, c->stream>>>(
-      Arrays{{nullptr, nullptr, nullptr}, {dst, nullptr, nullptr}}, N, c->logmx, nl, gpp, cp, cp,
+      arr, N, c->logmx, nl, gpp, cp, cp,
       nl * row, nl * row, 1, row, 1, row, 0, c->tw_x, fs);
   HIPF(c, hipGetLastError());
   return FLD_OK;
@@ -1188,17 +1471,22 @@ int fld_create(fld_ctx** out, const ibx_grid* gr, double rep, double dt, int dev
                           (int)LDS_MAX) != hipSuccess)
     return bail(FLD_E_HIP, "lds");
   // twiddles, eigenvalues, coefficients and the pivot tables of e = 1, 2, 3
-  const std::vector<double2> twx = twiddles(g.itot), twy = twiddles(g.jtot);
+  const std::vector<double2> twx = twiddles(g.itot, g.itot / 2), twy = twiddles(g.jtot, g.jtot / 2);
+  const std::vector<double2> twxm = twiddles(g.itot / 2, g.itot / 2), twyn = twiddles(g.jtot, g.jtot);
   const std::vector<double> xrt = eigen(g.itot, g.dxi), yrt = eigen(g.jtot, g.dyi);
   double *dx = nullptr, *dy = nullptr, *dabc = nullptr;
   bool ok = hipMalloc(&c->tw_x, twx.size() * sizeof(double2)) == hipSuccess &&
             hipMalloc(&c->tw_y, twy.size() * sizeof(double2)) == hipSuccess &&
+            hipMalloc(&c->tw_xm, twxm.size() * sizeof(double2)) == hipSuccess &&
+            hipMalloc(&c->tw_yn, twyn.size() * sizeof(double2)) == hipSuccess &&
             hipMalloc(&dx, xrt.size() * sizeof(double)) == hipSuccess &&
             hipMalloc(&dy, yrt.size() * sizeof(double)) == hipSuccess &&
             hipMalloc(&dabc, 3 * (size_t)g.ktot * sizeof(double)) == hipSuccess &&
             hipMalloc(&c->part, 2 * 1024 * sizeof(double)) == hipSuccess;
   ok = ok && hipMemcpy(c->tw_x, twx.data(), twx.size() * sizeof(double2), hipMemcpyHostToDevice) == hipSuccess &&
        hipMemcpy(c->tw_y, twy.data(), twy.size() * sizeof(double2), hipMemcpyHostToDevice) == hipSuccess &&
+       hipMemcpy(c->tw_xm, twxm.data(), twxm.size() * sizeof(double2), hipMemcpyHostToDevice) == hipSuccess &&
+       hipMemcpy(c->tw_yn, twyn.data(), twyn.size() * sizeof(double2), hipMemcpyHostToDevice) == hipSuccess &&
        hipMemcpy(dx, xrt.data(), xrt.size() * sizeof(double), hipMemcpyHostToDevice) == hipSuccess &&
        hipMemcpy(dy, yrt.data(), yrt.size() * sizeof(double), hipMemcpyHostToDevice) == hipSuccess;
   const int nkx = g.itot / 2 + 1, nky = g.jtot / 2 + 1;
@@ -1240,6 +1528,8 @@ void fld_destroy(fld_ctx* c) {
   }
   if (c->tw_x) (void)hipFree(c->tw_x);
   if (c->tw_y) (void)hipFree(c->tw_y);
+  if (c->tw_xm) (void)hipFree(c->tw_xm);
+  if (c->tw_yn) (void)hipFree(c->tw_yn);
   if (c->part) (void)hipFree(c->part);
   if (c->own) (void)hipStreamDestroy(c->own);
   delete c;
