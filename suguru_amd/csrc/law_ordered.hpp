@@ -8,7 +8,8 @@
 // 1e-12 instead of to that rounding: the Legendre sums of every ring in index order from the
 // ring's own table, the geometry through contravariant vectors and the derivatives of the
 // normal, every entry of a symmetric tensor by its own sum.  The law itself (k_nodes) does the
-// same with fewer operations: 8000 capsules take 2.4 ms in its node phase, about 4 ms in this one.
+// same with fewer operations: 1734 capsules of degree 16 take 0.47 ms in its node phase, 1.10 ms
+// in this one.
 // Shape and filter round at the size of their results and are the law's own.
 #pragma once
 

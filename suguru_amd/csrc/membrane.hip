@@ -30,7 +30,7 @@
 namespace memb {
 
 constexpr int NQ = 15;        // derivatives of total order <= 4
-constexpr int NREF = 36;      // reference-state doubles per fine node
+constexpr int NREF = 32;      // reference-state doubles per fine node
 constexpr int LMAX = 23;
 constexpr int ND_THREADS = 128;  // per workgroup of the node kernel (two wavefronts)
 constexpr int SH_THREADS = 256;  // per workgroup of the shape and filter kernels
@@ -48,6 +48,8 @@ __host__ __device__ constexpr int tidx(int N, int d, int m) { return d * N - d *
 // Colatitudes come in pairs (theta, pi - theta): P_n^m(pi - theta) = (-1)^(n + m) P_n^m(theta),
 // and each theta-derivative adds a sign, so tables hold the northern ring of a pair only.
 struct Tables {
+  // lanes of a ring in the node kernel: its quads are phi_j, -phi_j and both plus pi, j <= N
+  __host__ __device__ int slots() const { return 4 * (N + 1); }
   int L, N, np2, nt, np, NT;   // N = L+1 coarse latitudes; nt = 2N, np = 2 np2; NT harmonics
   const double* w2;            // [N] coarse Gauss weights
   const double* s2;            // [N] sin(theta) coarse
@@ -58,7 +60,7 @@ struct Tables {
   const double* WPf;           // [N][NT] w Pbar, fine northern rings (the filter's quadrature)
   const double2* e2;           // [np2] cos, sin(2 pi q / np2)
   const double2* ef;           // [np] cos, sin(2 pi q / np)
-  const double* ref;           // [NREF][nt*np] unit-sphere state (the law reads it)
+  const double* ref;           // [NREF][nt*slots] unit-sphere state (the law reads it)
 };
 
 __device__ inline double dot3(const double* u, const double* v) {
@@ -70,14 +72,17 @@ __device__ inline void cross3(const double* u, const double* v, double* r) {
   r[2] = u[0] * v[1] - u[1] * v[0];
 }
 
-// v of the adjacent lane (lanes 2k and 2k + 1 swap): DPP quad_perm [1, 0, 3, 2] on the two
-// halves, a VALU move instead of an LDS-crossbar permute; both lanes of a pair must be active
-__device__ __forceinline__ double swap_pair(double v) {
+// v of another lane of the quad, the DPP quad_perm CTRL on the two halves: a VALU move instead of
+// an LDS-crossbar permute; the lanes of a quad must be active
+template <int CTRL>
+__device__ __forceinline__ double quad_perm(double v) {
   const unsigned long long b = (unsigned long long)__double_as_longlong(v);
-  const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)b, 0xB1, 0xF, 0xF, false);
-  const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)(b >> 32), 0xB1, 0xF, 0xF, false);
+  const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)b, CTRL, 0xF, 0xF, false);
+  const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)(b >> 32), CTRL, 0xF, 0xF, false);
   return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
+__device__ __forceinline__ double swap_pair(double v) { return quad_perm<0xB1>(v); }  // lane ^ 1
+__device__ __forceinline__ double swap_half(double v) { return quad_perm<0x4E>(v); }  // lane ^ 2
 
 // ---- per-node geometry and law -----------------------------------------------------------------
 // Tensors that are symmetric in a pair of indices keep one value per sum of the pair: a metric
@@ -86,7 +91,8 @@ __device__ __forceinline__ double swap_pair(double v) {
 // the second derivative) and so on, the Christoffel symbols are Gam[l][s] = G[l][p] D21[s][p],
 // n_,c = -b_cl a^l turns the derivatives of the curvature into products of b, Gam and
 // H[l][s] = x_,s(third) . a^l, and no contravariant vector or derivative of the normal is formed:
-// about 430 FMAs a node instead of 1000, with 36 instead of 56 values of reference state.
+// less than half of the products a node, with 32 instead of 56 values of reference state (the
+// reference's mixed curvature and its derivatives as products).
 struct Geom {
   double n[3], x1[2][3];
   double g[3], gd[2][3], G[3], Gd[2][3], Gdd[3][3];
@@ -100,6 +106,35 @@ __device__ __forceinline__ void mul_fs(const double X[2][2], const double S[3], 
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) R[i][j] = X[i][0] * S[j] + X[i][1] * S[1 + j];
+}
+
+// P^pa Q_cp and its first and second derivatives (P symmetric contravariant, Q covariant), the
+// mixed curvature of the current and of the reference state
+__device__ __forceinline__ double mixed(const double P[3], const double Q[3], int c, int a) {
+  return P[a] * Q[c] + P[1 + a] * Q[c + 1];
+}
+__device__ __forceinline__ double mixed_d(const double P[3], const double Pl[3], const double Q[3],
+                                          const double Ql[3], int c, int a) {
+  return Pl[a] * Q[c] + Pl[1 + a] * Q[c + 1] + P[a] * Ql[c] + P[1 + a] * Ql[c + 1];
+}
+__device__ __forceinline__ double mixed_dd(const double P[3], const double (&Pd)[2][3],
+                                           const double Plk[3], const double Q[3],
+                                           const double (&Qd)[2][3], const double Qlk[3], int l,
+                                           int k, int c, int a) {
+  double v = 0.0;
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    v += Plk[p + a] * Q[c + p] + P[p + a] * Qlk[c + p];
+    if (l == k)
+      v += 2.0 * (Pd[l][p + a] * Qd[l][c + p]);
+    else
+      v += Pd[k][p + a] * Qd[l][c + p] + Pd[l][p + a] * Qd[k][c + p];
+  }
+  return v;
+}
+// field of the reference's second derivative e of K^a_c: (a, b) with a + b = e only is read
+__host__ __device__ constexpr int ref_dd(int e, int c, int a) {
+  return e == 1 ? 26 + 2 * c + a : (e == 0 ? 24 : 30) + c;
 }
 
 // X[c][q]: derivatives of coordinate c.  BEND: the second derivatives of metric and curvature
@@ -235,7 +270,7 @@ __device__ __forceinline__ void law(const Geom& o, const double* __restrict__ R,
 #pragma unroll
     for (int c = 0; c < 2; ++c) Ad[c][s] = R[(3 + 3 * c + s) * rs];
   }
-  const double detA = A[0] * A[2] - A[1] * A[1];
+  const double detA = R[9 * rs];
   const double deta = o.g[0] * o.g[2] - o.g[1] * o.g[1];
   const double I2 = detA * deta - 1.0;
   const double Js = sqrt(1.0 + I2);
@@ -248,7 +283,7 @@ __device__ __forceinline__ void law(const Geom& o, const double* __restrict__ R,
   for (int s = 0; s < 3; ++s) T[s] = tA * A[s] + tG * o.G[s];
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
-    const double dA = Ad[c][0] * A[2] + A[0] * Ad[c][2] - 2.0 * A[1] * Ad[c][1];
+    const double dA = R[(10 + c) * rs];
     const double da = o.gd[c][0] * o.g[2] + o.g[0] * o.gd[c][2] - 2.0 * o.g[1] * o.gd[c][1];
     const double I2d = dA * deta + da * detA;
     const double Jsd = 0.5 * rJs * I2d;
@@ -268,13 +303,6 @@ __device__ __forceinline__ void law(const Geom& o, const double* __restrict__ R,
            (o.Gam[b][0] * T[0] + 2.0 * o.Gam[b][1] * T[1] + o.Gam[b][2] * T[2]);
   double q3 = T[0] * o.b[0] + 2.0 * T[1] * o.b[1] + T[2] * o.b[2];
   if (BEND) {
-    double B[3], Bd[2][3];
-#pragma unroll
-    for (int s = 0; s < 3; ++s) {
-      B[s] = R[(18 + s) * rs];
-#pragma unroll
-      for (int c = 0; c < 2; ++c) Bd[c][s] = R[(21 + 3 * c + s) * rs];
-    }
     // K^a_c = A^pa B_cp - G^pa b_cp, its first derivatives, and in dds the contraction of
     // (G^bc K^a_c),ab; K[c][a], Kd[l][c][a]
     double K[2][2], Kd[2][2][2];
@@ -282,41 +310,15 @@ __device__ __forceinline__ void law(const Geom& o, const double* __restrict__ R,
     for (int c = 0; c < 2; ++c)
 #pragma unroll
       for (int a = 0; a < 2; ++a) {
-        K[c][a] = (A[a] * B[c] + A[1 + a] * B[c + 1]) - (o.G[a] * o.b[c] + o.G[1 + a] * o.b[c + 1]);
+        K[c][a] = R[(12 + 2 * c + a) * rs] - mixed(o.G, o.b, c, a);
 #pragma unroll
         for (int l = 0; l < 2; ++l)
-          Kd[l][c][a] = (Ad[l][a] * B[c] + Ad[l][1 + a] * B[c + 1] + A[a] * Bd[l][c] +
-                         A[1 + a] * Bd[l][c + 1]) -
-                        (o.Gd[l][a] * o.b[c] + o.Gd[l][1 + a] * o.b[c + 1] + o.G[a] * o.bd[l][c] +
-                         o.G[1 + a] * o.bd[l][c + 1]);
+          Kd[l][c][a] = R[(16 + 4 * l + 2 * c + a) * rs] - mixed_d(o.G, o.Gd[l], o.b, o.bd[l], c, a);
       }
     double dds = 0.0;
 #pragma unroll
     for (int e = 0; e < 3; ++e) {  // derivatives l, k with l + k = e
       const int l = e >> 1, k = (e + 1) >> 1;
-      double Add[3], Bdd[3];
-#pragma unroll
-      for (int s = 0; s < 3; ++s) Add[s] = R[(9 + 3 * e + s) * rs], Bdd[s] = R[(27 + 3 * e + s) * rs];
-      double Kdd[2][2];
-#pragma unroll
-      for (int c = 0; c < 2; ++c)
-#pragma unroll
-        for (int a = 0; a < 2; ++a) {
-          double u = 0.0, v = 0.0;
-#pragma unroll
-          for (int p = 0; p < 2; ++p) {
-            u += Add[p + a] * B[c + p] + A[p + a] * Bdd[c + p];
-            v += o.Gdd[e][p + a] * o.b[c + p] + o.G[p + a] * o.bdd[e][c + p];
-            if (l == k) {
-              u += 2.0 * (Ad[l][p + a] * Bd[l][c + p]);
-              v += 2.0 * (o.Gd[l][p + a] * o.bd[l][c + p]);
-            } else {
-              u += Ad[k][p + a] * Bd[l][c + p] + Ad[l][p + a] * Bd[k][c + p];
-              v += o.Gd[k][p + a] * o.bd[l][c + p] + o.Gd[l][p + a] * o.bd[k][c + p];
-            }
-          }
-          Kdd[c][a] = u - v;
-        }
       // (a, b) with a + b = e: once for a = b, both orders for e = 1
 #pragma unroll
       for (int a = 0; a < 2; ++a) {
@@ -324,7 +326,9 @@ __device__ __forceinline__ void law(const Geom& o, const double* __restrict__ R,
         if (b < 0 || b > 1) continue;
 #pragma unroll
         for (int c = 0; c < 2; ++c)
-          dds += (o.Gdd[e][b + c] * K[c][a] + o.G[b + c] * Kdd[c][a]) +
+          dds += (o.Gdd[e][b + c] * K[c][a] +
+                  o.G[b + c] * (R[ref_dd(e, c, a) * rs] -
+                                mixed_dd(o.G, o.Gd, o.Gdd[e], o.b, o.bd, o.bdd[e], l, k, c, a))) +
                  (o.Gd[a][b + c] * Kd[b][c][a] + o.Gd[b][b + c] * Kd[a][c][a]);
       }
     }
@@ -375,9 +379,9 @@ __device__ __forceinline__ void law(const Geom& o, const double* __restrict__ R,
 // As one kernel a capsule was one chain of 19 node chunks on one CU (478 us at degree 16,
 // whether 1 capsule or 1000 ran), with the registers of the node phase (256, 42 spilled) held
 // through the transforms.  Apart, the node phase spreads a few capsules over the chip (8
-// capsules: 56 us in all) and holds 232 registers, none spilled; the transforms run 16 wavefronts
-// a CU on tables read coalesced.  8000 capsules of degree 16: 4.74 -> 3.02 ms (shape 0.25, nodes
-// 2.40, filter 0.39); 301 of degree 23 without bending: 1053 -> 316 us.
+// capsules: 55 us in all) and holds 220 registers, none spilled; the transforms run 16 wavefronts
+// a CU on tables read coalesced.  8000 capsules of degree 16: 4.74 -> 2.8 ms (shape 0.25, nodes
+// 2.14, filter 0.39); 301 of degree 23 without bending: 1053 -> 275 us.
 // Capsules: slot q holds capsule list[q], q < *cnt (list null: capsule c0 + q, q < n).
 struct Work {
   int n;              // slots (list null), or the most there can be
@@ -566,22 +570,37 @@ __global__ void __launch_bounds__(SH_THREADS)
 // A unit of work is a run of rings of one capsule; rings go in the order north, south, north
 // ... (ring 0, nt - 1, 1, nt - 2, ...).  A few capsules are cut into so many runs that the
 // workgroups in flight are all used (8 capsules of degree 16: one ring each), many are one run
-// each: a ring's sums do not depend on the cut.  Within a run, chunks of W consecutive nodes, one per
-// thread.  A chunk of W <= 2 np nodes touches at most three rings; ring r's coefficients live in
-// slot r % AB_SLOTS and are summed (with those of its pair) before the first chunk that touches
-// it, its outputs live in slot r % F_SLOTS until the DFT after the chunk that completes it.
+// each: a ring's sums do not depend on the cut.  Within a run, chunks of W consecutive lanes' nodes.
+// A chunk of W <= 2 rings touches at most three; ring r's coefficients live in slot
+// r % AB_SLOTS and are summed (with those of its pair) before the first chunk that touches it, its
+// outputs live in slot r % F_SLOTS until the DFT after the chunk that completes it.
+//
+// Lanes 4j .. 4j + 3 of a ring are the nodes phi_j, phi_j + pi, -phi_j, -phi_j + pi (j <= N; the
+// quads j = 0 and j = N hold two nodes twice).  With (A, B)_m the ring's coefficients the four
+// are the same sums up to signs: A cos and B sin over even and over odd m.  Each lane takes one of
+// the four sums and two exchanges give every lane its node's values.
+// A lane that reads A or B reads half of the LDS that one which needs both does and multiplies
+// half as much, and the DFT of the quads' sums and differences runs over N + 1 instead of 2 N
+// points: 3250 -> 2340 vector instructions a node with the reference's products taken from the
+// table.  8000 capsules of degree 16: 2.40 -> 2.14 ms; 301 of degree 23 without bending
+// 316 -> 275 us in all.  What is left waits half its time at two wavefronts per SIMD (the vector
+// units are busy 63 %, LDS 29 %), in no one place: without the coefficients' sums, the DFT, the
+// reference loads or the rest of the law it takes 0.34, 0.24, 0.26, 0.08 ms less; reading the
+// tables ten at a time in the sums changes nothing.
 // Registers: two wavefronts per SIMD.
 template <bool REF, bool BEND>
 __global__ void __launch_bounds__(ND_THREADS, 2)
     k_nodes(Tables T, Work wk, int most, double gs, double eb, double* __restrict__ refout) {
   extern __shared__ double lds[];
   constexpr int NK = BEND ? 5 : 3, NX = BEND ? NQ : 6;  // theta-derivatives, derivatives
+  constexpr int NKG = (NK + 1) / 2;
   const int tid = threadIdx.x;
-  const int N = T.N, nt = T.nt, np = T.np, hp = np / 2, NT = T.NT;
-  double2* te = reinterpret_cast<double2*>(lds);  // [np]
-  double2* cf = te + np;                          // [3][NT]
-  double2* AB = cf + 3 * NT;                      // [AB_SLOTS][N][3][NK]
-  double* F = reinterpret_cast<double*>(AB + AB_SLOTS * 3 * NK * N);  // [F_SLOTS][hp][2][6]
+  const int N = T.N, nt = T.nt, np = T.np, NT = T.NT;
+  const int RS = T.slots();
+  double2* te = reinterpret_cast<double2*>(lds);   // [np]
+  double2* cf = te + np;                           // [3][NT]
+  double* AB = reinterpret_cast<double*>(cf + 3 * NT);  // [AB_SLOTS][N][A, B][3][NK]
+  double* F = AB + AB_SLOTS * 6 * NK * N;          // [F_SLOTS][N + 1][even, odd m][cos, sin][6]
   for (int q = tid; q < np; q += ND_THREADS) te[q] = T.ef[q];
   // runs of rp rings (an even number, so that pairs stay together, or single rings)
   const int n = work_n(wk);
@@ -590,148 +609,186 @@ __global__ void __launch_bounds__(ND_THREADS, 2)
   int rp = (nt + want - 1) / want;
   if (rp > 1) rp += rp & 1;
   const int parts = (nt + rp - 1) / rp;
-  const int W = min(ND_THREADS, 2 * np);  // even: node pairs stay in one chunk
+  const int W = min(ND_THREADS, 2 * RS);  // a multiple of 4: quads stay in one chunk
   for (int u = blockIdx.x; u < n * parts; u += gridDim.x) {
     const int slot = u / parts, s0 = (u - slot * parts) * rp, s1 = min(s0 + rp, nt);
     __syncthreads();
     for (int t = tid; t < 3 * NT; t += ND_THREADS) cf[t] = wk.coef[(size_t)slot * 3 * NT + t];
     __syncthreads();
-    const int node0 = s0 * np, node1 = s1 * np;
+    const int node0 = s0 * RS, node1 = s1 * RS;
     int rnext = s0, rdone = s0;  // first ring without coefficients / without its DFT
     for (int n0 = node0; n0 < node1; n0 += W) {
       const int n1 = min(n0 + W, node1);
-      const int rhi = (n1 - 1) / np;  // last ring of the chunk
+      const int rhi = (n1 - 1) / RS;  // last ring of the chunk
       if (rhi >= rnext) {
-        // one thread per (ring pair, k, m) for the three coordinates: each table load feeds
-        // six FMAs and both rings of the pair, north E + O, south (-1)^k (E - O) of the sums over
-        // even and odd n - m
+        // one thread per (ring pair, two k, m) for the three coordinates: a coefficient read feeds
+        // two FMAs, a table load three and both rings of the pair, north E + O, south
+        // (-1)^k (E - O) of the sums over even and odd n - m
         const int p0 = rnext >> 1, p1 = rhi >> 1;
-        for (int t = tid; t < (p1 - p0 + 1) * NK * N; t += ND_THREADS) {
-          const int p = p0 + t / (NK * N), k = (t / N) % NK, m = t % N;
-          const double* P = T.Pfd + ((size_t)p * 5 + k) * NT;
-          double2 s[2][3];
+        for (int t = tid; t < (p1 - p0 + 1) * NKG * N; t += ND_THREADS) {
+          const int p = p0 + t / (NKG * N), k0 = 2 * ((t / N) % NKG), m = t % N;
+          const bool both = k0 + 1 < NK;
+          const double* P = T.Pfd + ((size_t)p * 5 + k0) * NT;
+          const int kp = both ? NT : 0;
+          double2 s[2][2][3];  // [k - k0][n - m even, odd][coordinate]
 #pragma unroll
-          for (int c = 0; c < 3; ++c) s[0][c] = s[1][c] = make_double2(0.0, 0.0);
+          for (int c = 0; c < 12; ++c) (&s[0][0][0])[c] = make_double2(0.0, 0.0);
           int q = m;  // tidx(N, d, m)
-          #pragma unroll 2
           for (int d = 0; d < N - m; d += 2) {
             const bool two = d + 1 < N - m;
             const int q1 = two ? q + N - d : q;
-            const double e0 = P[q], e1 = two ? P[q1] : 0.0;
+            double e[2][2] = {{P[q], P[q1]}, {P[kp + q], P[kp + q1]}};
+            if (!two) e[0][1] = e[1][1] = 0.0;
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
               const double2 v0 = cf[c * NT + q], v1 = cf[c * NT + q1];
-              s[0][c].x += e0 * v0.x, s[0][c].y += e0 * v0.y;
-              s[1][c].x += e1 * v1.x, s[1][c].y += e1 * v1.y;
+#pragma unroll
+              for (int i = 0; i < 2; ++i) {
+                s[i][0][c].x += e[i][0] * v0.x, s[i][0][c].y += e[i][0] * v0.y;
+                s[i][1][c].x += e[i][1] * v1.x, s[i][1][c].y += e[i][1] * v1.y;
+              }
             }
             q += 2 * (N - d) - 1;
           }
-          const double h = m == 0 ? 0.5 : 1.0, hs = (k & 1) ? -h : h;
+          const double h = m == 0 ? 0.5 : 1.0;
 #pragma unroll
-          for (int c = 0; c < 3; ++c) {
-            const int a = m * 3 * NK + c * NK + k;
-            AB[((2 * p) % AB_SLOTS) * 3 * NK * N + a] =
-                make_double2(h * (s[0][c].x + s[1][c].x), h * (s[0][c].y + s[1][c].y));
-            AB[((2 * p + 1) % AB_SLOTS) * 3 * NK * N + a] =
-                make_double2(hs * (s[0][c].x - s[1][c].x), hs * (s[0][c].y - s[1][c].y));
+          for (int i = 0; i < 2; ++i) {
+            if (i && !both) break;
+            const double hs = i ? -h : h;  // k0 is even
+            double* north = AB + (((2 * p) % AB_SLOTS) * N + m) * 6 * NK + k0 + i;
+            double* south = AB + (((2 * p + 1) % AB_SLOTS) * N + m) * 6 * NK + k0 + i;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+              const double2 E = s[i][0][c], O = s[i][1][c];
+              north[c * NK] = h * (E.x + O.x), north[c * NK + 3 * NK] = h * (E.y + O.y);
+              south[c * NK] = hs * (E.x - O.x), south[c * NK + 3 * NK] = hs * (E.y - O.y);
+            }
           }
         }
         rnext = 2 * p1 + 2;
       }
       __syncthreads();
-      // Lanes 2k and 2k + 1 take the node pair (jj, jj + np/2) of one ring, whose factors
-      // agree up to (-1)^m (phi -> phi + pi): lane 2k sums the even-m terms E and lane 2k + 1
-      // the odd-m terms O, both at phi_jj; after one exchange node jj holds E + O and node
-      // jj + np/2 holds E - O, and each lane goes on with its own node.
+      // lane bits: par, the parity of the m it sums and phi + pi; neg, B's sums and -phi
       if (n0 + tid < n1) {
         const int pn = n0 + tid;
-        const int par = pn & 1, pr = pn >> 1;
-        const int ring = pr / hp, jj = pr - ring * hp;
+        const int ring = pn / RS, jq = (pn - ring * RS) >> 2;
+        const int par = pn & 1;
+        const bool neg = pn & 2, twice = jq == 0 || jq == N;
+        const double sp = par ? -1.0 : 1.0, sn = neg ? -1.0 : 1.0;
         double X[3][NX];
 #pragma unroll
         for (int c = 0; c < 3; ++c)
 #pragma unroll
           for (int q = 0; q < NX; ++q) X[c][q] = 0.0;
-        int q = par * jj;  // (m jj) mod np
-        int dq = 2 * jj;
-        if (dq >= np) dq -= np;
-        const double2* ab = AB + (ring % AB_SLOTS) * 3 * NK * N + par * 3 * NK;
-        for (int m = par; m < N; m += 2, ab += 6 * NK) {
+        int q = par * jq;  // (m jq) mod np
+        const int dq = 2 * jq;
+        const double* ab = AB + ((ring % AB_SLOTS) * N + par) * 6 * NK + (neg ? 3 * NK : 0);
+        for (int m = par; m < N; m += 2, ab += 12 * NK) {
           const double2 w = te[q];
           q += dq;
           if (q >= np) q -= np;
-          const double m1 = (double)m, m2 = m1 * m1, m3 = m2 * m1, m4 = m2 * m2;
+          // phi-derivatives of A cos, or of -B sin
+          const double m1 = (double)m, m2 = -(m1 * m1);
+          const double w0 = neg ? -w.y : w.x, w1 = m1 * (neg ? -w.x : -w.y);
+          const double w2 = m2 * w0, w3 = m2 * w1, w4 = m2 * w2;
 #pragma unroll
           for (int c = 0; c < 3; ++c)
 #pragma unroll
             for (int kt = 0; kt < NK; ++kt) {
-              const double2 v = ab[c * NK + kt];
-              const double h0 = v.x * w.x - v.y * w.y, h1 = -v.x * w.y - v.y * w.x;
-              X[c][qidx(kt, 0)] += h0;
-              if (kt <= NK - 2) X[c][qidx(kt, 1)] += m1 * h1;
-              if (kt <= NK - 3) X[c][qidx(kt, 2)] -= m2 * h0;
-              if (BEND && kt <= 1) X[c][BEND ? qidx(kt, 3) : 0] -= m3 * h1;
-              if (BEND && kt == 0) X[c][BEND ? qidx(0, 4) : 0] += m4 * h0;
+              const double v = ab[c * NK + kt];
+              X[c][qidx(kt, 0)] += v * w0;
+              if (kt <= NK - 2) X[c][qidx(kt, 1)] += v * w1;
+              if (kt <= NK - 3) X[c][qidx(kt, 2)] += v * w2;
+              if (BEND && kt <= 1) X[c][BEND ? qidx(kt, 3) : 0] += v * w3;
+              if (BEND && kt == 0) X[c][BEND ? qidx(0, 4) : 0] += v * w4;
             }
         }
+        // even + odd m, minus at phi + pi; then A's + B's: at -phi what holds a sine changes its
+        // sign (B's in an even phi-derivative, A's in an odd one)
 #pragma unroll
         for (int c = 0; c < 3; ++c)
 #pragma unroll
-          for (int qq = 0; qq < NX; ++qq) {
-            const double other = swap_pair(X[c][qq]);
-            X[c][qq] = par ? other - X[c][qq] : X[c][qq] + other;
-          }
+          for (int kt = 0; kt < NK; ++kt)
+#pragma unroll
+            for (int kp = 0; kp < NK - kt; ++kp) {
+              double& v = X[c][qidx(kt, kp)];
+              double other = swap_pair(v);
+              v = sp * v + other;
+              other = swap_half(v);
+              v = kp & 1 ? sn * other + v : sn * v + other;
+            }
         Geom o;
         geometry<BEND>(X, o);
-        const long long nodes = (long long)nt * np;
+        const long long nodes = (long long)nt * RS;
         if (REF) {
           double* R = refout + pn;
-#pragma unroll
           for (int s = 0; s < 3; ++s) {
-            R[s * nodes] = o.G[s], R[(18 + s) * nodes] = o.b[s];
+            R[s * nodes] = o.G[s];
 #pragma unroll
-            for (int c = 0; c < 2; ++c)
-              R[(3 + 3 * c + s) * nodes] = o.Gd[c][s], R[(21 + 3 * c + s) * nodes] = o.bd[c][s];
+            for (int c = 0; c < 2; ++c) R[(3 + 3 * c + s) * nodes] = o.Gd[c][s];
+          }
+          R[9 * nodes] = o.G[0] * o.G[2] - o.G[1] * o.G[1];
 #pragma unroll
-            for (int e = 0; e < 3; ++e)
-              R[(9 + 3 * e + s) * nodes] = o.Gdd[e][s], R[(27 + 3 * e + s) * nodes] = o.bdd[e][s];
+          for (int c = 0; c < 2; ++c) {
+            R[(10 + c) * nodes] =
+                o.Gd[c][0] * o.G[2] + o.G[0] * o.Gd[c][2] - 2.0 * o.G[1] * o.Gd[c][1];
+#pragma unroll
+            for (int a = 0; a < 2; ++a) {
+              R[(12 + 2 * c + a) * nodes] = mixed(o.G, o.b, c, a);
+#pragma unroll
+              for (int l = 0; l < 2; ++l)
+                R[(16 + 4 * l + 2 * c + a) * nodes] = mixed_d(o.G, o.Gd[l], o.b, o.bd[l], c, a);
+#pragma unroll
+              for (int b = 0; b < 2; ++b) {
+                const int e = a + b;
+                R[ref_dd(e, c, a) * nodes] = mixed_dd(o.G, o.Gd, o.Gdd[e], o.b, o.bd, o.bdd[e],
+                                                      e >> 1, (e + 1) >> 1, c, a);
+              }
+            }
           }
         } else {
           double f[6];
           law<BEND>(o, T.ref + pn, nodes, gs, eb, f);
 #pragma unroll
           for (int k = 0; k < 3; ++k) f[3 + k] = o.n[k];
-          // the DFT needs v_j + v_{j + np/2} for even and v_j - v_{j + np/2} for odd m
-          double* Fo = F + ((size_t)((ring % F_SLOTS) * hp + jj) * 2 + par) * 6;
+          // the DFT needs v(phi) + v(phi + pi) for even and the difference for odd m, and of these
+          // the sum over phi and -phi for cos and the difference for sin
+          double* Fo = F + (((size_t)(ring % F_SLOTS) * (N + 1) + jq) * 4 + par * 2 + neg) * 6;
 #pragma unroll
           for (int k = 0; k < 6; ++k) {
-            const double other = swap_pair(f[k]);
-            Fo[k] = par ? other - f[k] : f[k] + other;
+            double v = f[k], other = swap_pair(v);
+            v = sp * v + other;
+            other = swap_half(v);
+            Fo[k] = twice ? (neg ? other : v) : sn * v + other;
           }
         }
       }
       __syncthreads();
-      if (!REF && n1 / np > rdone) {
-        // rings rdone .. n1 / np - 1 are complete: longitude DFT of their six outputs, a thread
-        // for two outputs of one (ring, m)
-        for (int t = tid; t < (n1 / np - rdone) * 3 * N; t += ND_THREADS) {
-          const int ring = rdone + t / (3 * N), g = (t / N) % 3, m = t % N;
-          const double2* v =
-              reinterpret_cast<const double2*>(F + ((size_t)(ring % F_SLOTS) * hp * 2 + (m & 1)) * 6) + g;
-          double2 s0 = {0.0, 0.0}, s1 = {0.0, 0.0};
+      if (!REF && n1 / RS > rdone) {
+        // rings rdone .. n1 / RS - 1 are complete: longitude DFT of their six outputs, a thread
+        // for the cos or the sin sums of one (ring, m); from the last thread on, since the first
+        // ones go on to the next coefficients without a barrier
+        for (int t = ND_THREADS - 1 - tid; t < (n1 / RS - rdone) * 2 * N; t += ND_THREADS) {
+          const int ring = rdone + t / (2 * N), m = (t >> 1) % N, sc = t & 1;
+          const double2* v = reinterpret_cast<const double2*>(
+              F + ((size_t)(ring % F_SLOTS) * (N + 1) * 4 + (m & 1) * 2 + sc) * 6);
+          const double* e = reinterpret_cast<const double*>(te) + sc;
+          double2 sum[3] = {{0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}};
           int q = 0;  // (m j) mod np
-          #pragma unroll 4
-          for (int j = 0; j < hp; ++j) {
-            const double2 e = te[q], w = v[6 * j];
+          #pragma unroll 3
+          for (int j = 0; j <= N; ++j, v += 12) {
+            const double ev = e[2 * q];
             q += m;
             if (q >= np) q -= np;
-            s0.x += w.x * e.x, s0.y += w.x * e.y;
-            s1.x += w.y * e.x, s1.y += w.y * e.y;
+#pragma unroll
+            for (int g = 0; g < 3; ++g) sum[g].x += v[g].x * ev, sum[g].y += v[g].y * ev;
           }
-          double2* r = wk.rows + (((size_t)slot * nt + ring) * N + m) * 6 + 2 * g;
-          r[0] = s0, r[1] = s1;
+          double* r =
+              reinterpret_cast<double*>(wk.rows + (((size_t)slot * nt + ring) * N + m) * 6) + sc;
+#pragma unroll
+          for (int g = 0; g < 3; ++g) r[4 * g] = sum[g].x, r[4 * g + 2] = sum[g].y;
         }
-        rdone = n1 / np;
+        rdone = n1 / RS;
       }
     }
   }
@@ -1323,7 +1380,7 @@ size_t lds_shape(const Tables& T) {
 }
 size_t lds_nodes(const Tables& T, bool bend) {
   return (size_t)(T.np + 3 * T.NT + AB_SLOTS * 3 * (bend ? 5 : 3) * T.N) * sizeof(double2) +
-         (size_t)F_SLOTS * T.np * 6 * sizeof(double);
+         (size_t)F_SLOTS * T.slots() * 6 * sizeof(double);
 }
 size_t lds_filter(const Tables& T) {
   const int NN = T.N * T.N;
@@ -1436,7 +1493,7 @@ int memb_plan_create(memb_plan** out, int L, int device) {
   if (!alloc(&p->coef, (size_t)p->slots * 3 * NT * sizeof(double2)) ||
       !alloc(&p->rows, (size_t)p->slots * nt * N * 6 * sizeof(double2)) ||
       !alloc(&p->list, (size_t)(p->slots + 1) * sizeof(int)) ||
-      !alloc(&p->ref, (size_t)NREF * nt * np * sizeof(double)))
+      !alloc(&p->ref, (size_t)NREF * nt * T.slots() * sizeof(double)))
     return bail(fail(p, MEMB_E_HIP, "hipMalloc of the plan's work arrays failed"));
   // the reference state: the unit sphere through the same kernels (sph.f90:56-70, 152-161)
   std::vector<double> sx((size_t)N * np2 * 3);
