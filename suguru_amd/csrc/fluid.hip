@@ -127,6 +127,13 @@ __device__ __forceinline__ int xcd_logical_block() {
   return (int)((blockIdx.x & 7u) * (nb >> 3) + (blockIdx.x >> 3));
 }
 
+// The same for any number nb of workgroups: the blockIdx-th of the launch, which the hardware
+// deals out over the eight XCDs in turn, as its place in eight contiguous ranges.
+__device__ __forceinline__ unsigned xcd_contiguous(unsigned id, unsigned nb) {
+  const unsigned x = id & 7u, q = nb >> 3, r = nb & 7u;
+  return x * q + min(x, r) + (id >> 3);
+}
+
 __device__ __forceinline__ int brev(int n, int logm) {
   return logm ? (int)(__brev((unsigned)n) >> (32 - logm)) : 0;
 }
@@ -586,8 +593,8 @@ __global__ void __launch_bounds__(TRI_MODES)
   }
 }
 
-// One pass over the array for the same elimination.  A workgroup takes TRI_MODES modes (the
-// lanes) and splits rows 0..ktot-2 into segments of TRS_LSEG rows, one wavefront each, held in
+// One pass over the array for the same elimination.  A workgroup takes TRS_MODES modes (the
+// lanes) and splits rows 0..ktot-2 into segments of TRS_LSEG rows, half a wavefront each, held in
 // registers with their reciprocal pivots.  Each recurrence of the sweep is affine in the value
 // it carries in from the previous segment, so
 //   forward  y_k = (r_k - a_k y_k-1) z_k      over a segment: y_end = y0_end + G y_in,
@@ -595,26 +602,33 @@ __global__ void __launch_bounds__(TRI_MODES)
 // where (y0, G) and (x0, H) come from a first pass started at 0 (G, H the products of the
 // coefficients -a z and -d).  The carried values are composed through LDS, then every segment
 // runs the sweep again from its true incoming value (the same expressions as k_tri inside a
-// segment; only the carried values are re-associated).  The last wavefront also solves the
+// segment; only the carried values are re-associated).  The last segment also solves the
 // last row (solver.f90:103-107, with its zero-pivot guard).  Reads the array and the pivots
 // once and writes the solution once, against twice each for k_tri.
+// Bound by memory, and by how much of it a compute unit keeps in flight: a workgroup loads, sweeps
+// and stores in turn.  With 64 modes only one of 1024 threads fits (its registers hold the rows and
+// pivots); 32 modes, whose rows are still two whole cache lines, let two take turns.  The systems of
+// one launch and the rows 2j, 2j + 1, which read the same pivots, run close together on one XCD.
+// 512 x 512 x 250, four systems: 1287 us with 64 modes, 1168 now (4.0 TB/s), 1460 with 16.
 constexpr int TRS_LSEG = 16;                   // rows per segment (registers per lane: 2 x 16)
-constexpr int TRS_MAXSEG = 16;                 // segments (wavefronts) per workgroup
-__global__ void __launch_bounds__(TRI_MODES * TRS_MAXSEG)
-    k_tri_seg(Systems sys, int itot, int jtot, int ktot) {
-  double* __restrict__ p = sys.p[blockIdx.y];
-  const double* __restrict__ a = sys.a[blockIdx.y];
-  const double* __restrict__ c = sys.c[blockIdx.y];
-  const double* __restrict__ ztab = sys.ztab[blockIdx.y];
-  __shared__ double fy0[TRS_MAXSEG][TRI_MODES], fg[TRS_MAXSEG][TRI_MODES];
-  __shared__ double bx0[TRS_MAXSEG][TRI_MODES], bh[TRS_MAXSEG][TRI_MODES];
-  __shared__ double xlast[TRI_MODES];
-  const int lane = threadIdx.x & (TRI_MODES - 1);
-  // the segment is uniform over the wavefront: its rows and coefficients live in scalars
-  const int s = __builtin_amdgcn_readfirstlane(threadIdx.x / TRI_MODES);
-  const int nseg = blockDim.x / TRI_MODES;
+constexpr int TRS_MAXSEG = 16;                 // segments per workgroup
+constexpr int TRS_MODES = 32;                  // modes per workgroup
+__global__ void __launch_bounds__(TRS_MODES * TRS_MAXSEG, 4)
+    k_tri_seg(Systems sys, int nsys, int itot, int jtot, int ktot) {
+  const unsigned blk = xcd_contiguous(blockIdx.x, gridDim.x), sy = blk % nsys;
+  double* __restrict__ p = sys.p[sy];
+  const double* __restrict__ a = sys.a[sy];
+  const double* __restrict__ c = sys.c[sy];
+  const double* __restrict__ ztab = sys.ztab[sy];
+  __shared__ double fy0[TRS_MAXSEG][TRS_MODES], fg[TRS_MAXSEG][TRS_MODES];
+  __shared__ double bx0[TRS_MAXSEG][TRS_MODES], bh[TRS_MAXSEG][TRS_MODES];
+  __shared__ double xlast[TRS_MODES];
+  __shared__ double sa[TRS_MAXSEG * TRS_LSEG], sc[TRS_MAXSEG * TRS_LSEG];
+  const int lane = threadIdx.x & (TRS_MODES - 1);
+  const int s = threadIdx.x / TRS_MODES;
+  const int nseg = blockDim.x / TRS_MODES;
   const long long plane = (long long)itot * jtot;
-  const long long m = (long long)blockIdx.x * TRI_MODES + lane;
+  const long long m = (long long)(blk / nsys) * TRS_MODES + lane;
   const bool live = m < plane;
   const int nk = ktot - 1;  // rows of the two recurrences
   const int k0 = min(s * TRS_LSEG, nk), n = min(TRS_LSEG, nk - k0);
@@ -628,14 +642,11 @@ __global__ void __launch_bounds__(TRI_MODES * TRS_MAXSEG)
   // (selects, so that the arrays stay in registers)
   // (every load is in bounds: lanes past the last mode read mode 0, then discard it)
   const long long mm = live ? m : 0;
-  // (a and c of the segment's rows first: uniform over the wavefront and before any store, they
-  // are scalar loads)
-  double r[TRS_LSEG], z[TRS_LSEG], ak[TRS_LSEG], ck[TRS_LSEG];
-#pragma unroll
-  for (int t = 0; t < TRS_LSEG; ++t) {
-    const int k = k0 + min(t, max(n - 1, 0));
-    ak[t] = a[k], ck[t] = c[k];
-  }
+  // a and c of the rows from LDS (as registers they would leave one workgroup a compute unit)
+  for (int q = threadIdx.x; q < nseg * TRS_LSEG; q += blockDim.x)
+    sa[q] = a[min(q, nk - 1)], sc[q] = c[min(q, nk - 1)];
+  const double *ak = sa + s * TRS_LSEG, *ck = sc + s * TRS_LSEG;
+  double r[TRS_LSEG], z[TRS_LSEG];
   const double alast = a[ktot - 1];
 #pragma unroll
   for (int t = 0; t < TRS_LSEG; ++t) {
@@ -644,6 +655,7 @@ __global__ void __launch_bounds__(TRI_MODES * TRS_MAXSEG)
     r[t] = live && n > 0 ? rv : 0.0;
     z[t] = live && n > 0 ? zv : 1.0;
   }
+  __syncthreads();
   // forward, first pass: the segment's map y_in -> y_end = y0 + G y_in
   {
     double y = 0.0, gm = 1.0;
@@ -1349,11 +1361,12 @@ int tri(fld_ctx* c, int n, double* const* a, const int* ne) {
     sys.p[i] = a[i], sys.a[i] = c->coef[ne[i]], sys.c[i] = c->coef[ne[i]] + g.ktot,
     sys.ztab[i] = c->ztab[ne[i]];
   const int nseg = std::max(1, (g.ktot - 1 + TRS_LSEG - 1) / TRS_LSEG);
-  const dim3 nb(nblocks(modes, TRI_MODES), (unsigned)n);
   if (nseg <= TRS_MAXSEG)
-    k_tri_seg<<<nb, TRI_MODES * nseg, 0, c->stream>>>(sys, g.itot, g.jtot, g.ktot);
+    k_tri_seg<<<nblocks(modes, TRS_MODES) * (unsigned)n, TRS_MODES * nseg, 0, c->stream>>>(
+        sys, n, g.itot, g.jtot, g.ktot);
   else
-    k_tri<<<nb, TRI_MODES, 0, c->stream>>>(sys, g.itot, g.jtot, g.ktot);
+    k_tri<<<dim3(nblocks(modes, TRI_MODES), (unsigned)n), TRI_MODES, 0, c->stream>>>(
+        sys, g.itot, g.jtot, g.ktot);
   HIPF(c, hipGetLastError());
   return FLD_OK;
 }
