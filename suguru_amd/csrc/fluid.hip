@@ -729,19 +729,16 @@ __global__ void __launch_bounds__(TRS_MODES * TRS_MAXSEG, 4)
 // mom.f90:9-50 (momxad)
 template <class A>
 __device__ __forceinline__ double momxad(const FGrid& g, const A& Uo, const A& Vo, const A& Wo,
-                                         const A& Uoo, const A& Voo, const A& Woo) {
+                                         const A& Uoo, const A& Voo, const A& Woo, double uwkm,
+                                         double uwkp, double uwkmo, double uwkpo) {
   const double uuip = 0.25 * (Uo(1, 0, 0) + Uo(0, 0, 0)) * (Uo(1, 0, 0) + Uo(0, 0, 0));
   const double uuim = 0.25 * (Uo(-1, 0, 0) + Uo(0, 0, 0)) * (Uo(-1, 0, 0) + Uo(0, 0, 0));
   const double uvjp = 0.25 * (Uo(0, 1, 0) + Uo(0, 0, 0)) * (Vo(1, 0, 0) + Vo(0, 0, 0));
   const double uvjm = 0.25 * (Uo(0, -1, 0) + Uo(0, 0, 0)) * (Vo(1, -1, 0) + Vo(0, -1, 0));
-  const double uwkp = 0.25 * (Uo(0, 0, 1) + Uo(0, 0, 0)) * (Wo(1, 0, 0) + Wo(0, 0, 0));
-  const double uwkm = 0.25 * (Uo(0, 0, -1) + Uo(0, 0, 0)) * (Wo(1, 0, -1) + Wo(0, 0, -1));
   const double uuipo = 0.25 * (Uoo(1, 0, 0) + Uoo(0, 0, 0)) * (Uoo(1, 0, 0) + Uoo(0, 0, 0));
   const double uuimo = 0.25 * (Uoo(-1, 0, 0) + Uoo(0, 0, 0)) * (Uoo(-1, 0, 0) + Uoo(0, 0, 0));
   const double uvjpo = 0.25 * (Uoo(0, 1, 0) + Uoo(0, 0, 0)) * (Voo(1, 0, 0) + Voo(0, 0, 0));
   const double uvjmo = 0.25 * (Uoo(0, -1, 0) + Uoo(0, 0, 0)) * (Voo(1, -1, 0) + Voo(0, -1, 0));
-  const double uwkpo = 0.25 * (Uoo(0, 0, 1) + Uoo(0, 0, 0)) * (Woo(1, 0, 0) + Woo(0, 0, 0));
-  const double uwkmo = 0.25 * (Uoo(0, 0, -1) + Uoo(0, 0, 0)) * (Woo(1, 0, -1) + Woo(0, 0, -1));
   return g.dxi * ((1.5 * (-uuip + uuim)) - (.5 * (-uuipo + uuimo))) +
          g.dyi * ((1.5 * (-uvjp + uvjm)) - (.5 * (-uvjpo + uvjmo))) +
          g.dzi * ((1.5 * (-uwkp + uwkm)) - (.5 * (-uwkpo + uwkmo)));
@@ -750,19 +747,16 @@ __device__ __forceinline__ double momxad(const FGrid& g, const A& Uo, const A& V
 // mom.f90:158-199 (momyad)
 template <class A>
 __device__ __forceinline__ double momyad(const FGrid& g, const A& Uo, const A& Vo, const A& Wo,
-                                         const A& Uoo, const A& Voo, const A& Woo) {
+                                         const A& Uoo, const A& Voo, const A& Woo, double wvkm,
+                                         double wvkp, double wvkmo, double wvkpo) {
   const double uvip = 0.25 * (Uo(0, 0, 0) + Uo(0, 1, 0)) * (Vo(0, 0, 0) + Vo(1, 0, 0));
   const double uvim = 0.25 * (Uo(-1, 0, 0) + Uo(-1, 1, 0)) * (Vo(0, 0, 0) + Vo(-1, 0, 0));
   const double vvjp = 0.25 * (Vo(0, 0, 0) + Vo(0, 1, 0)) * (Vo(0, 0, 0) + Vo(0, 1, 0));
   const double vvjm = 0.25 * (Vo(0, 0, 0) + Vo(0, -1, 0)) * (Vo(0, 0, 0) + Vo(0, -1, 0));
-  const double wvkp = 0.25 * (Wo(0, 0, 0) + Wo(0, 1, 0)) * (Vo(0, 0, 1) + Vo(0, 0, 0));
-  const double wvkm = 0.25 * (Wo(0, 0, -1) + Wo(0, 1, -1)) * (Vo(0, 0, -1) + Vo(0, 0, 0));
   const double uvipo = 0.25 * (Uoo(0, 0, 0) + Uoo(0, 1, 0)) * (Voo(0, 0, 0) + Voo(1, 0, 0));
   const double uvimo = 0.25 * (Uoo(-1, 0, 0) + Uoo(-1, 1, 0)) * (Voo(0, 0, 0) + Voo(-1, 0, 0));
   const double vvjpo = 0.25 * (Voo(0, 0, 0) + Voo(0, 1, 0)) * (Voo(0, 0, 0) + Voo(0, 1, 0));
   const double vvjmo = 0.25 * (Voo(0, 0, 0) + Voo(0, -1, 0)) * (Voo(0, 0, 0) + Voo(0, -1, 0));
-  const double wvkpo = 0.25 * (Woo(0, 0, 0) + Woo(0, 1, 0)) * (Voo(0, 0, 1) + Voo(0, 0, 0));
-  const double wvkmo = 0.25 * (Woo(0, 0, -1) + Woo(0, 1, -1)) * (Voo(0, 0, -1) + Voo(0, 0, 0));
   return g.dxi * ((1.5 * (-uvip + uvim)) - (.5 * (-uvipo + uvimo))) +
          g.dyi * ((1.5 * (-vvjp + vvjm)) - (.5 * (-vvjpo + vvjmo))) +
          g.dzi * ((1.5 * (-wvkp + wvkm)) - (.5 * (-wvkpo + wvkmo)));
@@ -771,31 +765,46 @@ __device__ __forceinline__ double momyad(const FGrid& g, const A& Uo, const A& V
 // mom.f90:286-327 (momzad)
 template <class A>
 __device__ __forceinline__ double momzad(const FGrid& g, const A& Uo, const A& Vo, const A& Wo,
-                                         const A& Uoo, const A& Voo, const A& Woo) {
+                                         const A& Uoo, const A& Voo, const A& Woo, double wwkm,
+                                         double wwkp, double wwkmo, double wwkpo) {
   const double uwip = 0.25 * (Wo(0, 0, 0) + Wo(1, 0, 0)) * (Uo(0, 0, 0) + Uo(0, 0, 1));
   const double uwim = 0.25 * (Wo(0, 0, 0) + Wo(-1, 0, 0)) * (Uo(-1, 0, 0) + Uo(-1, 0, 1));
   const double vwjp = 0.25 * (Wo(0, 0, 0) + Wo(0, 1, 0)) * (Vo(0, 0, 0) + Vo(0, 0, 1));
   const double vwjm = 0.25 * (Wo(0, 0, 0) + Wo(0, -1, 0)) * (Vo(0, -1, 0) + Vo(0, -1, 1));
-  const double wwkp = 0.25 * (Wo(0, 0, 0) + Wo(0, 0, 1)) * (Wo(0, 0, 0) + Wo(0, 0, 1));
-  const double wwkm = 0.25 * (Wo(0, 0, 0) + Wo(0, 0, -1)) * (Wo(0, 0, 0) + Wo(0, 0, -1));
   const double uwipo = 0.25 * (Woo(0, 0, 0) + Woo(1, 0, 0)) * (Uoo(0, 0, 0) + Uoo(0, 0, 1));
   const double uwimo = 0.25 * (Woo(0, 0, 0) + Woo(-1, 0, 0)) * (Uoo(-1, 0, 0) + Uoo(-1, 0, 1));
   const double vwjpo = 0.25 * (Woo(0, 0, 0) + Woo(0, 1, 0)) * (Voo(0, 0, 0) + Voo(0, 0, 1));
   const double vwjmo = 0.25 * (Woo(0, 0, 0) + Woo(0, -1, 0)) * (Voo(0, -1, 0) + Voo(0, -1, 1));
-  const double wwkpo = 0.25 * (Woo(0, 0, 0) + Woo(0, 0, 1)) * (Woo(0, 0, 0) + Woo(0, 0, 1));
-  const double wwkmo = 0.25 * (Woo(0, 0, 0) + Woo(0, 0, -1)) * (Woo(0, 0, 0) + Woo(0, 0, -1));
   return g.dxi * ((1.5 * (-uwip + uwim)) - (.5 * (-uwipo + uwimo))) +
          g.dyi * ((1.5 * (-vwjp + vwjm)) - (.5 * (-vwjpo + vwjmo))) +
          g.dzi * ((1.5 * (-wwkp + wwkm)) - (.5 * (-wwkpo + wwkmo)));
 }
 
-// field(i + di, j + dj, k + dk) from the k-1, k, k+1 planes staged in LDS (row pitch w)
+// field(i + di, j + dj, k + dk), dk = 0 or 1, from the planes k and k+1 staged in LDS (row pitch w)
 struct LAcc {
-  const double* pl[3];  // &plane(i, j) of planes k-1, k, k+1
+  const double* pl[2];  // &plane(i, j) of planes k, k+1
   int w;
   __device__ __forceinline__ double operator()(int di, int dj, int dk) const {
-    return pl[dk + 1][di + w * dj];
+    return pl[dk][di + w * dj];
   }
+};
+
+// The fluxes through the face between planes k and k+1 (uwkp, wvkp, wwkp of mom.f90): the face
+// below plane k+1 is the same, with its sums the other way round (uwkm, wvkm, wwkm), so the march
+// carries them to the next plane.
+struct FaceK {
+  double u, v, w;
+};
+template <class A>
+__device__ __forceinline__ FaceK face_k(const A& U, const A& V, const A& W) {
+  return {0.25 * (U(0, 0, 1) + U(0, 0, 0)) * (W(1, 0, 0) + W(0, 0, 0)),
+          0.25 * (W(0, 0, 0) + W(0, 1, 0)) * (V(0, 0, 1) + V(0, 0, 0)),
+          0.25 * (W(0, 0, 0) + W(0, 0, 1)) * (W(0, 0, 0) + W(0, 0, 1))};
+}
+
+// p at a cell and its three next neighbours, and the forces there
+struct CellIn {
+  double p, pi, pj, pk, fx, fy, fz;
 };
 
 // The three right-hand sides of fftuvw.f90:30-105 at one interior cell, scaled by Rep
@@ -803,36 +812,44 @@ struct LAcc {
 template <class A>
 __device__ __forceinline__ void mom_cell(const FGrid& g, double rep, double dt, const A& U,
                                          const A& V, const A& W, const A& UU, const A& VV,
-                                         const A& WW, const double* __restrict__ p,
-                                         long long q, double fxq, double fyq, double fzq, int k,
-                                         double& du, double& dv, double& dw) {
-  const double durk = (-g.dxi * ((p[q + 1] - p[q]))) + fxq;
-  const double dvrk = (-g.dyi * (p[q + g.sy] - p[q])) + fyq;
-  const double dwrk = (-g.dzi * (p[q + g.sz] - p[q])) + fzq;
+                                         const A& WW, const CellIn& in, int k,
+                                         FaceK& f, FaceK& fo, double& du, double& dv,
+                                         double& dw) {
+  const FaceK fp = face_k(U, V, W), fpo = face_k(UU, VV, WW);
+  const double durk = (-g.dxi * ((in.pi - in.p))) + in.fx;
+  const double dvrk = (-g.dyi * (in.pj - in.p)) + in.fy;
+  const double dwrk = (-g.dzi * (in.pk - in.p)) + in.fz;
   du = -durk, dv = -dvrk, dw = -dwrk;
-  du = du - momxad(g, U, V, W, UU, VV, WW);
-  dv = dv - momyad(g, U, V, W, UU, VV, WW);
-  dw = dw - momzad(g, U, V, W, UU, VV, WW);
+  du = du - momxad(g, U, V, W, UU, VV, WW, f.u, fp.u, fo.u, fpo.u);
+  dv = dv - momyad(g, U, V, W, UU, VV, WW, f.v, fp.v, fo.v, fpo.v);
+  dw = dw - momzad(g, U, V, W, UU, VV, WW, f.w, fp.w, fo.w, fpo.w);
   du = du - (U(0, 0, 0) / dt);
   dv = dv - (V(0, 0, 0) / dt);
   dw = dw - (W(0, 0, 0) / dt);
   du = du * rep;
   dv = dv * rep;
   dw = (k == g.ktot) ? 0.0 : dw * rep;
+  f = fp, fo = fpo;
 }
 
 // fftuvw.f90:30-105 per interior cell, k-marching, into the compact arrays: a workgroup owns
-// an MR_TI x MR_TJ tile of (i, j) columns and KB consecutive planes.  The six velocity fields' planes k-1, k, k+1 of the tile plus a
-// one-cell apron sit in an LDS ring of three; each step prefetches plane k+2 into registers
-// while it computes plane k, then stores it over plane k-1.  Every velocity value is read
-// from HBM once per tile (plus the apron and the two extra planes); p and the forces are read
-// directly.
+// an MR_TI x MR_TJ tile of (i, j) columns and KB consecutive planes.  The six velocity fields'
+// planes k and k+1 of the tile plus a one-cell apron sit in LDS; the fluxes through the face below
+// plane k are carried in registers, so plane k-1 is not needed.  Each step starts the loads of
+// plane k+2 and of the next cell's p and forces, computes plane k from what is there, and stores
+// plane k+2 over plane k: no load is waited for before the arithmetic.  Every velocity value is
+// read from HBM once per tile (plus the apron and the two extra planes).
+// Bound by memory latency: 512 x 512 x 250 cells (6.9 GB) 1610 us with three planes in LDS and p
+// and the forces loaded at their use, 1650 with the carried fluxes alone, 1484 with both (4.6 TB/s).
+// At most three workgroups a compute unit: held to 128 registers for four, it spills (3330 us).
+// 64 x 4 tiles: 1580; the tiles of an XCD made contiguous: slower (1650 -> 1700 before the
+// earlier loads).
 constexpr int MR_TI = 32, MR_TJ = 8;
 constexpr int MR_W = MR_TI + 2, MR_H = MR_TJ + 2, MR_PL = MR_W * MR_H;
 constexpr int MR_T = MR_TI * MR_TJ;
 constexpr int MR_LD = (MR_PL + MR_T - 1) / MR_T;  // apron-plane cells per thread
 
-__global__ void __launch_bounds__(MR_T)
+__global__ void __launch_bounds__(MR_T, 3)
     k_mom_rhs_march(FGrid g, int KB, double rep, double dt, const double* __restrict__ uo,
                     const double* __restrict__ vo, const double* __restrict__ wo,
                     const double* __restrict__ uoo, const double* __restrict__ voo,
@@ -840,7 +857,7 @@ __global__ void __launch_bounds__(MR_T)
                     const double* __restrict__ fx, const double* __restrict__ fy,
                     const double* __restrict__ fz, double* __restrict__ cu,
                     double* __restrict__ cv, double* __restrict__ cw) {
-  __shared__ double sp[6][3][MR_PL];
+  __shared__ double sp[6][2][MR_PL];
   const double* src[6] = {uo, vo, wo, uoo, voo, woo};
   const int tx = threadIdx.x % MR_TI, ty = threadIdx.x / MR_TI;
   const int i0 = blockIdx.x * MR_TI, j0 = blockIdx.y * MR_TJ;  // apron origin (halo index)
@@ -856,8 +873,8 @@ __global__ void __launch_bounds__(MR_T)
     ok[r] = c < MR_PL && i0 + ii <= g.itot + 1 && j0 + jj <= g.jtot + 1;
     off[r] = ok[r] ? (long long)(i0 + ii) + g.sy * (j0 + jj) : 0;
   }
-  // planes kb0-1, kb0, kb0+1 into ring slots 0, 1, 2 (plane kk lives in slot (kk-kb0+1) % 3)
-  for (int s0 = 0; s0 < 3; ++s0) {
+  // planes kb0-1 and kb0 into slots 0 and 1 (plane kk lives in slot (kk-kb0+1) & 1)
+  for (int s0 = 0; s0 < 2; ++s0) {
     const long long kz = g.sz * (kb0 - 1 + s0);
 #pragma unroll
     for (int f = 0; f < 6; ++f)
@@ -869,10 +886,20 @@ __global__ void __launch_bounds__(MR_T)
   const int i = i0 + tx + 1, j = j0 + ty + 1;
   const bool live = i <= g.itot && j <= g.jtot;
   const int me = (tx + 1) + MR_W * (ty + 1);
-  for (int k = kb0; k <= kb1; ++k) {
-    const int sm = (k - kb0) % 3, s0 = (k - kb0 + 1) % 3, sp1 = (k - kb0 + 2) % 3;
+  FaceK face{}, faceo{};
+  const long long q0 = live ? fidx(g, i, j, 0) : 0;
+  CellIn in{}, nx{};
+  nx.pk = live ? p[q0 + g.sz * kb0] : 0.0;
+  // plane kb0-1 gives the faces below plane kb0 alone
+  for (int k = kb0 - 1; k <= kb1; ++k) {
+    const int s0 = (k - kb0 + 1) & 1, sp1 = s0 ^ 1;
     // prefetch plane k + 2 (the next step's k + 1)
     const bool more = k + 2 <= kb1 + 1;
+    in = nx;
+    if (live && more) {
+      const long long q = q0 + g.sz * (k + 1);
+      nx = CellIn{in.pk, p[q + 1], p[q + g.sy], p[q + g.sz], fx[q], fy[q], fz[q]};
+    }
     double pre[6][MR_LD];
     if (more) {
       const long long kz = g.sz * (k + 2);
@@ -882,27 +909,27 @@ __global__ void __launch_bounds__(MR_T)
         for (int r = 0; r < MR_LD; ++r) pre[f][r] = ok[r] ? src[f][off[r] + kz] : 0.0;
     }
     if (live) {
-      const long long q = fidx(g, i, j, k);
-      const double fxq = fx[q], fyq = fy[q], fzq = fz[q];
       LAcc A[6];
 #pragma unroll
-      for (int f = 0; f < 6; ++f)
-        A[f] = LAcc{{&sp[f][sm][me], &sp[f][s0][me], &sp[f][sp1][me]}, MR_W};
-      double du, dv, dw;
-      mom_cell(g, rep, dt, A[0], A[1], A[2], A[3], A[4], A[5], p, q, fxq, fyq, fzq, k, du, dv,
-               dw);
-      const long long t = (long long)(i - 1) + (long long)g.itot * ((j - 1) + (long long)g.jtot * (k - 1));
-      cu[t] = du;
-      cv[t] = dv;
-      cw[t] = dw;
+      for (int f = 0; f < 6; ++f) A[f] = LAcc{{&sp[f][s0][me], &sp[f][sp1][me]}, MR_W};
+      if (k < kb0) {
+        face = face_k(A[0], A[1], A[2]), faceo = face_k(A[3], A[4], A[5]);
+      } else {
+        double du, dv, dw;
+        mom_cell(g, rep, dt, A[0], A[1], A[2], A[3], A[4], A[5], in, k, face, faceo, du, dv, dw);
+        const long long t = (long long)(i - 1) + (long long)g.itot * ((j - 1) + (long long)g.jtot * (k - 1));
+        cu[t] = du;
+        cv[t] = dv;
+        cw[t] = dw;
+      }
     }
-    __syncthreads();  // plane k-1 is no longer read
+    __syncthreads();  // plane k is no longer read
     if (more) {
 #pragma unroll
       for (int f = 0; f < 6; ++f)
 #pragma unroll
         for (int r = 0; r < MR_LD; ++r)
-          if (threadIdx.x + r * MR_T < MR_PL) sp[f][sm][threadIdx.x + r * MR_T] = pre[f][r];
+          if (threadIdx.x + r * MR_T < MR_PL) sp[f][s0][threadIdx.x + r * MR_T] = pre[f][r];
     }
     __syncthreads();
   }
@@ -1583,8 +1610,9 @@ int fld_fftuvw_dev(fld_ctx* c, double* unew, double* vnew, double* wnew, const d
   if (!(unew && vnew && wnew && uo && vo && wo && uoo && voo && woo && pnew && fx && fy && fz))
     return fail(c, FLD_E_ARG, "null field");
   HIPF(c, hipSetDevice(c->device));
-  // planes per workgroup: 32 (two extra planes read per 32) while that gives a workgroup for each
-  // of the two the LDS lets a compute unit hold, fewer on smaller grids, where the march along k
+  // planes per workgroup: 32 (two extra planes read per 32) while that gives two workgroups a
+  // compute unit (asking for four changes nothing: 441 against 439 us for a step at
+  // 256 x 128 x 128), fewer on smaller grids, where the march along k
   // is a serial chain of plane loads (64^3 cells: 66 us with 32 planes, 32 workgroups)
   const unsigned ti = (unsigned)((c->grid.itot + MR_TI - 1) / MR_TI);
   const unsigned tj = (unsigned)((c->grid.jtot + MR_TJ - 1) / MR_TJ);
