@@ -342,20 +342,12 @@ struct XLine {
   static constexpr int M = Line::N, TPL = Line::TPL, PER = REG_T / TPL, PITCH = fft::pad(M) + 1;
 };
 
+// values 2q, 2q + 1 (q = t + TPL u) of x line (j, k): from `src`, the line's first value, or with
+// FILL the divergence
 template <int LOGM, bool FILL>
-__global__ void __launch_bounds__(REG_T)
-    k_x_fwd(Arrays arr, Rows rs, Rows rd, int logj, int lines, const double2* __restrict__ tw,
-            const double2* __restrict__ twm, FillSrc fs) {
-  using X = XLine<LOGM>;
-  constexpr int M = X::M, TPL = X::TPL;
-  constexpr bool WG = LOGM > 9;
-  __shared__ double2 sm[X::PER * X::PITCH];
-  const int t = threadIdx.x & (TPL - 1), own = threadIdx.x / TPL;
-  const int line = blockIdx.x * X::PER + own;
-  const bool live = line < lines;
-  const int ln = live ? line : lines - 1, k = ln >> logj, j = ln & ((1 << logj) - 1);
-  double2* buf = sm + own * X::PITCH;
-  double2 a[8];
+__device__ __forceinline__ void x_load(double2 (&a)[8], int t, const double* src,
+                                       const FillSrc& fs, int j, int k) {
+  constexpr int TPL = XLine<LOGM>::TPL;
   if constexpr (FILL) {
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
@@ -371,10 +363,19 @@ __global__ void __launch_bounds__(REG_T)
                           ((w0.y - w1.y) * fs.cz + (v0.y - v1.y) * fs.cy + (u0.y - u1.y) * fs.cx));
     }
   } else {
-    const double* src = arr.src[blockIdx.y] + rs.at(j, k);
 #pragma unroll
     for (int u = 0; u < 8; ++u) a[u] = load2(src + 2 * (t + TPL * u));
   }
+}
+
+// the line's values into its packed half spectrum, a[u] = values 2q, 2q + 1 of it
+template <int LOGM>
+__device__ __forceinline__ void x_spectrum(double2 (&a)[8], double2* buf, int t,
+                                           const double2* __restrict__ tw,
+                                           const double2* __restrict__ twm) {
+  using X = XLine<LOGM>;
+  constexpr int M = X::M, TPL = X::TPL;
+  constexpr bool WG = LOGM > 9;
   typename X::Line lw;
   lw.load(twm, t);
   lw.template run<false>(a, buf, t);
@@ -383,7 +384,6 @@ __global__ void __launch_bounds__(REG_T)
 #pragma unroll
   for (int u = 0; u < 8; ++u) buf[fft::pad(t + TPL * u)] = a[u];
   fft::line_sync<WG>();
-  double* dst = arr.dst[blockIdx.y] + rd.at(j, k);
 #pragma unroll
   for (int u = 0; u < 8; ++u) {
     const int q = t + TPL * u;
@@ -392,27 +392,19 @@ __global__ void __launch_bounds__(REG_T)
     const double2 O = make_double2(0.5 * (a[u].y + b.y), -0.5 * (a[u].x - b.x));
     double2 v = fft::add(E, fft::mul(w, O));
     if (u == 0 && t == 0) v = make_double2(a[0].x + a[0].y, a[0].x - a[0].y);
-    if (live) store2(dst + 2 * q, v);
+    a[u] = v;
   }
 }
 
+// and back
 template <int LOGM>
-__global__ void __launch_bounds__(REG_T)
-    k_x_inv(Arrays arr, Rows rs, Rows rd, int logj, int lines, const double2* __restrict__ tw,
-            const double2* __restrict__ twm) {
+__device__ __forceinline__ void x_values(double2 (&a)[8], double2* buf, int t,
+                                         const double2* __restrict__ tw,
+                                         const double2* __restrict__ twm) {
   using X = XLine<LOGM>;
   constexpr int M = X::M, TPL = X::TPL;
   constexpr bool WG = LOGM > 9;
-  __shared__ double2 sm[X::PER * X::PITCH];
-  const int t = threadIdx.x & (TPL - 1), own = threadIdx.x / TPL;
-  const int line = blockIdx.x * X::PER + own;
-  const bool live = line < lines;
-  const int ln = live ? line : lines - 1, k = ln >> logj, j = ln & ((1 << logj) - 1);
-  double2* buf = sm + own * X::PITCH;
-  const double* src = arr.src[blockIdx.y] + rs.at(j, k);
-  double2 a[8];
-#pragma unroll
-  for (int u = 0; u < 8; ++u) a[u] = load2(src + 2 * (t + TPL * u));
+  fft::line_sync<WG>();
 #pragma unroll
   for (int u = 0; u < 8; ++u) buf[fft::pad(t + TPL * u)] = a[u];
   fft::line_sync<WG>();
@@ -433,11 +425,47 @@ __global__ void __launch_bounds__(REG_T)
   lw.load(twm, t);
   lw.template run<true>(a, buf, t);
   const double sc = 1.0 / (double)M;
+#pragma unroll
+  for (int u = 0; u < 8; ++u) a[u] = make_double2(a[u].x * sc, a[u].y * sc);
+}
+
+template <int LOGM, bool FILL>
+__global__ void __launch_bounds__(REG_T)
+    k_x_fwd(Arrays arr, Rows rs, Rows rd, int logj, int lines, const double2* __restrict__ tw,
+            const double2* __restrict__ twm, FillSrc fs) {
+  using X = XLine<LOGM>;
+  __shared__ double2 sm[X::PER * X::PITCH];
+  const int t = threadIdx.x & (X::TPL - 1), own = threadIdx.x / X::TPL;
+  const int line = blockIdx.x * X::PER + own;
+  const bool live = line < lines;
+  const int ln = live ? line : lines - 1, k = ln >> logj, j = ln & ((1 << logj) - 1);
+  double2 a[8];
+  x_load<LOGM, FILL>(a, t, FILL ? nullptr : arr.src[blockIdx.y] + rs.at(j, k), fs, j, k);
+  x_spectrum<LOGM>(a, sm + own * X::PITCH, t, tw, twm);
   double* dst = arr.dst[blockIdx.y] + rd.at(j, k);
   if (live) {
 #pragma unroll
-    for (int u = 0; u < 8; ++u)
-      store2(dst + 2 * (t + TPL * u), make_double2(a[u].x * sc, a[u].y * sc));
+    for (int u = 0; u < 8; ++u) store2(dst + 2 * (t + X::TPL * u), a[u]);
+  }
+}
+
+template <int LOGM>
+__global__ void __launch_bounds__(REG_T)
+    k_x_inv(Arrays arr, Rows rs, Rows rd, int logj, int lines, const double2* __restrict__ tw,
+            const double2* __restrict__ twm) {
+  using X = XLine<LOGM>;
+  __shared__ double2 sm[X::PER * X::PITCH];
+  const int t = threadIdx.x & (X::TPL - 1), own = threadIdx.x / X::TPL;
+  const int line = blockIdx.x * X::PER + own;
+  const bool live = line < lines;
+  const int ln = live ? line : lines - 1, k = ln >> logj, j = ln & ((1 << logj) - 1);
+  double2 a[8];
+  x_load<LOGM, false>(a, t, arr.src[blockIdx.y] + rs.at(j, k), FillSrc{}, j, k);
+  x_values<LOGM>(a, sm + own * X::PITCH, t, tw, twm);
+  double* dst = arr.dst[blockIdx.y] + rd.at(j, k);
+  if (live) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) store2(dst + 2 * (t + X::TPL * u), a[u]);
   }
 }
 
@@ -529,6 +557,113 @@ __global__ void __launch_bounds__(YLine<LOGN>::T)
 #pragma unroll
       for (int u = 0; u < 8; ++u)
         p[(t + Y::TPL * u) * pitch] = make_double2(a[u].x * sc, a[u].y * sc);
+    }
+  }
+}
+
+// Planes of up to 8192 cells (itot, jtot >= 32): x and y transforms of a plane in one workgroup, the
+// plane between them in LDS.  Bound by latency: on such grids a launch and its drain cost more than
+// the pass over memory.  A step at 64^3 takes 68 us like this (82 with a launch per direction: 4.6
+// and 5.2 us, against 6.6 for both), 64 x 64 x 256 126 (152), 128 x 64 x 250 218 (250), 32 x 32 x 16
+// 47 (59).  A plane of 16384 values and the exchange buffer do not fit in LDS.
+template <int LOGI, int LOGJ>
+struct Plane {
+  using X = XLine<LOGI - 1>;
+  using Y = YLine<LOGJ>;
+  static constexpr int PAIRS = 1 << (LOGI - 1), J = 1 << LOGJ;
+  // rows of the columns that a wavefront's lanes hold together lie in different banks
+  static constexpr int PITCH = PAIRS + (Y::COLS < 16 ? Y::COLS : 0);
+  static constexpr int EX = X::PER * X::PITCH > Y::COLS * Y::PITCH ? X::PER * X::PITCH
+                                                                   : Y::COLS * Y::PITCH;
+};
+
+template <int LOGI, int LOGJ, bool FILL>
+__global__ void __launch_bounds__(REG_T)
+    k_plane_fwd(Arrays arr, Rows rs, const double2* __restrict__ tw,
+                const double2* __restrict__ twm, const double2* __restrict__ twn, FillSrc fs) {
+  using P = Plane<LOGI, LOGJ>;
+  using X = typename P::X;
+  using Y = typename P::Y;
+  static_assert(Y::T == REG_T, "one workgroup shape for both directions");
+  __shared__ double2 pl[P::J * P::PITCH], ex[P::EX];
+  const int k = blockIdx.x;
+  double2 a[8], row[8];
+  for (int j0 = 0; j0 < P::J; j0 += X::PER) {
+    const int t = threadIdx.x & (X::TPL - 1), own = threadIdx.x / X::TPL;
+    const bool live = j0 + own < P::J;
+    const int j = live ? j0 + own : P::J - 1;
+    x_load<LOGI - 1, FILL>(a, t, FILL ? nullptr : arr.src[blockIdx.y] + rs.at(j, k), fs, j, k);
+    x_spectrum<LOGI - 1>(a, ex + own * X::PITCH, t, tw, twm);
+    if (live) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) pl[j * P::PITCH + t + X::TPL * u] = a[u];
+    }
+  }
+  __syncthreads();
+  double2* out = reinterpret_cast<double2*>(arr.dst[blockIdx.y]) + (long long)k * P::PAIRS * P::J;
+  typename Y::Line lw;
+  const int col = threadIdx.x & (Y::COLS - 1), t = threadIdx.x / Y::COLS;
+  lw.load(twn, t);
+  for (int c0 = 0; c0 < P::PAIRS; c0 += Y::COLS) {
+    const bool live = c0 + col < P::PAIRS;
+    const int c = live ? c0 + col : P::PAIRS - 1;
+    double2* buf = ex + col * Y::PITCH;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) a[u] = pl[(t + Y::TPL * u) * P::PITCH + c];
+    lw.template run<false>(a, buf, t);
+    y_split<LOGJ>(a, buf, t, row);
+    if (live) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) out[(2 * (t + Y::TPL * (u >> 1)) + (u & 1)) * P::PAIRS + c] = row[u];
+    }
+  }
+}
+
+template <int LOGI, int LOGJ>
+__global__ void __launch_bounds__(REG_T)
+    k_plane_inv(Arrays arr, Rows rd, const double2* __restrict__ tw,
+                const double2* __restrict__ twm, const double2* __restrict__ twn) {
+  using P = Plane<LOGI, LOGJ>;
+  using X = typename P::X;
+  using Y = typename P::Y;
+  __shared__ double2 pl[P::J * P::PITCH], ex[P::EX];
+  const int k = blockIdx.x;
+  const double2* in =
+      reinterpret_cast<const double2*>(arr.src[blockIdx.y]) + (long long)k * P::PAIRS * P::J;
+  double2 a[8], row[8];
+  {
+    typename Y::Line lw;
+    const int col = threadIdx.x & (Y::COLS - 1), t = threadIdx.x / Y::COLS;
+    lw.load(twn, t);
+    const double sc = 1.0 / (double)Y::N;
+    for (int c0 = 0; c0 < P::PAIRS; c0 += Y::COLS) {
+      const bool live = c0 + col < P::PAIRS;
+      const int c = live ? c0 + col : P::PAIRS - 1;
+      double2* buf = ex + col * Y::PITCH;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) row[u] = in[(2 * (t + Y::TPL * (u >> 1)) + (u & 1)) * P::PAIRS + c];
+      __syncthreads();  // the columns before these are done with buf
+      y_join<LOGJ>(row, buf, t, a);
+      lw.template run<true>(a, buf, t);
+      if (live) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+          pl[(t + Y::TPL * u) * P::PITCH + c] = make_double2(a[u].x * sc, a[u].y * sc);
+      }
+    }
+  }
+  __syncthreads();
+  for (int j0 = 0; j0 < P::J; j0 += X::PER) {
+    const int t = threadIdx.x & (X::TPL - 1), own = threadIdx.x / X::TPL;
+    const bool live = j0 + own < P::J;
+    const int j = live ? j0 + own : P::J - 1;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) a[u] = pl[j * P::PITCH + t + X::TPL * u];
+    x_values<LOGI - 1>(a, ex + own * X::PITCH, t, tw, twm);
+    double* dst = arr.dst[blockIdx.y] + rd.at(j, k);
+    if (live) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) store2(dst + 2 * (t + X::TPL * u), a[u]);
     }
   }
 }
@@ -1414,39 +1549,15 @@ int tri(fld_ctx* c, int n, double* const* a, const int* ne) {
   return FLD_OK;
 }
 
-// n solver1d after the forward x transforms: y transforms, eliminations, inverses into the
-// interiors of `out`
-int solve_after_x(fld_ctx* c, int n, double* const* a, const int* ne, double* const* out) {
-  Arrays arr{};
-  for (int i = 0; i < n; ++i) arr.src[i] = a[i], arr.dst[i] = out[i];
-  int rc;
-  if ((rc = fft_y(c, false, n, a)) || (rc = tri(c, n, a, ne)) || (rc = fft_y(c, true, n, a)) ||
-      (rc = fft_x(c, true, n, arr, false, true)))
-    return rc;
-  return FLD_OK;
-}
-
-// n solver1d on compact right-hand sides, results into the interiors of `out`
-int solve_compact(fld_ctx* c, int n, double* const* a, const int* ne, double* const* out) {
-  Arrays arr{};
-  for (int i = 0; i < n; ++i) arr.src[i] = arr.dst[i] = a[i];
-  int rc;
-  if ((rc = fft_x(c, false, n, arr, false, false))) return rc;
-  return solve_after_x(c, n, a, ne, out);
-}
-
-// fillps (the divergence of u, v, w over dt) already transformed in x, into the compact
+// fillps (the divergence fs) already transformed in x, into the compact
 // array dst: k_fillps and the pressure solve's forward x transform in one pass
-int fft_x_fill(fld_ctx* c, const double* u, const double* v, const double* w, double* dst) {
+int fft_x_fill(fld_ctx* c, const FillSrc& fs, double* dst) {
   const FGrid& g = c->g;
   const int N = g.itot, nl = c->xlines;
   const int gpp = g.jtot / nl;
   const long long cp = (long long)g.itot * g.jtot, row = g.itot;
   const size_t lds = (size_t)nl * (N / 2 + 1) * sizeof(double2);
   const unsigned nb = (unsigned)(gpp * g.ktot);
-  const double dti = 1.0 / c->dt;
-  const FillSrc fs{u,    v,    w,      dti * g.dxi, dti * g.dyi, dti * g.dzi,
-                   g.sy, g.sz, g.itot, g.jtot,      g.ktot};
   const Arrays arr{{nullptr, nullptr, nullptr}, {dst, nullptr, nullptr}};
   if (reg_x(c)) return reg_fft_x(c, false, 1, arr, false, false, &fs);
   k_rfft_fwd<true, true><<<nb, FFT_THREADS, lds, c->stream>>>(
@@ -1454,6 +1565,70 @@ int fft_x_fill(fld_ctx* c, const double* u, const double* v, const double* w, do
       nl * row, nl * row, 1, row, 1, row, 0, c->tw_x, fs);
   HIPF(c, hipGetLastError());
   return FLD_OK;
+}
+
+// f(LOGI, LOGJ as integral constants) where the plane kernels hold such a plane; the largest from
+// 32 planes on (128 x 64 x 16: 68.4 us a step with them, 68.0 without)
+template <class F>
+bool with_plane(const fld_ctx* c, F&& f) {
+  const int li = c->logmx + 1, lj = c->logmy + 1;
+  if (li < 5 || lj < 5 || li + lj > (c->g.ktot >= 32 ? 13 : 12)) return false;
+  with_log<5, 8>(li, [&](auto i) {
+    constexpr int LI = decltype(i)::value;
+    with_log<5, 13 - LI>(lj, [&](auto j) { f(i, j); });
+  });
+  return true;
+}
+
+// Forward x and y transforms of n systems io (fields or compact arrays, or the divergence fs) into
+// the compact arrays a
+int fft_xy(fld_ctx* c, int n, double* const* io, bool field, const FillSrc* fs, double* const* a) {
+  const FGrid& g = c->g;
+  const Rows rf{1 + g.sy + g.sz, g.sy, g.sz}, rc{0, g.itot, (long long)g.itot * g.jtot};
+  Arrays arr{};
+  for (int i = 0; i < n; ++i) arr.src[i] = io[i], arr.dst[i] = a[i];
+  if (with_plane(c, [&](auto i, auto j) {
+        constexpr int LI = decltype(i)::value, LJ = decltype(j)::value;
+        const dim3 nb((unsigned)g.ktot, (unsigned)n);
+        if (fs)
+          k_plane_fwd<LI, LJ, true>
+              <<<nb, REG_T, 0, c->stream>>>(arr, rc, c->tw_x, c->tw_xm, c->tw_yn, *fs);
+        else
+          k_plane_fwd<LI, LJ, false><<<nb, REG_T, 0, c->stream>>>(
+              arr, field ? rf : rc, c->tw_x, c->tw_xm, c->tw_yn, FillSrc{});
+      })) {
+    HIPF(c, hipGetLastError());
+    return FLD_OK;
+  }
+  const int rv = fs ? fft_x_fill(c, *fs, a[0]) : fft_x(c, false, n, arr, field, false);
+  return rv ? rv : fft_y(c, false, n, a);
+}
+
+// and back, into the interiors of the fields out
+int ifft_xy(fld_ctx* c, int n, double* const* a, double* const* out) {
+  const FGrid& g = c->g;
+  const Rows rf{1 + g.sy + g.sz, g.sy, g.sz};
+  Arrays arr{};
+  for (int i = 0; i < n; ++i) arr.src[i] = a[i], arr.dst[i] = out[i];
+  if (with_plane(c, [&](auto i, auto j) {
+        constexpr int LI = decltype(i)::value, LJ = decltype(j)::value;
+        k_plane_inv<LI, LJ><<<dim3((unsigned)g.ktot, (unsigned)n), REG_T, 0, c->stream>>>(
+            arr, rf, c->tw_x, c->tw_xm, c->tw_yn);
+      })) {
+    HIPF(c, hipGetLastError());
+    return FLD_OK;
+  }
+  const int rv = fft_y(c, true, n, a);
+  return rv ? rv : fft_x(c, true, n, arr, false, true);
+}
+
+// n solver1d of the sources io (as fft_xy's), through the compact arrays a, into the interiors of
+// the fields out
+int solve(fld_ctx* c, int n, double* const* io, bool field, const FillSrc* fs, double* const* a,
+          const int* ne, double* const* out) {
+  int rc;
+  if ((rc = fft_xy(c, n, io, field, fs, a)) || (rc = tri(c, n, a, ne))) return rc;
+  return ifft_xy(c, n, a, out);
 }
 
 // halos and wall ghosts of nfields fields; kinds: kstep's kind of each, four bits
@@ -1612,11 +1787,7 @@ int fld_solver1d_dev(fld_ctx* c, double* p, int ne) {
   if (!p) return fail(c, FLD_E_ARG, "null field");
   if (ne < 1 || ne > 3) return fail(c, FLD_E_ARG, "ne must be 1, 2 or 3");
   HIPF(c, hipSetDevice(c->device));
-  Arrays arr{};
-  arr.src[0] = p, arr.dst[0] = c->work[0];
-  int rc = fft_x(c, false, 1, arr, true, false);
-  if (rc) return rc;
-  return solve_after_x(c, 1, c->work, &ne, &p);
+  return solve(c, 1, &p, true, nullptr, c->work, &ne, &p);
 }
 
 int fld_fftuvw_dev(fld_ctx* c, double* unew, double* vnew, double* wnew, const double* uo,
@@ -1642,7 +1813,7 @@ int fld_fftuvw_dev(fld_ctx* c, double* unew, double* vnew, double* wnew, const d
   HIPF(c, hipGetLastError());
   const int ne[3] = {2, 2, 3};
   double* const out[3] = {unew, vnew, wnew};
-  return solve_compact(c, 3, c->work, ne, out);
+  return solve(c, 3, c->work, false, nullptr, c->work, ne, out);
 }
 
 int fld_bounduvw_dev(fld_ctx* c, double* u, double* v, double* w) {
@@ -1689,10 +1860,12 @@ int fld_step_dev(fld_ctx* c, double* unew, double* vnew, double* wnew, double* p
   const int ne = 1;
   // the reference sets the halos of the velocities before fillps and those of p before correc:
   // the two passes read the interior values behind them instead, and one launch sets all at the
-  // end (64^3 cells: 13 launches instead of 15, 87.4 -> 82.3 us a step)
-  if ((rc = fft_x_fill(c, unew, vnew, wnew, c->work[0])) ||
-      (rc = solve_after_x(c, 1, c->work, &ne, &p)))
-    return rc;
+  // end (64^3 cells: 87.4 -> 82.3 us a step)
+  const FGrid& g = c->g;
+  const double dti = 1.0 / c->dt;
+  const FillSrc fs{unew, vnew, wnew,   dti * g.dxi, dti * g.dyi, dti * g.dzi,
+                   g.sy, g.sz, g.itot, g.jtot,      g.ktot};
+  if ((rc = solve(c, 1, c->work, false, &fs, c->work, &ne, &p))) return rc;
   // correc and pnew += p fused (the reference's bounduvw between them reads neither p nor
   // pnew), then bounduvw, boundp(pnew) and boundp(p)
   k_correc_addp<<<nblocks(c->ncomp, 256), 256, 0, c->stream>>>(c->g, c->dt, unew, vnew, wnew, p,
@@ -1756,7 +1929,7 @@ int fld_indicator_dev(fld_ctx* c, const double* gx, const double* gy, const doub
   k_ind_div<<<nblocks(c->ncomp, 256), 256, 0, c->stream>>>(c->g, gx, gy, gz, c->work[0], nullptr);
   HIPF(c, hipGetLastError());
   const int ne = 1;
-  int rc = solve_compact(c, 1, c->work, &ne, &indi);
+  int rc = solve(c, 1, c->work, false, nullptr, c->work, &ne, &indi);
   if (rc) return rc;
   return ind_finish(c, indi, indic, visc, forcey, forcez, lambda, visc0, sin_t, cos_t, tcoef);
 }
