@@ -44,9 +44,10 @@ class CoupledStep:
     """Device state and the stage launches of the coupled step (module docstring).
     overlap: run the interpolation on a second stream beside the traction stage in the graphs
     and in untimed eager steps (steps timed with events stay sequential).  None (default):
-    only with a traction object -- beside the FP64 law, whose persistent workgroups then
-    share the compute units, the step was slower (37.3 against 36.5 ms at 8000 capsules); beside
-    the surrogate stage it saves 0.17 ms (25.15 against 25.33 ms).
+    only with a traction object -- beside the FP64 law, which fills the compute units itself,
+    it gives 0.25 % at 8000 capsules (23.77 against 23.71 ms) and costs the second stream's
+    joins below some hundred (887 against 909 us with 30); beside the surrogate stage it
+    saves 0.17 ms (25.15 against 25.33 ms when measured).
 
     grid: ibx-style grid (itot, jtot powers of two); cap_off: every capsule has the points of
     degree `degree`, latitude-major; gs, eb: the law's moduli; rep, dt: param.f90:57 and
