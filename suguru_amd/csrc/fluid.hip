@@ -1130,28 +1130,32 @@ __global__ void __launch_bounds__(256) k_correc(FGrid g, double dt, double* __re
 // correc (correc.f90:11-38) and pnew += p (main.f90:406-408) in one pass over the cells: the
 // two touch disjoint outputs and both read p, which is then read once.  The p beyond the last cell
 // of a line or row is the first one, above the last plane the cell's own (bound.f90:93-98): read
-// there, so that p's halos are set with all others after this pass.
-__global__ void __launch_bounds__(256) k_correc_addp(FGrid g, double dt, double* __restrict__ u,
+// there, so that p's halos are set with all others after this pass.  Two neighbouring cells a
+// thread (itot is even).  Bound by memory: 1024 x 512 x 256 (9.7 GB) 1905 us a cell a thread from
+// halos, 2010 from the interior, 1966 two cells a thread (4.9 TB/s); a step at 256 x 128 x 128
+// 437 -> 432 us with the two cells.
+__global__ void __launch_bounds__(256) k_correc_addp(FGrid g, int logh, int logj, double dt,
+                                                     double* __restrict__ u,
                                                      double* __restrict__ v,
                                                      double* __restrict__ w,
                                                      const double* __restrict__ p,
                                                      double* __restrict__ pn) {
-  const long long n = (long long)g.itot * g.jtot * g.ktot;
+  const long long n = (long long)(g.itot / 2) * g.jtot * g.ktot;
   const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= n) return;
-  const int i = (int)(t % g.itot) + 1;
-  const long long r = t / g.itot;
-  const int j = (int)(r % g.jtot) + 1, k = (int)(r / g.jtot) + 1;
+  const int h = (int)(t & ((1 << logh) - 1)), r = (int)(t >> logh);
+  const int j = (r & ((1 << logj) - 1)) + 1, k = (r >> logj) + 1;
   const double factori = dt * g.dxi, factorj = dt * g.dyi, factork = dt * g.dzi;
-  const long long q = fidx(g, i, j, k);
-  const double pq = p[q];
-  const double pi = p[i < g.itot ? q + 1 : q - (g.itot - 1)];
-  const double pj = p[j < g.jtot ? q + g.sy : q - (g.jtot - 1) * g.sy];
-  const double pk = k < g.ktot ? p[q + g.sz] : pq;
-  u[q] = u[q] - factori * (pi - pq);
-  v[q] = v[q] - factorj * (pj - pq);
-  w[q] = w[q] - factork * (pk - pq);
-  pn[q] = pn[q] + pq;
+  const long long q = fidx(g, 2 * h + 1, j, k);
+  const double2 pq = load2(p + q);
+  const double2 pi = make_double2(pq.y, p[h < (1 << logh) - 1 ? q + 2 : q + 2 - g.itot]);
+  const double2 pj = load2(p + (j < g.jtot ? q + g.sy : q - (g.jtot - 1) * g.sy));
+  const double2 pk = load2(p + (k < g.ktot ? q + g.sz : q));
+  const double2 uq = load2(u + q), vq = load2(v + q), wq = load2(w + q), nq = load2(pn + q);
+  store2(u + q, make_double2(uq.x - factori * (pi.x - pq.x), uq.y - factori * (pi.y - pq.y)));
+  store2(v + q, make_double2(vq.x - factorj * (pj.x - pq.x), vq.y - factorj * (pj.y - pq.y)));
+  store2(w + q, make_double2(wq.x - factork * (pk.x - pq.x), wq.y - factork * (pk.y - pq.y)));
+  store2(pn + q, make_double2(nq.x + pq.x, nq.y + pq.y));
 }
 
 // Final value of a wall ghost / top face after the k step of bounduvw (bound.f90:38-56) or
@@ -1868,8 +1872,8 @@ int fld_step_dev(fld_ctx* c, double* unew, double* vnew, double* wnew, double* p
   if ((rc = solve(c, 1, c->work, false, &fs, c->work, &ne, &p))) return rc;
   // correc and pnew += p fused (the reference's bounduvw between them reads neither p nor
   // pnew), then bounduvw, boundp(pnew) and boundp(p)
-  k_correc_addp<<<nblocks(c->ncomp, 256), 256, 0, c->stream>>>(c->g, c->dt, unew, vnew, wnew, p,
-                                                               pnew);
+  k_correc_addp<<<nblocks(c->ncomp / 2, 256), 256, 0, c->stream>>>(
+      c->g, c->logmx, c->logmy + 1, c->dt, unew, vnew, wnew, p, pnew);
   HIPF(c, hipGetLastError());
   return bound(c, Fields{{unew, vnew, wnew, pnew, p}}, 5, KIND_STEP);
 }
