@@ -16,7 +16,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 LIB = os.path.join(HERE, "libibx.so")
 SOURCES = [os.path.join(HERE, "csrc", "ibx.hip")]
-DEPS = SOURCES + [os.path.join(HERE, "csrc", "ibx_device.hpp"), os.path.join(ROOT, "include", "ibx.h")]
+DEPS = SOURCES + [os.path.join(HERE, "csrc", "ibx_device.hpp"),
+                  os.path.join(HERE, "csrc", "obj_items.hpp"), os.path.join(ROOT, "include", "ibx.h")]
 # the capsule-membrane library: FP64 membrane law and the BF16-MFMA surrogate
 MEMB_LIB = os.path.join(HERE, "libmemb.so")
 MEMB_SOURCES = [os.path.join(HERE, "csrc", "membrane.hip"), os.path.join(HERE, "csrc", "mlp.hip")]

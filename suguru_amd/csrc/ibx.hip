@@ -244,7 +244,6 @@ struct ObjBufs {
   unsigned* cover;           // coverage bitmap, 1 bit per cell
   int* meta;                 // OB_META queue counters
   long long icap;            // item capacity
-  ObjLimit lim;              // item extent
 };
 
 // Items of a launch: 2048 cells where there are enough of them to fill the chip, fewer where a
@@ -255,20 +254,17 @@ struct ObjBufs {
 // with items of 2048 / 1024 / 512 / 256 cells: 1 capsule of radius 8h (4 items of 2048) 107 / 96 /
 // 91 / 83 us; radius 10.6h: 4 capsules (32) 156 / 132 / 117 / 105, 16 (127) 162 / 130 / 118 / 129,
 // 30 (240) 171 / 138 / 144 / -, 60 (480) 181 / 160 / 177 / -, 1000 (7900) 1108 / 1306 / 1725 / -.
-// times: the most items one of 2048 cells can turn into.
-struct ObjChoice {
-  ObjLimit lim;
-  int times;
-};
-ObjChoice obj_choice(long long ncap, long long npts) {
-  if (ncap > 0 && ncap <= 256 && npts > 0) {
+// Index of the limit (obj_limit); the launch falls back to larger ones as its buffers need
+// (obj_fit).
+int obj_choice(long long ncap, long long npts) {
+  if (ncap > 0 && ncap <= OB_SMALL && npts > 0) {
     const double edge = 2.0 * std::sqrt((double)npts / (double)ncap / (4.0 * M_PI)) + 4.0;
     const double est = (double)ncap * std::max(1.0, edge * edge * edge / 2048.0);
-    if (est <= 64) return {{16, 256}, 16};
-    if (est <= 160) return {{16, 512}, 8};
-    if (est <= 600) return {{16, 1024}, 4};
+    if (est <= 64) return 3;
+    if (est <= 160) return 2;
+    if (est <= 600) return 1;
   }
-  return {{OB_BX, OB_NC}, 1};
+  return 0;
 }
 
 // Sizes (bytes) of the object-spread work buffers for ncap capsules on the context's grid;
@@ -291,7 +287,7 @@ ObjSizes obj_sizes(const ibx_ctx* c, long long ncap) {
                           ((c->grid.jtot + OB_BIN - 1) / OB_BIN) *
                           ((c->grid.ktot + 2 + OB_BIN - 1) / OB_BIN);
   z.nbw = nbins * z.nwd;
-  z.icap_want = std::max<long long>(1024, 64 * ncap + 1024);
+  z.icap_want = obj_item_capacity(ncap);
   z.boxes = (size_t)std::max<long long>(1, 9 * ncap) * 6 * sizeof(int);
   z.nbm = (size_t)std::max<long long>(1, ncap * z.nwd) * 8;
   z.cnt = (size_t)std::max<long long>(1, ncap) * sizeof(int);
@@ -303,11 +299,9 @@ ObjSizes obj_sizes(const ibx_ctx* c, long long ncap) {
 }
 
 // The allocating path: context-owned buffers, grown on demand.
-int obj_bufs_alloc(ibx_ctx* c, long long ncap, long long npts, ObjBufs& ob) {
+int obj_bufs_alloc(ibx_ctx* c, long long ncap, ObjBufs& ob) {
   const ObjSizes z = obj_sizes(c, ncap);
-  const ObjChoice ch = obj_choice(ncap, npts);
-  const long long icap = z.icap_want * ch.times;
-  ob.lim = ch.lim;
+  const long long icap = z.icap_want;
   int rc;
   if ((rc = ensure(c, c->oboxes, z.boxes)) || (rc = ensure(c, c->onbm, z.nbm)) ||
       (rc = ensure(c, c->ocnt, z.cnt)) || (rc = ensure(c, c->obinm, z.binm)) ||
@@ -329,7 +323,7 @@ int obj_bufs_alloc(ibx_ctx* c, long long ncap, long long npts, ObjBufs& ob) {
 // The no-allocation path: the same buffers carved out of this device's fixed work array, each
 // aligned to 256 bytes.  The item capacity is what the array has left (at most the allocating
 // path's); a call that needs more items than that reports IBX_E_CAPACITY at the next ibx_sync.
-int obj_bufs_scratch(ibx_ctx* c, long long ncap, long long npts, ObjBufs& ob) {
+int obj_bufs_scratch(ibx_ctx* c, long long ncap, ObjBufs& ob) {
   if (!c->scratch) return fail(c, IBX_E_STATE, "no work array address for this device");
   const ObjSizes z = obj_sizes(c, ncap);
   auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
@@ -343,11 +337,7 @@ int obj_bufs_scratch(ibx_ctx* c, long long ncap, long long npts, ObjBufs& ob) {
                     " MiB of work buffers, more than the fixed " +
                     std::to_string(kScratchBytes >> 20) + " MiB array");
   const long long fit = (long long)((kScratchBytes - fixed - 3 * 256) / ObjSizes::per_item);
-  // small items only where the array holds all that the larger ones could turn into
-  ObjChoice ch = obj_choice(ncap, npts);
-  if (fit < z.icap_want * ch.times) ch = {{OB_BX, OB_NC}, 1};
-  const long long icap = std::min<long long>(z.icap_want * ch.times, fit);
-  ob.lim = ch.lim;
+  const long long icap = std::min<long long>(z.icap_want, fit);
   unsigned char* p = (unsigned char*)c->scratch;
   auto take = [&](size_t b) {
     unsigned char* q = p;
@@ -382,7 +372,7 @@ int enqueue_spread_obj(ibx_ctx* c, const TileCfg& cf, bool cc, long long ncap,
   const ObjSizes zs = obj_sizes(c, ncap);
   const long long nw = zs.nw, nbw = zs.nbw, icap = ob.icap;
   const int nwd = zs.nwd;
-  const ObjLimit lim = ob.lim;
+  const int want = obj_choice(ncap, npts);
   int* meta = ob.meta;
   unsigned* cover = ob.cover;
   const bool chk = check && ncap > 0;
@@ -390,12 +380,14 @@ int enqueue_spread_obj(ibx_ctx* c, const TileCfg& cf, bool cc, long long ncap,
                 c->stream>>>(nw, cover, nbw, ob.binm, meta, ncap, chk ? d_off : nullptr, npts,
                              c->d_err);
   if (npts > 0 && ncap > 0) {
+    // (the neighbour masks' memory: k_obj_items<true> keeps the masks in LDS)
+    unsigned long long* small = ncap <= OB_SMALL ? ob.nbm : nullptr;
     k_obj_boxes<<<(unsigned)ncap, 256, 0, c->stream>>>(
-        c->gd, klo, khi, lim, d_off, x, y, z, ob.boxes, ob.cnt,
+        c->gd, klo, khi, d_off, x, y, z, ob.boxes, ob.cnt, small,
         nwd, ob.binm, c->d_err);
 #define ITEM_ARGS                                                                              \
-  c->gd, lim, ncap, nwd, ob.boxes, ob.binm, ob.off, ob.cnt, ob.items, (int)icap, cover, ob.nbm, \
-      ob.src, ob.nsrc, meta, c->d_err
+  c->gd, want, ncap, nwd, ob.boxes, ob.binm, ob.off, ob.cnt, small, ob.items, (int)icap, cover, \
+      ob.nbm, ob.src, ob.nsrc, meta, c->d_err
     if (ncap <= OB_FUSE) {
       k_obj_items<true><<<(unsigned)ncap, 256, 0, c->stream>>>(ITEM_ARGS);
     } else {
@@ -451,7 +443,7 @@ int enqueue_spread(ibx_ctx* c, int cfgid, bool cc, long long ncap, const long lo
   const TileCfg& cf = kCfgs[cfgid];
   if (cf.obj) {
     ObjBufs ob;
-    int rc = obj_bufs_alloc(c, ncap, npts, ob);
+    int rc = obj_bufs_alloc(c, ncap, ob);
     if (rc) return rc;
     return enqueue_spread_obj(c, cf, cc, ncap, d_off, npts, x, y, z, f1, f2, f3, area, o1, o2,
                               o3, ob, check, ev_tile, ev_tile_end, ev_split, ev_before);
@@ -796,7 +788,7 @@ int ibx_spread_f64_dev_noalloc(ibx_ctx* c, int64_t ncap, const int64_t* cap_off,
                            forcez);
   if (rc) return rc;
   ObjBufs ob;
-  if ((rc = obj_bufs_scratch(c, ncap, npts, ob))) return rc;
+  if ((rc = obj_bufs_scratch(c, ncap, ob))) return rc;
   HIPCHK(c, hipSetDevice(c->device));
   // the context's configuration when it is an object one, else the default object one (the
   // tile spread sizes its candidate list per call)

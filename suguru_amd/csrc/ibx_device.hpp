@@ -9,6 +9,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "obj_items.hpp"
+
 #pragma clang fp contract(off)
 
 namespace ibx {
@@ -909,9 +911,6 @@ __global__ void __launch_bounds__(SP_THREADS)
 // k_obj_scan (item offsets); k_obj_items (items, bitmap, neighbouring capsules);
 // k_obj_sources (source lists); k_obj_spread (items and zero units); k_jhalo.
 // ---------------------------------------------------------------------------------------
-constexpr int OB_BX = 32;          // item extent limit in x and y (cells)
-constexpr int OB_NZ = 32;          // item extent limit in z
-constexpr int OB_NC = 2048;        // cells per item
 constexpr int OB_THREADS = 256;
 constexpr int OB_CPT = OB_NC / OB_THREADS;  // cells per thread
 constexpr int OB_PEND = 64 + OB_THREADS;    // pending candidate list
@@ -950,25 +949,6 @@ __global__ void __launch_bounds__(256) k_obj_clear(long long nw, unsigned* __res
   if (q < OB_META) meta[q] = 0;
 }
 
-// Extent of the items of a launch: at most bx cells in x and y and nc cells.
-struct ObjLimit {
-  int bx, nc;
-};
-
-// Item grid of one object box: cx x cy x cz sub-boxes of extent nx x ny x nz (the last ones
-// cut short), within the launch's limit and OB_NZ planes each.
-struct ObjGrid {
-  int cx, cy, cz, nx, ny, nz;
-  __device__ explicit ObjGrid(const int* b, ObjLimit l) {
-    const int X = b[1] - b[0] + 1, Y = b[3] - b[2] + 1, Z = b[5] - b[4] + 1;
-    cx = (X + l.bx - 1) / l.bx, cy = (Y + l.bx - 1) / l.bx;
-    nx = (X + cx - 1) / cx, ny = (Y + cy - 1) / cy;
-    nz = max(1, min(min(Z, OB_NZ), l.nc / (nx * ny)));
-    cz = (Z + nz - 1) / nz;
-  }
-  __device__ int count() const { return cx * cy * cz; }
-};
-
 constexpr int OB_NBL = 256;  // bins of one capsule's boxes held in LDS
 constexpr int OB_NQL = 512;  // candidate capsules per mask chunk held in LDS
 constexpr int OB_NWC = 64;   // neighbour-mask words per chunk
@@ -993,19 +973,20 @@ struct ObjBins {
 };
 
 // One workgroup per capsule: the clamped window boxes of its nine objects (boxes[o], o =
-// 9 p + nb), its registration in the coarse bins, and its number of items (cnt[p]).
-__global__ void __launch_bounds__(256) k_obj_boxes(GridD g, int klo, int khi, ObjLimit lim,
+// 9 p + nb), its registration in the coarse bins, and its number of items of the largest limit
+// (cnt[p]); with `small`, of the smaller limits too (small[p], obj_pack).
+__global__ void __launch_bounds__(256) k_obj_boxes(GridD g, int klo, int khi,
                                                    const long long* __restrict__ cap_off,
                                                    const double* __restrict__ x,
                                                    const double* __restrict__ y,
                                                    const double* __restrict__ z,
                                                    int* __restrict__ boxes,
-                                                   int* __restrict__ cnt, int nwd,
+                                                   int* __restrict__ cnt,
+                                                   unsigned long long* __restrict__ small, int nwd,
                                                    unsigned long long* __restrict__ binm,
                                                    int* __restrict__ err) {
   if (offsets_bad(err)) return;
   __shared__ int red[4][9][6];
-  __shared__ int ncnt[9];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const long long p = blockIdx.x;
   const long long lo = cap_off[p], hi = cap_off[p + 1];
@@ -1068,7 +1049,6 @@ __global__ void __launch_bounds__(256) k_obj_boxes(GridD g, int klo, int khi, Ob
     const int nb = tid;
     const bool has = B[nb][0] <= B[nb][1];
     for (int e = 0; e < 6; ++e) boxes[(p * 9 + nb) * 6 + e] = has ? B[nb][e] : (e & 1 ? 0 : 1);
-    ncnt[nb] = has ? ObjGrid(B[nb], lim).count() : 0;
     if (has) {
       const ObjBins bins(g);
       int r[6];
@@ -1080,11 +1060,19 @@ __global__ void __launch_bounds__(256) k_obj_boxes(GridD g, int klo, int khi, Ob
             atomicOr(&binm[bins.index(bx_, by, bz) * nwd + (p >> 6)], bit);
     }
   }
-  __syncthreads();
-  if (tid == 0) {
-    int total = 0;
-    for (int nb = 0; nb < 9; ++nb) total += ncnt[nb];
-    cnt[p] = total;
+  if (wv == 1) {  // meanwhile: lanes 16 e + nb count object nb at limit e
+    const int nb = lane & 15, e = lane >> 4;
+    int n = 0;
+    if (nb < 9 && (e == 0 || small) && B[nb][0] <= B[nb][1]) n = ObjGrid(B[nb], obj_limit(e)).count();
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1) n += __shfl_xor(n, o);
+    int total[OB_LIMITS];
+#pragma unroll
+    for (int l = 0; l < OB_LIMITS; ++l) total[l] = __shfl(n, 16 * l);
+    if (lane == 0) {
+      cnt[p] = total[0];
+      if (small) small[p] = obj_pack(total);
+    }
   }
 }
 
@@ -1194,13 +1182,17 @@ __device__ __forceinline__ void obj_item_sources(const ObjItem& it, int item, in
 // FUSE (at most OB_FUSE capsules): the workgroup also adds up the item counts before its own
 // (k_obj_scan's work) and lists its items' sources (k_obj_sources'), whose neighbour mask it
 // holds in LDS: two launches fewer, 7 us of the 83 us a transfer of one capsule takes.
+// small (with FUSE, at most 256 capsules; null: items of the largest limit): the launch takes items
+// of limit `want`, or of the next larger one that the buffers hold.
 constexpr int OB_FUSE = 1024;
+constexpr int OB_SMALL = 256;
 template <bool FUSE>
-__global__ void __launch_bounds__(256) k_obj_items(GridD g, ObjLimit lim, long long ncap, int nwd,
+__global__ void __launch_bounds__(256) k_obj_items(GridD g, int want, long long ncap, int nwd,
                                                    const int* __restrict__ boxes,
                                                    const unsigned long long* __restrict__ binm,
                                                    const int* __restrict__ off,
                                                    const int* __restrict__ cnt,
+                                                   const unsigned long long* __restrict__ small,
                                                    ObjItem* __restrict__ items, int icap,
                                                    unsigned* __restrict__ cover,
                                                    unsigned long long* __restrict__ nbm,
@@ -1209,23 +1201,40 @@ __global__ void __launch_bounds__(256) k_obj_items(GridD g, ObjLimit lim, long l
                                                    int* __restrict__ err) {
   if (offsets_bad(err)) return;
   __shared__ int B[9][6];
-  __shared__ int first;
+  __shared__ int first, tot[OB_LIMITS];
   const int tid = threadIdx.x;
   const long long p = blockIdx.x;
   if (tid < 54) B[tid / 6][tid % 6] = boxes[p * 54 + tid];
   if (FUSE && tid == 0) first = 0;
+  if (FUSE && tid < OB_LIMITS) tot[tid] = 0;
+  // with `small` a capsule per thread
+  const bool mine = FUSE && small && tid < ncap;
+  const int c0 = mine ? cnt[tid] : 0;
+  const unsigned long long cs = mine ? small[tid] : 0ull;
   __syncthreads();
-  int at;
+  int at, e = 0;
   if (FUSE) {
-    int v = 0;
-    for (long long q = tid; q < p; q += 256) v += cnt[q];
+    const auto add = [&](int v, int* to) {  // the workgroup's sum
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o);
-    if ((tid & 63) == 0 && v) atomicAdd(&first, v);
+      for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o);
+      if ((tid & 63) == 0 && v) atomicAdd(to, v);
+    };
+    int v = 0;
+    if (small) {
+      add(c0, &tot[0]);
+#pragma unroll
+      for (int l = 1; l < OB_LIMITS; ++l) add(obj_unpack(cs, l), &tot[l]);
+      __syncthreads();
+      e = obj_fit(want, tot, icap);
+      v = tid < p ? (e ? obj_unpack(cs, e) : c0) : 0;
+    } else {
+      for (long long q = tid; q < p; q += 256) v += cnt[q];
+    }
+    add(v, &first);
     __syncthreads();
     at = first;
     if (tid == 0 && p == ncap - 1) {
-      meta[0] = at + cnt[p];
+      meta[0] = small ? tot[e] : at + cnt[p];
       if (meta[0] > icap) atomicOr(err, ERR_CAPACITY);
     }
   } else {
@@ -1234,9 +1243,9 @@ __global__ void __launch_bounds__(256) k_obj_items(GridD g, ObjLimit lim, long l
   const int at0 = at;
   for (int nb = 0; nb < 9; ++nb) {
     if (B[nb][0] > B[nb][1]) continue;  // uniform
-    const ObjGrid og(B[nb], lim);
+    const ObjGrid og(B[nb], obj_limit(e));
     for (int t = tid; t < og.count(); t += 256) {
-      if (at + t >= icap) break;  // flagged by k_obj_scan
+      if (at + t >= icap) break;  // flagged above, or by k_obj_scan
       const int a = t / (og.cy * og.cz), b = (t / og.cz) % og.cy, c = t % og.cz;
       ObjItem it;
       it.p = (int)p, it.nb = nb;

@@ -1,0 +1,64 @@
+// obj_items.hpp -- how the spread by capsule objects cuts an object's box into work items, and how
+// many items its buffers hold (constant expressions: the same on host and device).
+#pragma once
+
+namespace ibx {
+
+constexpr int OB_BX = 32;    // item extent limit in x and y (cells)
+constexpr int OB_NZ = 32;    // item extent limit in z
+constexpr int OB_NC = 2048;  // cells per item
+
+// Extent of the items of a launch: at most bx cells in x and y and nc cells.
+struct ObjLimit {
+  int bx, nc;
+};
+
+// The extents that a launch chooses from: 2048, 1024, 512 and 256 cells.
+constexpr int OB_LIMITS = 4;
+constexpr ObjLimit obj_limit(int e) { return {e ? OB_BX / 2 : OB_BX, OB_NC >> e}; }
+
+// Item grid of one object box (its bounds xa, xb, ya, yb, za, zb): cx x cy x cz sub-boxes of extent
+// nx x ny x nz (the last ones cut short), within the launch's limit and OB_NZ planes each.
+struct ObjGrid {
+  int cx, cy, cz, nx, ny, nz;
+  constexpr ObjGrid(const int* b, ObjLimit l)
+      : ObjGrid(b[1] - b[0] + 1, b[3] - b[2] + 1, b[5] - b[4] + 1, l) {}
+  constexpr ObjGrid(int X, int Y, int Z, ObjLimit l) : cx(0), cy(0), cz(0), nx(0), ny(0), nz(0) {
+    cx = (X + l.bx - 1) / l.bx, cy = (Y + l.bx - 1) / l.bx;
+    nx = (X + cx - 1) / cx, ny = (Y + cy - 1) / cy;
+    const int most = Z < OB_NZ ? Z : OB_NZ, fit = l.nc / (nx * ny);
+    nz = most < fit ? most : fit;
+    if (nz < 1) nz = 1;
+    cz = (Z + nz - 1) / nz;
+  }
+  constexpr int count() const { return cx * cy * cz; }
+};
+
+// Items that the buffers hold for ncap capsules.  By the capsule count alone and never fewer for
+// more capsules: a call with fewer capsules than an earlier one leaves the buffers where they are,
+// which a captured graph of the earlier call relies on.
+constexpr long long obj_item_capacity(long long ncap) {
+  return 64 * (ncap < 16 ? 16 : ncap) + 1024;
+}
+
+// The limit of a launch that wants limit e and whose boxes make tot[e] items at each: the next
+// larger one whose items fit.  (The largest is taken whether they fit or not, and its overflow
+// reported.)
+constexpr int obj_fit(int e, const int* tot, int icap) {
+  while (e > 0 && tot[e] > icap) --e;
+  return e;
+}
+
+// Counts of the three smaller limits in one word, 21 bits each, saturated.
+constexpr int OB_CBITS = 21, OB_CMAX = 1 << 20;
+constexpr unsigned long long obj_pack(const int* cnt) {
+  unsigned long long v = 0;
+  for (int e = 1; e < OB_LIMITS; ++e)
+    v |= (unsigned long long)(cnt[e] < OB_CMAX ? cnt[e] : OB_CMAX) << (OB_CBITS * (e - 1));
+  return v;
+}
+constexpr int obj_unpack(unsigned long long v, int e) {
+  return (int)(v >> (OB_CBITS * (e - 1))) & ((1 << OB_CBITS) - 1);
+}
+
+}  // namespace ibx
