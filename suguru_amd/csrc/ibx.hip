@@ -246,27 +246,6 @@ struct ObjBufs {
   long long icap;            // item capacity
 };
 
-// Items of a launch: 2048 cells where there are enough of them to fill the chip, fewer where a
-// capsule or a few would otherwise leave it idle: an item is one workgroup's chain over its
-// candidates, so that smaller items end sooner, while candidates near an item's faces are prepared
-// once for each item they reach.  The line lies at the items that 2048 cells would give,
-// estimated from the points per capsule (about one per h^2 of surface).  Spread + interpolation
-// with items of 2048 / 1024 / 512 / 256 cells: 1 capsule of radius 8h (4 items of 2048) 107 / 96 /
-// 91 / 83 us; radius 10.6h: 4 capsules (32) 156 / 132 / 117 / 105, 16 (127) 162 / 130 / 118 / 129,
-// 30 (240) 171 / 138 / 144 / -, 60 (480) 181 / 160 / 177 / -, 1000 (7900) 1108 / 1306 / 1725 / -.
-// Index of the limit (obj_limit); the launch falls back to larger ones as its buffers need
-// (obj_fit).
-int obj_choice(long long ncap, long long npts) {
-  if (ncap > 0 && ncap <= OB_SMALL && npts > 0) {
-    const double edge = 2.0 * std::sqrt((double)npts / (double)ncap / (4.0 * M_PI)) + 4.0;
-    const double est = (double)ncap * std::max(1.0, edge * edge * edge / 2048.0);
-    if (est <= 64) return 3;
-    if (est <= 160) return 2;
-    if (est <= 600) return 1;
-  }
-  return 0;
-}
-
 // Sizes (bytes) of the object-spread work buffers for ncap capsules on the context's grid;
 // items are sized separately (ObjSizes::per_item bytes per item of capacity).
 struct ObjSizes {
@@ -372,7 +351,6 @@ int enqueue_spread_obj(ibx_ctx* c, const TileCfg& cf, bool cc, long long ncap,
   const ObjSizes zs = obj_sizes(c, ncap);
   const long long nw = zs.nw, nbw = zs.nbw, icap = ob.icap;
   const int nwd = zs.nwd;
-  const int want = obj_choice(ncap, npts);
   int* meta = ob.meta;
   unsigned* cover = ob.cover;
   const bool chk = check && ncap > 0;
@@ -386,7 +364,7 @@ int enqueue_spread_obj(ibx_ctx* c, const TileCfg& cf, bool cc, long long ncap,
         c->gd, klo, khi, d_off, x, y, z, ob.boxes, ob.cnt, small,
         nwd, ob.binm, c->d_err);
 #define ITEM_ARGS                                                                              \
-  c->gd, want, ncap, nwd, ob.boxes, ob.binm, ob.off, ob.cnt, small, ob.items, (int)icap, cover, \
+  c->gd, ncap, nwd, ob.boxes, ob.binm, ob.off, ob.cnt, small, ob.items, (int)icap, cover, \
       ob.nbm, ob.src, ob.nsrc, meta, c->d_err
     if (ncap <= OB_FUSE) {
       k_obj_items<true><<<(unsigned)ncap, 256, 0, c->stream>>>(ITEM_ARGS);

@@ -1182,12 +1182,11 @@ __device__ __forceinline__ void obj_item_sources(const ObjItem& it, int item, in
 // FUSE (at most OB_FUSE capsules): the workgroup also adds up the item counts before its own
 // (k_obj_scan's work) and lists its items' sources (k_obj_sources'), whose neighbour mask it
 // holds in LDS: two launches fewer, 7 us of the 83 us a transfer of one capsule takes.
-// small (with FUSE, at most 256 capsules; null: items of the largest limit): the launch takes items
-// of limit `want`, or of the next larger one that the buffers hold.
+// small (with FUSE, at most OB_SMALL capsules; null: items of the largest limit): obj_choice's limit.
 constexpr int OB_FUSE = 1024;
 constexpr int OB_SMALL = 256;
 template <bool FUSE>
-__global__ void __launch_bounds__(256) k_obj_items(GridD g, int want, long long ncap, int nwd,
+__global__ void __launch_bounds__(256) k_obj_items(GridD g, long long ncap, int nwd,
                                                    const int* __restrict__ boxes,
                                                    const unsigned long long* __restrict__ binm,
                                                    const int* __restrict__ off,
@@ -1225,7 +1224,7 @@ __global__ void __launch_bounds__(256) k_obj_items(GridD g, int want, long long 
 #pragma unroll
       for (int l = 1; l < OB_LIMITS; ++l) add(obj_unpack(cs, l), &tot[l]);
       __syncthreads();
-      e = obj_fit(want, tot, icap);
+      e = obj_choice(tot, icap);
       v = tid < p ? (e ? obj_unpack(cs, e) : c0) : 0;
     } else {
       for (long long q = tid; q < p; q += 256) v += cnt[q];

@@ -41,10 +41,21 @@ constexpr long long obj_item_capacity(long long ncap) {
   return 64 * (ncap < 16 ? 16 : ncap) + 1024;
 }
 
-// The limit of a launch that wants limit e and whose boxes make tot[e] items at each: the next
-// larger one whose items fit.  (The largest is taken whether they fit or not, and its overflow
-// reported.)
-constexpr int obj_fit(int e, const int* tot, int icap) {
+// The limit of a launch whose boxes make tot[e] items at each: 2048 cells where there are enough of
+// them to fill the chip, fewer where a capsule or a few would otherwise leave it idle: an item is one
+// workgroup's chain over its candidates, so that smaller items end sooner, while candidates near an
+// item's faces are prepared once for each item they reach.  The lines lie at the items of 2048
+// cells, counted from the boxes.  Capsules of degree 16 and radius 10.6h (8 items each) on
+// 256 x 256 x 128 cells, spread with items of 2048 / 1024 / 512 / 256 cells: 1 (8 items) 93 / 78 / 76 /
+// 75 us; 8 (64) 98 / 86 / 80 / 82; 16 (127) 106 / 91 / 87 / 101; 24 (190) 107 / 99 / 91 / 121;
+// 30 (240) 105 / 96 / 93 / 131; 45 (360) 108 / 96 / 109 / 155; 60 (480) 107 / 108 / 120 / 180;
+// 76 (600) 116 / 119 / 138 / 221; 100 (790) 122 / 134 / 158 / 255; 226 (1790) 203 / 226 / 284 / 534.
+// Spread and interpolation on a denser channel: 4 (32) 156 / 132 / 117 / 105; 16 162 / 130 / 118 / 129;
+// 30 171 / 138 / 144 / -; 60 181 / 160 / 177 / -; 1000 1108 / 1306 / 1725 / -.
+// Smaller items are taken only where the buffers hold them: the next larger ones otherwise.  (The
+// largest are taken whether they fit or not, and their overflow reported.)
+constexpr int obj_choice(const int* tot, int icap) {
+  int e = tot[0] <= 48 ? 3 : tot[0] <= 200 ? 2 : tot[0] <= 500 ? 1 : 0;
   while (e > 0 && tot[e] > icap) --e;
   return e;
 }

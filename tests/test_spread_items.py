@@ -16,7 +16,7 @@ HOST = """
 using namespace ibx;
 extern "C" {
 long long capacity(long long n) { return obj_item_capacity(n); }
-int fit(int e, const int* tot, int icap) { return obj_fit(e, tot, icap); }
+int choice(const int* tot, int icap) { return obj_choice(tot, icap); }
 void limit(int e, int* o) { o[0] = obj_limit(e).bx, o[1] = obj_limit(e).nc; }
 void grid(int x, int y, int z, int e, int* o) {
   const int b[6] = {1, x, 1, y, 0, z - 1};
@@ -70,11 +70,23 @@ def test_items_cover_a_box_within_their_limit(items):
 def test_small_items_only_where_they_fit(items):
     rng = np.random.default_rng(3)
     for _ in range(2000):
-        tot = np.cumsum(rng.integers(1, 2000, 4))
-        icap, want = int(rng.integers(1, 5000)), int(rng.integers(0, 4))
-        e = items.fit(want, ints(*map(int, tot)), icap)
-        fits = [k for k in range(want + 1) if tot[k] <= icap]
+        tot = np.cumsum(rng.integers(1, 600, 4))
+        icap = int(rng.integers(1, 2500))
+        e, free = (items.choice(ints(*map(int, tot)), c) for c in (icap, 1 << 20))
+        fits = [k for k in range(free + 1) if tot[k] <= icap]
         assert e == (max(fits) if fits else 0)
+
+
+@pytest.mark.parametrize("ncap,limit", [(4, 3), (16, 2), (24, 2), (30, 1), (60, 1), (76, 0), (226, 0)])
+def test_size_by_the_items_of_the_boxes(items, ncap, limit):
+    """Degree-16 capsules of radius 10.6h, 24 or 25 cells wide with their windows: 8 items of 2048
+    cells each, whose 578 points would suggest 3."""
+    tot, o = [], ints(*[0] * 7)
+    for e in range(4):
+        items.grid(25, 24, 24, e, o)
+        tot.append(ncap * o[6])
+    assert tot[0] == 8 * ncap
+    assert items.choice(ints(*tot), items.capacity(ncap)) == limit
 
 
 def test_counts_survive_the_packing(items):
