@@ -480,7 +480,40 @@ struct YLine {
   // the pairs of a row lie in different banks: pitch = 16 / COLS mod 16 sixteen-byte slots
   static constexpr int SKEW = COLS >= 16 ? 1 : 16 / COLS;
   static constexpr int PITCH = fft::pad(N) + (SKEW - fft::pad(N) % 16 + 16) % 16;
+  static constexpr int WAVES = T / 64;
 };
+
+// The two columns of a pair share their rounding: each gets about 1e-16 of the other's largest
+// value, no more than the x transform left in either from the same row, except where a column is
+// zero: in a flow uniform in x every column but the first is, and has to stay so for the flow to stay
+// uniform to the last bit.  So a column of zeros gives zeros.
+// y_mark: from the eight values a thread holds of each column, a bit per lane (nz: the first
+// column's of each wavefront, then the second's); y_clear, a barrier later: the zero columns'
+// values of v.
+template <int LOGN>
+__device__ __forceinline__ void y_mark(const double2 (&v)[8], unsigned long long* nz) {
+  using Y = YLine<LOGN>;
+  bool x = false, y = false;
+#pragma unroll
+  for (int u = 0; u < 8; ++u) x |= v[u].x != 0.0, y |= v[u].y != 0.0;
+  const unsigned long long bx = __ballot(x), by = __ballot(y);
+  if ((threadIdx.x & 63) == 0) nz[threadIdx.x >> 6] = bx, nz[Y::WAVES + (threadIdx.x >> 6)] = by;
+}
+template <int LOGN>
+__device__ __forceinline__ void y_clear(double2 (&v)[8], const unsigned long long* nz, int col) {
+  using Y = YLine<LOGN>;
+  // wavefronts and, in each, lanes with values of column col
+  constexpr int STEP = Y::COLS > 64 ? Y::COLS / 64 : 1;
+  unsigned long long bx = 0, by = 0, lanes = 1;
+#pragma unroll
+  for (int l = Y::COLS; l < 64; l += Y::COLS) lanes |= 1ull << l;
+  const int w0 = Y::COLS > 64 ? col >> 6 : 0;
+#pragma unroll
+  for (int w = 0; w < Y::WAVES; w += STEP) bx |= nz[w0 + w], by |= nz[Y::WAVES + w0 + w];
+  const bool x = (bx >> (col & 63)) & lanes, y = (by >> (col & 63)) & lanes;
+#pragma unroll
+  for (int u = 0; u < 8; ++u) v[u] = make_double2(x ? v[u].x : 0.0, y ? v[u].y : 0.0);
+}
 
 // the packed half spectra of a pair of columns from its complex spectrum: rows 2k and 2k + 1
 // (k = t + TPL u, u < 4) get Re and Im of X_k, rows 0 and 1 X_0 and X_N/2
@@ -527,6 +560,7 @@ __global__ void __launch_bounds__(YLine<LOGN>::T)
     k_y(Arrays arr, int logc, long long pairs, const double2* __restrict__ twn) {
   using Y = YLine<LOGN>;
   __shared__ double2 sm[Y::COLS * Y::PITCH];
+  __shared__ unsigned long long nz[2 * Y::WAVES];
   const int col = threadIdx.x & (Y::COLS - 1), t = threadIdx.x / Y::COLS;
   const long long g = (long long)xcd_logical_block<false>() * Y::COLS + col;
   const bool live = g < pairs;
@@ -540,8 +574,10 @@ __global__ void __launch_bounds__(YLine<LOGN>::T)
 #pragma unroll
     for (int u = 0; u < 8; ++u) a[u] = p[(t + Y::TPL * u) * pitch];
     lw.load(twn, t);
+    y_mark<LOGN>(a, nz);
     lw.template run<false>(a, buf, t);
     y_split<LOGN>(a, buf, t, row);
+    y_clear<LOGN>(row, nz, col);
     if (live) {
 #pragma unroll
       for (int u = 0; u < 8; ++u) p[(2 * (t + Y::TPL * (u >> 1)) + (u & 1)) * pitch] = row[u];
@@ -550,8 +586,10 @@ __global__ void __launch_bounds__(YLine<LOGN>::T)
 #pragma unroll
     for (int u = 0; u < 8; ++u) row[u] = p[(2 * (t + Y::TPL * (u >> 1)) + (u & 1)) * pitch];
     lw.load(twn, t);
+    y_mark<LOGN>(row, nz);
     y_join<LOGN>(row, buf, t, a);
     lw.template run<true>(a, buf, t);
+    y_clear<LOGN>(a, nz, col);
     const double sc = 1.0 / (double)Y::N;
     if (live) {
 #pragma unroll
@@ -586,6 +624,7 @@ __global__ void __launch_bounds__(REG_T)
   using Y = typename P::Y;
   static_assert(Y::T == REG_T, "one workgroup shape for both directions");
   __shared__ double2 pl[P::J * P::PITCH], ex[P::EX];
+  __shared__ unsigned long long nz[2][2 * Y::WAVES];  // in turn: read until the next columns' barriers
   const int k = blockIdx.x;
   double2 a[8], row[8];
   for (int j0 = 0; j0 < P::J; j0 += X::PER) {
@@ -610,8 +649,11 @@ __global__ void __launch_bounds__(REG_T)
     double2* buf = ex + col * Y::PITCH;
 #pragma unroll
     for (int u = 0; u < 8; ++u) a[u] = pl[(t + Y::TPL * u) * P::PITCH + c];
+    unsigned long long* z = nz[(c0 / Y::COLS) & 1];
+    y_mark<LOGJ>(a, z);
     lw.template run<false>(a, buf, t);
     y_split<LOGJ>(a, buf, t, row);
+    y_clear<LOGJ>(row, z, col);
     if (live) {
 #pragma unroll
       for (int u = 0; u < 8; ++u) out[(2 * (t + Y::TPL * (u >> 1)) + (u & 1)) * P::PAIRS + c] = row[u];
@@ -627,6 +669,7 @@ __global__ void __launch_bounds__(REG_T)
   using X = typename P::X;
   using Y = typename P::Y;
   __shared__ double2 pl[P::J * P::PITCH], ex[P::EX];
+  __shared__ unsigned long long nz[2 * Y::WAVES];
   const int k = blockIdx.x;
   const double2* in =
       reinterpret_cast<const double2*>(arr.src[blockIdx.y]) + (long long)k * P::PAIRS * P::J;
@@ -642,9 +685,11 @@ __global__ void __launch_bounds__(REG_T)
       double2* buf = ex + col * Y::PITCH;
 #pragma unroll
       for (int u = 0; u < 8; ++u) row[u] = in[(2 * (t + Y::TPL * (u >> 1)) + (u & 1)) * P::PAIRS + c];
-      __syncthreads();  // the columns before these are done with buf
+      __syncthreads();  // the columns before these are done with buf and nz
+      y_mark<LOGJ>(row, nz);
       y_join<LOGJ>(row, buf, t, a);
       lw.template run<true>(a, buf, t);
+      y_clear<LOGJ>(a, nz, col);
       if (live) {
 #pragma unroll
         for (int u = 0; u < 8; ++u)
