@@ -1049,7 +1049,8 @@ struct memb_plan {
   double2* rows = nullptr;
   int* list = nullptr;
   int slots = 0;
-  int num_wg = 0;  // node workgroups in flight
+  int num_wg = 0;         // shape and filter workgroups in flight, about
+  int nodes_wg[2] = {};   // node workgroups that fit the device, without and with bending
   ordered::OrderedTables O{};  // built at the first use of the ordered law
 };
 
@@ -1392,7 +1393,7 @@ int run_law(memb_plan* p, long long ncap, double gs, double eb, const double* x,
             const double* z, double* fx, double* fy, double* fz, double* nx, double* ny,
             double* nz, double* area, const int* sel) {
   const Tables& T = p->T;
-  const int most = p->num_wg;
+  const int most = p->nodes_wg[eb != 0.0];
   for (long long c0 = 0; c0 < ncap; c0 += p->slots) {
     const int n = (int)std::min<long long>(p->slots, ncap - c0);
     Work w{};
@@ -1410,8 +1411,8 @@ int run_law(memb_plan* p, long long ncap, double gs, double eb, const double* x,
     else
       k_nodes<false, false><<<gn, ND_THREADS, lds_nodes(T, false), p->stream>>>(T, w, most, gs,
                                                                                eb, nullptr);
-    k_filter<<<2 * n <= most ? 2 * n : n, SH_THREADS, lds_filter(T), p->stream>>>(
-        T, w, most, fx, fy, fz, nx, ny, nz);
+    k_filter<<<2 * n <= p->num_wg ? 2 * n : n, SH_THREADS, lds_filter(T), p->stream>>>(
+        T, w, p->num_wg, fx, fy, fz, nx, ny, nz);
   }
   MCHK(p, hipGetLastError());
   return MEMB_OK;
@@ -1481,7 +1482,7 @@ int memb_plan_create(memb_plan** out, int L, int device) {
   T.e2 = reinterpret_cast<const double2*>(e2), T.ef = reinterpret_cast<const double2*>(ef);
   int cus = 256;
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device);
-  p->num_wg = 4 * cus;  // node workgroups in flight: four per CU (LDS and registers allow it)
+  p->num_wg = 4 * cus;
   p->slots = 8 * cus;   // capsules per batch: two full rounds of them
   auto alloc = [&](auto** d, size_t bytes) {
     void* q = nullptr;
@@ -1512,6 +1513,19 @@ int memb_plan_create(memb_plan** out, int L, int device) {
       !big((const void*)k_nodes<false, false>, lds_nodes(T, false)) ||
       !big((const void*)k_filter, lds_filter(T)))
     return bail(fail(p, MEMB_E_HIP, "hipFuncSetAttribute failed"));
+  // four per CU by the registers, three by the LDS from degree 19 on (without bending 22): cut for
+  // four all the same, the runs of some hundred capsules made a thin second round (301 capsules of
+  // degree 23: 425 us with bending and 278 without, 376 and 254 cut for three).  Low degrees without
+  // bending have room for more, which is not always better: 301 capsules of degree 16 take
+  // 109 us cut for four and 113 for five.
+  for (int bend = 0; bend < 2; ++bend) {
+    int per_cu = 0;
+    const void* f = bend ? (const void*)k_nodes<false, true> : (const void*)k_nodes<false, false>;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, ND_THREADS,
+                                                     lds_nodes(T, bend)) != hipSuccess)
+      return bail(fail(p, MEMB_E_HIP, "occupancy of the node kernel failed"));
+    p->nodes_wg[bend] = std::min(4, std::max(1, per_cu)) * cus;
+  }
   T.ref = nullptr;
   Work wk{};
   wk.n = 1, wk.coef = p->coef, wk.rows = p->rows;
