@@ -61,7 +61,7 @@ struct GemmArgs {
   const float* omean;    // EPI_OUT, EPI_LOSS
   const float* oscale;
   const float* wt;       // EPI_LOSS: per-output weights or null
-  float* part;           // EPI_LOSS: one partial sum per workgroup
+  float* part;           // EPI_LOSS: one partial sum per workgroup, or null
   int batch, dout;       // EPI_OUT, EPI_LOSS: the unpadded extents
 };
 
@@ -241,7 +241,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& q, int m0, int n0) {
     for (int s = 32; s > 0; s >>= 1) loss += __shfl_down(loss, s);
     if (lane == 0) red[wv] = loss;
     __syncthreads();
-    if (tid == 0) q.part[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
+    if (tid == 0 && q.part) q.part[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
   }
 }
 
@@ -400,8 +400,11 @@ struct memb_mlp {
   std::vector<float*> Z;           // hidden pre-activations [Mp][Wp]
   std::vector<__bf16*> H;          // hidden activations [Mp][Wp]
   std::vector<__bf16*> dZ;         // per layer, gradient of the pre-activation [Mp][out_p]
-  float* hpart = nullptr;          // loss partials, one per workgroup of the last layer, in
-  float* part = nullptr;           // pinned host memory; its device address
+  // loss partials, one per workgroup of the last layer, in pinned host memory, and its device
+  // address: allocated by the first call that asks for the loss (an allocation and its release take
+  // 0.5 ms, which a network that only infers need not pay; such a call waits, so it is not captured)
+  float* hpart = nullptr;
+  float* part = nullptr;
   size_t npart = 0;
   float *mean = nullptr, *scale = nullptr;    // input normalisation [Dp]
   float *omean = nullptr, *oscale = nullptr;  // output de-normalisation [Op]
@@ -476,16 +479,21 @@ GemmArgs last_layer(const memb_mlp* m, int batch) {
   return q;
 }
 
-// Forward, loss and every gradient, enqueued; the nloss loss partials are in hpart once the
-// stream has come this far.
+// Forward, loss and every gradient, enqueued; with want_loss the nloss loss partials are in hpart
+// once the stream has come this far.
 int backward(memb_mlp* m, int batch, const float* x, const float* t, const float* wt,
-             size_t& nloss) {
+             bool want_loss, size_t& nloss) {
+  if (want_loss && !m->hpart) {
+    const size_t parts = (size_t)(m->Mp / 32) * (m->Op / 32);  // the smallest tile's workgroups
+    XCHK(m, hipHostMalloc((void**)&m->hpart, parts * sizeof(float), hipHostMallocMapped));
+    XCHK(m, hipHostGetDevicePointer((void**)&m->part, m->hpart, 0));
+  }
   int rc = forward_hidden(m, batch, x, true);
   if (rc) return rc;
   const int Mp = pad128(batch), last = m->nl - 1;
   {
     GemmArgs q = last_layer(m, batch);
-    q.aux = t, q.wt = wt, q.out1 = m->dZ[last], q.part = m->part;
+    q.aux = t, q.wt = wt, q.out1 = m->dZ[last], q.part = want_loss ? m->part : nullptr;
     if ((rc = gemm<false, true, EPI_LOSS>(m, Mp, m->out_p[last], q))) return rc;
     nloss = m->npart;
   }
@@ -573,9 +581,6 @@ int memb_mlp_create(memb_mlp** out, int din, int width, int nhidden, int dout, i
     if ((rc = dalloc(m, &d, (size_t)m->Mp * m->out_p[i]))) return rc;
     m->dZ.push_back(d);
   }
-  const size_t parts = (size_t)(m->Mp / 32) * (m->Op / 32);  // the smallest tile's workgroups
-  XCHK(m, hipHostMalloc((void**)&m->hpart, parts * sizeof(float), hipHostMallocMapped));
-  XCHK(m, hipHostGetDevicePointer((void**)&m->part, m->hpart, 0));
   if ((rc = dalloc(m, &m->X, (size_t)m->Mp * m->Dp)) ||
       (rc = dalloc(m, &m->mean, (size_t)m->Dp)) || (rc = dalloc(m, &m->scale, (size_t)m->Dp)) ||
       (rc = dalloc(m, &m->omean, (size_t)m->Op)) || (rc = dalloc(m, &m->oscale, (size_t)m->Op)))
@@ -698,7 +703,7 @@ int memb_mlp_grad_only(memb_mlp* m, int batch, const float* x, const float* t, c
   if (!m || batch <= 0 || batch > m->maxb || !x || !t) return MEMB_E_ARG;
   XCHK(m, hipSetDevice(m->device));
   size_t nloss = 0;
-  int rc = backward(m, batch, x, t, wt, nloss);
+  int rc = backward(m, batch, x, t, wt, loss != nullptr, nloss);
   if (rc || !loss) return rc;
   return read_loss(m, nloss, loss);
 }
@@ -708,7 +713,7 @@ int memb_mlp_train_step(memb_mlp* m, int batch, const float* x, const float* t, 
   if (!m || batch <= 0 || batch > m->maxb || !x || !t) return MEMB_E_ARG;
   XCHK(m, hipSetDevice(m->device));
   size_t nloss = 0;
-  int rc = backward(m, batch, x, t, wt, nloss);
+  int rc = backward(m, batch, x, t, wt, loss != nullptr, nloss);
   if (rc) return rc;
   ++m->step;
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
