@@ -46,7 +46,9 @@ typedef struct memb_plan memb_plan;
 
 /* Tables (Gauss grid, Legendre functions and their theta-derivatives up to 4th order, the
  * unit-sphere reference state on the 2x grid) for degree L (2 <= L <= 23) on HIP device
- * `device`.  Replaces capsule_init_cal_coeff (sph.f90:16-191). */
+ * `device`, and work arrays for 2048 capsules at a time on 256 compute units whatever the plan
+ * will see: 128 MB at degree 16, 256 MB at degree 23.  Replaces capsule_init_cal_coeff
+ * (sph.f90:16-191). */
 int memb_plan_create(memb_plan** out, int L, int device);
 void memb_plan_destroy(memb_plan* p);
 const char* memb_last_error(const memb_plan* p);

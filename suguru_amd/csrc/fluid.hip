@@ -117,9 +117,9 @@ __device__ void fft_stages(double2* s, int nl, int M, int logm, int logn,
 // Workgroup b runs on XCD b % 8 (round-robin dispatch).  With a grid of a multiple of 8
 // workgroups, the y transforms take logical block (b % 8) (grid / 8) + b / 8, so that each XCD
 // works through one contiguous eighth of the lines: neighbouring groups of y lines share their
-// 128-byte rows, and these are then fetched once, into one L2 (y transforms 941 -> 883 us
-// forward, 874 -> 739 us inverse at 1024 x 512 x 256).  The x lines are whole rows and keep
-// the dispatch order.
+// 128-byte rows, and these are then fetched once, into one L2 (k_y: a step at 1024 x 512 x 256
+// 15.79 -> 14.36 ms, 512 x 512 x 250 7.63 -> 6.93).  The x lines are whole rows and keep the dispatch
+// order.
 template <bool XMAJOR>
 __device__ __forceinline__ int xcd_logical_block() {
   const unsigned nb = gridDim.x;
@@ -744,9 +744,6 @@ __global__ void __launch_bounds__(256) k_ztab(int nkx, int nky, int ktot, int ne
   ztab[(long long)(ktot - 1) * st + t] = bb - a[ktot - 1] * d;
 }
 
-// One lane per (i, j) mode of the compact spectral array, the forward sweep's values stored
-// back into the array and read again by the back substitution (the path above 257 planes;
-// k_tri_seg below takes every smaller grid in one pass).
 // The systems of one launch: workgroup row blockIdx.y solves array p[y] with its coefficients.
 struct Systems {
   double* p[3];
@@ -755,6 +752,9 @@ struct Systems {
   const double* ztab[3];
 };
 
+// One lane per (i, j) mode of the compact spectral array, the forward sweep's values stored
+// back into the array and read again by the back substitution (the path above 257 planes;
+// k_tri_seg below takes every smaller grid in one pass).
 __global__ void __launch_bounds__(TRI_MODES)
     k_tri(Systems sys, int itot, int jtot, int ktot) {
   double* __restrict__ p = sys.p[blockIdx.y];
@@ -1716,8 +1716,9 @@ int fld_create(fld_ctx** out, const ibx_grid* gr, double rep, double dt, int dev
   c->ncomp = (long long)g.itot * g.jtot * g.ktot;
   c->logmx = ilog2(g.itot / 2), c->logmy = ilog2(g.jtot / 2);
   c->xlines = std::min(g.jtot, std::max(1, 2048 / g.itot));
-  // 8 columns per workgroup both ways (at 1024 x 512 x 256: forward 543 us against 604 with 4
-  // and 744 with 2; inverse 602 us against 674 with 16)
+  // columns per workgroup of the LDS y transforms (jtot of 4, or above 1024); 8 both ways was best
+  // when they took every length (512 rows: forward 543 us against 604 with 4 and 744 with 2;
+  // inverse 602 us against 674 with 16)
   auto lines = [&](int want) {
     int nl = std::min(g.itot, want);
     while (nl > 1 && (size_t)nl * (g.jtot / 2 + 1) * sizeof(double2) > LDS_MAX / 2) nl >>= 1;

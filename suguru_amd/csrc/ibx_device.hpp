@@ -908,8 +908,9 @@ __global__ void __launch_bounds__(SP_THREADS)
 // included).  Cells outside every item box are zeroed by the same persistent launch (zero
 // units interleaved with the items), which finds them in a bitmap of the covered cells.
 // Steps: k_obj_clear (bitmap, counters); k_obj_boxes (object boxes, items per capsule);
-// k_obj_scan (item offsets); k_obj_items (items, bitmap, neighbouring capsules);
-// k_obj_sources (source lists); k_obj_spread (items and zero units); k_jhalo.
+// k_obj_scan (item offsets); k_obj_items (items, bitmap, neighbouring capsules); k_obj_sources
+// (source lists; up to OB_FUSE capsules k_obj_items does these two's work too); k_obj_spread
+// (items and zero units); k_jhalo.
 // ---------------------------------------------------------------------------------------
 constexpr int OB_THREADS = 256;
 constexpr int OB_CPT = OB_NC / OB_THREADS;  // cells per thread
@@ -1200,40 +1201,56 @@ __global__ void __launch_bounds__(256) k_obj_items(GridD g, long long ncap, int 
                                                    int* __restrict__ err) {
   if (offsets_bad(err)) return;
   __shared__ int B[9][6];
-  __shared__ int first, tot[OB_LIMITS];
+  __shared__ int first;
   const int tid = threadIdx.x;
   const long long p = blockIdx.x;
   if (tid < 54) B[tid / 6][tid % 6] = boxes[p * 54 + tid];
   if (FUSE && tid == 0) first = 0;
-  if (FUSE && tid < OB_LIMITS) tot[tid] = 0;
-  // with `small` a capsule per thread
-  const bool mine = FUSE && small && tid < ncap;
-  const int c0 = mine ? cnt[tid] : 0;
-  const unsigned long long cs = mine ? small[tid] : 0ull;
-  __syncthreads();
-  int at, e = 0;
-  if (FUSE) {
-    const auto add = [&](int v, int* to) {  // the workgroup's sum
+  // with `small` every wavefront adds up all counts, of all capsules and of those before its own
+  int tot[OB_LIMITS] = {}, before[OB_LIMITS] = {};
+  if (FUSE && small) {
 #pragma unroll
-      for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o);
-      if ((tid & 63) == 0 && v) atomicAdd(to, v);
-    };
-    int v = 0;
-    if (small) {
-      add(c0, &tot[0]);
+    for (int i = 0; i < OB_SMALL / 64; ++i) {
+      const int q = (tid & 63) + 64 * i;
+      if (q >= ncap) break;
+      const unsigned long long cs = small[q];
 #pragma unroll
-      for (int l = 1; l < OB_LIMITS; ++l) add(obj_unpack(cs, l), &tot[l]);
-      __syncthreads();
-      e = obj_choice(tot, icap);
-      v = tid < p ? (e ? obj_unpack(cs, e) : c0) : 0;
-    } else {
-      for (long long q = tid; q < p; q += 256) v += cnt[q];
+      for (int l = 0; l < OB_LIMITS; ++l) {
+        const int v = l ? obj_unpack(cs, l) : cnt[q];
+        tot[l] += v;
+        before[l] += q < p ? v : 0;
+      }
     }
-    add(v, &first);
+  }
+  __syncthreads();
+  int at = 0, e = 0;
+  if (FUSE && small) {
+#pragma unroll
+    for (int l = 0; l < OB_LIMITS; ++l)
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) {
+        tot[l] += __shfl_xor(tot[l], o);
+        before[l] += __shfl_xor(before[l], o);
+      }
+    e = obj_choice(tot, icap);
+    int n = 0;
+#pragma unroll
+    for (int l = 0; l < OB_LIMITS; ++l)
+      if (l == e) at = before[l], n = tot[l];
+    if (tid == 0 && p == ncap - 1) {
+      meta[0] = n;
+      if (n > icap) atomicOr(err, ERR_CAPACITY);
+    }
+  } else if (FUSE) {
+    int v = 0;
+    for (long long q = tid; q < p; q += 256) v += cnt[q];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o);
+    if ((tid & 63) == 0 && v) atomicAdd(&first, v);
     __syncthreads();
     at = first;
     if (tid == 0 && p == ncap - 1) {
-      meta[0] = small ? tot[e] : at + cnt[p];
+      meta[0] = at + cnt[p];
       if (meta[0] > icap) atomicOr(err, ERR_CAPACITY);
     }
   } else {

@@ -381,7 +381,7 @@ __device__ __forceinline__ void law(const Geom& o, const double* __restrict__ R,
 // through the transforms.  Apart, the node phase spreads a few capsules over the chip (8
 // capsules: 55 us in all) and holds 220 registers, none spilled; the transforms run 16 wavefronts
 // a CU on tables read coalesced.  8000 capsules of degree 16: 4.74 -> 2.8 ms (shape 0.25, nodes
-// 2.14, filter 0.39); 301 of degree 23 without bending: 1053 -> 275 us.
+// 2.14, filter 0.39); 301 of degree 23 without bending: 1053 -> 252 us.
 // Capsules: slot q holds capsule list[q], q < *cnt (list null: capsule c0 + q, q < n).
 struct Work {
   int n;              // slots (list null), or the most there can be
@@ -583,10 +583,10 @@ __global__ void __launch_bounds__(SH_THREADS)
 // half as much, and the DFT of the quads' sums and differences runs over N + 1 instead of 2 N
 // points: 3250 -> 2340 vector instructions a node with the reference's products taken from the
 // table.  8000 capsules of degree 16: 2.40 -> 2.14 ms; 301 of degree 23 without bending
-// 316 -> 275 us in all.  What is left waits half its time at two wavefronts per SIMD (the vector
-// units are busy 63 %, LDS 29 %), in no one place: without the coefficients' sums, the DFT, the
-// reference loads or the rest of the law it takes 0.34, 0.24, 0.26, 0.08 ms less; reading the
-// tables ten at a time in the sums changes nothing.
+// 316 -> 275 us in all, 252 with the runs cut for the workgroups that fit.  What is left waits half
+// its time at two wavefronts per SIMD (the vector units are busy 63 %, LDS 29 %), in no one place:
+// without the coefficients' sums, the DFT, the reference loads or the rest of the law it takes
+// 0.34, 0.24, 0.26, 0.08 ms less; reading the tables ten at a time in the sums changes nothing.
 // Registers: two wavefronts per SIMD.
 template <bool REF, bool BEND>
 __global__ void __launch_bounds__(ND_THREADS, 2)
@@ -1483,7 +1483,9 @@ int memb_plan_create(memb_plan** out, int L, int device) {
   int cus = 256;
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device);
   p->num_wg = 4 * cus;
-  p->slots = 8 * cus;   // capsules per batch: two full rounds of them
+  // capsules per batch; half as many would halve the plan's 128 MB (degree 16), but 8000 capsules
+  // then take 2866 us instead of 2811, a ragged end more often
+  p->slots = 8 * cus;
   auto alloc = [&](auto** d, size_t bytes) {
     void* q = nullptr;
     if (hipMalloc(&q, bytes) != hipSuccess) return false;

@@ -56,7 +56,8 @@ constexpr long long obj_item_capacity(long long ncap) {
 // largest are taken whether they fit or not, and their overflow reported.)
 constexpr int obj_choice(const int* tot, int icap) {
   int e = tot[0] <= 48 ? 3 : tot[0] <= 200 ? 2 : tot[0] <= 500 ? 1 : 0;
-  while (e > 0 && tot[e] > icap) --e;
+  for (int l = OB_LIMITS - 1; l > 0; --l)  // (constant indices: tot may be registers)
+    if (e == l && tot[l] > icap) e = l - 1;
   return e;
 }
 
